@@ -74,8 +74,8 @@ EXPORTS = [
 
 
 # one object per translation unit; compiled side by side, then linked
-SOURCES = ["capi_gemm.hip", "capi_harness.hip", "capi_api_gemm.hip"]
-ASM_MFMA_SOURCES = ["capi_gemm.hip"]
+ASM_MFMA_SOURCES = ["gemm_f16.hip", "gemm_bf16.hip", "gemm_bf16x3.hip"]
+SOURCES = ["capi_gemm.hip", "capi_harness.hip", "capi_api_gemm.hip"] + ASM_MFMA_SOURCES
 
 
 def device_asm_path(name):

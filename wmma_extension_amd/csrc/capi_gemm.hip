@@ -1,794 +1,28 @@
 // extern "C" boundary of libwmmae_tcec.so, GEMM driver part: argument
-// validation, kernel selection and launches of the split pass, the packed
-// GEMM and the single-kernel GEMM.  Declarations and per-entry documentation
+// validation and path selection; the kernels live in the gemm_*.hip
+// translation units, one per policy.  Declarations and per-entry documentation
 // live in include/wmmae_tcec.h.
-#include "capi_common.hpp"
-#include <limits>
-#include "tcec_gemm_fused_kernel.hpp"
-#include "tcec_gemm_kernels.hpp"
+#include "gemm_plan.hpp"
 
 namespace {
-using namespace wmmae_capi;
-using wmmae_gemm::u32x4;
+using namespace wmmae_driver;
 
-// ------------------------------------------------------------ policy table
-struct PolicyInfo {
-  int terms;       // stored terms per operand
-  bool bf16;       // MFMA element type
-  float inv_scale; // factor applied to the error accumulator
-};
-inline bool policy_info(const int policy, PolicyInfo &p) {
-  switch (policy) {
-  case WMMAE_POLICY_F16_EC:
-    p = {2, false, 1.f / 2048.f};
-    return true;
-  case WMMAE_POLICY_F16_NOEC:
-    p = {1, false, 1.f};
-    return true;
-  case WMMAE_POLICY_BF16X3_EC:
-    p = {3, true, 1.f};
-    return true;
-  case WMMAE_POLICY_BF16X2_EC:
-    p = {2, true, 1.f};
-    return true;
-  case WMMAE_POLICY_BF16_NOEC:
-    p = {1, true, 1.f};
-    return true;
-  default:
-    return false;
-  }
-}
-
-// packed operand geometry: 16-row blocks, 32-wide k chunks
-inline long long packed_row_blocks(const int rows) { return ceil_div(rows, 16); }
-inline int packed_k_tiles(const int k) {
-  return static_cast<int>(ceil_div(k, 32));
-}
-// u32x4 elements of one packed matrix
-inline long long packed_elems(const int rows, const int k, const int terms) {
-  return packed_row_blocks(rows) * packed_k_tiles(k) * terms * 64;
-}
-
-// ------------------------------------------------------------------ pack
-// One operand of a split launch as the caller describes it.
-struct PackSource {
-  int rows;
-  const float *X;
-  const float *const *ptrs;
-  long long row_stride, k_stride, batch_stride;
-  void *packed;
-};
-
-inline wmmae_gemm::PackOperand pack_operand(const PackSource &src,
-                                            const int KT) {
-  wmmae_gemm::PackOperand o;
-  o.X = src.X;
-  o.ptrs = src.ptrs;
-  o.row_stride = src.row_stride;
-  o.k_stride = src.k_stride;
-  o.batch_stride = src.batch_stride;
-  o.rows = src.rows;
-  o.chunks = packed_row_blocks(src.rows) * KT;
-  o.out = static_cast<u32x4 *>(src.packed);
-  return o;
-}
-
-// The batch index of the split, scale and fold kernels is the grid's y
-// coordinate, which ends at 65535: longer batches take one launch per 65535
-// entries.
-constexpr int kMaxGridY = 65535;
-
-// Splits one operand (b == nullptr) or both operands of a product in a single
-// launch.
-template <class T, int TERMS>
-int launch_pack(const int k, const int batch, const PackSource &a,
-                const PackSource *const b, hipStream_t stream) {
-  const int KT = packed_k_tiles(k);
-  const wmmae_gemm::PackOperand oa = pack_operand(a, KT);
-  const long long blocks_a = ceil_div(oa.chunks * 64, 256);
-  if (b == nullptr) {
-    if (blocks_a > 0x7fffffffLL)
-      return WMMAE_STATUS_NOT_SUPPORTED;
-    for (int e0 = 0; e0 < batch; e0 += kMaxGridY)
-      hipLaunchKernelGGL((wmmae_gemm::split_pack_kernel<T, TERMS>),
-                         dim3(static_cast<unsigned>(blocks_a),
-                              std::min(batch - e0, kMaxGridY)),
-                         dim3(256), 0, stream, oa, k, KT,
-                         static_cast<unsigned>(e0));
-    return launch_status();
-  }
-  const wmmae_gemm::PackOperand ob = pack_operand(*b, KT);
-  const long long blocks_b = ceil_div(ob.chunks * 64, 256);
-  if (blocks_a + blocks_b > 0x7fffffffLL)
-    return WMMAE_STATUS_NOT_SUPPORTED;
-  for (int e0 = 0; e0 < batch; e0 += kMaxGridY)
-    hipLaunchKernelGGL((wmmae_gemm::split_pack_pair_kernel<T, TERMS>),
-                       dim3(static_cast<unsigned>(blocks_a + blocks_b),
-                            std::min(batch - e0, kMaxGridY)),
-                       dim3(256), 0, stream, oa, ob,
-                       static_cast<unsigned>(blocks_a), k, KT,
-                       static_cast<unsigned>(e0));
-  return launch_status();
-}
-
-int pack_dispatch(const int policy, const int k, const int batch,
-                  const PackSource &a, const PackSource *const b,
-                  hipStream_t stream) {
-  switch (policy) {
-  case WMMAE_POLICY_F16_EC:
-    return launch_pack<w::half, 2>(k, batch, a, b, stream);
-  case WMMAE_POLICY_F16_NOEC:
-    return launch_pack<w::half, 1>(k, batch, a, b, stream);
-  case WMMAE_POLICY_BF16X3_EC:
-    return launch_pack<w::precision::tf32, 3>(k, batch, a, b, stream);
-  case WMMAE_POLICY_BF16X2_EC:
-    return launch_pack<w::bfloat16, 2>(k, batch, a, b, stream);
-  case WMMAE_POLICY_BF16_NOEC:
-    return launch_pack<w::bfloat16, 1>(k, batch, a, b, stream);
-  default:
-    return WMMAE_STATUS_INVALID_VALUE;
-  }
-}
-
-// ------------------------------------------------------------------ gemm
-struct GemmArgs {
-  const u32x4 *a, *b;
-  float *c;
-  int m, n, k;
-  long long ldc, stride_c;
-  float alpha, beta, inv_scale;
-  int batch, terms;
-  float *const *c_ptrs; // device array of C pointers, or nullptr
-  float *partial;  // split-K slices, or nullptr
-  int splits;      // >= 1
-  // room for the K slices of the tiles of a partly empty last round (used
-  // only without split-K), or nullptr
-  float *tail_ws;
-  size_t tail_ws_bytes;
-  hipStream_t stream;
-  // fp32 operands for the kernel variant that splits them itself (a and b are
-  // null then)
-  bool is_direct = false;
-  wmmae_gemm::DirectSource direct = {};
-};
-
-// Compute units of the current device, looked up once per device.
-inline int device_cus() {
-  static std::atomic<int> cached[64];
-  int dev = 0;
-  if (hipGetDevice(&dev) != hipSuccess)
-    return 256; // MI355X; also the answer when no device is visible
-  const bool tracked = dev >= 0 && dev < 64;
-  if (tracked) {
-    const int c = cached[dev].load(std::memory_order_relaxed);
-    if (c > 0)
-      return c;
-  }
-  hipDeviceProp_t prop;
-  if (hipGetDeviceProperties(&prop, dev) != hipSuccess ||
-      prop.multiProcessorCount <= 0)
-    return 256;
-  if (tracked)
-    cached[dev].store(prop.multiProcessorCount, std::memory_order_relaxed);
-  return prop.multiProcessorCount;
-}
-
-// ------------------------------------------------ fitted cost parameters
-// Every number the path and tile choices below are made with, in one place.
-// All are fits to measurements on MI355X (256 compute units, one box of the
-// pool each; the boxes differ by 3 to 5 % in what they sustain under the power
-// limit).  The estimates have one form: launch cost + rounds of tiles over the
-// compute units x (k stages of 32 x time per stage + time per tile), bounded
-// below by the bytes moved.
-namespace fit {
-// -- packed GEMM, time of one k stage of one tile, by stored terms (1, 2, 3).
-//    Sweep: 216 products, m = n = 512 .. 2048, k = 512 .. 4096, each run with
-//    1, 2, 3, 4, 6 and 8 K slices; the slice count chosen with them is within
-//    0.7 % of the best measured one on average (1.9 % on 120 random products
-//    with m, n = 64 .. 2900, k = 400 .. 32000, 1 .. 100 entries, 1 .. 32
-//    slices forced).
-constexpr double kStage256x128[3] = {0.8e-6, 1.0e-6, 1.82e-6};
-constexpr double kStage128x128[3] = {0.45e-6, 0.6e-6, 0.99e-6};
-constexpr double kStage64x64 = 0.25e-6;
-constexpr double kTileOverhead = 7e-6;    // pipeline fill + epilogue of a tile
-constexpr double kFoldLaunch = 6e-6;      // the pass that adds the K slices
-constexpr double kFoldBytesPerS = 3e12;   // ... reads and writes its planes at
-constexpr double kSplitMustBeat = 0.95;   // a split has to win by 5 %
-// -- tile choice, cost of a tile in units of one 128x128 tile.  Sweep: both
-//    tiles forced on 124 products, 1024^2 .. 8192^2, k = 256 .. 4096, some
-//    batched: the choice is within 0.4 % of the faster tile on average.
-constexpr double kUnits256x128 = 2.0;
-constexpr double kUnits128x128 = 1.2;     // one and two terms
-//    Three terms (sweep: both tiles forced on 36 products, 1024^2 .. 8192^2,
-//    k = 1024 .. 5000, some batched or rectangular: a round of 256x128 tiles
-//    costs 1.8 rounds of 128x128 tiles, so the large tile wins when it halves
-//    the rounds, 8 to 14 %, and loses otherwise, 3 % at 7 -> 4 rounds, 17 to
-//    20 % at 3 -> 2).
-constexpr double kUnits256x128Terms3 = 1.8;
-constexpr double kUnits128x128Terms3 = 1.0;
-constexpr double kUnits64x64 = 0.4;
-constexpr double units256x128(const int terms) {
-  return terms == 3 ? kUnits256x128Terms3 : kUnits256x128;
-}
-constexpr double units128x128(const int terms) {
-  return terms == 3 ? kUnits128x128Terms3 : kUnits128x128;
-}
-// -- K slices for a partly empty last round: slices, pipeline refills, fold.
-//    Sweep: 126 products, 2304^2 .. 8192^2, k = 2048 .. 8192, two policies.
-constexpr double kTailOverhead = 0.2;
-// -- which path: the single kernel, split passes + GEMM on packed operands, or
-//    the GEMM kernel that splits the fp32 operands itself.  Fit: 1860 random
-//    products (m, n = 45 .. 5000, k = 32 .. 32768, 1 .. 1024 entries, half of
-//    them with dimensions that are multiples of nothing, all five policies),
-//    each run with every path forced; the constants below minimise the
-//    squared log error of each path's estimate on 1060 of them and on 137
-//    structured products (the reference harness's grid with 256 entries,
-//    squares 1024 .. 8192, the baseline workloads; weighted four times).  On
-//    the 800 held out the path chosen with them is 1.4 % slower than always
-//    taking the fastest forced path on average (37 of 800 above 1.10 x, six
-//    above 1.25 x), on the structured ones 0.5 % (two above 1.10 x); the
-//    constants before (fits to the harness's grid and to square products)
-//    were 3 to 6 % slower on the same 800, 3.1 x at worst.  Whole default
-//    calls on 400 further random products: 1.1 % (worst 1.48 x).
-//    Rows: one, two, three terms.
-struct PathRates {
-  double launch, stage, tile, bytes_per_s; // seconds, seconds, seconds, B/s
-  double split_bytes_per_s;                // packed path only
-  // A k stage takes longer the fuller the chip is (power limit, contention in
-  // L2 and HBM): stage * (1 + busy * (compute units with a tile / all compute
-  // units, averaged over the rounds))
-  double busy;
-};
-constexpr PathRates kFused[3] = {
-    {6.01e-6, 0.643e-6, 2.88e-6, 5.32e12, 0., 0.101},
-    {6.50e-6, 0.992e-6, 1.85e-6, 5.27e12, 0., 0.170},
-    {5.37e-6, 1.39e-6, 2.22e-6, 5.14e12, 0., 0.141}};
-constexpr PathRates kPacked[3] = {
-    {8.35e-6, 0.131e-6, 3.07e-6, 3.65e12, 5.61e12, 0.359},
-    {8.17e-6, 0.287e-6, 3.69e-6, 6.50e12, 5.57e12, 0.649},
-    {7.10e-6, 0.652e-6, 4.65e-6, 6.50e12, 4.92e12, 0.361}};
-// -- the packed path's GEMM kernel reading and splitting the fp32 operands
-//    itself (256x128 tiles only; rows: one, two terms)
-constexpr PathRates kDirect[2] = {
-    {3.41e-6, 0.173e-6, 3.76e-6, 4.62e12, 0., 1.18},
-    {5.00e-6, 0.355e-6, 3.65e-6, 4.92e12, 0., 0.750}};
-// ... as the host sees it when it decides whether a launch of that kernel is
-// bound by its bytes and should start its workgroups staggered (a fit of its
-// own, to the reference harness's grid: 0.8 / 1.5 us per k stage of a 256x128
-// tile and 6 us per tile, in units of half a tile)
-constexpr PathRates kDirectStagger[2] = {
-    {6.0e-6, 0.40e-6, 3.0e-6, 5.0e12, 0., 0.},
-    {6.0e-6, 0.75e-6, 3.0e-6, 5.0e12, 0., 0.}};
-// with K slices: the GEMM's time against the packed kernel's estimate for the
-// same slices of 256x128 tiles (two terms: twelve K-sliced products, m, n =
-// 64 .. 4096, k = 2048 .. 262144, each run on either path: with 1.4 the faster
-// path is chosen for all of them, with 1.5 for eleven)
-constexpr double kDirectSliceRatio[2] = {1.5, 1.4};
-// Products that are cut into K slices (few output tiles): what the slice
-// planner's time (split_time, whose constants are fitted for choosing the slice
-// count) has to be scaled and shifted by to be the time of the whole call on
-// each path; same fit as above.  Rows: scale, shift in seconds; by terms.
-constexpr double kSlicedFused[2][3] = {{1.16, 1.08, 1.03},
-                                       {-3.73e-6, -2.84e-6, -2.89e-6}};
-constexpr double kSlicedPacked[2][3] = {{0.724, 0.954, 0.955},
-                                        {-0.65e-6, -6.0e-6, -6.0e-6}};
-constexpr double kSlicedDirect[2][2] = {{0.759, 0.890}, {-6.0e-6, -6.0e-6}};
-// Calls issued back to back cannot complete faster than the host issues their
-// launches (250 products below 1.5e8 flop, called in a loop: 11, 14.5 and 12 us
-// per call in the median): what decides among the paths for tiny products -
-// one launch for the single kernel and the direct kernel, two or three for
-// the packed path.  Order: single kernel, packed, direct.
-constexpr double kCallFloor[3] = {11.0e-6, 14.3e-6, 11.5e-6};
-// k % 32 != 0: the kernel variant that reads a shorter last stage (1024^2 x 1000
-// against x 1024, batch 256: 301 against 336 TFLOPS, of which 2.4 % are the k)
-constexpr double kDirectTailStage = 1.47;
-// the single kernel's 64x64 tile against its 128x128 tile (1024^3: 41 -> 27 us)
-constexpr double kFusedSmallTileTime = 0.65; // whole tile, latency-bound sizes
-constexpr double kFusedSmallStage = 0.599, kFusedSmallTile = 0.467;
-// 4-byte instead of 16-byte requests: 114 random products with k % 4 != 0 ran
-// at 0.55 of the packed path's speed in the median
-constexpr double kFusedNarrowRequests = 3.50;
-} // namespace fit
-
-// XCDs (chiplets with an L2 of their own) behind the current device.  HIP does
-// not report them; a gfx950 XCD has 32 active compute units in every partition
-// mode (SPX 256 = 8 x 32, DPX 128, QPX 64, CPX 32), so the count follows from
-// the compute units.  Consecutive workgroup ids go round-robin over the XCDs;
-// the kernels' XCD-aware item lists are written for eight of them and are used
-// only then (other counts take the plain shared list: same results, tiles not
-// grouped by L2).
-inline int device_xcds() {
-  const int cus = device_cus();
-  return cus % 32 == 0 ? cus / 32 : 1;
-}
-constexpr int kKernelXcds = 8; // the constant XCDS of the kernels' item lists
-
-// Number of K slices of every tile, when the 256x128 output tiles cannot fill
-// half the chip.  For every candidate (at most 32 slices of at least 6 stages)
-// the GEMM's time is estimated the way gemm_by_size will run it: the tile that
-// the slice count leads to, rounds of those tiles over the compute units,
-// stages per slice at that tile's time per stage, a fixed time per tile, and
-// for more than one slice the fold (a launch plus the planes written and
-// read).  The cheapest count is taken, any split having to beat the uncut run
-// by 5 %.  Times per stage and tile: fits to measurements on MI355X (216
-// products, m = n = 512 .. 2048, k = 512 .. 4096, one to three terms, each run
-// with 1, 2, 3, 4, 6 and 8 slices: the choice is within 0.7 % of the best measured count on
-// average; "as many slices as fill the chip with 256x128 tiles" was 7 % off,
-// over-cutting outputs from 1280^2 up and not cutting short loops at all).
-// Whether the 256x128 tile is a candidate at all: only where the 128x128 tiles
-// need more than one round over the compute units (in a single round the
-// smaller tile always finishes first), and not for the one-term kernels on
-// loops of 32 stages or fewer, where the stores of C dominate and the smaller
-// tile measured 8 to 12 % faster.  (Forced-tile runs of 124 products: the
-// choice below is within 0.4 % of the faster tile on average; requiring a full
-// round of 256x128 tiles instead had cost 2 %, up to 13 % at 2560^2 .. 2816^2.)
-inline bool big_tile_candidate(const int terms, const long long mid,
-                               const int kt) {
-  return mid > device_cus() && !(terms == 1 && kt <= 32);
-}
-// `direct`: the kernel that splits the fp32 operands itself, which has the
-// 256x128 tile only and takes kDirectSliceRatio times the packed kernel's time
-// (its slice count must be planned with its own tiles: 4096 x 64 x 4096 cut
-// for the 128x128 tiles of the packed path left half the compute units
-// without a 256x128 item, 48 against 39 us).
-inline double split_time(const int terms, const int m, const int n,
-                         const int batch, const int kt, const int slices,
-                         const bool direct = false) {
-  const long long cus = device_cus();
-  const int stages = static_cast<int>(ceil_div(kt, slices));
-  const long long z = ceil_div(kt, stages);
-  const long long big = ceil_div(m, 256) * ceil_div(n, 128) * batch * z;
-  const long long mid = ceil_div(m, 128) * ceil_div(n, 128) * batch * z;
-  double stage_time, rounds;
-  const double r_big = static_cast<double>(ceil_div(big, cus));
-  const double r_mid = static_cast<double>(ceil_div(mid, cus));
-  if (direct ||
-      (big_tile_candidate(terms, mid, stages) &&
-       r_big * fit::units256x128(terms) <= r_mid * fit::units128x128(terms))) {
-    stage_time = fit::kStage256x128[terms - 1];
-    rounds = r_big;
-  } else if (mid >= cus || (m > 64 && n > 64)) {
-    stage_time = fit::kStage128x128[terms - 1];
-    rounds = r_mid;
-  } else {
-    stage_time = fit::kStage64x64;
-    rounds = static_cast<double>(
-        ceil_div(ceil_div(m, 64) * ceil_div(n, 64) * batch * z, cus));
-  }
-  double t = rounds * (stages * stage_time + fit::kTileOverhead);
-  if (z > 1)
-    t += fit::kFoldLaunch + static_cast<double>(z + 1) * m * n * batch * 4.0 /
-                                fit::kFoldBytesPerS;
-  return direct ? t * fit::kDirectSliceRatio[terms - 1] : t;
-}
-// Test hook (wmmae_tcec_force_k_slices): a slice count for the calling thread's
-// next calls instead of the estimates' choice, so that two kernels can be run on
-// the same cut of K and compared bit by bit.  0: the estimates choose.
-thread_local int t_forced_k_slices = 0;
-// Measurement hook (wmmae_tcec_time_gemm_kernel): events this thread's calls
-// record on their stream right before the MFMA GEMM kernel and right after it
-// (after the fold of its K slices where there is one).
-thread_local hipEvent_t t_gemm_begin = nullptr, t_gemm_end = nullptr;
-constexpr int kMaxSplits = 32, kMinStagesPerSplit = 6;
-inline int choose_splits(const int terms, const int m, const int n, const int k,
-                         const int batch, const bool direct = false) {
-  const long long tiles = ceil_div(m, 256) * ceil_div(n, 128) * batch;
-  const int kt = static_cast<int>(ceil_div(k, 32));
-  if (t_forced_k_slices > 0) {
-    const int s = std::max(
-        1, std::min({t_forced_k_slices, kMaxSplits, kt / kMinStagesPerSplit}));
-    return static_cast<int>(ceil_div(kt, ceil_div(kt, s)));
-  }
-  if (tiles * 2 > device_cus())
-    return 1;
-  int best = 1;
-  double t_best =
-      fit::kSplitMustBeat * split_time(terms, m, n, batch, kt, 1, direct);
-  for (int s = 2; s <= kMaxSplits && s * kMinStagesPerSplit <= kt; s++) {
-    if (ceil_div(kt, ceil_div(kt, s)) != s)
-      continue; // the same slices as a smaller count
-    const double t = split_time(terms, m, n, batch, kt, s, direct);
-    if (t < t_best) {
-      t_best = t;
-      best = s;
-    }
-  }
-  return best;
-}
-
-// K slices for the tiles of the last round only.  `tiles` output tiles run in
-// rounds of `resident` (one workgroup per item, long K loops); when the last
-// round is less than half full its tiles are cut into `slices` K slices of at
-// least 32 stages each, so that the round takes about 1/slices of a tile's
-// time (plus the pass that folds the slices).  slices == 1: not worth it.
-struct TailPlan {
-  long long full = 0, tail = 0; // tiles in whole rounds, tiles in the last
-  int slices = 1, stages = 0;   // K slices of a tail tile, stages per slice
-};
-inline TailPlan plan_tail(const long long tiles, const long long resident,
-                          const int KT) {
-  TailPlan t;
-  t.full = tiles / resident * resident;
-  t.tail = tiles - t.full;
-  if (t.full == 0 || t.tail == 0 || t.tail * 2 > resident || KT < 64)
-    return t;
-  long long s = std::min<long long>({resident / t.tail, KT / 32, 16});
-  if (s < 2)
-    return t;
-  t.stages = static_cast<int>(ceil_div(KT, s));
-  t.slices = static_cast<int>(ceil_div(KT, t.stages));
-  return t;
-}
-// Time of `tiles` tiles in units of one tile, with and without that plan.
-inline double rounds_cost(const long long tiles, const long long resident,
-                          const int KT, const bool tail_allowed) {
-  const TailPlan t = plan_tail(tiles, resident, KT);
-  const double full_rounds = static_cast<double>(t.full / resident);
-  if (t.tail == 0)
-    return full_rounds;
-  if (!tail_allowed || t.slices < 2)
-    return full_rounds + 1.0;
-  return full_rounds + 1.0 / t.slices + fit::kTailOverhead;
-}
-
-// Deepest LDS ring (at most 4 stages) that fits the 160 KiB of a compute unit.
-constexpr int ring_depth(const int bm, const int bn, const int terms) {
-  const int stage_bytes = (bm / 16 + bn / 16) * terms * 1024;
-  const int fit = (160 * 1024) / stage_bytes;
-  return fit > 4 ? 4 : fit;
-}
-
-// Workgroups of one GEMM kernel that a compute unit holds at a time: what the
-// runtime's occupancy query says (registers, LDS and wave slots together),
-// looked up once per kernel and device; the LDS bound alone where the query
-// gives nothing (no device visible).  The persistent work-item modes give
-// every resident workgroup a fixed share of the items, so a count the
-// registers do not allow would leave the extra workgroups' shares to run after
-// everything else (the one-term direct kernel: 48 KiB of LDS, three by that
-// bound, but 512 registers a lane).
-template <class MT, int TERMS, int BM, int BN, int WGM, int WGN, bool RN,
-          int DIRECT = 0>
-int workgroups_per_cu() {
-  constexpr int NSTAGE = DIRECT ? 2 : ring_depth(BM, BN, TERMS);
-  using Cfg =
-      wmmae_gemm::GemmConfig<MT, TERMS, BM, BN, WGM, WGN, NSTAGE, RN, DIRECT>;
-  constexpr int by_lds =
-      (160 * 1024) / Cfg::LDS_BYTES > 4 ? 4 : (160 * 1024) / Cfg::LDS_BYTES;
-  static std::atomic<int> cached[64];
-  static std::atomic<unsigned long long> lds_allowed{0};
-  int dev = 0;
-  if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) {
-    (void)hipGetLastError();
-    return by_lds;
-  }
-  const int c = cached[dev].load(std::memory_order_relaxed);
-  if (c > 0)
-    return c;
-  auto kernel = wmmae_gemm::tcec_gemm_kernel<MT, TERMS, BM, BN, WGM, WGN,
-                                             NSTAGE, RN, DIRECT>;
-  int n = 0;
-  if (allow_dynamic_lds(reinterpret_cast<const void *>(kernel), Cfg::LDS_BYTES,
-                        lds_allowed) != hipSuccess ||
-      hipOccupancyMaxActiveBlocksPerMultiprocessor(
-          &n, reinterpret_cast<const void *>(kernel), Cfg::NTHREADS,
-          Cfg::LDS_BYTES) != hipSuccess ||
-      n <= 0) {
-    (void)hipGetLastError();
-    return by_lds;
-  }
-  n = n < by_lds ? n : by_lds;
-  cached[dev].store(n, std::memory_order_relaxed);
-  return n;
-}
-
-template <class MT, int TERMS, int BM, int BN, int WGM, int WGN, bool RN,
-          int DIRECT = 0>
-int launch_gemm(const GemmArgs &g) {
-  constexpr int NSTAGE = DIRECT ? 2 : ring_depth(BM, BN, TERMS);
-  using Cfg =
-      wmmae_gemm::GemmConfig<MT, TERMS, BM, BN, WGM, WGN, NSTAGE, RN, DIRECT>;
-  auto kernel = wmmae_gemm::tcec_gemm_kernel<MT, TERMS, BM, BN, WGM, WGN,
-                                             NSTAGE, RN, DIRECT>;
-  static std::atomic<unsigned long long> lds_allowed{0};
-  WMMAE_HIP_TRY(allow_dynamic_lds(reinterpret_cast<const void *>(kernel),
-                                  Cfg::LDS_BYTES, lds_allowed));
-  const int tiles_m = static_cast<int>(ceil_div(g.m, BM));
-  const int tiles_n = static_cast<int>(ceil_div(g.n, BN));
-  const int KT = packed_k_tiles(g.k);
-  const int rb_a = static_cast<int>(packed_row_blocks(g.m));
-  const int rb_b = static_cast<int>(packed_row_blocks(g.n));
-  // 16-byte stores need ldc % 4 == 0 and an aligned base; the base of each
-  // batch entry is checked again inside the kernel
-  const int vec_store =
-      (g.ldc % 4 == 0) &&
-      (g.c_ptrs != nullptr || (reinterpret_cast<uintptr_t>(g.c) % 16 == 0 &&
-                               g.stride_c % 4 == 0));
-  const int splits = g.partial != nullptr ? g.splits : 1;
-  const int split_stages = static_cast<int>(ceil_div(KT, splits));
-  const int zdim = static_cast<int>(ceil_div(KT, split_stages));
-  const long long items =
-      static_cast<long long>(tiles_m) * tiles_n * g.batch * zdim;
-  if (items >= (1ll << 31)) // the kernel counts items in 32 bits
-    return WMMAE_STATUS_INVALID_VALUE;
-  // Who takes which item (the large tiles take most of a compute unit's LDS,
-  // so one workgroup per unit is resident):
-  //  * 8 or more batch entries: an XCD owns whole entries, so that an entry's
-  //    operands are read into one L2 only (batch 256 of 1024x1024x256:
-  //    196 -> 256 effective TFLOPS), persistent workgroups when there are
-  //    more items than resident workgroups;
-  // and with more items than resident workgroups otherwise
-  //  * short K loops: persistent workgroups walking one shared list, their
-  //    requests running ahead into the next item;
-  //  * long K loops (64 stages = 2048 of k or more per item) of few entries:
-  //    one workgroup per item, handed out by the hardware as compute units
-  //    become free, which evens out compute units of unequal speed over many
-  //    rounds (a fixed share per workgroup measured 7 % slower at 16384^3).
-  const int per_cu =
-      workgroups_per_cu<MT, TERMS, BM, BN, WGM, WGN, RN, DIRECT>();
-  const long long resident = static_cast<long long>(device_cus()) * per_cu;
-  int grid = static_cast<int>(std::min(items, resident));
-  int entry_per_xcd = 0;
-  const bool eight_xcds = device_xcds() == kKernelXcds;
-  if (zdim > 1 && eight_xcds && resident >= 8 && resident % 8 == 0) {
-    // split-K: eight runs of the item list, one per XCD, so that an XCD holds
-    // as few K slices as possible; the grid is padded to whole runs
-    entry_per_xcd = 2;
-    grid = static_cast<int>(std::min(8 * ceil_div(items, 8), resident));
-  }
-  unsigned tail_begin = 0xffffffffu; // no tail slices
-  TailPlan tail;
-  // (an XCD that owns one entry more than the others must not cost more
-  // rounds than the shared list would take: 9 entries of 128 tiles are 8
-  // rounds on the XCD with two entries, 5 on the shared list)
-  const bool by_xcd = eight_xcds && resident >= 8 && resident % 8 == 0;
-  const long long owned_rounds =
-      by_xcd ? ceil_div(static_cast<long long>(tiles_m) * tiles_n *
-                            ceil_div(g.batch, 8),
-                        resident / 8)
-             : 0;
-  if (zdim == 1 && g.batch >= 8 && by_xcd &&
-      owned_rounds * 100 <= ceil_div(items, resident) * 115) {
-    // also when every item gets a workgroup of its own: a workgroup for every
-    // item of the XCD that owns the most entries
-    entry_per_xcd = 1;
-    grid = static_cast<int>(std::min(
-        8ll * tiles_m * tiles_n * ceil_div(g.batch, 8), resident));
-  } else if (items > resident && entry_per_xcd == 0) {
-    if (split_stages >= 64) {
-      grid = static_cast<int>(items);
-      // one entry, no split-K, room for the slices: the tiles of a partly
-      // empty last round are cut along K
-      if (g.batch == 1 && zdim == 1 && g.c_ptrs == nullptr &&
-          g.tail_ws != nullptr) {
-        tail = plan_tail(items, resident, KT);
-        const size_t need =
-            static_cast<size_t>(tail.slices) * tail.tail * BM * BN * 4u;
-        if (tail.slices >= 2 && need <= g.tail_ws_bytes) {
-          tail_begin = static_cast<unsigned>(tail.full);
-          grid = static_cast<int>(tail.full + tail.tail * tail.slices);
-        } else {
-          tail.slices = 1;
-        }
-      }
-    }
-  }
-  if (t_gemm_begin != nullptr)
-    WMMAE_HIP_TRY(hipEventRecord(t_gemm_begin, g.stream));
-  hipLaunchKernelGGL(kernel, dim3(grid), dim3(Cfg::NTHREADS), Cfg::LDS_BYTES,
-                     g.stream, g.a, g.b,
-                     g.c, g.m, g.n, KT, rb_a, rb_b, g.ldc, g.alpha, g.beta,
-                     g.inv_scale, tiles_m, tiles_n, vec_store,
-                     static_cast<long long>(rb_a) * KT * TERMS * 64,
-                     static_cast<long long>(rb_b) * KT * TERMS * 64,
-                     g.stride_c, split_stages,
-                     zdim > 1 ? g.partial : static_cast<float *>(nullptr),
-                     g.c_ptrs, g.batch, zdim, entry_per_xcd, tail_begin,
-                     tail.stages, g.tail_ws, g.direct);
-  int st = launch_status();
-  if (st == WMMAE_STATUS_SUCCESS && tail_begin != 0xffffffffu) {
-    hipLaunchKernelGGL((wmmae_gemm::reduce_tail_kernel<BM, BN>),
-                       dim3(static_cast<unsigned>(tail.tail), BM * BN / 1024),
-                       dim3(256), 0, g.stream, g.tail_ws, tail.slices,
-                       tail_begin, static_cast<unsigned>(tiles_m * tiles_n),
-                       tiles_m, tiles_n, g.c, g.m, g.n, g.ldc, g.alpha, g.beta);
-    st = launch_status();
-  }
-  if (st == WMMAE_STATUS_SUCCESS && zdim > 1) {
-    // 16 bytes per access where every slice column and every column of C starts
-    // on a 16-byte boundary (entries of a pointer array: not known here)
-    const bool vec = g.m % 4 == 0 && g.ldc % 4 == 0 && g.c_ptrs == nullptr &&
-                     reinterpret_cast<uintptr_t>(g.c) % 16 == 0 &&
-                     g.stride_c % 4 == 0 &&
-                     reinterpret_cast<uintptr_t>(g.partial) % 16 == 0;
-    const long long blocks =
-        ceil_div(static_cast<long long>(g.m) * g.n, vec ? 1024 : 256);
-    for (int e0 = 0; e0 < g.batch; e0 += kMaxGridY) {
-      const dim3 grid(static_cast<unsigned>(blocks),
-                      std::min(g.batch - e0, kMaxGridY));
-      if (vec)
-        hipLaunchKernelGGL(wmmae_gemm::reduce_splits_kernel<4>, grid, dim3(256),
-                           0, g.stream, g.partial, zdim, g.c, g.m, g.n, g.ldc,
-                           g.stride_c, g.c_ptrs, g.alpha, g.beta,
-                           static_cast<long long>(g.batch),
-                           static_cast<unsigned>(e0));
-      else
-        hipLaunchKernelGGL(wmmae_gemm::reduce_splits_kernel<1>, grid, dim3(256),
-                           0, g.stream, g.partial, zdim, g.c, g.m, g.n, g.ldc,
-                           g.stride_c, g.c_ptrs, g.alpha, g.beta,
-                           static_cast<long long>(g.batch),
-                           static_cast<unsigned>(e0));
-    }
-    st = launch_status();
-  }
-  if (st == WMMAE_STATUS_SUCCESS && t_gemm_end != nullptr)
-    WMMAE_HIP_TRY(hipEventRecord(t_gemm_end, g.stream));
-  return st;
-}
-
-// Tile choice: the 256x128 tile moves the fewest operand bytes per flop and is
-// the choice whenever its rounds cost less; the tiles run in rounds
-// of one per compute unit, so when the last round would be mostly empty the
-// 128x128 tile (5 to 25 % slower per flop) can still finish sooner; 64x64
-// tiles for problems too small to give the larger ones work.
-template <class MT, int TERMS, bool RN> int gemm_by_size(const GemmArgs &g) {
-  const int cus = device_cus();
-  const long long z = g.partial != nullptr ? g.splits : 1;
-  const long long big =
-      ceil_div(g.m, 256) * ceil_div(g.n, 128) * g.batch * z;
-  const long long mid =
-      ceil_div(g.m, 128) * ceil_div(g.n, 128) * g.batch * z;
-  if constexpr (TERMS <= 2 && !RN) {
-    // (k a multiple of 32, or the variant with a shorter last stage)
-    if (g.is_direct)
-      return g.k % 32 == 0 ? launch_gemm<MT, TERMS, 256, 128, 2, 2, RN, 1>(g)
-                           : launch_gemm<MT, TERMS, 256, 128, 2, 2, RN, 2>(g);
-  }
-  // (not with the separate fp32 adds of RN: their temporaries do not fit the
-  // register file next to the large tile's accumulators)
-  if constexpr (!RN) {
-    const int KT = packed_k_tiles(g.k);
-    if (big_tile_candidate(TERMS, mid, static_cast<int>(ceil_div(KT, z)))) {
-      // time in units of one 128x128 tile: rounds * tile cost
-      const bool tail_ok = g.batch == 1 && z == 1 && g.c_ptrs == nullptr &&
-                           g.tail_ws != nullptr;
-      const double t_big =
-          rounds_cost(big, cus, KT, tail_ok) * fit::units256x128(TERMS);
-      // (a 128x128 tile measured at 1.2 to 1.25 times half a 256x128 tile in
-      // runs of two to eight rounds, 1.05 in long ones)
-      const double t_mid =
-          rounds_cost(mid, cus, KT, tail_ok) * fit::units128x128(TERMS);
-      if (t_big <= t_mid)
-        return launch_gemm<MT, TERMS, 256, 128, 2, 2, RN>(g);
-    }
-  }
-  if (mid >= cus || (g.m > 64 && g.n > 64))
-    return launch_gemm<MT, TERMS, 128, 128, 2, 2, RN>(g);
-  return launch_gemm<MT, TERMS, 64, 64, 2, 2, RN>(g);
-}
-
-int gemm_dispatch(const int policy, const int flags, const GemmArgs &g) {
-  const bool rn = (flags & WMMAE_FLAG_RN_MAIN) != 0;
-  switch (policy) {
-  case WMMAE_POLICY_F16_EC:
-    return rn ? gemm_by_size<_Float16, 2, true>(g)
-              : gemm_by_size<_Float16, 2, false>(g);
-  case WMMAE_POLICY_F16_NOEC:
-    return rn ? WMMAE_STATUS_NOT_SUPPORTED
-              : gemm_by_size<_Float16, 1, false>(g);
-  case WMMAE_POLICY_BF16X3_EC:
-    return rn ? gemm_by_size<__bf16, 3, true>(g)
-              : gemm_by_size<__bf16, 3, false>(g);
-  case WMMAE_POLICY_BF16X2_EC:
-    return rn ? WMMAE_STATUS_NOT_SUPPORTED
-              : gemm_by_size<__bf16, 2, false>(g);
-  case WMMAE_POLICY_BF16_NOEC:
-    return rn ? WMMAE_STATUS_NOT_SUPPORTED : gemm_by_size<__bf16, 1, false>(g);
-  default:
-    return WMMAE_STATUS_INVALID_VALUE;
-  }
-}
-
-// Resident workgroups per compute unit of the packed kernel a policy runs with
-// tile shape 0 (256x128), 1 (128x128) or 2 (64x64): the number launch_gemm
-// plans its rounds with, for the workspace query.
-template <class MT, int TERMS> int per_cu_by_shape(const int shape) {
-  switch (shape) {
-  case 0:
-    return workgroups_per_cu<MT, TERMS, 256, 128, 2, 2, false>();
-  case 1:
-    return workgroups_per_cu<MT, TERMS, 128, 128, 2, 2, false>();
-  default:
-    return workgroups_per_cu<MT, TERMS, 64, 64, 2, 2, false>();
-  }
-}
-int per_cu_of(const int policy, const int shape) {
-  switch (policy) {
-  case WMMAE_POLICY_F16_EC:
-    return per_cu_by_shape<_Float16, 2>(shape);
-  case WMMAE_POLICY_F16_NOEC:
-    return per_cu_by_shape<_Float16, 1>(shape);
-  case WMMAE_POLICY_BF16X3_EC:
-    return per_cu_by_shape<__bf16, 3>(shape);
-  case WMMAE_POLICY_BF16X2_EC:
-    return per_cu_by_shape<__bf16, 2>(shape);
-  default:
-    return per_cu_by_shape<__bf16, 1>(shape);
-  }
-}
-
-// ------------------------------------------------------ fused small GEMM
-struct FusedArgs {
-  wmmae_gemm::FusedParams p;
-  hipStream_t stream;
-};
-
-template <class T, int TERMS, int BM, int BN> int launch_fused(FusedArgs f) {
-  using Cfg = wmmae_gemm::FusedConfig<TERMS, BM, BN>;
-  auto kernel = wmmae_gemm::tcec_gemm_fused_kernel<T, TERMS, BM, BN>;
-  static std::atomic<unsigned long long> lds_allowed{0};
-  WMMAE_HIP_TRY(allow_dynamic_lds(reinterpret_cast<const void *>(kernel),
-                                  Cfg::LDS_BYTES, lds_allowed));
-  wmmae_gemm::FusedParams &p = f.p;
-  p.tiles_m = static_cast<int>(ceil_div(p.M, BM));
-  p.tiles_per_batch = p.tiles_m * static_cast<int>(ceil_div(p.N, BN));
-  // one persistent workgroup per compute unit at most; with 8 or more batch
-  // entries an XCD (block index mod 8) owns whole entries
-  const int per_xcd_max = device_cus() / 8 > 0 ? device_cus() / 8 : 1;
-  // (not when the XCD that owns one entry more than the others would need
-  // over 15 % more rounds of tiles than an even spread)
-  const long long all_tiles =
-      static_cast<long long>(p.batch) * p.tiles_per_batch;
-  p.grouped =
-      device_xcds() == kKernelXcds && p.batch >= 8 &&
-      ceil_div(ceil_div(p.batch, 8) * p.tiles_per_batch, per_xcd_max) * 100 <=
-          ceil_div(all_tiles, 8ll * per_xcd_max) * 115;
-  long long per_xcd = p.grouped
-                          ? ceil_div(p.batch, 8) * p.tiles_per_batch
-                          : ceil_div(static_cast<long long>(p.batch) *
-                                         p.tiles_per_batch,
-                                     8);
-  if (per_xcd > per_xcd_max)
-    per_xcd = per_xcd_max;
-  const int grid = 8 * static_cast<int>(per_xcd);
-  hipLaunchKernelGGL(kernel, dim3(grid), dim3(Cfg::NTHREADS), Cfg::LDS_BYTES,
-                     f.stream,
-                     p);
-  return launch_status();
-}
-
-// 128x128 tiles, unless they leave compute units without work and 64x64 tiles
-// (four times as many workgroups; one takes 0.65 of a 128x128 tile's time at
-// these latency-bound sizes) finish sooner: 1024^3 went from 41 to 27 us.
-inline bool fused_small_tiles(const int m, const int n, const int batch) {
-  const long long cus = device_cus();
-  const long long tiles128 = ceil_div(m, 128) * ceil_div(n, 128) * batch;
-  const long long tiles64 = ceil_div(m, 64) * ceil_div(n, 64) * batch;
-  return (m <= 64 && n <= 64) ||
-         (tiles128 < cus && fit::kFusedSmallTileTime *
-                                    static_cast<double>(ceil_div(tiles64, cus)) <
-                                static_cast<double>(ceil_div(tiles128, cus)));
-}
-template <class T, int TERMS> int fused_by_size(const FusedArgs &f) {
-  if (fused_small_tiles(f.p.M, f.p.N, f.p.batch))
-    return launch_fused<T, TERMS, 64, 64>(f);
-  return launch_fused<T, TERMS, 128, 128>(f);
-}
-
-int fused_dispatch(const int policy, const FusedArgs &f) {
-  switch (policy) {
-  case WMMAE_POLICY_F16_EC:
-    return fused_by_size<w::half, 2>(f);
-  case WMMAE_POLICY_F16_NOEC:
-    return fused_by_size<w::half, 1>(f);
-  case WMMAE_POLICY_BF16X3_EC:
-    return fused_by_size<w::precision::tf32, 3>(f);
-  case WMMAE_POLICY_BF16X2_EC:
-    return fused_by_size<w::bfloat16, 2>(f);
-  case WMMAE_POLICY_BF16_NOEC:
-    return fused_by_size<w::bfloat16, 1>(f);
-  default:
-    return WMMAE_STATUS_INVALID_VALUE;
-  }
+// --------------------------------------------------------------------------
+// scale_c_kernel: C = beta * C, the whole result when k == 0.
+// --------------------------------------------------------------------------
+__global__ void __launch_bounds__(256)
+    scale_c_kernel(float *__restrict__ C, const int M, const int N,
+                   const long long ldc, const long long batch_stride_c,
+                   float *const *__restrict__ c_ptrs, const float beta,
+                   const unsigned entry0) {
+  const long long e = static_cast<long long>(blockIdx.x) * 256 + threadIdx.x;
+  if (e >= static_cast<long long>(M) * N)
+    return;
+  const long long entry = entry0 + blockIdx.y;
+  float *const cb =
+      c_ptrs != nullptr ? c_ptrs[entry] : C + entry * batch_stride_c;
+  float *const p = cb + (e % M) + (e / M) * ldc;
+  *p = beta == 0.f ? 0.f : beta * *p;
 }
 
 // Which of the three paths?  The single ("fused") kernel moves only the fp32
@@ -1077,8 +311,8 @@ int pack_impl(const int policy, const int rows, const int k,
   if (st != WMMAE_STATUS_SUCCESS || nothing)
     return st;
   const PackSource src{rows, X, ptrs, row_stride, k_stride, batch_stride, packed};
-  return pack_dispatch(policy, k, batch, src, nullptr,
-                       static_cast<hipStream_t>(stream));
+  return policy_kernels(policy)->pack(k, batch, src, nullptr,
+                                      static_cast<hipStream_t>(stream));
 }
 
 // split-K, or K slices for a partly empty last round, only when the caller
@@ -1132,7 +366,7 @@ int gemm_packed_impl(const int policy, const int m, const int n, const int k,
     if (blocks > 0x7fffffffLL)
       return WMMAE_STATUS_NOT_SUPPORTED;
     for (int e0 = 0; e0 < batch; e0 += kMaxGridY)
-      hipLaunchKernelGGL(wmmae_gemm::scale_c_kernel,
+      hipLaunchKernelGGL(scale_c_kernel,
                          dim3(static_cast<unsigned>(blocks),
                               std::min(batch - e0, kMaxGridY)),
                          dim3(256), 0, static_cast<hipStream_t>(stream), C, m, n,
@@ -1157,7 +391,11 @@ int gemm_packed_impl(const int policy, const int m, const int n, const int k,
   g.terms = p.terms;
   g.stream = static_cast<hipStream_t>(stream);
   plan_k_slices(g, workspace, workspace_bytes);
-  return gemm_dispatch(policy, flags, g);
+  const PolicyKernels *const kernels = policy_kernels(policy);
+  if ((flags & WMMAE_FLAG_RN_MAIN) == 0)
+    return kernels->gemm(g);
+  return kernels->gemm_rn != nullptr ? kernels->gemm_rn(g)
+                                     : WMMAE_STATUS_NOT_SUPPORTED;
 }
 
 int sgemm_impl(const char transa, const char transb, const int m, const int n,
@@ -1257,7 +495,7 @@ int sgemm_impl(const char transa, const char transb, const int m, const int n,
         direct_times(m, n, k, batch, fit::kDirectStagger[p.terms - 1]);
     if (g.splits <= 1 && batch >= 8 && dt.bytes > dt.tiles)
       g.direct.stagger = 1;
-    int st = gemm_dispatch(policy, 0, g);
+    int st = policy_kernels(policy)->gemm(g);
     if (own && hipFreeAsync(ws, s) != hipSuccess && st == WMMAE_STATUS_SUCCESS)
       st = WMMAE_STATUS_RUNTIME_ERROR;
     return st;
@@ -1294,7 +532,7 @@ int sgemm_impl(const char transa, const char transb, const int m, const int n,
     q.beta = *beta;
     q.inv_scale = p.inv_scale;
     f.stream = static_cast<hipStream_t>(stream);
-    return fused_dispatch(policy, f);
+    return policy_kernels(policy)->fused(f);
   }
 
   size_t bytes_a = 0, bytes_b = 0, bytes_c = 0;
@@ -1338,7 +576,7 @@ int sgemm_impl(const char transa, const char transb, const int m, const int n,
                       sb.k_stride, batch, pb, bytes_b, none_b);
     // (m, n, k and batch are all positive here: both operands have work)
     if (st == WMMAE_STATUS_SUCCESS && !none_a && !none_b)
-      st = pack_dispatch(policy, k, batch, sa, &sb, s); // one launch for both
+      st = policy_kernels(policy)->pack(k, batch, sa, &sb, s); // one launch
   }
   if (st == WMMAE_STATUS_SUCCESS)
     st = gemm_packed_impl(policy, m, n, k, alpha, pa, pb, beta, C, c_ptrs, ldc,
@@ -1405,7 +643,7 @@ int wmmae_tcec_gemm_packed_workspace_bytes(const int policy, const int m,
     const int shapes[3][2] = {{256, 128}, {128, 128}, {64, 64}};
     for (int i = 0; i < 3; i++) {
       const int *const sh = shapes[i];
-      const int per_cu = per_cu_of(policy, i);
+      const int per_cu = policy_kernels(policy)->per_cu(i);
       const TailPlan t =
           plan_tail(ceil_div(m, sh[0]) * ceil_div(n, sh[1]),
                     static_cast<long long>(device_cus()) * per_cu, KT);

@@ -1,0 +1,445 @@
+// What the host side of the GEMM driver decides with: policies, packed operand
+// geometry, the fitted cost parameters, K-slice plans.  Shared by the C boundary
+// (capi_gemm.hip) and the translation units that hold the kernels of one or two
+// policies each (gemm_*.hip, through gemm_launch.hpp).
+#pragma once
+#include "capi_common.hpp"
+#include <limits>
+#include "tcec_gemm_fused_kernel.hpp"
+#include "tcec_gemm_kernels.hpp"
+
+namespace wmmae_driver {
+using namespace wmmae_capi;
+using wmmae_gemm::u32x4;
+
+// ------------------------------------------------------------ policy table
+struct PolicyInfo {
+  int terms;       // stored terms per operand
+  bool bf16;       // MFMA element type
+  float inv_scale; // factor applied to the error accumulator
+};
+inline bool policy_info(const int policy, PolicyInfo &p) {
+  switch (policy) {
+  case WMMAE_POLICY_F16_EC:
+    p = {2, false, 1.f / 2048.f};
+    return true;
+  case WMMAE_POLICY_F16_NOEC:
+    p = {1, false, 1.f};
+    return true;
+  case WMMAE_POLICY_BF16X3_EC:
+    p = {3, true, 1.f};
+    return true;
+  case WMMAE_POLICY_BF16X2_EC:
+    p = {2, true, 1.f};
+    return true;
+  case WMMAE_POLICY_BF16_NOEC:
+    p = {1, true, 1.f};
+    return true;
+  default:
+    return false;
+  }
+}
+
+// packed operand geometry: 16-row blocks, 32-wide k chunks
+inline long long packed_row_blocks(const int rows) { return ceil_div(rows, 16); }
+inline int packed_k_tiles(const int k) {
+  return static_cast<int>(ceil_div(k, 32));
+}
+// u32x4 elements of one packed matrix
+inline long long packed_elems(const int rows, const int k, const int terms) {
+  return packed_row_blocks(rows) * packed_k_tiles(k) * terms * 64;
+}
+
+// ------------------------------------------------------------------ pack
+// One operand of a split launch as the caller describes it.
+struct PackSource {
+  int rows;
+  const float *X;
+  const float *const *ptrs;
+  long long row_stride, k_stride, batch_stride;
+  void *packed;
+};
+
+inline wmmae_gemm::PackOperand pack_operand(const PackSource &src,
+                                            const int KT) {
+  wmmae_gemm::PackOperand o;
+  o.X = src.X;
+  o.ptrs = src.ptrs;
+  o.row_stride = src.row_stride;
+  o.k_stride = src.k_stride;
+  o.batch_stride = src.batch_stride;
+  o.rows = src.rows;
+  o.chunks = packed_row_blocks(src.rows) * KT;
+  o.out = static_cast<u32x4 *>(src.packed);
+  return o;
+}
+
+// The batch index of the split, scale and fold kernels is the grid's y
+// coordinate, which ends at 65535: longer batches take one launch per 65535
+// entries.
+constexpr int kMaxGridY = 65535;
+
+// ------------------------------------------------------------------ gemm
+struct GemmArgs {
+  const u32x4 *a, *b;
+  float *c;
+  int m, n, k;
+  long long ldc, stride_c;
+  float alpha, beta, inv_scale;
+  int batch, terms;
+  float *const *c_ptrs; // device array of C pointers, or nullptr
+  float *partial;  // split-K slices, or nullptr
+  int splits;      // >= 1
+  // room for the K slices of the tiles of a partly empty last round (used
+  // only without split-K), or nullptr
+  float *tail_ws;
+  size_t tail_ws_bytes;
+  hipStream_t stream;
+  // fp32 operands for the kernel variant that splits them itself (a and b are
+  // null then)
+  bool is_direct = false;
+  wmmae_gemm::DirectSource direct = {};
+};
+
+// Compute units of the current device, looked up once per device.
+inline int device_cus() {
+  static std::atomic<int> cached[64];
+  int dev = 0;
+  if (hipGetDevice(&dev) != hipSuccess)
+    return 256; // MI355X; also the answer when no device is visible
+  const bool tracked = dev >= 0 && dev < 64;
+  if (tracked) {
+    const int c = cached[dev].load(std::memory_order_relaxed);
+    if (c > 0)
+      return c;
+  }
+  hipDeviceProp_t prop;
+  if (hipGetDeviceProperties(&prop, dev) != hipSuccess ||
+      prop.multiProcessorCount <= 0)
+    return 256;
+  if (tracked)
+    cached[dev].store(prop.multiProcessorCount, std::memory_order_relaxed);
+  return prop.multiProcessorCount;
+}
+
+// ------------------------------------------------ fitted cost parameters
+// Every number the path and tile choices below are made with, in one place.
+// All are fits to measurements on MI355X (256 compute units, one box of the
+// pool each; the boxes differ by 3 to 5 % in what they sustain under the power
+// limit).  The estimates have one form: launch cost + rounds of tiles over the
+// compute units x (k stages of 32 x time per stage + time per tile), bounded
+// below by the bytes moved.
+namespace fit {
+// -- packed GEMM, time of one k stage of one tile, by stored terms (1, 2, 3).
+//    Sweep: 216 products, m = n = 512 .. 2048, k = 512 .. 4096, each run with
+//    1, 2, 3, 4, 6 and 8 K slices; the slice count chosen with them is within
+//    0.7 % of the best measured one on average (1.9 % on 120 random products
+//    with m, n = 64 .. 2900, k = 400 .. 32000, 1 .. 100 entries, 1 .. 32
+//    slices forced).
+constexpr double kStage256x128[3] = {0.8e-6, 1.0e-6, 1.82e-6};
+constexpr double kStage128x128[3] = {0.45e-6, 0.6e-6, 0.99e-6};
+constexpr double kStage64x64 = 0.25e-6;
+constexpr double kTileOverhead = 7e-6;    // pipeline fill + epilogue of a tile
+constexpr double kFoldLaunch = 6e-6;      // the pass that adds the K slices
+constexpr double kFoldBytesPerS = 3e12;   // ... reads and writes its planes at
+constexpr double kSplitMustBeat = 0.95;   // a split has to win by 5 %
+// -- tile choice, cost of a tile in units of one 128x128 tile.  Sweep: both
+//    tiles forced on 124 products, 1024^2 .. 8192^2, k = 256 .. 4096, some
+//    batched: the choice is within 0.4 % of the faster tile on average.
+constexpr double kUnits256x128 = 2.0;
+constexpr double kUnits128x128 = 1.2;     // one and two terms
+//    Three terms (sweep: both tiles forced on 36 products, 1024^2 .. 8192^2,
+//    k = 1024 .. 5000, some batched or rectangular: a round of 256x128 tiles
+//    costs 1.8 rounds of 128x128 tiles, so the large tile wins when it halves
+//    the rounds, 8 to 14 %, and loses otherwise, 3 % at 7 -> 4 rounds, 17 to
+//    20 % at 3 -> 2).
+constexpr double kUnits256x128Terms3 = 1.8;
+constexpr double kUnits128x128Terms3 = 1.0;
+constexpr double kUnits64x64 = 0.4;
+constexpr double units256x128(const int terms) {
+  return terms == 3 ? kUnits256x128Terms3 : kUnits256x128;
+}
+constexpr double units128x128(const int terms) {
+  return terms == 3 ? kUnits128x128Terms3 : kUnits128x128;
+}
+// -- K slices for a partly empty last round: slices, pipeline refills, fold.
+//    Sweep: 126 products, 2304^2 .. 8192^2, k = 2048 .. 8192, two policies.
+constexpr double kTailOverhead = 0.2;
+// -- which path: the single kernel, split passes + GEMM on packed operands, or
+//    the GEMM kernel that splits the fp32 operands itself.  Fit: 1860 random
+//    products (m, n = 45 .. 5000, k = 32 .. 32768, 1 .. 1024 entries, half of
+//    them with dimensions that are multiples of nothing, all five policies),
+//    each run with every path forced; the constants below minimise the
+//    squared log error of each path's estimate on 1060 of them and on 137
+//    structured products (the reference harness's grid with 256 entries,
+//    squares 1024 .. 8192, the baseline workloads; weighted four times).  On
+//    the 800 held out the path chosen with them is 1.4 % slower than always
+//    taking the fastest forced path on average (37 of 800 above 1.10 x, six
+//    above 1.25 x), on the structured ones 0.5 % (two above 1.10 x); the
+//    constants before (fits to the harness's grid and to square products)
+//    were 3 to 6 % slower on the same 800, 3.1 x at worst.  Whole default
+//    calls on 400 further random products: 1.1 % (worst 1.48 x).
+//    Rows: one, two, three terms.
+struct PathRates {
+  double launch, stage, tile, bytes_per_s; // seconds, seconds, seconds, B/s
+  double split_bytes_per_s;                // packed path only
+  // A k stage takes longer the fuller the chip is (power limit, contention in
+  // L2 and HBM): stage * (1 + busy * (compute units with a tile / all compute
+  // units, averaged over the rounds))
+  double busy;
+};
+constexpr PathRates kFused[3] = {
+    {6.01e-6, 0.643e-6, 2.88e-6, 5.32e12, 0., 0.101},
+    {6.50e-6, 0.992e-6, 1.85e-6, 5.27e12, 0., 0.170},
+    {5.37e-6, 1.39e-6, 2.22e-6, 5.14e12, 0., 0.141}};
+constexpr PathRates kPacked[3] = {
+    {8.35e-6, 0.131e-6, 3.07e-6, 3.65e12, 5.61e12, 0.359},
+    {8.17e-6, 0.287e-6, 3.69e-6, 6.50e12, 5.57e12, 0.649},
+    {7.10e-6, 0.652e-6, 4.65e-6, 6.50e12, 4.92e12, 0.361}};
+// -- the packed path's GEMM kernel reading and splitting the fp32 operands
+//    itself (256x128 tiles only; rows: one, two terms)
+constexpr PathRates kDirect[2] = {
+    {3.41e-6, 0.173e-6, 3.76e-6, 4.62e12, 0., 1.18},
+    {5.00e-6, 0.355e-6, 3.65e-6, 4.92e12, 0., 0.750}};
+// ... as the host sees it when it decides whether a launch of that kernel is
+// bound by its bytes and should start its workgroups staggered (a fit of its
+// own, to the reference harness's grid: 0.8 / 1.5 us per k stage of a 256x128
+// tile and 6 us per tile, in units of half a tile)
+constexpr PathRates kDirectStagger[2] = {
+    {6.0e-6, 0.40e-6, 3.0e-6, 5.0e12, 0., 0.},
+    {6.0e-6, 0.75e-6, 3.0e-6, 5.0e12, 0., 0.}};
+// with K slices: the GEMM's time against the packed kernel's estimate for the
+// same slices of 256x128 tiles (two terms: twelve K-sliced products, m, n =
+// 64 .. 4096, k = 2048 .. 262144, each run on either path: with 1.4 the faster
+// path is chosen for all of them, with 1.5 for eleven)
+constexpr double kDirectSliceRatio[2] = {1.5, 1.4};
+// Products that are cut into K slices (few output tiles): what the slice
+// planner's time (split_time, whose constants are fitted for choosing the slice
+// count) has to be scaled and shifted by to be the time of the whole call on
+// each path; same fit as above.  Rows: scale, shift in seconds; by terms.
+constexpr double kSlicedFused[2][3] = {{1.16, 1.08, 1.03},
+                                       {-3.73e-6, -2.84e-6, -2.89e-6}};
+constexpr double kSlicedPacked[2][3] = {{0.724, 0.954, 0.955},
+                                        {-0.65e-6, -6.0e-6, -6.0e-6}};
+constexpr double kSlicedDirect[2][2] = {{0.759, 0.890}, {-6.0e-6, -6.0e-6}};
+// Calls issued back to back cannot complete faster than the host issues their
+// launches (250 products below 1.5e8 flop, called in a loop: 11, 14.5 and 12 us
+// per call in the median): what decides among the paths for tiny products -
+// one launch for the single kernel and the direct kernel, two or three for
+// the packed path.  Order: single kernel, packed, direct.
+constexpr double kCallFloor[3] = {11.0e-6, 14.3e-6, 11.5e-6};
+// k % 32 != 0: the kernel variant that reads a shorter last stage (1024^2 x 1000
+// against x 1024, batch 256: 301 against 336 TFLOPS, of which 2.4 % are the k)
+constexpr double kDirectTailStage = 1.47;
+// the single kernel's 64x64 tile against its 128x128 tile (1024^3: 41 -> 27 us)
+constexpr double kFusedSmallTileTime = 0.65; // whole tile, latency-bound sizes
+constexpr double kFusedSmallStage = 0.599, kFusedSmallTile = 0.467;
+// 4-byte instead of 16-byte requests: 114 random products with k % 4 != 0 ran
+// at 0.55 of the packed path's speed in the median
+constexpr double kFusedNarrowRequests = 3.50;
+} // namespace fit
+
+// XCDs (chiplets with an L2 of their own) behind the current device.  HIP does
+// not report them; a gfx950 XCD has 32 active compute units in every partition
+// mode (SPX 256 = 8 x 32, DPX 128, QPX 64, CPX 32), so the count follows from
+// the compute units.  Consecutive workgroup ids go round-robin over the XCDs;
+// the kernels' XCD-aware item lists are written for eight of them and are used
+// only then (other counts take the plain shared list: same results, tiles not
+// grouped by L2).
+inline int device_xcds() {
+  const int cus = device_cus();
+  return cus % 32 == 0 ? cus / 32 : 1;
+}
+constexpr int kKernelXcds = 8; // the constant XCDS of the kernels' item lists
+
+// Number of K slices of every tile, when the 256x128 output tiles cannot fill
+// half the chip.  For every candidate (at most 32 slices of at least 6 stages)
+// the GEMM's time is estimated the way gemm_by_size will run it: the tile that
+// the slice count leads to, rounds of those tiles over the compute units,
+// stages per slice at that tile's time per stage, a fixed time per tile, and
+// for more than one slice the fold (a launch plus the planes written and
+// read).  The cheapest count is taken, any split having to beat the uncut run
+// by 5 %.  Times per stage and tile: fits to measurements on MI355X (216
+// products, m = n = 512 .. 2048, k = 512 .. 4096, one to three terms, each run
+// with 1, 2, 3, 4, 6 and 8 slices: the choice is within 0.7 % of the best measured count on
+// average; "as many slices as fill the chip with 256x128 tiles" was 7 % off,
+// over-cutting outputs from 1280^2 up and not cutting short loops at all).
+// Whether the 256x128 tile is a candidate at all: only where the 128x128 tiles
+// need more than one round over the compute units (in a single round the
+// smaller tile always finishes first), and not for the one-term kernels on
+// loops of 32 stages or fewer, where the stores of C dominate and the smaller
+// tile measured 8 to 12 % faster.  (Forced-tile runs of 124 products: the
+// choice below is within 0.4 % of the faster tile on average; requiring a full
+// round of 256x128 tiles instead had cost 2 %, up to 13 % at 2560^2 .. 2816^2.)
+inline bool big_tile_candidate(const int terms, const long long mid,
+                               const int kt) {
+  return mid > device_cus() && !(terms == 1 && kt <= 32);
+}
+// `direct`: the kernel that splits the fp32 operands itself, which has the
+// 256x128 tile only and takes kDirectSliceRatio times the packed kernel's time
+// (its slice count must be planned with its own tiles: 4096 x 64 x 4096 cut
+// for the 128x128 tiles of the packed path left half the compute units
+// without a 256x128 item, 48 against 39 us).
+inline double split_time(const int terms, const int m, const int n,
+                         const int batch, const int kt, const int slices,
+                         const bool direct = false) {
+  const long long cus = device_cus();
+  const int stages = static_cast<int>(ceil_div(kt, slices));
+  const long long z = ceil_div(kt, stages);
+  const long long big = ceil_div(m, 256) * ceil_div(n, 128) * batch * z;
+  const long long mid = ceil_div(m, 128) * ceil_div(n, 128) * batch * z;
+  double stage_time, rounds;
+  const double r_big = static_cast<double>(ceil_div(big, cus));
+  const double r_mid = static_cast<double>(ceil_div(mid, cus));
+  if (direct ||
+      (big_tile_candidate(terms, mid, stages) &&
+       r_big * fit::units256x128(terms) <= r_mid * fit::units128x128(terms))) {
+    stage_time = fit::kStage256x128[terms - 1];
+    rounds = r_big;
+  } else if (mid >= cus || (m > 64 && n > 64)) {
+    stage_time = fit::kStage128x128[terms - 1];
+    rounds = r_mid;
+  } else {
+    stage_time = fit::kStage64x64;
+    rounds = static_cast<double>(
+        ceil_div(ceil_div(m, 64) * ceil_div(n, 64) * batch * z, cus));
+  }
+  double t = rounds * (stages * stage_time + fit::kTileOverhead);
+  if (z > 1)
+    t += fit::kFoldLaunch + static_cast<double>(z + 1) * m * n * batch * 4.0 /
+                                fit::kFoldBytesPerS;
+  return direct ? t * fit::kDirectSliceRatio[terms - 1] : t;
+}
+// Test hook (wmmae_tcec_force_k_slices): a slice count for the calling thread's
+// next calls instead of the estimates' choice, so that two kernels can be run on
+// the same cut of K and compared bit by bit.  0: the estimates choose.
+inline thread_local int t_forced_k_slices = 0;
+// Measurement hook (wmmae_tcec_time_gemm_kernel): events this thread's calls
+// record on their stream right before the MFMA GEMM kernel and right after it
+// (after the fold of its K slices where there is one).
+inline thread_local hipEvent_t t_gemm_begin = nullptr, t_gemm_end = nullptr;
+constexpr int kMaxSplits = 32, kMinStagesPerSplit = 6;
+inline int choose_splits(const int terms, const int m, const int n, const int k,
+                         const int batch, const bool direct = false) {
+  const long long tiles = ceil_div(m, 256) * ceil_div(n, 128) * batch;
+  const int kt = static_cast<int>(ceil_div(k, 32));
+  if (t_forced_k_slices > 0) {
+    const int s = std::max(
+        1, std::min({t_forced_k_slices, kMaxSplits, kt / kMinStagesPerSplit}));
+    return static_cast<int>(ceil_div(kt, ceil_div(kt, s)));
+  }
+  if (tiles * 2 > device_cus())
+    return 1;
+  int best = 1;
+  double t_best =
+      fit::kSplitMustBeat * split_time(terms, m, n, batch, kt, 1, direct);
+  for (int s = 2; s <= kMaxSplits && s * kMinStagesPerSplit <= kt; s++) {
+    if (ceil_div(kt, ceil_div(kt, s)) != s)
+      continue; // the same slices as a smaller count
+    const double t = split_time(terms, m, n, batch, kt, s, direct);
+    if (t < t_best) {
+      t_best = t;
+      best = s;
+    }
+  }
+  return best;
+}
+
+// K slices for the tiles of the last round only.  `tiles` output tiles run in
+// rounds of `resident` (one workgroup per item, long K loops); when the last
+// round is less than half full its tiles are cut into `slices` K slices of at
+// least 32 stages each, so that the round takes about 1/slices of a tile's
+// time (plus the pass that folds the slices).  slices == 1: not worth it.
+struct TailPlan {
+  long long full = 0, tail = 0; // tiles in whole rounds, tiles in the last
+  int slices = 1, stages = 0;   // K slices of a tail tile, stages per slice
+};
+inline TailPlan plan_tail(const long long tiles, const long long resident,
+                          const int KT) {
+  TailPlan t;
+  t.full = tiles / resident * resident;
+  t.tail = tiles - t.full;
+  if (t.full == 0 || t.tail == 0 || t.tail * 2 > resident || KT < 64)
+    return t;
+  long long s = std::min<long long>({resident / t.tail, KT / 32, 16});
+  if (s < 2)
+    return t;
+  t.stages = static_cast<int>(ceil_div(KT, s));
+  t.slices = static_cast<int>(ceil_div(KT, t.stages));
+  return t;
+}
+// Time of `tiles` tiles in units of one tile, with and without that plan.
+inline double rounds_cost(const long long tiles, const long long resident,
+                          const int KT, const bool tail_allowed) {
+  const TailPlan t = plan_tail(tiles, resident, KT);
+  const double full_rounds = static_cast<double>(t.full / resident);
+  if (t.tail == 0)
+    return full_rounds;
+  if (!tail_allowed || t.slices < 2)
+    return full_rounds + 1.0;
+  return full_rounds + 1.0 / t.slices + fit::kTailOverhead;
+}
+
+// Deepest LDS ring (at most 4 stages) that fits the 160 KiB of a compute unit.
+constexpr int ring_depth(const int bm, const int bn, const int terms) {
+  const int stage_bytes = (bm / 16 + bn / 16) * terms * 1024;
+  const int fit = (160 * 1024) / stage_bytes;
+  return fit > 4 ? 4 : fit;
+}
+
+// ------------------------------------------------------ fused small GEMM
+struct FusedArgs {
+  wmmae_gemm::FusedParams p;
+  hipStream_t stream;
+};
+
+// 128x128 tiles, unless they leave compute units without work and 64x64 tiles
+// (four times as many workgroups; one takes 0.65 of a 128x128 tile's time at
+// these latency-bound sizes) finish sooner: 1024^3 went from 41 to 27 us.
+inline bool fused_small_tiles(const int m, const int n, const int batch) {
+  const long long cus = device_cus();
+  const long long tiles128 = ceil_div(m, 128) * ceil_div(n, 128) * batch;
+  const long long tiles64 = ceil_div(m, 64) * ceil_div(n, 64) * batch;
+  return (m <= 64 && n <= 64) ||
+         (tiles128 < cus && fit::kFusedSmallTileTime *
+                                    static_cast<double>(ceil_div(tiles64, cus)) <
+                                static_cast<double>(ceil_div(tiles128, cus)));
+}
+// The kernels of one policy, as the driver calls them: one table per policy,
+// filled in the gemm_*.hip translation units, which is what lets the kernels
+// compile side by side.
+struct PolicyKernels {
+  // splits one operand (b == nullptr) or both of a product
+  int (*pack)(int k, int batch, const PackSource &a, const PackSource *b,
+              hipStream_t stream);
+  int (*gemm)(const GemmArgs &g);
+  int (*gemm_rn)(const GemmArgs &g); // nullptr: the policy has no such variant
+  int (*fused)(const FusedArgs &f);
+  // resident workgroups per compute unit of the packed kernel with tile shape
+  // 0 (256x128), 1 (128x128) or 2 (64x64): the number the launch plans its
+  // rounds with, for the workspace query
+  int (*per_cu)(int shape);
+};
+const PolicyKernels &kernels_f16_ec();
+const PolicyKernels &kernels_f16_noec();
+const PolicyKernels &kernels_bf16x3_ec();
+const PolicyKernels &kernels_bf16x2_ec();
+const PolicyKernels &kernels_bf16_noec();
+inline const PolicyKernels *policy_kernels(const int policy) {
+  switch (policy) {
+  case WMMAE_POLICY_F16_EC:
+    return &kernels_f16_ec();
+  case WMMAE_POLICY_F16_NOEC:
+    return &kernels_f16_noec();
+  case WMMAE_POLICY_BF16X3_EC:
+    return &kernels_bf16x3_ec();
+  case WMMAE_POLICY_BF16X2_EC:
+    return &kernels_bf16x2_ec();
+  case WMMAE_POLICY_BF16_NOEC:
+    return &kernels_bf16_noec();
+  default:
+    return nullptr;
+  }
+}
+
+} // namespace wmmae_driver

@@ -264,24 +264,6 @@ __global__ void __launch_bounds__(256)
 }
 
 // --------------------------------------------------------------------------
-// scale_c_kernel: C = beta * C, the whole result when k == 0.
-// --------------------------------------------------------------------------
-__global__ void __launch_bounds__(256)
-    scale_c_kernel(float *__restrict__ C, const int M, const int N,
-                   const long long ldc, const long long batch_stride_c,
-                   float *const *__restrict__ c_ptrs, const float beta,
-                   const unsigned entry0) {
-  const long long e = static_cast<long long>(blockIdx.x) * 256 + threadIdx.x;
-  if (e >= static_cast<long long>(M) * N)
-    return;
-  const long long entry = entry0 + blockIdx.y;
-  float *const cb =
-      c_ptrs != nullptr ? c_ptrs[entry] : C + entry * batch_stride_c;
-  float *const p = cb + (e % M) + (e / M) * ldc;
-  *p = beta == 0.f ? 0.f : beta * *p;
-}
-
-// --------------------------------------------------------------------------
 // reduce_splits_kernel: C = alpha * sum_z partial[z] + beta * C for split-K.
 // partial[z][batch] are dense column-major M x N slices; the sum runs over z
 // in ascending order in double precision, so the result does not depend on
