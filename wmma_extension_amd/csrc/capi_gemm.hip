@@ -525,8 +525,6 @@ int sgemm_impl(const char transa, const char transb, const int m, const int n,
     q.batch = batch;
     q.vec_a = vec_a;
     q.vec_b = vec_b;
-    q.vec_store = (ldc % 4 == 0) &&
-                  (c_ptrs != nullptr || (aligned16(C) && stride_c % 4 == 0));
     q.rn_main = (flags & WMMAE_FLAG_RN_MAIN) != 0;
     q.alpha = *alpha;
     q.beta = *beta;

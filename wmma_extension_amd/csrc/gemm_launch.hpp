@@ -97,12 +97,6 @@ int launch_gemm(const GemmArgs &g) {
   const int KT = packed_k_tiles(g.k);
   const int rb_a = static_cast<int>(packed_row_blocks(g.m));
   const int rb_b = static_cast<int>(packed_row_blocks(g.n));
-  // 16-byte stores need ldc % 4 == 0 and an aligned base; the base of each
-  // batch entry is checked again inside the kernel
-  const int vec_store =
-      (g.ldc % 4 == 0) &&
-      (g.c_ptrs != nullptr || (reinterpret_cast<uintptr_t>(g.c) % 16 == 0 &&
-                               g.stride_c % 4 == 0));
   const int splits = g.partial != nullptr ? g.splits : 1;
   const int split_stages = static_cast<int>(ceil_div(KT, splits));
   const int zdim = static_cast<int>(ceil_div(KT, split_stages));
@@ -177,7 +171,7 @@ int launch_gemm(const GemmArgs &g) {
   hipLaunchKernelGGL(kernel, dim3(grid), dim3(Cfg::NTHREADS), Cfg::LDS_BYTES,
                      g.stream, g.a, g.b,
                      g.c, g.m, g.n, KT, rb_a, rb_b, g.ldc, g.alpha, g.beta,
-                     g.inv_scale, tiles_m, tiles_n, vec_store,
+                     g.inv_scale, tiles_m, tiles_n,
                      static_cast<long long>(rb_a) * KT * TERMS * 64,
                      static_cast<long long>(rb_b) * KT * TERMS * 64,
                      g.stride_c, split_stages,

@@ -76,11 +76,153 @@ __device__ __forceinline__ f32x4 epilogue_beta(const f32x4 scaled,
   return __builtin_elementwise_fma(f32x4{beta, beta, beta, beta}, c_old,
                                    scaled);
 }
-__device__ __forceinline__ float epilogue_beta(const float scaled,
-                                               const float beta,
-                                               const float c_old) {
-  return __builtin_fmaf(beta, c_old, scaled);
+// --------------------------------------------------------------------------
+// store_piece: the epilogue's memory side, shared by the GEMM kernels.  A wave
+// stores its piece of MT_ x NT_ accumulator tiles (16 x 16, a lane holds rows
+// 4*(lane/16) .. +3 of column lane%16) whose first element is (row0, col0) of
+// the column-major M x N matrix at Cb; value(i, j) is the scaled result of tile
+// (i, j), to which beta * C is added.
+//   * C is read GROUP tiles at a time before any of them is stored: a load next
+//     to every store makes the wave sit out one memory round trip per tile
+//     (nothing else runs on its SIMD).  All of a piece of up to sixteen tiles,
+//     one tile column (32 registers) of the largest kernels' pieces, whose
+//     other registers hold the next item's operands.
+//   * 16-byte accesses whatever the alignment: the hardware takes a dwordx4 at
+//     any address that is a multiple of four.  With one load next to every
+//     store, and four bytes at a time where ldc or the base is no multiple of
+//     four floats, 7 x 777x1333x515 with three bf16 terms and beta took 136 us,
+//     now 86; 1024x3072x4096 with beta 100.0, now 93.5; beta = 0 the same.
+//   * PAIRS: two vertically adjacent tiles at a time, the lanes of neighbouring
+//     columns swapping one tile's values, so that eight lanes hold 32
+//     consecutive rows of one column and an instruction writes 128 contiguous
+//     bytes instead of 64 of each of 16 columns (1024^2 x 128 x 256 entries
+//     0.458 -> 0.434 ms, 4096^3 0.322 -> 0.318).
+//   * One decision per piece: all of it inside C, no guards at all, or the
+//     guarded loop (with the choice made per pair of tiles the compiler keeps
+//     the accumulators in sight of several store paths, and values of the
+//     direct kernel's K loop go to scratch: c5b 1.45 -> 1.60 ms).
+// --------------------------------------------------------------------------
+template <int MT_, int NT_, bool PAIRS, int GROUP, class Value>
+__device__ __forceinline__ void
+store_piece(const Value &value, float *const Cb, const long long ld,
+            const int row0, const int col0, const int M, const int N,
+            const float beta, unsigned lane) {
+  static_assert(MT_ * NT_ % GROUP == 0 &&
+                    (!PAIRS || (MT_ % 2 == 0 && GROUP % 2 == 0)),
+                "whole groups");
+  // (device memory: global instructions, not generic ones, which count as LDS
+  // operations too)
+  typedef __attribute__((address_space(1))) float gfloat;
+  typedef f32x4 __attribute__((aligned(4))) f32x4_u;
+  typedef __attribute__((address_space(1))) f32x4_u gf32x4;
+  // (redefined in place: the lane's row and column are worked out here and not
+  // carried through the K loop, whose registers are all taken)
+  asm volatile("" : "+v"(lane));
+  const int q4 = 4 * static_cast<int>(lane >> 4);
+  const int c16 = static_cast<int>(lane & 15u);
+  if (row0 + 16 * MT_ <= M && col0 + 16 * NT_ <= N) { // wave-uniform
+    const int odd = static_cast<int>(lane & 1u);
+    // place of the lane's f32x4 number i of tile column j: rows of tile i, or
+    // of the pair's two instructions (even columns, then odd ones)
+    const auto place = [&](const int i, const int j) {
+      const int row =
+          row0 + q4 + (PAIRS ? 16 * ((i & ~1) + odd) : 16 * i);
+      const int col = col0 + 16 * j +
+                      (PAIRS ? ((i & 1) ? (c16 | 1) : (c16 & ~1)) : c16);
+      return reinterpret_cast<gf32x4 *>(
+          (gfloat *)(Cb + row + static_cast<long long>(col) * ld));
+    };
+#pragma unroll
+    for (int t0 = 0; t0 < MT_ * NT_; t0 += GROUP) {
+      f32x4 old[GROUP];
+      if (beta != 0.f) {
+#pragma unroll
+        for (int g = 0; g < GROUP; g++)
+          old[g] = *place((t0 + g) % MT_, (t0 + g) / MT_);
+      }
+      if constexpr (PAIRS) {
+#pragma unroll
+        for (int g = 0; g < GROUP; g += 2) {
+          const int i = (t0 + g) % MT_, j = (t0 + g) / MT_;
+          const f32x4 v0 = value(i, j), v1 = value(i + 1, j);
+          f32x4 d0, d1;
+#pragma unroll
+          for (int x = 0; x < 4; x++) {
+            // (through a function taking the element by value:
+            // __builtin_bit_cast applied to `v0[x]` directly read element 0
+            // for every x)
+            const float n0 = neighbour_lane(v0[x]), n1 = neighbour_lane(v1[x]);
+            d0[x] = odd ? n1 : v0[x]; // even column: own rows | neighbour's next 16
+            d1[x] = odd ? v1[x] : n0; // odd column
+          }
+          if (beta != 0.f) {
+            d0 = epilogue_beta(d0, beta, old[g]);
+            d1 = epilogue_beta(d1, beta, old[g + 1]);
+          }
+          *place(i, j) = d0;
+          *place(i + 1, j) = d1;
+        }
+      } else {
+#pragma unroll
+        for (int g = 0; g < GROUP; g++) {
+          const int i = (t0 + g) % MT_, j = (t0 + g) / MT_;
+          f32x4 v = value(i, j);
+          if (beta != 0.f)
+            v = epilogue_beta(v, beta, old[g]);
+          *place(i, j) = v;
+        }
+      }
+    }
+    return;
+  }
+#pragma unroll
+  for (int j = 0; j < NT_; j++) {
+    const int col = col0 + 16 * j + c16;
+    if (col >= N)
+      continue;
+    gfloat *const dst =
+        (gfloat *)(Cb + row0 + q4 + static_cast<long long>(col) * ld);
+    constexpr int HALF = MT_ > 4 ? 4 : MT_; // tiles whose C is read at a time
+    static_assert(MT_ % HALF == 0, "whole groups");
+#pragma unroll
+    for (int i0 = 0; i0 < MT_; i0 += HALF) {
+      f32x4 old[HALF];
+      if (beta != 0.f) {
+#pragma unroll
+        for (int g = 0; g < HALF; g++) {
+          const int i = i0 + g;
+          const int left = M - (row0 + 16 * i + q4); // rows from the lane's first
+          if (left > 3) {
+            old[g] = *reinterpret_cast<gf32x4 *>(dst + 16 * i);
+          } else {
+#pragma unroll
+            for (int x = 0; x < 4; x++)
+              old[g][x] = x < left ? dst[16 * i + x] : 0.f;
+          }
+        }
+      }
+#pragma unroll
+      for (int g = 0; g < HALF; g++) {
+        const int i = i0 + g;
+        const int left = M - (row0 + 16 * i + q4);
+        // (also for the rows past the end: a load whose register nothing reads
+        // would be waited for where the K loop next writes that register)
+        f32x4 v = value(i, j);
+        if (beta != 0.f)
+          v = epilogue_beta(v, beta, old[g]);
+        if (left > 3) {
+          *reinterpret_cast<gf32x4 *>(dst + 16 * i) = v;
+        } else {
+#pragma unroll
+          for (int x = 0; x < 3; x++)
+            if (x < left)
+              dst[16 * i + x] = v[x];
+        }
+      }
+    }
+  }
 }
+
 // Row permutation of k group q (0..3) of a chunk written by the DIRECT
 // variant of tcec_gemm_kernel.
 __host__ __device__ constexpr unsigned direct_swizzle(const unsigned q) {
@@ -497,8 +639,7 @@ __global__ void __launch_bounds__(WGM *WGN * 64)
                      const int KT, const int rb_a, const int rb_b,
                      const long long ldc, const float alpha,
                      const float beta, const float inv_scale, const int tiles_m,
-                     const int tiles_n, const int vec_store,
-                     const long long batch_stride_a,
+                     const int tiles_n, const long long batch_stride_a,
                      const long long batch_stride_b,
                      const long long batch_stride_c, const int split_stages,
                      float *__restrict__ partial,
@@ -927,15 +1068,23 @@ __global__ void __launch_bounds__(WGM *WGN * 64)
   // wait states (the compiler emits none for the builtin either).  Small wave
   // tiles use the builtin.
   constexpr bool USE_ASM = MT_ * NT_ >= 8;
+  // (The round-to-nearest variants keep fragments in accumulation registers and
+  // copy them back right in front of the MFMAs that read them: a wait of two
+  // states in front of each makes that safe.)
   auto mfma_acc = [](f32x4 &z, const ab_vec x, const ab_vec y) {
-    if constexpr (std::is_same<MT, _Float16>::value)
-      asm volatile(WMMAE_MFMA_GUARD "v_mfma_f32_16x16x32_f16 %0, %1, %2, %0"
-                   : "+a"(z)
-                   : "v"(x), "v"(y));
+#define WMMAE_MFMA_ACC(GUARD, TYPE)                                            \
+  asm volatile(GUARD "v_mfma_f32_16x16x32_" TYPE " %0, %1, %2, %0"             \
+               : "+a"(z)                                                       \
+               : "v"(x), "v"(y))
+    if constexpr (std::is_same<MT, _Float16>::value && RN_MAIN)
+      WMMAE_MFMA_ACC("s_nop 1\n\t", "f16");
+    else if constexpr (std::is_same<MT, _Float16>::value)
+      WMMAE_MFMA_ACC(WMMAE_MFMA_GUARD, "f16");
+    else if constexpr (RN_MAIN)
+      WMMAE_MFMA_ACC("s_nop 1\n\t", "bf16");
     else
-      asm volatile(WMMAE_MFMA_GUARD "v_mfma_f32_16x16x32_bf16 %0, %1, %2, %0"
-                   : "+a"(z)
-                   : "v"(x), "v"(y));
+      WMMAE_MFMA_ACC(WMMAE_MFMA_GUARD, "bf16");
+#undef WMMAE_MFMA_ACC
   };
   auto mfma = [](const ab_vec x, const ab_vec y, const f32x4 z) -> f32x4 {
     if constexpr (std::is_same<MT, _Float16>::value)
@@ -1174,14 +1323,6 @@ __global__ void __launch_bounds__(WGM *WGN * 64)
     const long long ld_out = to_tail ? BM : (to_partial ? M : ldc);
     const float a_out = to_partial ? 1.f : alpha;
     const float b_out = to_partial ? 0.f : beta;
-    const int vec_out =
-        to_tail      ? 1
-        : to_partial ? (M % 4 == 0)
-                     : (vec_store && (reinterpret_cast<uintptr_t>(Cb) & 15u) == 0);
-    const int row_base = (to_tail ? 0 : it.tm * BM) + wm * Cfg::WM +
-                         4 * static_cast<int>(lane >> 4);
-    const int col_base = (to_tail ? 0 : it.tn * BN) + wn * Cfg::WN +
-                         static_cast<int>(lane & 15u);
     // the value of tile (i, j) as it goes to memory, before beta
     const auto out_value = [&](const int i, const int j) {
       f32x4 v = acc_main[i][j];
@@ -1189,146 +1330,9 @@ __global__ void __launch_bounds__(WGM *WGN * 64)
         v = epilogue_fold(v, acc_err[i][j], inv_scale);
       return v * a_out;
     };
-    // (every destination is device memory: global-memory instructions, not
-    // generic ones, which would also count as LDS operations and make the
-    // compiler drain both memory counters before the next step's first
-    // dependent instruction)
-    typedef __attribute__((address_space(1))) float gfloat;
-    typedef __attribute__((address_space(1))) f32x4 gf32x4;
-    // one 16x16 tile: a lane stores rows 4q .. 4q+3 of its column, 16 bytes
-    const auto store_tile = [&](const int i, const int j) {
-      const int col = col_base + 16 * j;
-      const int row = row_base + 16 * i;
-      if (col >= N || row >= M)
-        return;
-      f32x4 v = out_value(i, j);
-      gfloat *const dst =
-          (gfloat *)(Cb + row + static_cast<long long>(col) * ld_out);
-      if (vec_out && row + 3 < M) {
-        if (b_out != 0.f)
-          v = epilogue_beta(v, b_out, *reinterpret_cast<const gf32x4 *>(dst));
-        *reinterpret_cast<gf32x4 *>(dst) = v;
-      } else {
-#pragma unroll
-        for (int x = 0; x < 4; x++) {
-          if (row + x < M) {
-            float o = v[x];
-            if (b_out != 0.f)
-              o = epilogue_beta(o, b_out, dst[x]);
-            dst[x] = o;
-          }
-        }
-      }
-    };
-    // Two tiles of one tile column (32 rows x 16 columns, all inside C): as
-    // above a store instruction would write 64 bytes of every column.  The
-    // lanes of neighbouring columns swap one tile's values instead, so that
-    // eight lanes cover 32 consecutive rows of one column: an instruction
-    // writes whole 128-byte lines, first of the even columns, then of the odd.
-    // Forced packed path, same box: 1024^2 x 128 x 256 entries 0.458 -> 0.434
-    // ms, 2048^2 x 256 x 16 0.152 -> 0.145, one term 0.336 -> 0.314, 4096^3
-    // 0.322 -> 0.318.  The kernel that splits the fp32 operands itself has no
-    // register to spare: with the choice made per pair of tiles, as here, the
-    // compiler keeps the accumulators' values in sight of three store paths
-    // at once, and two more of its K loop's values went to scratch (c5b 1.45
-    // -> 1.60 ms).  It decides once per item instead (below): the wave's whole
-    // piece inside C -> every pair by the swap, else the plain loop; that
-    // costs no scratch at all, and 1024 entries of 256^3 go from 0.175 to
-    // 0.166 ms, 1024^2 x 128 x 256 entries from 0.389 to 0.355.  Not in the
-    // round-to-nearest variants (their fragments then come back from AGPR
-    // copies right in front of the MFMAs that read them, see
-    // wmma_extension_amd/isa_check.py).
-    constexpr bool WHOLE_LINES = !DIRECT && !RN_MAIN && MT_ % 2 == 0;
-    const int odd = static_cast<int>(lane & 1u);
-    const int blk_row0 = (to_tail ? 0 : it.tm * BM) + wm * Cfg::WM;
-    const int blk_col0 = (to_tail ? 0 : it.tn * BN) + wn * Cfg::WN;
-    const auto store_tile_pair = [&](const int i, const int j) {
-      const f32x4 v0 = out_value(i, j), v1 = out_value(i + 1, j);
-      f32x4 d1, d2;
-#pragma unroll
-      for (int x = 0; x < 4; x++) {
-        // (through a function taking the element by value: __builtin_bit_cast
-        // applied to `v0[x]` directly read element 0 for every x)
-        const float n0 = neighbour_lane(v0[x]), n1 = neighbour_lane(v1[x]);
-        d1[x] = odd ? n1 : v0[x]; // even column: own rows | neighbour's next 16
-        d2[x] = odd ? v1[x] : n0; // odd column
-      }
-      const int row = row_base + 16 * (i + odd);
-      const int col = col_base + 16 * j;
-      gfloat *const dst1 =
-          (gfloat *)(Cb + row + static_cast<long long>(col & ~1) * ld_out);
-      gfloat *const dst2 =
-          (gfloat *)(Cb + row + static_cast<long long>(col | 1) * ld_out);
-      if (b_out != 0.f) {
-        d1 = epilogue_beta(d1, b_out, *reinterpret_cast<const gf32x4 *>(dst1));
-        d2 = epilogue_beta(d2, b_out, *reinterpret_cast<const gf32x4 *>(dst2));
-      }
-      *reinterpret_cast<gf32x4 *>(dst1) = d1;
-      *reinterpret_cast<gf32x4 *>(dst2) = d2;
-    };
-    if constexpr (DIRECT && !RN_MAIN && MT_ % 2 == 0) {
-      // the wave's whole piece inside C: every pair by the swap, no other
-      // path in sight of the accumulators (one decision per item)
-      if (vec_out && blk_row0 + Cfg::WM <= M && blk_col0 + Cfg::WN <= N) {
-#pragma unroll
-        for (int j = 0; j < NT_; j++)
-#pragma unroll
-          for (int i = 0; i < MT_; i += 2)
-            store_tile_pair(i, j);
-        return;
-      }
-    }
-#pragma unroll
-    for (int j = 0; j < NT_; j++) {
-      const bool cols_inside = blk_col0 + 16 * j + 16 <= N;
-      if constexpr (WHOLE_LINES) {
-#pragma unroll
-        for (int i = 0; i < MT_; i += 2) {
-          // (wave-uniform: both lanes of a swap take the same branch)
-          if (vec_out && cols_inside && blk_row0 + 16 * i + 32 <= M) {
-            store_tile_pair(i, j);
-          } else {
-            store_tile(i, j);
-            store_tile(i + 1, j);
-          }
-        }
-      } else {
-        // (the loop as one piece, with the compiler's own contraction of
-        // a * x + b * y, which comes out in the helpers' form: the kernel that
-        // splits its own operands has no register to spare, and through
-        // store_tile one more of its K loop's values went to scratch)
-        const int col = col_base + 16 * j;
-        if (col >= N)
-          continue;
-#pragma unroll
-        for (int i = 0; i < MT_; i++) {
-          const int row = row_base + 16 * i;
-          if (row >= M)
-            continue;
-          f32x4 v = acc_main[i][j];
-          if constexpr (TERMS >= 2)
-            v += acc_err[i][j] * inv_scale;
-          v *= a_out;
-          gfloat *const dst =
-              (gfloat *)(Cb + row + static_cast<long long>(col) * ld_out);
-          if (vec_out && row + 3 < M) {
-            if (b_out != 0.f)
-              v += b_out * *reinterpret_cast<const gf32x4 *>(dst);
-            *reinterpret_cast<gf32x4 *>(dst) = v;
-          } else {
-#pragma unroll
-            for (int x = 0; x < 4; x++) {
-              if (row + x < M) {
-                float o = v[x];
-                if (b_out != 0.f)
-                  o += b_out * dst[x];
-                dst[x] = o;
-              }
-            }
-          }
-        }
-      }
-    }
+    store_piece<MT_, NT_, MT_ % 2 == 0, (MT_ * NT_ <= 16 ? MT_ * NT_ : MT_)>(
+        out_value, Cb, ld_out, (to_tail ? 0 : it.tm * BM) + wm * Cfg::WM,
+        (to_tail ? 0 : it.tn * BN) + wn * Cfg::WN, M, N, b_out, lane);
   };
 
   // DIRECT, launches bound by their bytes (batches of small matrices with few
