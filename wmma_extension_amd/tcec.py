@@ -32,12 +32,21 @@ TYPE_HALF, TYPE_BF16, TYPE_TF32 = 0, 1, 2
 USE_A, USE_B, USE_ACC = 0, 1, 2
 
 
+# The current stream's handle without the torch.cuda.Stream object around it: building that object
+# took 2.7 of the 10.3 us that a call of sgemm on a 64^3 product took to issue.
+_raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)
+_raw_device = getattr(torch._C, "_cuda_getDevice", None)
+
+
 def _stream():
-    return ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
+    """hipStream_t of the current device's current stream (0: the default stream)."""
+    if _raw_stream is None or _raw_device is None or not torch.cuda.is_initialized():
+        return torch.cuda.current_stream().cuda_stream
+    return _raw_stream(_raw_device())
 
 
 def _ptr(t):
-    return ctypes.c_void_p(t.data_ptr()) if t is not None else ctypes.c_void_p(0)
+    return t.data_ptr() if t is not None else None
 
 
 def _f(v):
@@ -55,7 +64,11 @@ def _room(t):
     return t.untyped_storage().nbytes() - t.storage_offset() * t.element_size()
 
 
-def _check_matrix(name, t, rows, cols, ld, batch=1, stride=0, device=None):
+def _bytes(t):
+    return t.numel() * t.element_size() if t is not None else 0
+
+
+def _check_matrix(name, t, rows, cols, ld, batch=1, stride=0, like=None):
     """A column-major rows x cols fp32 matrix (leading dimension ld, `batch` of them `stride`
     apart) must lie inside the tensor's storage: the kernels take raw pointers, so a wrong dtype
     or a short tensor would read or write out of bounds on the GPU."""
@@ -63,24 +76,24 @@ def _check_matrix(name, t, rows, cols, ld, batch=1, stride=0, device=None):
         return
     if t.dtype != torch.float32:
         raise ValueError(f"{name}: float32 tensor required, got {t.dtype}")
-    if device is not None and t.device != device:
-        raise ValueError(f"{name}: on {t.device}, expected {device}")
+    if like is not None and t is not like and t.get_device() != like.get_device():
+        raise ValueError(f"{name}: on {t.device}, expected {like.device}")
     if rows <= 0 or cols <= 0 or batch <= 0:
         return
     if stride < 0:
         raise ValueError(f"{name}: negative batch stride")
-    need = ((batch - 1) * stride + (cols - 1) * ld + rows) * 4
-    if ld >= rows and _room(t) < need:
-        raise ValueError(f"{name}: needs {need} bytes from its first element, tensor has {_room(t)}")
+    need = (batch - 1) * stride + (cols - 1) * ld + rows
+    # (a contiguous tensor with that many elements has them all; asking its storage takes longer)
+    if ld >= rows and not (t.numel() >= need and t.is_contiguous()) and _room(t) < 4 * need:
+        raise ValueError(f"{name}: needs {4 * need} bytes from its first element, tensor has {_room(t)}")
 
 
 def _check_gemm_operands(transa, transb, m, n, k, A, lda, B, ldb, C, ldc, batch=1,
                          stride_a=0, stride_b=0, stride_c=0):
-    dev = C.device if C is not None else None
     ta, tb = transa in "Nn", transb in "Nn"
-    _check_matrix("A", A, m if ta else k, k if ta else m, lda, batch, stride_a, dev)
-    _check_matrix("B", B, k if tb else n, n if tb else k, ldb, batch, stride_b, dev)
-    _check_matrix("C", C, m, n, ldc, batch, stride_c, dev)
+    _check_matrix("A", A, m if ta else k, k if ta else m, lda, batch, stride_a, C)
+    _check_matrix("B", B, k if tb else n, n if tb else k, ldb, batch, stride_b, C)
+    _check_matrix("C", C, m, n, ldc, batch, stride_c)
 
 
 def _check_bytes(name, t, need, device=None):
@@ -88,7 +101,7 @@ def _check_bytes(name, t, need, device=None):
         return
     if device is not None and t.device != device:
         raise ValueError(f"{name}: on {t.device}, expected {device}")
-    if _room(t) < need:
+    if not (t.numel() * t.element_size() >= need and t.is_contiguous()) and _room(t) < need:
         raise ValueError(f"{name}: needs {need} bytes, tensor has {_room(t)}")
 
 
@@ -185,7 +198,7 @@ def sgemm(transa, transb, m, n, k, alpha, A, lda, B, ldb, beta, C, ldc,
     """C = alpha*op(A)*op(B) + beta*C, column-major BLAS convention."""
     _need_cuda(A, B, C, workspace)
     _check_gemm_operands(transa, transb, m, n, k, A, lda, B, ldb, C, ldc)
-    ws_bytes = workspace.numel() * workspace.element_size() if workspace is not None else 0
+    ws_bytes = _bytes(workspace)
     st = _lib.lib().wmmae_tcec_sgemm(transa.encode(), transb.encode(), m, n, k, _f(alpha),
                                      _ptr(A), lda, _ptr(B), ldb, _f(beta), _ptr(C), ldc,
                                      int(policy), flags, _ptr(workspace), ws_bytes, _stream())
@@ -212,7 +225,7 @@ def sgemm_strided_batched(transa, transb, m, n, k, alpha, A, lda, stride_a, B, l
     _need_cuda(A, B, C, workspace)
     _check_gemm_operands(transa, transb, m, n, k, A, lda, B, ldb, C, ldc, batch,
                          stride_a, stride_b, stride_c)
-    ws_bytes = workspace.numel() * workspace.element_size() if workspace is not None else 0
+    ws_bytes = _bytes(workspace)
     st = _lib.lib().wmmae_tcec_sgemm_strided_batched(
         transa.encode(), transb.encode(), m, n, k, _f(alpha), _ptr(A), lda, stride_a,
         _ptr(B), ldb, stride_b, _f(beta), _ptr(C), ldc, stride_c, batch, int(policy), flags,
@@ -228,7 +241,7 @@ def sgemm_batched(transa, transb, m, n, k, alpha, A_array, lda, B_array, ldb, be
     for name, arr in (("A_array", A_array), ("B_array", B_array), ("C_array", C_array)):
         if arr is not None and (arr.dtype != torch.int64 or arr.numel() < batch):
             raise ValueError(f"{name}: int64 tensor of at least {batch} device pointers required")
-    ws_bytes = workspace.numel() * workspace.element_size() if workspace is not None else 0
+    ws_bytes = _bytes(workspace)
     st = _lib.lib().wmmae_tcec_sgemm_batched(
         transa.encode(), transb.encode(), m, n, k, _f(alpha), _ptr(A_array), lda, _ptr(B_array), ldb,
         _f(beta), _ptr(C_array), ldc, batch, int(policy), flags, _ptr(workspace), ws_bytes, _stream())
@@ -263,7 +276,7 @@ def gemm_packed(policy, m, n, k, alpha, packed_a, packed_b, beta, C, ldc, batch=
     if k > 0 and m > 0 and n > 0 and batch > 0:
         _check_bytes("packed_a", packed_a, pack_bytes(m, k, batch, policy), C.device)
         _check_bytes("packed_b", packed_b, pack_bytes(n, k, batch, policy), C.device)
-    ws_bytes = workspace.numel() * workspace.element_size() if workspace is not None else 0
+    ws_bytes = _bytes(workspace)
     st = _lib.lib().wmmae_tcec_gemm_packed(int(policy), m, n, k, _f(alpha), _ptr(packed_a),
                                            _ptr(packed_b), _f(beta), _ptr(C), ldc, stride_c,
                                            batch, flags, _ptr(workspace), ws_bytes, _stream())
@@ -278,7 +291,7 @@ def matmul_tn(A, B, policy=Policy.F16_EC, flags=0, workspace=None, out=None):
     n, k2 = B.shape
     assert k == k2 and A.is_contiguous() and B.is_contiguous()
     if out is None:
-        out = torch.empty((n, m), dtype=torch.float32, device=A.device)
+        out = A.new_empty((n, m), dtype=torch.float32)
     elif tuple(out.shape) != (n, m) or not out.is_contiguous():
         raise ValueError(f"out: contiguous ({n}, {m}) tensor required, got {tuple(out.shape)}")
     sgemm("T", "N", m, n, k, 1.0, A, k, B, k, 0.0, out, m, policy, flags, workspace)
