@@ -100,9 +100,8 @@ int wmmae_query(int what, long long *out);
  * `stream`; measured at 3 to 9 us a call on MI355X, which a product of 20 us
  * feels - keep a workspace across calls where calls are small).  Products
  * whose operand elements are used by few tiles (small m and n, or a short k;
- * an estimate of both paths' times decides; no K slices; operands readable
- * 16 bytes at a time) are split inside the GEMM
- * kernel (as the reference's bgemm_kernel splits at fragment load,
+ * an estimate of the paths' times decides; no K slices) are split inside the
+ * GEMM kernel (as the reference's bgemm_kernel splits at fragment load,
  * batch_gemm.cu:196-386): they use no workspace, allocate nothing and ignore
  * the workspace arguments.  Batches of medium-sized matrices and K-heavy
  * products with k contiguous in both operands run the packed path's GEMM
@@ -129,13 +128,10 @@ int wmmae_tcec_sgemm_workspace_bytes(int m, int n, int k, int batch, int policy,
  * 2 packed operands and K slices (when the workspace has room for them),
  * 3 the packed path's GEMM kernel loading and splitting the fp32 operands
  * itself (no packed operands), 4 the same with K slices.  3 and 4 assume
- * k contiguous in both operands ('T','N') and need k >= 4; other layouts
- * take 1 and 2.
- * The answer is for op(A) = 'T', op(B) = 'N' with tight leading dimensions
- * (lda = ldb = k) and 16-byte aligned bases: with k a multiple of 4 the
- * single kernel reads such operands 16 bytes at a time, which is what the
- * time estimates behind the choice assume; other leading dimensions or bases
- * can move a product from path 0 to another one. */
+ * k contiguous in both operands ('T','N') and need k >= 4.
+ * The answer is for op(A) = 'T', op(B) = 'N', whatever the leading dimensions
+ * and bases.  Other layouts take 0, 1 or 2, and 0 more often: the single kernel
+ * runs them at the same speed, the split pass of 1 and 2 does not. */
 int wmmae_tcec_sgemm_path(int m, int n, int k, int batch, int policy, int flags,
                           int *path);
 

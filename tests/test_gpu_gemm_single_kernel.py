@@ -1,0 +1,68 @@
+"""The single-launch kernel at its edges: every way it reads an operand (k contiguous, rows
+contiguous, strides of 2^24 floats, k < 4), last stages of every length, row counts that end inside
+a load, one tile to several per workgroup with both tile sizes, with NaN around the operands.
+Expected: the bits of pack + GEMM on packed operands without K slices, whose own bits are pinned
+against the matrix core's model elsewhere."""
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+PACKED, FUSED = 2, 4
+
+
+def _operand(g, dev, batch, rows, k, k_contiguous, pad, off):
+    """(view of rows x k values inside NaN, leading dimension)"""
+    outer, inner = (rows, k) if k_contiguous else (k, rows)
+    ld = inner + pad
+    room = torch.full((off + batch * outer * ld + 8,), float("nan"), device=dev)
+    X = room[off:off + batch * outer * ld].view(batch, outer, ld)
+    X[:, :, :inner] = (torch.rand((batch, outer, inner), generator=g) * 2 - 1).to(dev)
+    return X, ld
+
+
+def _same_bits(tc, dev, ta, tb, m, n, k, batch, policy, rn, pad, off, beta):
+    g = torch.Generator(device="cpu").manual_seed(m + 1000 * n + 7 * k + policy)
+    A, lda = _operand(g, dev, batch, m, k, ta == "T", pad, off)
+    B, ldb = _operand(g, dev, batch, n, k, tb == "N", pad, off)
+    C0 = (torch.rand((batch, n, m), generator=g) * 2 - 1).to(dev)
+    out = []
+    for flag in (PACKED, FUSED):
+        C = C0.clone()
+        with tc.forced_k_slices(1):
+            # (no workspace of the caller: no K slices for the tiles of a last round either)
+            tc.sgemm_strided_batched(ta, tb, m, n, k, 1.25, A, lda, A.stride(0), B, ldb, B.stride(0), beta, C, m,
+                                     m * n, batch, policy, flag | rn, None)
+        out.append(C)
+    assert torch.isfinite(out[0]).all()
+    assert torch.equal(out[0].view(torch.int32), out[1].view(torch.int32)), (m, n, k, (out[0] - out[1]).abs().max())
+
+
+@pytest.mark.parametrize("ta,tb", [("T", "N"), ("N", "N"), ("N", "T"), ("T", "T")])
+@pytest.mark.parametrize("policy", [0, 1, 2, 3, 4])
+def test_same_bits_as_packed_operands(tc, dev, ta, tb, policy):
+    # k: 1 .. 3 (element by element), ends of a stage, ends of the ring of stages
+    for k in (1, 2, 3, 4, 5, 30, 31, 32, 33, 34, 35, 63, 64, 65, 96, 127, 131, 190, 225, 260):
+        _same_bits(tc, dev, ta, tb, 65 + k % 3, 130 - k % 5, k, 1, policy, 0, k % 4, k % 4, 0.0)
+    # row counts around tiles, 64-row loads and row blocks
+    for m, n in ((1, 1), (7, 66), (15, 17), (63, 129), (64, 64), (127, 257), (200, 8)):
+        _same_bits(tc, dev, ta, tb, m, n, 77, 2, policy, 0, 3, 1, -0.5)
+    # several tiles per workgroup: 64x64 and 128x128, shared list and entries owned by an XCD,
+    # odd and even stage counts, one stage per tile
+    for m, n, k, batch in ((60, 50, 37, 1100), (60, 50, 64, 1030), (130, 100, 29, 700), (1500, 1300, 131, 3),
+                           (1500, 1300, 64, 3), (900, 1000, 20, 9)):
+        _same_bits(tc, dev, ta, tb, m, n, k, batch, policy, 0, 0, 0, 0.0)
+
+
+@pytest.mark.parametrize("policy", [0, 2])
+def test_leading_product_outside_the_matrix_core(tc, dev, policy):
+    for ta, tb, m, n, k, batch in (("T", "N", 70, 130, 95, 1), ("N", "T", 300, 200, 161, 9),
+                                   ("N", "N", 1500, 1300, 100, 3)):
+        _same_bits(tc, dev, ta, tb, m, n, k, batch, policy, tc.FLAG_RN_MAIN, 1, 2, 0.5)
+
+
+def test_strides_beyond_the_offsets_of_a_load(tc, dev):
+    """Leading dimensions of 2^24 floats and more (a lane's offset from the wave's address then no
+    longer fits its 32 bits)."""
+    for ta, tb, m, n, k in (("T", "N", 5, 40, 36), ("N", "T", 40, 5, 6), ("N", "N", 33, 3, 5)):
+        _same_bits(tc, dev, ta, tb, m, n, k, 1, 0, 0, (1 << 24) + 1, 0, 0.0)

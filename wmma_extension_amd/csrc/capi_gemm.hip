@@ -25,25 +25,23 @@ __global__ void __launch_bounds__(256)
   *p = beta == 0.f ? 0.f : beta * *p;
 }
 
-// Which of the three paths?  The single ("fused") kernel moves only the fp32
-// operands and C but needs about twice as long per 128x128x32 tile step and
-// converts every element once per wave that uses it; the packed path first
-// writes and re-reads the split operands, which pays off when every operand
-// element is used by many tiles; the "direct" path is the packed path's GEMM
-// kernel (256x128 tiles) loading the fp32 operands itself and splitting them
-// on their way into LDS - no packed copy and no split pass, at 1.2 to 1.9
-// times the time per k stage; it wins where an operand element is used by
-// few tiles (batches of small and medium matrices, K-heavy products) and
-// needs k contiguous in both operands, k at least 4 and at most two terms;
-// same bits as the packed path.  All three times are estimated with the same
-// shape, a launch cost plus rounds of tiles over the compute units times (k
-// stages * time per stage + time per tile), bounded below by the bytes moved;
-// products that are cut into K slices take the slice planner's time, rescaled.
-// The constants and what they were fitted to: namespace fit.
-// fused_vec: the fused kernel can request 16 bytes per lane from both
-// operands (k contiguous, k and the strides multiples of 4, aligned bases).
-// Without that it issues four times as many requests (3.5 times the time per
-// stage), so such products take another path unless k is very short.
+// Which of the three paths?  The single ("fused") kernel reads the fp32 operands
+// once per 64 or 128 rows or columns of C and takes one launch, in any layout;
+// the packed path first writes and re-reads the split operands, which pays off
+// when every operand element is used by many tiles, and can cut K where there
+// are few; the "direct" path is the packed path's GEMM kernel (256x128 tiles)
+// loading the fp32 operands itself and splitting them on their way into LDS - no
+// packed copy and no split pass, at 1.2 to 1.9 times the time per k stage; it
+// wins where an operand element is used by few tiles (batches of medium
+// matrices, K-heavy products) and needs k contiguous in both operands, k at
+// least 4 and at most two terms; same bits as the packed path.  All three times
+// are estimated with the same shape, a launch cost plus rounds of tiles over the
+// compute units times (k stages * time per stage + time per tile), bounded below
+// by the bytes moved; products that are cut into K slices take the slice
+// planner's time, rescaled.  The constants and what they were fitted to:
+// namespace fit.
+//   fused_ok : the single kernel is considered (fused_considered)
+//   rows     : an operand does not have k contiguous
 enum class Path { Fused, Packed, Direct };
 // (see PathRates::busy)
 inline double busy_factor(const fit::PathRates &r, const long long tiles) {
@@ -83,10 +81,11 @@ struct PathEstimates {
 };
 inline PathEstimates estimate_paths(const int m, const int n, const int k,
                                     const int batch, const int terms,
-                                    const bool fused_vec, const bool direct_ok) {
+                                    const bool fused_ok, const bool rows,
+                                    const bool direct_ok) {
   constexpr double kNever = std::numeric_limits<double>::infinity();
   PathEstimates e{kNever, kNever, kNever};
-  const fit::PathRates &f = fit::kFused[terms - 1], &p = fit::kPacked[terms - 1];
+  const fit::PathRates &p = fit::kPacked[terms - 1];
   const long long cus = device_cus();
   const int kti = static_cast<int>(ceil_div(k, 32));
   const double kt = static_cast<double>(kti);
@@ -96,28 +95,18 @@ inline PathEstimates estimate_paths(const int m, const int n, const int k,
   const long long tiles128 = ceil_div(m, 128) * ceil_div(n, 128) * batch;
   const long long tiles256 = ceil_div(m, 256) * ceil_div(n, 128) * batch;
 
-  // fused kernel: 128x128 tiles, or 64x64 ones (a third of the stage time,
-  // half of the per-tile time) under fused_by_size's rule
-  if (fused_vec || k <= 96) {
-    const bool small = fused_small_tiles(m, n, batch);
-    const long long f_tiles = small ? tiles64 : tiles128;
-    const double f_rounds = static_cast<double>(ceil_div(f_tiles, cus));
-    e.fused =
-        f.launch +
-        std::max(f_rounds * (kt * f.stage * busy_factor(f, f_tiles) *
-                                 (fused_vec ? 1.0 : fit::kFusedNarrowRequests) *
-                                 (small ? fit::kFusedSmallStage : 1.0) +
-                             f.tile * (small ? fit::kFusedSmallTile : 1.0)),
-                 (c_bytes + 4.0 * ab) / f.bytes_per_s);
-  }
+  if (fused_ok)
+    e.fused = (rows || batch >= fit::kFusedTnMarginBatch
+                   ? 1.0
+                   : fit::kFusedTnMargin[terms - 1]) *
+              std::min(fused_time(terms, m, n, k, batch, true, rows),
+                       fused_time(terms, m, n, k, batch, false, rows));
   const double split_pass = (4.0 + 2.0 * terms) * ab / p.split_bytes_per_s;
   const int splits = choose_splits(terms, m, n, k, batch);
   if (splits != 1) {
     // K slices: the split pass and the packed kernel's slices against the
     // slower stages of the direct kernel (cut into the slices that suit its own
     // tile)
-    e.fused = e.fused * fit::kSlicedFused[0][terms - 1] +
-              fit::kSlicedFused[1][terms - 1];
     e.packed = (p.launch + split_pass +
                 split_time(terms, m, n, batch, kti, splits)) *
                    fit::kSlicedPacked[0][terms - 1] +
@@ -169,7 +158,8 @@ inline PathEstimates estimate_paths(const int m, const int n, const int k,
 }
 inline Path choose_path(const int m, const int n, const int k, const int batch,
                         const int flags, const int terms, const int policy,
-                        const bool fused_vec, const bool direct_ok) {
+                        const bool fused_ok, const bool rows,
+                        const bool direct_ok) {
   // (the round-to-nearest flag with a policy that has no such variant is
   // turned down by the packed path's dispatch)
   const bool rn_unsupported =
@@ -177,7 +167,7 @@ inline Path choose_path(const int m, const int n, const int k, const int batch,
       policy != WMMAE_POLICY_BF16X3_EC;
   if (k <= 0 || rn_unsupported)
     return Path::Packed;
-  PathEstimates e = estimate_paths(m, n, k, batch, terms, fused_vec, direct_ok);
+  PathEstimates e = estimate_paths(m, n, k, batch, terms, fused_ok, rows, direct_ok);
   e.fused = std::max(e.fused, fit::kCallFloor[0]);
   e.packed = std::max(e.packed, fit::kCallFloor[1]);
   e.direct = std::max(e.direct, fit::kCallFloor[2]);
@@ -191,12 +181,24 @@ inline Path choose_path(const int m, const int n, const int k, const int batch,
     best = Path::Direct;
   return best;
 }
+// ('T','N') products with k % 4 != 0 and more than three stages stay with the
+// other paths, as the path query has always answered.
+inline bool fused_considered(const int k) { return k % 4 == 0 || k <= 96; }
 // what the direct kernel needs of a product (the operands' k strides are 1)
 inline bool direct_possible(const int k, const int terms, const int flags,
                             const long long a_rs, const long long b_rs) {
   return k >= 4 && terms <= 2 &&
          (flags & WMMAE_FLAG_RN_MAIN) == 0 && a_rs < (1 << 24) &&
          b_rs < (1 << 24);
+}
+
+// how the single kernel reads an operand (see its head comment)
+inline int fused_source(const long long rs, const long long ks, const int k) {
+  if (ks == 1 && k >= 4 && rs < (1 << 24))
+    return wmmae_gemm::kFusedKRows;
+  if (rs == 1 && ks < (1 << 24))
+    return wmmae_gemm::kFusedRRows;
+  return wmmae_gemm::kFusedAny;
 }
 
 inline bool is_n(const char t) { return t == 'N' || t == 'n'; }
@@ -427,22 +429,14 @@ int sgemm_impl(const char transa, const char transb, const int m, const int n,
       ldc < m)
     return WMMAE_STATUS_BAD_LEADING_DIM;
 
-  const auto aligned16 = [](const void *ptr) {
-    return reinterpret_cast<uintptr_t>(ptr) % 16 == 0;
-  };
-  // 16-byte requests of the fused kernel (entries of pointer arrays are
-  // checked by the kernel itself)
   const long long a_rs = is_n(transa) ? 1 : lda, a_ks = is_n(transa) ? lda : 1;
   const long long b_rs = is_n(transb) ? ldb : 1, b_ks = is_n(transb) ? 1 : ldb;
-  const bool vec_a = a_ks == 1 && k % 4 == 0 && a_rs % 4 == 0 &&
-                     (a_ptrs != nullptr || (aligned16(A) && stride_a % 4 == 0));
-  const bool vec_b = b_ks == 1 && k % 4 == 0 && b_rs % 4 == 0 &&
-                     (b_ptrs != nullptr || (aligned16(B) && stride_b % 4 == 0));
+  const bool rows = a_ks != 1 || b_ks != 1;
   const bool direct_ok = a_ks == 1 && b_ks == 1 &&
                          direct_possible(k, p.terms, flags, a_rs, b_rs);
   const int rn = flags & WMMAE_FLAG_RN_MAIN;
-  Path path = choose_path(m, n, k, batch, rn, p.terms, policy, vec_a && vec_b,
-                          direct_ok);
+  Path path = choose_path(m, n, k, batch, rn, p.terms, policy,
+                          rows || fused_considered(k), rows, direct_ok);
   if ((flags & WMMAE_FLAG_PATH_DIRECT) != 0) {
     if (!direct_ok)
       return WMMAE_STATUS_NOT_SUPPORTED;
@@ -523,14 +517,14 @@ int sgemm_impl(const char transa, const char transb, const int m, const int n,
     q.N = n;
     q.K = k;
     q.batch = batch;
-    q.vec_a = vec_a;
-    q.vec_b = vec_b;
-    q.rn_main = (flags & WMMAE_FLAG_RN_MAIN) != 0;
+    q.a_source = fused_source(a_rs, a_ks, k);
+    q.b_source = fused_source(b_rs, b_ks, k);
     q.alpha = *alpha;
     q.beta = *beta;
     q.inv_scale = p.inv_scale;
     f.stream = static_cast<hipStream_t>(stream);
-    return policy_kernels(policy)->fused(f);
+    const PolicyKernels *const kernels = policy_kernels(policy);
+    return rn != 0 ? kernels->fused_rn(f) : kernels->fused(f);
   }
 
   size_t bytes_a = 0, bytes_b = 0, bytes_c = 0;
@@ -668,7 +662,8 @@ int wmmae_tcec_sgemm_path(const int m, const int n, const int k,
     return WMMAE_STATUS_INVALID_VALUE;
   const bool any = m > 0 && n > 0 && k > 0 && batch > 0;
   const bool slices = any && choose_splits(p.terms, m, n, k, batch) > 1;
-  switch (choose_path(m, n, k, batch, flags, p.terms, policy, k % 4 == 0,
+  switch (choose_path(m, n, k, batch, flags, p.terms, policy,
+                      fused_considered(k), false,
                       direct_possible(k, p.terms, flags, 1, 1))) {
   case Path::Fused:
     *path = 0;
@@ -690,7 +685,8 @@ int wmmae_tcec_path_estimates(const int m, const int n, const int k,
     return WMMAE_STATUS_NULL_POINTER;
   if (m <= 0 || n <= 0 || k <= 0 || batch <= 0 || !policy_info(policy, p))
     return WMMAE_STATUS_INVALID_VALUE;
-  const PathEstimates e = estimate_paths(m, n, k, batch, p.terms, k % 4 == 0,
+  const PathEstimates e = estimate_paths(m, n, k, batch, p.terms,
+                                         fused_considered(k), false,
                                          direct_possible(k, p.terms, 0, 1, 1));
   seconds[0] = e.fused;
   seconds[1] = e.packed;
@@ -730,7 +726,7 @@ int wmmae_tcec_sgemm_k_slices(const int m, const int n, const int k,
     return WMMAE_STATUS_SUCCESS;
   const bool direct_ok = direct_possible(k, p.terms, flags, 1, 1);
   Path path = choose_path(m, n, k, batch, flags & WMMAE_FLAG_RN_MAIN, p.terms,
-                          policy, k % 4 == 0, direct_ok);
+                          policy, fused_considered(k), false, direct_ok);
   if ((flags & WMMAE_FLAG_PATH_DIRECT) != 0) {
     if (!direct_ok)
       return WMMAE_STATUS_NOT_SUPPORTED;

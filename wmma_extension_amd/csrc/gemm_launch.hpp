@@ -270,44 +270,54 @@ template <class MT, int TERMS> int per_cu_by_shape(const int shape) {
     return workgroups_per_cu<MT, TERMS, 64, 64, 2, 2, false>();
   }
 }
-template <class T, int TERMS, int BM, int BN> int launch_fused(FusedArgs f) {
-  using Cfg = wmmae_gemm::FusedConfig<TERMS, BM, BN>;
-  auto kernel = wmmae_gemm::tcec_gemm_fused_kernel<T, TERMS, BM, BN>;
+template <class T, int TERMS, int BM, int BN, int CW, int PW, int DEPTH, bool RN,
+          bool STREAM>
+int launch_fused_grid(const FusedArgs &f, const long long grid) {
+  using Cfg = wmmae_gemm::FusedConfig<TERMS, BM, BN, CW, PW>;
+  auto kernel = wmmae_gemm::tcec_gemm_fused_kernel<T, TERMS, BM, BN, CW, PW,
+                                                   DEPTH, RN, STREAM>;
   static std::atomic<unsigned long long> lds_allowed{0};
   WMMAE_HIP_TRY(allow_dynamic_lds(reinterpret_cast<const void *>(kernel),
                                   Cfg::LDS_BYTES, lds_allowed));
-  wmmae_gemm::FusedParams &p = f.p;
-  p.tiles_m = static_cast<int>(ceil_div(p.M, BM));
-  p.tiles_per_batch = p.tiles_m * static_cast<int>(ceil_div(p.N, BN));
-  // one persistent workgroup per compute unit at most; with 8 or more batch
-  // entries an XCD (block index mod 8) owns whole entries
-  const int per_xcd_max = device_cus() / 8 > 0 ? device_cus() / 8 : 1;
-  // (not when the XCD that owns one entry more than the others would need
-  // over 15 % more rounds of tiles than an even spread)
-  const long long all_tiles =
-      static_cast<long long>(p.batch) * p.tiles_per_batch;
-  p.grouped =
-      device_xcds() == kKernelXcds && p.batch >= 8 &&
-      ceil_div(ceil_div(p.batch, 8) * p.tiles_per_batch, per_xcd_max) * 100 <=
-          ceil_div(all_tiles, 8ll * per_xcd_max) * 115;
-  long long per_xcd = p.grouped
-                          ? ceil_div(p.batch, 8) * p.tiles_per_batch
-                          : ceil_div(static_cast<long long>(p.batch) *
-                                         p.tiles_per_batch,
-                                     8);
-  if (per_xcd > per_xcd_max)
-    per_xcd = per_xcd_max;
-  const int grid = 8 * static_cast<int>(per_xcd);
-  hipLaunchKernelGGL(kernel, dim3(grid), dim3(Cfg::NTHREADS), Cfg::LDS_BYTES,
-                     f.stream,
-                     p);
+  hipLaunchKernelGGL(kernel, dim3(static_cast<unsigned>(grid)),
+                     dim3(Cfg::NTHREADS), Cfg::LDS_BYTES, f.stream, f.p);
   return launch_status();
 }
 
-template <class T, int TERMS> int fused_by_size(const FusedArgs &f) {
-  if (fused_small_tiles(f.p.M, f.p.N, f.p.batch))
-    return launch_fused<T, TERMS, 64, 64>(f);
-  return launch_fused<T, TERMS, 128, 128>(f);
+template <class T, int TERMS, int BM, int BN, int CW, int PW, int DEPTH, bool RN>
+int launch_fused(FusedArgs f) {
+  wmmae_gemm::FusedParams &p = f.p;
+  p.tiles_m = static_cast<int>(ceil_div(p.M, BM));
+  p.tiles_n = static_cast<int>(ceil_div(p.N, BN));
+  const long long tpb = static_cast<long long>(p.tiles_m) * p.tiles_n;
+  const long long items = p.batch * tpb;
+  if (items >= (1ll << 30)) // the kernel counts tiles in 32 bits
+    return WMMAE_STATUS_NOT_SUPPORTED;
+  // with 8 or more batch entries an XCD (block index mod 8) owns whole entries
+  // (not when the XCD that owns one entry more than the others would need over
+  // 15 % more rounds of tiles than an even spread)
+  const long long resident =
+      static_cast<long long>(device_cus()) * fit::fused_resident(BM);
+  const long long per_xcd = std::max(1ll, resident / 8);
+  p.grouped = device_xcds() == kKernelXcds && p.batch >= 8 &&
+              ceil_div(ceil_div(p.batch, 8) * tpb, per_xcd) * 100 <=
+                  ceil_div(items, 8 * per_xcd) * 115;
+  const long long spread = p.grouped ? 8 * ceil_div(p.batch, 8) * tpb : items;
+  // one workgroup per tile when all of them are resident together, else
+  // persistent workgroups
+  if (spread <= resident)
+    return launch_fused_grid<T, TERMS, BM, BN, CW, PW, DEPTH, RN, false>(f,
+                                                                         spread);
+  return launch_fused_grid<T, TERMS, BM, BN, CW, PW, DEPTH, RN, true>(
+      f, p.grouped ? 8 * per_xcd : resident);
+}
+
+template <class T, int TERMS, bool RN> int fused_by_size(const FusedArgs &f) {
+  if (fused_small_tiles(TERMS, f.p.M, f.p.N, f.p.K, f.p.batch,
+                        f.p.a_source != wmmae_gemm::kFusedKRows ||
+                            f.p.b_source != wmmae_gemm::kFusedKRows))
+    return launch_fused<T, TERMS, 64, 64, 4, 4, 4, RN>(f);
+  return launch_fused<T, TERMS, 128, 128, 8, 4, 2, RN>(f);
 }
 
 // The table of one policy: split tag T, MFMA element type MT, stored terms; RN:
@@ -318,9 +328,11 @@ constexpr PolicyKernels make_policy_kernels() {
   PolicyKernels k{};
   k.pack = launch_pack<T, TERMS>;
   k.gemm = gemm_by_size<MT, TERMS, false>;
-  if constexpr (RN)
+  if constexpr (RN) {
     k.gemm_rn = gemm_by_size<MT, TERMS, true>;
-  k.fused = fused_by_size<T, TERMS>;
+    k.fused_rn = fused_by_size<T, TERMS, true>;
+  }
+  k.fused = fused_by_size<T, TERMS, false>;
   k.per_cu = per_cu_by_shape<MT, TERMS>;
   return k;
 }

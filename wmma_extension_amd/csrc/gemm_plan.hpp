@@ -188,10 +188,6 @@ struct PathRates {
   // units, averaged over the rounds))
   double busy;
 };
-constexpr PathRates kFused[3] = {
-    {6.01e-6, 0.643e-6, 2.88e-6, 5.32e12, 0., 0.101},
-    {6.50e-6, 0.992e-6, 1.85e-6, 5.27e12, 0., 0.170},
-    {5.37e-6, 1.39e-6, 2.22e-6, 5.14e12, 0., 0.141}};
 constexpr PathRates kPacked[3] = {
     {8.35e-6, 0.131e-6, 3.07e-6, 3.65e12, 5.61e12, 0.359},
     {8.17e-6, 0.287e-6, 3.69e-6, 6.50e12, 5.57e12, 0.649},
@@ -217,8 +213,6 @@ constexpr double kDirectSliceRatio[2] = {1.5, 1.4};
 // planner's time (split_time, whose constants are fitted for choosing the slice
 // count) has to be scaled and shifted by to be the time of the whole call on
 // each path; same fit as above.  Rows: scale, shift in seconds; by terms.
-constexpr double kSlicedFused[2][3] = {{1.16, 1.08, 1.03},
-                                       {-3.73e-6, -2.84e-6, -2.89e-6}};
 constexpr double kSlicedPacked[2][3] = {{0.724, 0.954, 0.955},
                                         {-0.65e-6, -6.0e-6, -6.0e-6}};
 constexpr double kSlicedDirect[2][2] = {{0.759, 0.890}, {-6.0e-6, -6.0e-6}};
@@ -228,15 +222,43 @@ constexpr double kSlicedDirect[2][2] = {{0.759, 0.890}, {-6.0e-6, -6.0e-6}};
 // one launch for the single kernel and the direct kernel, two or three for
 // the packed path.  Order: single kernel, packed, direct.
 constexpr double kCallFloor[3] = {11.0e-6, 14.3e-6, 11.5e-6};
+// -- the single kernel (one launch, fp32 operands), by terms.  Its 64x64 tile
+//    runs alone on a compute unit (stage64, tile64) or as one of two (pair64,
+//    pair_tile64, for both), its 128x128 tile always alone; rows64 / rows128:
+//    factor on a stage when an operand does not have k contiguous; busy64 (for
+//    pairs) / busy128 as PathRates::busy.  Fit: 3000 random products (m, n =
+//    32 .. 4096, k = 32 .. 8192, 1 .. 1024 entries, three transpose
+//    combinations), each run with both tiles: 5 to 12 % rms, the tile chosen
+//    with them 0.03 to 0.3 % slower than the faster one on average; stage64 is
+//    that of operands that come from HBM (0.34, 0.40, 0.53 us; from L2 0.18,
+//    0.32, 0.47), which one workgroup of a compute unit cannot hide.  The launch
+//    is 0.8 us above the fit to those launches inside a graph, as the other
+//    paths' are.
+struct FusedRates {
+  double launch, stage64, tile64, pair64, pair_tile64, busy64, rows64;
+  double stage128, tile128, busy128, rows128, bytes_per_s;
+};
+constexpr FusedRates kFused[3] = {
+    {4.1e-6, 0.330e-6, 1.18e-6, 0.242e-6, 2.06e-6, 0.811, 1.232,
+     0.314e-6, 2.15e-6, 0.854, 1.114, 4.92e12},
+    {4.7e-6, 0.360e-6, 0.97e-6, 0.341e-6, 1.90e-6, 0.748, 1.185,
+     0.551e-6, 2.12e-6, 0.522, 1.157, 4.74e12},
+    {5.2e-6, 0.500e-6, 0.41e-6, 0.601e-6, 1.70e-6, 0.465, 1.101,
+     0.909e-6, 2.02e-6, 0.434, 1.084, 3.95e12}};
+// ('T','N') products of fewer than 16 entries take the single kernel only where
+// it is well ahead: its time counts this much there.  The path query answers for
+// exactly these, and callers size workspaces and K slices by its answers
+// (1160x1544x1056, two terms: packed operands, though the single kernel takes
+// 0.8 of the time).  Larger batches, and other layouts, which the query does not
+// speak for, go by the times alone.
+constexpr double kFusedTnMargin[3] = {1.25, 1.4, 1.25}; // by terms
+constexpr int kFusedTnMarginBatch = 16;
+// Its workgroups that are resident on a compute unit: 12 waves of up to 168
+// registers (128x128), twice 8 waves of up to 128.
+constexpr int fused_resident(const int bm) { return bm > 64 ? 1 : 2; }
 // k % 32 != 0: the kernel variant that reads a shorter last stage (1024^2 x 1000
 // against x 1024, batch 256: 301 against 336 TFLOPS, of which 2.4 % are the k)
 constexpr double kDirectTailStage = 1.47;
-// the single kernel's 64x64 tile against its 128x128 tile (1024^3: 41 -> 27 us)
-constexpr double kFusedSmallTileTime = 0.65; // whole tile, latency-bound sizes
-constexpr double kFusedSmallStage = 0.599, kFusedSmallTile = 0.467;
-// 4-byte instead of 16-byte requests: 114 random products with k % 4 != 0 ran
-// at 0.55 of the packed path's speed in the median
-constexpr double kFusedNarrowRequests = 3.50;
 } // namespace fit
 
 // XCDs (chiplets with an L2 of their own) behind the current device.  HIP does
@@ -393,17 +415,40 @@ struct FusedArgs {
   hipStream_t stream;
 };
 
-// 128x128 tiles, unless they leave compute units without work and 64x64 tiles
-// (four times as many workgroups; one takes 0.65 of a 128x128 tile's time at
-// these latency-bound sizes) finish sooner: 1024^3 went from 41 to 27 us.
-inline bool fused_small_tiles(const int m, const int n, const int batch) {
+// Time of a call of the single kernel with its 64x64 or 128x128 tiles.  `rows`:
+// an operand does not have k contiguous.
+inline double fused_time(const int terms, const int m, const int n, const int k,
+                         const int batch, const bool small, const bool rows) {
+  const fit::FusedRates &f = fit::kFused[terms - 1];
+  const double kt = static_cast<double>(ceil_div(k, 32));
   const long long cus = device_cus();
-  const long long tiles128 = ceil_div(m, 128) * ceil_div(n, 128) * batch;
-  const long long tiles64 = ceil_div(m, 64) * ceil_div(n, 64) * batch;
-  return (m <= 64 && n <= 64) ||
-         (tiles128 < cus && fit::kFusedSmallTileTime *
-                                    static_cast<double>(ceil_div(tiles64, cus)) <
-                                static_cast<double>(ceil_div(tiles128, cus)));
+  const int t = small ? 64 : 128;
+  const long long tiles = ceil_div(m, t) * ceil_div(n, t) * batch;
+  const long long rounds = ceil_div(tiles, cus);
+  const double full = static_cast<double>(tiles) /
+                      (static_cast<double>(rounds) * static_cast<double>(cus));
+  double time;
+  if (small) {
+    const double factor = rows ? f.rows64 : 1.0;
+    time = static_cast<double>(rounds / 2) *
+               (kt * f.pair64 * factor * (1.0 + f.busy64 * full) +
+                f.pair_tile64) +
+           static_cast<double>(rounds % 2) * (kt * f.stage64 * factor + f.tile64);
+  } else {
+    time = static_cast<double>(rounds) *
+           (kt * f.stage128 * (rows ? f.rows128 : 1.0) *
+                (1.0 + f.busy128 * full) +
+            f.tile128);
+  }
+  const double bytes =
+      4.0 * batch *
+      (static_cast<double>(m) * n + (static_cast<double>(m) + n) * k);
+  return f.launch + std::max(time, bytes / f.bytes_per_s);
+}
+inline bool fused_small_tiles(const int terms, const int m, const int n,
+                              const int k, const int batch, const bool rows) {
+  return fused_time(terms, m, n, k, batch, true, rows) <=
+         fused_time(terms, m, n, k, batch, false, rows);
 }
 // The kernels of one policy, as the driver calls them: one table per policy,
 // filled in the gemm_*.hip translation units, which is what lets the kernels
@@ -415,6 +460,7 @@ struct PolicyKernels {
   int (*gemm)(const GemmArgs &g);
   int (*gemm_rn)(const GemmArgs &g); // nullptr: the policy has no such variant
   int (*fused)(const FusedArgs &f);
+  int (*fused_rn)(const FusedArgs &f); // as gemm_rn
   // resident workgroups per compute unit of the packed kernel with tile shape
   // 0 (256x128), 1 (128x128) or 2 (64x64): the number the launch plans its
   // rounds with, for the workspace query

@@ -1,45 +1,59 @@
-// TCEC SGEMM for gfx950 straight from the fp32 operands, for products that are
-// bound by HBM rather than by the matrix cores (small matrices, usually
-// batched: every element is needed by only a few workgroups).  The packed path
-// (split_pack_kernel + tcec_gemm_kernel) would read and write every operand
-// once more.  Here one kernel does it all:
+// TCEC SGEMM for gfx950 in one launch, straight from the fp32 operands: for
+// products that are over before a split pass (split_pack_kernel) and a second
+// launch would pay, in any of the four transpose combinations, any leading
+// dimension and any alignment.
 //
-//   HBM --global_load_lds--> raw fp32 ring in LDS (NRAW stages of 32 k)
-//       --split in registers--> 16-bit terms in LDS, two stages, in the same
-//         fragment-major chunk order the packed kernel uses
-//       --ds_read_b128--> MFMA operands
+//   HBM/L2 --global loads--> registers (fp32, DEPTH stages of 32 k in flight)
+//       --split--> 16-bit terms in LDS, two stages, in the same fragment-major
+//         chunk order the packed kernel uses (slots of a k group permuted,
+//         direct_swizzle)
+//       --ds_read_b128--> MFMA operands of the next stage
 //
 // The reference's tiled GEMM has the same shape of data flow (fp32 tiles in
 // shared memory, split at fragment load: test/tcec/batch_gemm.cu:196-386,
 // tcec/tcec.hpp:213-229) but splits every element once per warp that needs it;
 // here every element of a tile is split once per workgroup.
 //
-// Each wave requests, and later converts, the same row blocks, so the raw ring
-// needs no workgroup barrier: the wave's own s_waitcnt vmcnt is enough.  The
-// only barrier of a stage publishes the converted terms.
+// What bounds it: at these sizes a compute unit has one or two workgroups, and a
+// k stage (32 of k) takes as long as its longest chain of instructions between
+// two barriers, not what any unit could do: of the 0.39 us of a stage of a 64x64
+// tile with two terms, done by four waves that load, split and multiply, the
+// matrix cores need 0.08, LDS 0.16.  Hence
+//   * two parts: PW producer waves load and split, CW consumer waves read
+//     fragments and multiply, one of each on every SIMD, one barrier a stage
+//     (0.39 -> 0.32 us; the kernel before, which took the fp32 values through an
+//     LDS ring and read them back, 0.8);
+//   * the fp32 values wait in the producers' registers, DEPTH stages in flight:
+//     no second LDS round trip, and the memory latency is covered;
+//   * the consumers read the fragments of stage s+1 while the MFMAs of stage s
+//     run;
+//   * few registers, so that two workgroups of the 64x64 tile share a compute
+//     unit (0.45 us for a stage of both);
+//   * with more tiles than resident workgroups the (tile, k stage) pairs of a
+//     workgroup are one stream, so that the next tile's stages are loaded and
+//     split while a tile is stored (STREAM).
+// Whole launches, two terms, before -> now: 1024^3 30.5 -> 16.2 us (two kernels
+// on packed operands 27.7), 512^3 16.7 -> 12.5, 256 entries of 256^3 with rows
+// contiguous 80.8 -> 54 (packed 96), 1024 entries of 100^3 35.2 -> 29.8; three
+// terms: 1024^3 packed 27.3 -> 20.7.
 //
-// Workgroups are persistent.  A workgroup walks a list of output tiles and
-// treats (tile, k stage) pairs as one stream, so the loads of the next tile
-// are in flight while the current one finishes and is written back: with
-// 8 stages a tile (k = 256) a pipeline refill per tile would cost as much as
-// the tile.  With eight or more batch entries, an XCD (blockIdx % 8) takes
-// whole batch entries, so the tiles that share an operand panel share an L2.
-//
-// Raw layout of one 16-row block of a stage (2 KiB = 16 rows x 128 bytes).
-// When k is contiguous and 16-byte aligned, two 16-byte requests per lane:
-// request h covers rows 8h..8h+7, lane l fetching row 8h + l/8, so that eight
-// lanes take one whole 128-byte line (requests that touch half lines ran the
-// read stream at 4.1 instead of 5.2-6 TB/s).  Within its row, lane l fetches
-// 16-byte piece (l%8) ^ (2*((l/16)%4) + h): the pieces of a row are stored
-// permuted so that the conversion - where lane l needs the 32 bytes
-// k = 8*(l/16) .. +7 of row r = l%16, found as two 16-byte halves at byte
-// r*128 + 32*((l/16) ^ ((r/2)%4)), in swapped order for r >= 8 - does
-// not have the sixteen rows of a read start in the same LDS banks (each
-// ds_read_b128 of sixteen lanes covers all 64 banks once).  Otherwise (any
-// stride, any alignment) eight 4-byte requests per lane, element e of the
-// lane's eight into slot [e][l], read back from the same slots.
+// How an operand is read (chosen by the host for each operand; the two halves
+// of a workgroup's waves load A and B, so a wave runs one of the three):
+//   kFusedKRows  k contiguous, k >= 4: a row block (16 rows x 32 k) in two
+//                16-byte loads per lane, load h covering rows 8h .. 8h+7, eight
+//                lanes to a row's 128 bytes.  16-byte loads need only a
+//                float's alignment.
+//   kFusedRRows  rows contiguous: 64 rows x 8 k in eight 4-byte loads per
+//                lane, lane = row, 256 contiguous bytes a load.
+//   kFusedAny    64 rows x 8 k with 64-bit addresses: k < 4, or strides of
+//                2^24 floats and more.
 // Rows past the matrix are clamped to the last row (their results are never
-// stored); k past K is clamped in the request and zeroed at the conversion.
+// stored).  In a last stage of fewer than 32 k no lane reads past the end of k
+// (load_tail_stage), and what lies there is zeroed before the split.
+//
+// Tiles: 128x128 (8 + 4 waves) reads an element half as often and takes 0.58 us
+// for a stage, 64x64 (4 + 4) gives four times the workgroups; the host's estimate
+// of either's time decides (fused_time).
 //
 // Operand element (r, l) of op(A) is A[r*a_rs + l*a_ks] (rows = m), of op(B) it
 // is B[r*b_rs + l*b_ks] (rows = n); batch entry y is base + y*stride or ptrs[y].
@@ -49,6 +63,8 @@
 #include "tcec_gemm_kernels.hpp"
 
 namespace wmmae_gemm {
+
+enum FusedSource { kFusedKRows = 0, kFusedRRows = 1, kFusedAny = 2 };
 
 struct FusedParams {
   const float *A;
@@ -61,67 +77,71 @@ struct FusedParams {
   float *const *c_ptrs;
   long long ldc, c_bs;
   int M, N, K, batch;
-  int tiles_m, tiles_per_batch;
+  int tiles_m, tiles_n;
   // XCD x (block index mod 8) owns the batch entries x, x+8, ... (set by the
   // launcher for 8 or more entries that spread evenly enough)
   int grouped;
-  // 16-byte requests are possible as far as the host can tell: k contiguous,
-  // K and the strides multiples of 4, base pointers aligned (pointer-array
-  // entries are checked by the kernel)
-  int vec_a, vec_b;
-  // accumulate the leading product with fp32 adds outside the matrix core
-  // (tcec_gemm_kernel's RN_MAIN; the reference's mma_rn_sync)
-  int rn_main;
+  int a_source, b_source; // FusedSource
   float alpha, beta, inv_scale;
 };
 
-template <int TERMS, int BM, int BN, int NW = (BM * BN >= 128 * 128 ? 8 : 4)>
-struct FusedConfig {
-  static constexpr int NWAVES = NW;       // 2 x NW/2 waves
-  static constexpr int NTHREADS = 64 * NW;
+// CW consumer waves (2 x CW/2 over the tile), PW producer waves
+template <int TERMS, int BM, int BN, int CW, int PW> struct FusedConfig {
+  static constexpr int NTHREADS = 64 * (CW + PW);
   static constexpr int RBA = BM / 16, RBB = BN / 16, NRB = RBA + RBB;
-  static constexpr int NQ = NRB / NW; // row blocks per wave and stage
-  static constexpr int RAW_STAGE_BYTES = NRB * 2048;
-  static constexpr int FRAG_BYTES = 2 * NRB * TERMS * 1024;
-  static constexpr int FIT = (160 * 1024 - FRAG_BYTES) / RAW_STAGE_BYTES;
-  static constexpr int NRAW = FIT > 4 ? 4 : FIT;
-  static constexpr int LDS_BYTES = NRAW * RAW_STAGE_BYTES + FRAG_BYTES;
-  static_assert(RBA % NW == 0 && RBB % NW == 0,
-                "row blocks divide over the waves");
-  static_assert(NRAW >= 2, "raw ring too shallow");
+  static constexpr int U = RBA / (PW / 2); // units of 512 floats per producer
+  static constexpr int BUF_BYTES = NRB * TERMS * 1024;
+  static constexpr int LDS_BYTES = 2 * BUF_BYTES;
+  static_assert(BM == BN && BM % 64 == 0 && RBA % (PW / 2) == 0,
+                "half the producers load A, half load B, in units of 64 x 8");
+  static_assert(LDS_BYTES <= 160 * 1024, "LDS of one compute unit");
 };
 
-template <int N> __device__ __forceinline__ void wait_vmcnt_at_most() {
-  asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N > 63 ? 63 : N) : "memory");
-}
-
-template <class T, int TERMS, int BM, int BN,
-          int NW = FusedConfig<TERMS, BM, BN>::NWAVES>
-__global__ void __launch_bounds__(64 * NW)
+//   RN_MAIN : accumulate the leading product with fp32 adds outside the matrix
+//             core (tcec_gemm_kernel's RN_MAIN; the reference's mma_rn_sync)
+//   STREAM  : a workgroup walks several tiles; else one, the grid covers them all
+//             (the cursor's step to the next tile costs a stage 5 to 10 %, a
+//             pipeline refill per tile 2 to 3 us: 4096 tiles of 64x64 at k = 128
+//             46.6 -> 30.3 us)
+//   DEPTH   : stages of fp32 values in flight in registers (even: the LDS
+//             buffer and fragment set of a step are then compile-time choices)
+template <class T, int TERMS, int BM, int BN, int CW, int PW, int DEPTH,
+          bool RN_MAIN, bool STREAM>
+__global__ void __launch_bounds__(64 * (CW + PW))
     tcec_gemm_fused_kernel(const FusedParams p) {
   using traits = mtk::wmma::tcec::detail::split_traits<T>;
   using S = typename traits::storage;
   typedef S ab_vec __attribute__((ext_vector_type(8)));
-  using Cfg = FusedConfig<TERMS, BM, BN, NW>;
-  constexpr int RBA = Cfg::RBA, NRB = Cfg::NRB, NQ = Cfg::NQ;
-  constexpr int NRAW = Cfg::NRAW;
-  constexpr int WGN = NW / 2;
-  constexpr int WM = BM / 2, WN = BN / WGN; // 2 x NW/2 waves
+  typedef S s2_t __attribute__((ext_vector_type(2)));
+  typedef unsigned u32x2 __attribute__((ext_vector_type(2)));
+  using Cfg = FusedConfig<TERMS, BM, BN, CW, PW>;
+  constexpr int RBA = Cfg::RBA, U = Cfg::U;
+  constexpr int WGN = CW / 2;
+  constexpr int WM = BM / 2, WN = BN / WGN;
   constexpr int MT_ = WM / 16, NT_ = WN / 16;
+  static_assert(DEPTH % 2 == 0 && DEPTH >= 2, "even ring");
+  // Two sets of fragments where they fit the registers that two workgroups (64x64
+  // tile) or three waves a SIMD (128x128) leave a wave; else one set, a term's
+  // fragments refilled for the next stage once its last product has been issued.
+  constexpr bool RECYCLE = TERMS == 3 || BM > 64;
 
   extern __shared__ __attribute__((aligned(1024))) unsigned char lds_raw[];
-  u32x4 *const frag =
-      reinterpret_cast<u32x4 *>(lds_raw + NRAW * Cfg::RAW_STAGE_BYTES);
 
   const unsigned lane = threadIdx.x & 63u;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int wm = wave & 1, wn = wave >> 1;
-  const int r16 = static_cast<int>(lane & 15u);
-  const int g8 = 8 * static_cast<int>(lane >> 4);
   const int M = p.M, N = p.N, K = p.K;
+  const int num_k = (K + 31) / 32;
+  const int k_left = K - 32 * (num_k - 1); // k of the last stage, 1 .. 32
+
+  // a producer's work: A or B, units unit0 .. unit0 + U-1 of it
+  const bool loads_a = wave - CW < PW / 2;
+  const int unit0 = (loads_a ? wave - CW : wave - CW - PW / 2) * U;
+  const int source =
+      __builtin_amdgcn_readfirstlane(loads_a ? p.a_source : p.b_source);
 
   // ---- this workgroup's tiles: v = first + i*stride while v < count
-  const int tpb = p.tiles_per_batch;
+  const int tpb = p.tiles_m * p.tiles_n;
   const bool grouped = p.grouped != 0;
   const int xcd = grouped ? static_cast<int>(blockIdx.x & 7u) : 0;
   const int first = grouped ? static_cast<int>(blockIdx.x >> 3)
@@ -130,193 +150,51 @@ __global__ void __launch_bounds__(64 * NW)
                              : static_cast<int>(gridDim.x);
   const int count = grouped ? ((p.batch - xcd + 7) >> 3) * tpb : p.batch * tpb;
   if (first >= count)
-    return;
-  const int n_my = (count - first + stride - 1) / stride;
-  auto decode = [&](const int i, int &entry, int &tm, int &tn) __attribute__((always_inline)) {
+    return; // nothing for this workgroup (before any barrier)
+  const int n_my = STREAM ? (count - first + stride - 1) / stride : 1;
+  auto decode = [&](const int i, int &entry, int &tm, int &tn) {
     const int v = first + i * stride;
     const int bi = v / tpb;
-    const int t = v - bi * tpb;
     entry = grouped ? bi * 8 + xcd : bi;
-    tn = t / p.tiles_m;
-    tm = t - tn * p.tiles_m;
+    tile_of<8>(static_cast<unsigned>(v - bi * tpb), static_cast<unsigned>(tpb),
+               static_cast<unsigned>(p.tiles_m),
+               static_cast<unsigned>(p.tiles_n), !grouped, tm, tn);
   };
 
-  // ---- request width (uniform over the workgroup)
-  int vec_a = p.vec_a, vec_b = p.vec_b;
-  if (p.a_ptrs != nullptr || p.b_ptrs != nullptr) {
-    int low_a = 0, low_b = 0;
-    for (int i = threadIdx.x; i < n_my; i += 64 * NW) {
-      int entry, tm, tn;
-      decode(i, entry, tm, tn);
-      if (p.a_ptrs != nullptr)
-        low_a |= static_cast<int>(
-            reinterpret_cast<uintptr_t>(p.a_ptrs[entry]) & 15u);
-      if (p.b_ptrs != nullptr)
-        low_b |= static_cast<int>(
-            reinterpret_cast<uintptr_t>(p.b_ptrs[entry]) & 15u);
+  f32x4 acc_main[MT_][NT_], acc_err[MT_][NT_];
+  struct Frags {
+    ab_vec a[TERMS][MT_], b[TERMS][NT_];
+  };
+  // 16-byte slot of this lane's fragment inside a chunk
+  const unsigned frag_off =
+      16u * ((lane & 48u) + ((lane & 15u) ^ direct_swizzle(lane >> 4)));
+  // the fragments of term TA of A and term TB of B (-1: none) of the stage in
+  // the LDS buffer at `base`
+  auto read_terms = [&](Frags &f, const unsigned base, auto TA, auto TB)
+                        __attribute__((always_inline)) {
+    constexpr int ta = decltype(TA)::value, tb = decltype(TB)::value;
+    const unsigned char *const buf =
+        lds_raw + base + frag_off;
+    const unsigned char *const sa = buf + wm * MT_ * TERMS * 1024;
+    const unsigned char *const sb = buf + (RBA + wn * NT_) * TERMS * 1024;
+    if constexpr (tb >= 0) {
+#pragma unroll
+      for (int j = 0; j < NT_; j++)
+        f.b[tb][j] =
+            *reinterpret_cast<const ab_vec *>(sb + (j * TERMS + tb) * 1024);
     }
-    // workgroup-wide OR through the (still unused) start of the LDS ring
-    int *const flags = reinterpret_cast<int *>(lds_raw);
-    const int any_a = __builtin_amdgcn_ballot_w64(low_a != 0) != 0;
-    const int any_b = __builtin_amdgcn_ballot_w64(low_b != 0) != 0;
-    if (lane == 0)
-      flags[wave] = any_a | (any_b << 1);
-    __syncthreads();
-    int all = 0;
+    if constexpr (ta >= 0) {
 #pragma unroll
-    for (int w = 0; w < NW; w++)
-      all |= flags[w];
-    __syncthreads();
-    if (all & 1)
-      vec_a = 0;
-    if (all & 2)
-      vec_b = 0;
-  }
-  vec_a = __builtin_amdgcn_readfirstlane(vec_a);
-  vec_b = __builtin_amdgcn_readfirstlane(vec_b);
-
-  const int num_k = (K + 31) / 32;
-  const int total = n_my * num_k; // stages in this workgroup's stream
-
-  // ---- requests
-  typedef const __attribute__((address_space(1))) float *gptr_t;
-  gptr_t rowptr[NQ][2]; // [.][h]: row of request h (16-byte mode); [.][0] else
-  auto set_rows = [&](auto VEC, const int i) __attribute__((always_inline)) {
-    int entry, tm, tn;
-    decode(i, entry, tm, tn);
-    // the pointer arrays are read with scalar loads (constant address space):
-    // a vector load here would make the compiler wait for every outstanding
-    // request of the ring before it can use the pointer
-    typedef const float *const __attribute__((address_space(4))) *ptr_array_t;
-    const float *const Ab = p.a_ptrs != nullptr
-                                ? ((ptr_array_t)p.a_ptrs)[entry]
-                                : p.A + static_cast<long long>(entry) * p.a_bs;
-    const float *const Bb = p.b_ptrs != nullptr
-                                ? ((ptr_array_t)p.b_ptrs)[entry]
-                                : p.B + static_cast<long long>(entry) * p.b_bs;
-#pragma unroll
-    for (int q = 0; q < NQ; q++) {
-      const int rbl = wave + NW * q;
-      const bool is_a = NW * q < RBA;
-      const int row0 = is_a ? tm * BM + rbl * 16 : tn * BN + (rbl - RBA) * 16;
-      const int last = is_a ? M - 1 : N - 1;
-      const float *const base = is_a ? Ab : Bb;
-      const long long rs = is_a ? p.a_rs : p.b_rs;
-#pragma unroll
-      for (int h = 0; h < 2; h++) {
-        // 16-byte mode: row 8h + lane/8; 4-byte mode: row lane%16
-        int r = row0 + (decltype(VEC)::value
-                            ? 8 * h + static_cast<int>(lane >> 3)
-                            : r16);
-        r = r < last ? r : last;
-        rowptr[q][h] = (gptr_t)(base + static_cast<long long>(r) * rs);
-      }
+      for (int i = 0; i < MT_; i++)
+        f.a[ta][i] =
+            *reinterpret_cast<const ab_vec *>(sa + (i * TERMS + ta) * 1024);
     }
   };
-  // VEC: std::true_type for 16-byte requests (both operands), else 4-byte ones
-  auto issue = [&](auto VEC, const int ks, const int slot) __attribute__((always_inline)) {
-#pragma unroll
-    for (int q = 0; q < NQ; q++) {
-      const int rbl = wave + NW * q;
-      unsigned char *const dst =
-          lds_raw + slot * Cfg::RAW_STAGE_BYTES + rbl * 2048;
-      if constexpr (decltype(VEC)::value) {
-        // K % 4 == 0 here: a piece is all in or all out
-        const int piece =
-            static_cast<int>((lane & 7u) ^ (2u * ((lane >> 4) & 3u)));
-#pragma unroll
-        for (int h = 0; h < 2; h++) {
-          int k = ks * 32 + 4 * (piece ^ h);
-          k = k < K ? k : 0;
-          __builtin_amdgcn_global_load_lds(
-              (const __attribute__((address_space(1))) void *)(rowptr[q][h] +
-                                                                k),
-              (__attribute__((address_space(3))) void *)(dst + h * 1024), 16, 0,
-              0);
-        }
-      } else {
-        const long long kst = NW * q < RBA ? p.a_ks : p.b_ks;
-#pragma unroll
-        for (int e = 0; e < 8; e++) {
-          int k = ks * 32 + g8 + e;
-          k = k < K ? k : K - 1;
-          __builtin_amdgcn_global_load_lds(
-              (const __attribute__((address_space(1))) void *)(rowptr[q][0] +
-                                                                k * kst),
-              (__attribute__((address_space(3))) void *)(dst + e * 256), 4, 0,
-              0);
-        }
-      }
-    }
-  };
-  // leave NRAW-1 stages of this wave's requests in flight
-  auto wait_oldest_stage = [&](auto VEC) __attribute__((always_inline)) {
-    constexpr int per_stage = NQ * (decltype(VEC)::value ? 2 : 8);
-    wait_vmcnt_at_most<(NRAW - 1) * per_stage>();
-  };
-  // byte offset of this lane's eight floats inside a raw row block (16-byte mode)
-  const int vec_off =
-      r16 * 128 + 32 * static_cast<int>((lane >> 4) ^ ((lane >> 1) & 3u));
-  const int vec_off_lo = vec_off + 16 * (r16 >> 3);
-  const int vec_off_hi = vec_off + 16 * (1 - (r16 >> 3));
-  // conversion, first half: this lane's eight floats of each of the wave's
-  // row blocks, out of raw slot `slot`
-  auto load_raw = [&](auto VEC, const int slot, float (&v)[NQ][8]) __attribute__((always_inline)) {
-#pragma unroll
-    for (int q = 0; q < NQ; q++) {
-      const int rbl = wave + NW * q;
-      const unsigned char *const src =
-          lds_raw + slot * Cfg::RAW_STAGE_BYTES + rbl * 2048;
-      if constexpr (decltype(VEC)::value) {
-        const f32x4 lo = *reinterpret_cast<const f32x4 *>(src + vec_off_lo);
-        const f32x4 hi = *reinterpret_cast<const f32x4 *>(src + vec_off_hi);
-#pragma unroll
-        for (int x = 0; x < 4; x++) {
-          v[q][x] = lo[x];
-          v[q][4 + x] = hi[x];
-        }
-      } else {
-#pragma unroll
-        for (int e = 0; e < 8; e++)
-          v[q][e] = reinterpret_cast<const float *>(src)[e * 64 + lane];
-      }
-    }
-  };
-  // conversion, second half: split and write the terms of k stage `ks` into
-  // fragment buffer `buf`
-  auto split_store = [&](const int ks, const int buf, float (&v)[NQ][8]) __attribute__((always_inline)) {
-#pragma unroll
-    for (int q = 0; q < NQ; q++) {
-      const int rbl = wave + NW * q;
-      // k past K was clamped in the request: zero it (last stage only)
-      if (ks * 32 + 32 > K) {
-        const int left = K - (ks * 32 + g8);
-#pragma unroll
-        for (int x = 0; x < 8; x++)
-          v[q][x] = x < left ? v[q][x] : 0.f;
-      }
-      // the split of split_traits<T>, four elements at a time in the form
-      // that uses the packed conversions (and for fp16 the mixed-precision
-      // fma): t0 = RN16(v), t1 = RN16((v - t0) * scale), t2 = RN16((v - t0) - t1)
-      S term[3][8];
-#pragma unroll
-      for (int x = 0; x < 8; x += 4) {
-        const mtk::wmma::tcec::detail::f32x4_t vv = {v[q][x], v[q][x + 1],
-                                                     v[q][x + 2], v[q][x + 3]};
-        mtk::wmma::tcec::detail::split4<T>(vv, &term[0][x], &term[1][x],
-                                           &term[2][x]);
-      }
-      ab_vec t[3];
-#pragma unroll
-      for (int c = 0; c < TERMS; c++)
-#pragma unroll
-        for (int x = 0; x < 8; x++)
-          t[c][x] = term[c][x];
-#pragma unroll
-      for (int c = 0; c < TERMS; c++)
-        frag[((buf * NRB + rbl) * TERMS + c) * 64 + lane] =
-            __builtin_bit_cast(u32x4, t[c]);
-    }
+  auto read_frags = [&](Frags &f, const unsigned base)
+                        __attribute__((always_inline)) {
+    static_for<0, TERMS>([&](auto T_) __attribute__((always_inline)) {
+      read_terms(f, base, T_, T_);
+    });
   };
   auto mfma = [](const ab_vec x, const ab_vec y, const f32x4 z) -> f32x4 {
     if constexpr (std::is_same<S, _Float16>::value)
@@ -324,9 +202,365 @@ __global__ void __launch_bounds__(64 * NW)
     else
       return __builtin_amdgcn_mfma_f32_16x16x32_bf16(x, y, z, 0, 0, 0);
   };
+  // MFMA n of a step.  Same products and, per accumulator, the same order as
+  // tcec_gemm_kernel, product by product over the wave's tiles (neighbouring
+  // MFMAs never wait for each other's accumulator).
+  constexpr int NPROD = TERMS == 1 ? 1 : (TERMS == 2 ? 3 : 6);
+  constexpr int NTILE = MT_ * NT_;
+  constexpr int NMFMA = NPROD * NTILE;
+  auto multiply = [&](const Frags &f, auto N_) __attribute__((always_inline)) {
+    constexpr int n = decltype(N_)::value, pr = n / NTILE;
+    constexpr int i = (n % NTILE) / NT_, j = n % NT_;
+    constexpr int first_product = TERMS == 1 ? 5 : (TERMS == 2 ? 3 : 0);
+    // (term of A, term of B): smallest products first, the main product last
+    constexpr int ta_of[6] = {2, 0, 1, 1, 0, 0}, tb_of[6] = {0, 2, 1, 0, 1, 0};
+    constexpr int ta = ta_of[first_product + pr], tb = tb_of[first_product + pr];
+    if constexpr (pr + 1 < NPROD)
+      acc_err[i][j] = mfma(f.a[ta][i], f.b[tb][j], acc_err[i][j]);
+    else if constexpr (RN_MAIN)
+      acc_main[i][j] +=
+          mfma(f.a[0][i], f.b[0][j], f32x4{0.f, 0.f, 0.f, 0.f});
+    else
+      acc_main[i][j] = mfma(f.a[0][i], f.b[0][j], acc_main[i][j]);
+  };
 
-  f32x4 acc_main[MT_][NT_], acc_err[MT_][NT_];
-  auto clear_acc = [&]() __attribute__((always_inline)) {
+  // A producer's part: the workgroup's (tile, k stage) pairs as one stream, so
+  // that the next tile's first stages are on their way while the consumers store
+  // a tile.  SRC: how this wave's operand is read.
+  auto produce = [&](auto SRC) __attribute__((always_inline)) {
+    constexpr int src_kind = decltype(SRC)::value;
+    constexpr int NOFF = src_kind == kFusedKRows ? 2 : 8;
+    // ---- source of this wave's operand
+    typedef const float *const __attribute__((address_space(4))) *ptr_array_t;
+    typedef const __attribute__((address_space(1))) char *gbytes_t;
+    const float *const *const ptrs = loads_a ? p.a_ptrs : p.b_ptrs;
+    const long long rs = loads_a ? p.a_rs : p.b_rs;
+    const long long ks = loads_a ? p.a_ks : p.b_ks;
+    const int last = (loads_a ? M : N) - 1;
+    // src[u]: wave-uniform address at the load cursor's stage, voff[u][.]: the
+    // lane's byte offsets from it
+    unsigned long long src[U];
+    unsigned voff[U][NOFF];
+    // the load cursor: tile and stage, first row of the tile
+    int ld_tile = 0, ld_stage = 0, tile_row = 0;
+    // first row of unit u (KRows: a row block, else 64 rows), its k group
+    auto unit_row = [&](const int u) {
+      const int row = tile_row + (src_kind == kFusedKRows
+                                      ? 16 * (unit0 + u)
+                                      : 64 * ((unit0 + u) >> 2));
+      return row < last ? row : last;
+    };
+    auto unit_k = [&](const int u) {
+      return src_kind == kFusedKRows ? 0 : 8 * ((unit0 + u) & 3);
+    };
+    // sources of the cursor's stage when it is the last one and shorter than
+    // 32: every lane reads inside the operand.  KRows: a lane whose four floats
+    // would end past the row reads the row's last four instead (the uniform
+    // address then starts four floats early where there are any, for the lanes
+    // that read up to three floats before the stage); RRows: k clamped to the
+    // last one.
+    auto load_tail_stage = [&]() __attribute__((always_inline)) {
+      const int k0 = 32 * ld_stage;
+      int left = k_left;
+      asm volatile("" : "+s"(left));
+#pragma unroll
+      for (int u = 0; u < U; u++) {
+        if constexpr (src_kind == kFusedKRows) {
+          const int bias = k0 > 0 ? kDirectBias : 0;
+          const int back = direct_tail_shift(lane, left);
+          src[u] -= 4ull * bias;
+#pragma unroll
+          for (int h = 0; h < 2; h++)
+            voff[u][h] += 4u * static_cast<unsigned>(bias - back);
+        } else if constexpr (src_kind == kFusedRRows) {
+          const int behind = left - 1 - unit_k(u); // k of the unit after its first
+          if (behind < 0)
+            src[u] += static_cast<long long>(behind) * ks * 4;
+#pragma unroll
+          for (int e = 0; e < 8; e++) {
+            const int back = e - (behind < 0 ? 0 : behind);
+            if (back > 0)
+              voff[u][e] -= static_cast<unsigned>(back * ks) * 4u;
+          }
+        }
+        asm volatile("" : "+s"(src[u]));
+      }
+    };
+    // the cursor's tile: sources of its first stage
+    auto set_tile = [&]() __attribute__((always_inline)) {
+      int entry, tm, tn;
+      decode(ld_tile, entry, tm, tn);
+      tile_row = loads_a ? tm * BM : tn * BN;
+      const float *const X =
+          ptrs != nullptr
+              ? ((ptr_array_t)ptrs)[entry]
+              : (loads_a ? p.A + entry * p.a_bs : p.B + entry * p.b_bs);
+#pragma unroll
+      for (int u = 0; u < U; u++) {
+        const int row0 = unit_row(u);
+        src[u] = reinterpret_cast<unsigned long long>(X + row0 * rs +
+                                                      unit_k(u) * ks);
+        asm volatile("" : "+s"(src[u]));
+#pragma unroll
+        for (int o = 0; o < NOFF; o++) {
+          const int r = row0 + (src_kind == kFusedKRows
+                                    ? 8 * o + static_cast<int>(lane >> 3)
+                                    : static_cast<int>(lane));
+          const int mine = (r < last ? r : last) - row0;
+          voff[u][o] =
+              src_kind == kFusedKRows
+                  ? static_cast<unsigned>(mine * rs) * 4u + 16u * (lane & 7u)
+              : src_kind == kFusedRRows
+                  ? static_cast<unsigned>(mine) * 4u +
+                        static_cast<unsigned>(o * ks) * 4u
+                  : static_cast<unsigned>(mine);
+        }
+      }
+      if (num_k == 1 && k_left < 32)
+        load_tail_stage();
+    };
+    set_tile();
+    auto advance = [&]() __attribute__((always_inline)) {
+      if (ld_stage + 1 < num_k) {
+        ld_stage++;
+#pragma unroll
+        for (int u = 0; u < U; u++) {
+          src[u] += src_kind == kFusedKRows ? 128ull : 128ull * ks;
+          asm volatile("" : "+s"(src[u]));
+        }
+        if (ld_stage + 1 == num_k && k_left < 32)
+          load_tail_stage();
+      } else if (STREAM && ld_tile + 1 < n_my) {
+        ld_tile++;
+        ld_stage = 0;
+        set_tile();
+      } // else: the last stage again, never used
+    };
+    // the tile stage that is split next
+    int conv_k = 0;
+    auto advance_conv = [&]() __attribute__((always_inline)) {
+      conv_k = conv_k + 1 == num_k ? 0 : conv_k + 1;
+    };
+    float raw[DEPTH][U][8];
+    auto load_unit = [&](auto SLOT, auto UN) __attribute__((always_inline)) {
+      constexpr int slot = decltype(SLOT)::value, u = decltype(UN)::value;
+      typedef f32x4 __attribute__((aligned(4))) f32x4_u;
+      typedef const __attribute__((address_space(1))) f32x4_u *vec_ptr;
+      typedef const __attribute__((address_space(1))) float *flt_ptr;
+      const gbytes_t base = reinterpret_cast<gbytes_t>(src[u]);
+      if constexpr (src_kind == kFusedAny) {
+        const int k0 = 32 * ld_stage + unit_k(u);
+#pragma unroll
+        for (int e = 0; e < 8; e++) {
+          const int k = k0 + e < K ? k0 + e : K - 1;
+          raw[slot][u][e] = *reinterpret_cast<flt_ptr>(
+              base + 4 * (static_cast<long long>(voff[u][e]) * rs +
+                          (k - k0) * ks));
+        }
+      } else {
+#pragma unroll
+        for (int o = 0; o < NOFF; o++) {
+          // (redefined in place so that the address is formed here, as the
+          // instruction's scalar base + 32-bit lane offset)
+          asm volatile("" : "+v"(voff[u][o]));
+          if constexpr (src_kind == kFusedKRows) {
+            const f32x4 x = *reinterpret_cast<vec_ptr>(base + voff[u][o]);
+#pragma unroll
+            for (int e = 0; e < 4; e++)
+              raw[slot][u][4 * o + e] = x[e];
+          } else {
+            raw[slot][u][o] = *reinterpret_cast<flt_ptr>(base + voff[u][o]);
+          }
+        }
+      }
+    };
+    // the values of a last, shorter stage waiting in `slot`: what lies past the
+    // end of k becomes zero (`left` is redefined in place so that the masks are
+    // worked out here and not kept through the loop)
+    auto zero_tail = [&](auto SLOT) __attribute__((always_inline)) {
+      constexpr int slot = decltype(SLOT)::value;
+      int left = k_left;
+      asm volatile("" : "+s"(left));
+      if constexpr (src_kind == kFusedKRows) {
+        const int shift = direct_tail_shift(lane, left);
+        const bool by1 = (shift & 1) != 0, by2 = (shift & 2) != 0;
+        const bool all = shift > 3;
+#pragma unroll
+        for (int u = 0; u < U; u++)
+#pragma unroll
+          for (int h = 0; h < 2; h++) {
+            float *const r = &raw[slot][u][4 * h];
+            float v0 = r[0], v1 = r[1], v2 = r[2], v3 = r[3];
+            v0 = by1 ? v1 : v0;
+            v1 = by1 ? v2 : v1;
+            v2 = by1 ? v3 : v2;
+            v3 = by1 || by2 || all ? 0.f : v3;
+            v0 = by2 ? v2 : v0;
+            v1 = by2 ? (by1 ? 0.f : r[3]) : v1;
+            v2 = by2 || all ? 0.f : v2;
+            r[0] = all ? 0.f : v0;
+            r[1] = all ? 0.f : v1;
+            r[2] = v2;
+            r[3] = v3;
+          }
+      } else {
+#pragma unroll
+        for (int u = 0; u < U; u++) {
+          const int mine = left - unit_k(u);
+#pragma unroll
+          for (int e = 0; e < 8; e++)
+            raw[slot][u][e] = e < mine ? raw[slot][u][e] : 0.f;
+        }
+      }
+    };
+    // split the stage in `slot` into LDS buffer BUF and load the cursor's stage
+    // into the slot, unit by unit
+    auto convert = [&](auto SLOT, auto BUF) __attribute__((always_inline)) {
+      constexpr int slot = decltype(SLOT)::value;
+      unsigned char *const buf = lds_raw + decltype(BUF)::value * Cfg::BUF_BYTES +
+                                 (loads_a ? 0 : RBA * TERMS * 1024);
+      static_for<0, U>([&](auto UN) __attribute__((always_inline)) {
+        constexpr int u = decltype(UN)::value;
+        unsigned term[TERMS][4];
+#pragma unroll
+        for (int q = 0; q < 4; q++) {
+          s2_t h[3];
+          mtk::wmma::tcec::detail::split2<T>(
+              mtk::wmma::tcec::detail::f32x2_t{raw[slot][u][2 * q],
+                                               raw[slot][u][2 * q + 1]},
+              h[0], h[1], h[2]);
+#pragma unroll
+          for (int t = 0; t < TERMS; t++)
+            term[t][q] = __builtin_bit_cast(unsigned, h[t]);
+          if (src_kind == kFusedKRows && q % 2 == 1) {
+            // the lane's four floats of load q/2: half of position (row, k group)
+            unsigned char *const chunk = buf + (unit0 + u) * TERMS * 1024;
+            const unsigned g = (lane & 7u) >> 1, r = 8u * (q / 2) + (lane >> 3);
+            const unsigned off =
+                256u * g + 16u * (r ^ direct_swizzle(g)) + 8u * (lane & 1u);
+#pragma unroll
+            for (int t = 0; t < TERMS; t++)
+              *reinterpret_cast<u32x2 *>(chunk + t * 1024 + off) =
+                  u32x2{term[t][q - 1], term[t][q]};
+          }
+        }
+        if constexpr (src_kind != kFusedKRows) {
+          const unsigned g = static_cast<unsigned>((unit0 + u) & 3);
+          unsigned char *const chunk =
+              buf + (4 * ((unit0 + u) >> 2) + static_cast<int>(lane >> 4)) *
+                        (TERMS * 1024);
+          const unsigned off =
+              256u * g + 16u * ((lane & 15u) ^ direct_swizzle(g));
+#pragma unroll
+          for (int t = 0; t < TERMS; t++)
+            *reinterpret_cast<u32x4 *>(chunk + t * 1024 + off) =
+                u32x4{term[t][0], term[t][1], term[t][2], term[t][3]};
+        }
+        load_unit(SLOT, UN);
+        __builtin_amdgcn_sched_barrier(0);
+      });
+    };
+
+    // ---- prologue: stages 0 .. DEPTH-1 requested, 0 and 1 converted (their
+    // slots take the stages DEPTH and DEPTH+1), stage 0's fragments read
+    static_for<0, DEPTH>([&](auto SLOT) __attribute__((always_inline)) {
+      static_for<0, U>([&](auto UN) __attribute__((always_inline)) {
+        load_unit(SLOT, UN);
+      });
+      advance();
+    });
+    static_for<0, 2>([&](auto SLOT) __attribute__((always_inline)) {
+      if (conv_k + 1 == num_k && k_left < 32)
+        zero_tail(SLOT);
+      convert(SLOT, SLOT);
+      advance();
+      advance_conv();
+    });
+    asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+    asm volatile("s_barrier" ::: "memory"); // (the consumers hold stage 0)
+
+    // step s of the stream: stage s+2 into the buffer stage s has left, stage
+    // s+2+DEPTH requested
+    int left = n_my * num_k;
+    auto steps = [&](auto self, auto D_) __attribute__((always_inline)) {
+      constexpr int d = decltype(D_)::value;
+      if (conv_k + 1 == num_k && k_left < 32)
+        zero_tail(ic<(d + 2) % DEPTH>{});
+      convert(ic<(d + 2) % DEPTH>{}, ic<d & 1>{});
+      advance();
+      advance_conv();
+      asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+      left--;
+      if constexpr (d + 1 < DEPTH)
+        if (left > 0)
+          self(self, ic<d + 1>{});
+    };
+    while (left > 0)
+      steps(steps, ic<0>{});
+  };
+
+  // (the waves of a workgroup meet at the same number of barriers, two and one
+  // a stage, whatever their part; the producers' vector instructions are the
+  // longest part of a step: they go first where they share a SIMD with a
+  // consumer: 128x128 tile, per k stage, 657 -> 580 ns, rows contiguous 757 ->
+  // 660; 64x64 465 -> 437 with two workgroups on a compute unit)
+  if (wave >= CW) {
+    __builtin_amdgcn_s_setprio(2);
+    if (source == kFusedKRows)
+      produce(ic<kFusedKRows>{});
+    else if (source == kFusedRRows)
+      produce(ic<kFusedRRows>{});
+    else
+      produce(ic<kFusedAny>{});
+    return;
+  }
+
+  // ---- consumer: step s of the stream, the MFMAs of stage s while the fragments
+  // of stage s+1 (after a tile's last stage the next tile's first) are read
+  asm volatile("s_barrier" ::: "memory"); // stages 0 and 1 are there
+  Frags f[RECYCLE ? 1 : 2];
+  unsigned held = 0; // LDS offset of the buffer whose stage is in registers
+  read_frags(f[0], 0u);
+  asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+  // (LAST with RECYCLE: the fragments are read after the tile has been stored,
+  // whose addresses and old values need their registers)
+  auto step = [&](auto D_, auto LAST) __attribute__((always_inline)) {
+    constexpr int d = decltype(D_)::value;
+    const unsigned next = Cfg::BUF_BYTES - held; // buffer of stage s+1
+    if constexpr (!RECYCLE) {
+      read_frags(f[1 - d], next);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+    static_for<0, NMFMA>([&](auto N_) __attribute__((always_inline)) {
+      constexpr int n = decltype(N_)::value;
+      multiply(f[RECYCLE ? 0 : d], N_);
+      if constexpr (RECYCLE && !decltype(LAST)::value &&
+                    (n + 1) % NTILE == 0) {
+        // the terms whose last product has just been issued
+        constexpr int pr = n / NTILE + (6 - NPROD);
+        constexpr int ta = TERMS == 1   ? 0
+                           : TERMS == 2 ? (pr == 3 ? 1 : pr == 5 ? 0 : -1)
+                                        : (pr == 0   ? 2
+                                           : pr == 3 ? 1
+                                           : pr == 5 ? 0
+                                                     : -1);
+        constexpr int tb = TERMS == 1   ? 0
+                           : TERMS == 2 ? (pr == 4 ? 1 : pr == 5 ? 0 : -1)
+                                        : (pr == 1   ? 2
+                                           : pr == 4 ? 1
+                                           : pr == 5 ? 0
+                                                     : -1);
+        __builtin_amdgcn_sched_barrier(0);
+        read_terms(f[0], next, ic<ta>{}, ic<tb>{});
+        __builtin_amdgcn_sched_barrier(0);
+      }
+    });
+    if constexpr (!(RECYCLE && decltype(LAST)::value)) {
+      asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+      held = next;
+    }
+  };
+  for (int tile = 0; tile < n_my; tile++) {
 #pragma unroll
     for (int i = 0; i < MT_; i++)
 #pragma unroll
@@ -334,10 +568,20 @@ __global__ void __launch_bounds__(64 * NW)
         acc_main[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
         acc_err[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
       }
-  };
-  auto store_tile = [&](const int i_tile) __attribute__((always_inline)) {
+    int s = num_k;
+    for (; s > (RECYCLE ? 2 : 1); s -= 2) {
+      step(ic<0>{}, std::false_type{});
+      step(ic<1>{}, std::false_type{});
+    }
+    if (RECYCLE && s == 2)
+      step(ic<0>{}, std::false_type{});
+    if (RECYCLE || s == 1) { // the next tile's first fragments arrive in the other set
+      step(ic<0>{}, std::true_type{});
+      if constexpr (!RECYCLE)
+        f[0] = f[1];
+    }
     int entry, tm, tn;
-    decode(i_tile, entry, tm, tn);
+    decode(tile, entry, tm, tn);
     typedef float *const __attribute__((address_space(4))) *out_array_t;
     float *const Cb = p.c_ptrs != nullptr
                           ? ((out_array_t)p.c_ptrs)[entry]
@@ -349,152 +593,16 @@ __global__ void __launch_bounds__(64 * NW)
         o = epilogue_fold(o, acc_err[i][j], p.inv_scale);
       return o * alpha;
     };
-    store_piece<MT_, NT_, MT_ % 2 == 0, MT_ * NT_>(out_value, Cb, p.ldc,
-                                             tm * BM + wm * WM,
-                                             tn * BN + wn * WN, M, N, p.beta,
-                                             lane);
-  };
-
-  // Pipeline, per wave and stream stage s (one iteration of the k loop):
-  //   request stage s+1+NRAW into the raw slot that stage s+1 has left
-  //   wait until the wave's requests of stage s+2 have landed, read them
-  //   issue the MFMAs of stage s (fragments are in registers)
-  //   read the fragments of stage s+1 (converted last iteration) into the
-  //     same registers - the matrix core has fetched them by then
-  //   split stage s+2 and write its terms over the fragment buffer of stage s
-  //   barrier
-  // so the LDS latencies sit behind the MFMAs and the conversion arithmetic,
-  // and NRAW stages of requests are in flight while the wave computes.
-  auto run = [&](auto VEC) __attribute__((always_inline)) {
-    int req_tile = 0, req_ks = 0; // next (tile, k stage) to request
-    auto advance_request = [&]() __attribute__((always_inline)) {
-      if (req_ks + 1 < num_k) {
-        req_ks++;
-      } else if (req_tile + 1 < n_my) {
-        req_tile++;
-        req_ks = 0;
-        set_rows(VEC, req_tile);
-      } // else: stay on the last stage; the redundant requests land in free
-        // slots and keep the in-flight count constant
-    };
-    int conv_ks = 0; // k stage of the stream stage converted next
-    auto advance_conv = [&]() __attribute__((always_inline)) {
-      conv_ks = conv_ks + 1 == num_k ? 0 : conv_ks + 1;
-    };
-    ab_vec a[TERMS][MT_], b[TERMS][NT_];
-    auto read_frags = [&](const int buf) __attribute__((always_inline)) {
-      const u32x4 *const sa =
-          frag + ((buf * NRB + wm * MT_) * TERMS) * 64 + lane;
-      const u32x4 *const sb =
-          frag + ((buf * NRB + RBA + wn * NT_) * TERMS) * 64 + lane;
-#pragma unroll
-      for (int j = 0; j < NT_; j++)
-#pragma unroll
-        for (int t = 0; t < TERMS; t++)
-          b[t][j] = __builtin_bit_cast(ab_vec, sb[(j * TERMS + t) * 64]);
-#pragma unroll
-      for (int i = 0; i < MT_; i++)
-#pragma unroll
-        for (int t = 0; t < TERMS; t++)
-          a[t][i] = __builtin_bit_cast(ab_vec, sa[(i * TERMS + t) * 64]);
-    };
-    float v[NQ][8];
-
-    // ---- prologue: fill the raw ring, convert stages 0 and 1, load stage 0
-    set_rows(VEC, 0);
-    for (int s = 0; s < NRAW; s++) {
-      issue(VEC, req_ks, s);
-      advance_request();
+    store_piece<MT_, NT_, MT_ % 2 == 0, MT_>(
+        out_value, Cb, p.ldc, tm * BM + wm * WM, tn * BN + wn * WN, M, N,
+        p.beta, lane);
+    if constexpr (RECYCLE) {
+      held = Cfg::BUF_BYTES - held;
+      if (STREAM)
+        read_frags(f[0], held);
+      asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
     }
-    wait_oldest_stage(VEC); // stage 0
-    load_raw(VEC, 0, v);
-    split_store(conv_ks, 0, v);
-    advance_conv();
-    issue(VEC, req_ks, 0); // stage NRAW into the slot stage 0 has left
-    advance_request();
-    wait_oldest_stage(VEC); // stage 1
-    load_raw(VEC, 1 % NRAW, v);
-    split_store(conv_ks, 1, v);
-    advance_conv();
-    asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
-    read_frags(0);
-    // every wave has stage 0 in registers before anybody overwrites its buffer
-    asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
-
-    // The k loop of a tile is a loop of its own so that the accumulators are
-    // touched by nothing but MFMAs inside it (they stay in AGPRs); the stream
-    // of requests and conversions runs on across the tile boundary.
-    int slot_conv = 2 % NRAW; // raw slot of stage s+2
-    int s = 0;                // stream index of the stage being multiplied
-    for (int cur_tile = 0; cur_tile < n_my; cur_tile++) {
-      clear_acc();
-      for (int cur_ks = 0; cur_ks < num_k; cur_ks++, s++) {
-        const int buf = s & 1;
-        // refill the slot that stage s+1 has left (it was converted last
-        // iteration): it is the one before slot_conv
-        issue(VEC, req_ks, slot_conv == 0 ? NRAW - 1 : slot_conv - 1);
-        advance_request();
-        wait_oldest_stage(VEC); // stage s+2 (past the end: a redundant tail stage)
-        load_raw(VEC, slot_conv, v);
-
-        auto sweep = [&](f32x4(&acc)[MT_][NT_], const int ta, const int tb) __attribute__((always_inline)) {
-#pragma unroll
-          for (int i = 0; i < MT_; i++)
-#pragma unroll
-            for (int j = 0; j < NT_; j++)
-              acc[i][j] = mfma(a[ta][i], b[tb][j], acc[i][j]);
-        };
-        auto multiply = [&]() __attribute__((always_inline)) {
-          // same products and, per accumulator, the same order as
-          // tcec_gemm_kernel.  (That kernel's tile-major issue order, a
-          // tile's products back to back, was measured here too: this kernel
-          // is not limited by the matrix core's power and ran 7 % slower.)
-          if constexpr (TERMS >= 3) {
-            sweep(acc_err, 2, 0);
-            sweep(acc_err, 0, 2);
-            sweep(acc_err, 1, 1);
-          }
-          if constexpr (TERMS >= 2) {
-            sweep(acc_err, 1, 0);
-            sweep(acc_err, 0, 1);
-          }
-          if (p.rn_main) {
-#pragma unroll
-            for (int i = 0; i < MT_; i++)
-#pragma unroll
-              for (int j = 0; j < NT_; j++)
-                acc_main[i][j] +=
-                    mfma(a[0][i], b[0][j], f32x4{0.f, 0.f, 0.f, 0.f});
-          } else {
-            sweep(acc_main, 0, 0);
-          }
-          // stage s+1 into the registers the MFMAs above have been fed from
-          read_frags(buf ^ 1);
-        };
-        // The two waves that share a SIMD run the matrix phase and the
-        // conversion phase in opposite order, so that one wave's MFMAs overlap
-        // the other's vector arithmetic instead of colliding with its MFMAs.
-        const bool matrix_first = NW < 8 || wave < NW / 2;
-        if (matrix_first)
-          multiply();
-        // stage s+2 over the buffer of stage s, which every wave took into
-        // registers before the last barrier
-        split_store(conv_ks, buf, v);
-        if (!matrix_first)
-          multiply();
-        advance_conv();
-        slot_conv = slot_conv + 1 == NRAW ? 0 : slot_conv + 1;
-        asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
-      }
-      store_tile(cur_tile);
-    }
-  };
-  if (vec_a && vec_b)
-    run(std::true_type{});
-  else
-    run(std::false_type{});
-  // the redundant tail requests still write LDS: drain them before the end
-  asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
+  }
 }
 
 } // namespace wmmae_gemm
