@@ -175,8 +175,15 @@ store_piece(const Value &value, float *const Cb, const long long ld,
     }
     return;
   }
+  // (a piece, or a column of its tiles, that lies outside C altogether is left
+  // by the wave as a whole: with the other edge tiles' per-lane guards alone the
+  // planes of K slices of 160x72x2051 cost 0.6 us more)
+  if (row0 >= M || col0 >= N)
+    return;
 #pragma unroll
   for (int j = 0; j < NT_; j++) {
+    if (col0 + 16 * j >= N)
+      return;
     const int col = col0 + 16 * j + c16;
     if (col >= N)
       continue;
