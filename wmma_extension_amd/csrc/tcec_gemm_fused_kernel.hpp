@@ -33,8 +33,8 @@
 //     workgroup are one stream, so that the next tile's stages are loaded and
 //     split while a tile is stored (STREAM).
 // Whole launches, two terms, before -> now: 1024^3 30.5 -> 16.2 us (two kernels
-// on packed operands 27.7), 512^3 16.7 -> 12.5, 256 entries of 256^3 with rows
-// contiguous 80.8 -> 54 (packed 96), 1024 entries of 100^3 35.2 -> 29.8; three
+// on packed operands 27.7), 512^3 16.7 -> 9.8, 7 x 777x1333x515 with rows
+// contiguous 127 -> 58 (packed 61), 1024 entries of 100^3 35.2 -> 29.8; three
 // terms: 1024^3 packed 27.3 -> 20.7.
 //
 // How an operand is read (chosen by the host for each operand; the two halves
