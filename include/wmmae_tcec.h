@@ -100,10 +100,11 @@ int wmmae_query(int what, long long *out);
  * `stream`; measured at 3 to 9 us a call on MI355X, which a product of 20 us
  * feels - keep a workspace across calls where calls are small).  Products
  * whose operand elements are used by few tiles (small m and n, or a short k;
- * an estimate of the paths' times decides; no K slices) are split inside the
- * GEMM kernel (as the reference's bgemm_kernel splits at fragment load,
+ * an estimate of the paths' times decides) are split inside the GEMM kernel
+ * (as the reference's bgemm_kernel splits at fragment load,
  * batch_gemm.cu:196-386): they use no workspace, allocate nothing and ignore
- * the workspace arguments.  Batches of medium-sized matrices and K-heavy
+ * the workspace arguments.  Where one of the other paths would cut K, that
+ * kernel makes the same slices itself, with the same bits.  Batches of medium-sized matrices and K-heavy
  * products with k contiguous in both operands run the packed path's GEMM
  * kernel on the fp32 operands directly (it splits them on their way into LDS):
  * no packed copy; the workspace then only holds K slices.  All paths give the
@@ -125,13 +126,17 @@ int wmmae_tcec_sgemm_workspace_bytes(int m, int n, int k, int batch, int policy,
  * reference, whose harness fixes one kernel configuration at compile time,
  * batch_gemm.cu:408-431, 659): *path = 0 the single kernel that splits the
  * operands on the fly (no workspace), 1 packed operands in the workspace,
- * 2 packed operands and K slices (when the workspace has room for them),
+ * 2 packed operands and K slices (when the workspace has room for them; or the
+ * same slices, without a workspace, inside the single kernel, where that is
+ * estimated to take less time),
  * 3 the packed path's GEMM kernel loading and splitting the fp32 operands
- * itself (no packed operands), 4 the same with K slices.  3 and 4 assume
+ * itself (no packed operands), 4 the same with K slices (or inside the single
+ * kernel, as 2).  3 and 4 assume
  * k contiguous in both operands ('T','N') and need k >= 4.
  * The answer is for op(A) = 'T', op(B) = 'N', whatever the leading dimensions
- * and bases.  Other layouts take 0, 1 or 2, and 0 more often: the single kernel
- * runs them at the same speed, the split pass of 1 and 2 does not. */
+ * and bases.  Other layouts take 0, 1 or 2, and the single kernel more often: it
+ * runs them at the same speed, the split pass of 1 and 2 does not.  Whichever
+ * kernel runs them, they have the bits of the packed path. */
 int wmmae_tcec_sgemm_path(int m, int n, int k, int batch, int policy, int flags,
                           int *path);
 

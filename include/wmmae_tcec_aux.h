@@ -54,10 +54,13 @@ int wmmae_direct_read_first(int tail, int k, int stage, int lane,
 /* Host only (no counterpart in the reference): the number of K slices
  * wmmae_tcec_sgemm* cuts a product into on the path it takes for these
  * arguments (flags as there, path flags included; a workspace of
- * wmmae_tcec_sgemm_workspace_bytes assumed).  1: K is not cut, or the single
- * kernel runs.  The two GEMM kernels plan their slices for their own tiles, so
- * the counts of the forced packed and the forced direct path may differ - and
- * with them the last bits of C, since the slices' partial sums are rounded. */
+ * wmmae_tcec_sgemm_workspace_bytes assumed), whichever kernel makes them.  1: K
+ * is not cut; always with WMMAE_FLAG_PATH_FUSED.  The two GEMM kernels plan their
+ * slices for their own tiles, so the counts of the forced packed and the forced
+ * direct path may differ - and with them the last bits of C, since the slices'
+ * partial sums are rounded.  Without a path flag the answer is for op(A) = 'T',
+ * op(B) = 'N'; products of other layouts are cut as the packed path cuts them,
+ * which is what the query answers with WMMAE_FLAG_PATH_PACKED. */
 int wmmae_tcec_sgemm_k_slices(int m, int n, int k, int batch, int policy,
                               int flags, int *slices);
 
@@ -66,8 +69,14 @@ int wmmae_tcec_sgemm_k_slices(int m, int n, int k, int batch, int policy,
  * leading dimensions and aligned bases: seconds[0] the single kernel,
  * seconds[1] split passes + GEMM on packed operands, seconds[2] the GEMM kernel
  * that splits the fp32 operands itself; infinity for a path the product cannot
- * take.  The smallest is the path wmmae_tcec_sgemm* takes.  For checking the
- * estimates against measured times. */
+ * take.  The smallest is the path wmmae_tcec_sgemm* takes for these layouts
+ * (none below the time the host needs to issue its launches).  For checking the
+ * estimates against measured times.  seconds[0] is more than a time in two
+ * cases: single products and batches of fewer than 16 take the single kernel
+ * only where it is well ahead, and their seconds[0] holds that factor (1.25,
+ * 1.4, 1.25 for one, two, three terms); and a product whose K the faster of the
+ * other two paths cuts does not run over an uncut K in the single kernel at all:
+ * its seconds[0] lies above that path's. */
 int wmmae_tcec_path_estimates(int m, int n, int k, int batch, int policy,
                               double *seconds);
 

@@ -350,3 +350,31 @@ def test_direct_kernel_reads_stay_inside_their_rows(h):
     assert h.wmmae_direct_read_first(1, 33, 2, 0, ctypes.byref(first)) == -1
     assert h.wmmae_direct_read_first(1, 33, 0, 64, ctypes.byref(first)) == -1
     assert h.wmmae_direct_read_first(1, 33, 0, 0, None) == -2
+
+
+def test_single_kernel_over_an_uncut_k_only_where_no_path_would_cut_it(h):
+    """Path 0 sums all of k in one chain of the matrix core's fp32 accumulators: it is taken only for
+    products whose K the faster of the other two paths leaves whole too.  The slice count of a cut
+    product is that path's, whichever kernel makes the slices."""
+    import random
+    est = (ctypes.c_double * 3)()
+    out = ctypes.c_int(-1)
+    rnd = random.Random(9)
+
+    def slices(args, flag):
+        status = h.wmmae_tcec_sgemm_k_slices(*args, flag, ctypes.byref(out))
+        return out.value if status == 0 else 1
+    seen = set()
+    for _ in range(4000):
+        m, n = int(2 ** rnd.uniform(3, 12)), int(2 ** rnd.uniform(3, 12))
+        k = 32 * int(2 ** rnd.uniform(0, 9)) + rnd.choice([0, 0, 4, 1])
+        args = (m, n, k, rnd.choice([1, 1, 2, 8, 64]), rnd.randrange(5))
+        assert h.wmmae_tcec_path_estimates(*args, est) == 0
+        assert h.wmmae_tcec_sgemm_path(*args, 0, ctypes.byref(out)) == 0
+        path = out.value
+        planned = slices(args, 8 if max(est[2], 11.5e-6) < max(est[1], 14.3e-6) else 2)
+        assert (path in (2, 4)) == (planned > 1), (args, path, planned)
+        assert slices(args, 0) == planned, (args, path, planned)
+        seen.add(path)
+    assert seen == {0, 1, 2, 3, 4}
+    assert slices((1024, 1024, 1024, 1, 0), 0) == 4 and slices((1024, 1024, 1024, 1, 2), 0) == 4

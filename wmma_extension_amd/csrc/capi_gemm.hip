@@ -3,6 +3,7 @@
 // translation units, one per policy.  Declarations and per-entry documentation
 // live in include/wmmae_tcec.h.
 #include "gemm_plan.hpp"
+#include <cmath>
 
 namespace {
 using namespace wmmae_driver;
@@ -42,6 +43,12 @@ __global__ void __launch_bounds__(256)
 // namespace fit.
 //   fused_ok : the single kernel is considered (fused_considered)
 //   rows     : an operand does not have k contiguous
+// The single kernel stands in for the faster of the other two, with that path's
+// K slices (SLICED in its head comment): the choice never changes a bit, and no
+// product is summed in a longer fp32 chain for being small.  (Taken by its time
+// alone, over an uncut K, it left 1024^3 in two fp16 terms with a relative
+// error of 2.2e-7 where the four slices give 1.3e-7, 8 x 320x321x12900 in three
+// bf16 terms of one sign with 5.8e-7 for 0.8e-7.)
 enum class Path { Fused, Packed, Direct };
 // (see PathRates::busy)
 inline double busy_factor(const fit::PathRates &r, const long long tiles) {
@@ -77,14 +84,39 @@ inline bool one_path_at_most(const int flags) {
 // Estimated time of a call on each path, in seconds; a path that cannot run
 // the product (or is not considered for it) has infinity.
 struct PathEstimates {
-  double fused, packed, direct;
+  double packed, direct;
+  Path base;          // the faster of the two ...
+  int slices;         // ... the K slices it makes, 1: none ...
+  double base_time;   // ... and its time, no less than issuing its launches takes
+  double fused;       // the single kernel with that cut of K
 };
 inline PathEstimates estimate_paths(const int m, const int n, const int k,
                                     const int batch, const int terms,
                                     const bool fused_ok, const bool rows,
                                     const bool direct_ok) {
   constexpr double kNever = std::numeric_limits<double>::infinity();
-  PathEstimates e{kNever, kNever, kNever};
+  PathEstimates e{kNever, kNever, Path::Packed, 1, kNever, kNever};
+  const auto finish = [&]() {
+    e.base_time = std::max(e.packed, fit::kCallFloor[1]);
+    const double direct = std::max(e.direct, fit::kCallFloor[2]);
+    if (direct < e.base_time) {
+      e.base = Path::Direct;
+      e.base_time = direct;
+    }
+    e.slices = choose_splits(terms, m, n, k, batch, e.base == Path::Direct);
+    if (!fused_ok)
+      return e;
+    if (e.slices > 1)
+      e.fused = fit::kFusedSlicedMargin *
+                fused_time(terms, m, n, k, batch, true, rows, e.slices);
+    else
+      e.fused = (rows || batch >= fit::kFusedTnMarginBatch
+                     ? 1.0
+                     : fit::kFusedTnMargin[terms - 1]) *
+                std::min(fused_time(terms, m, n, k, batch, true, rows),
+                         fused_time(terms, m, n, k, batch, false, rows));
+    return e;
+  };
   const fit::PathRates &p = fit::kPacked[terms - 1];
   const long long cus = device_cus();
   const int kti = static_cast<int>(ceil_div(k, 32));
@@ -95,12 +127,6 @@ inline PathEstimates estimate_paths(const int m, const int n, const int k,
   const long long tiles128 = ceil_div(m, 128) * ceil_div(n, 128) * batch;
   const long long tiles256 = ceil_div(m, 256) * ceil_div(n, 128) * batch;
 
-  if (fused_ok)
-    e.fused = (rows || batch >= fit::kFusedTnMarginBatch
-                   ? 1.0
-                   : fit::kFusedTnMargin[terms - 1]) *
-              std::min(fused_time(terms, m, n, k, batch, true, rows),
-                       fused_time(terms, m, n, k, batch, false, rows));
   const double split_pass = (4.0 + 2.0 * terms) * ab / p.split_bytes_per_s;
   const int splits = choose_splits(terms, m, n, k, batch);
   if (splits != 1) {
@@ -118,7 +144,7 @@ inline PathEstimates estimate_paths(const int m, const int n, const int k,
                       choose_splits(terms, m, n, k, batch, true), true)) *
               fit::kSlicedDirect[0][terms - 1] +
           fit::kSlicedDirect[1][terms - 1];
-    return e;
+    return finish();
   }
   // packed path: rounds in units of one 128x128 tile as gemm_by_size counts
   // them (a 256x128 tile 2.0 and a 128x128 tile 1.2 for one and two terms,
@@ -154,32 +180,34 @@ inline PathEstimates estimate_paths(const int m, const int n, const int k,
                       fit::kSlicedDirect[1][terms - 1]
                 : fit::kDirect[terms - 1].launch + std::max(d.tiles, d.bytes);
   }
-  return e;
+  return finish();
 }
-inline Path choose_path(const int m, const int n, const int k, const int batch,
-                        const int flags, const int terms, const int policy,
-                        const bool fused_ok, const bool rows,
-                        const bool direct_ok) {
+// How a product runs: the path whose bits it has, that path's K slices, and
+// whether the single kernel makes them.
+struct Choice {
+  Path path; // Path::Fused: the single kernel over an uncut K
+  int slices;
+  bool single;
+};
+inline Choice choose_path(const int m, const int n, const int k, const int batch,
+                          const int flags, const int terms, const int policy,
+                          const bool fused_ok, const bool rows,
+                          const bool direct_ok) {
   // (the round-to-nearest flag with a policy that has no such variant is
   // turned down by the packed path's dispatch)
   const bool rn_unsupported =
       (flags & WMMAE_FLAG_RN_MAIN) != 0 && policy != WMMAE_POLICY_F16_EC &&
       policy != WMMAE_POLICY_BF16X3_EC;
-  if (k <= 0 || rn_unsupported)
-    return Path::Packed;
-  PathEstimates e = estimate_paths(m, n, k, batch, terms, fused_ok, rows, direct_ok);
-  e.fused = std::max(e.fused, fit::kCallFloor[0]);
-  e.packed = std::max(e.packed, fit::kCallFloor[1]);
-  e.direct = std::max(e.direct, fit::kCallFloor[2]);
-  Path best = Path::Packed;
-  double t_best = e.packed;
-  if (e.fused < t_best) {
-    t_best = e.fused;
-    best = Path::Fused;
-  }
-  if (e.direct < t_best)
-    best = Path::Direct;
-  return best;
+  if (m <= 0 || n <= 0 || k <= 0 || batch <= 0)
+    return {Path::Packed, 1, false};
+  if (rn_unsupported)
+    return {Path::Packed, choose_splits(terms, m, n, k, batch), false};
+  const PathEstimates e =
+      estimate_paths(m, n, k, batch, terms, fused_ok, rows, direct_ok);
+  const double fused = std::max(e.fused, fit::kCallFloor[0]);
+  const bool single = e.base == Path::Direct ? fused <= e.base_time
+                                             : fused < e.base_time;
+  return {single && e.slices == 1 ? Path::Fused : e.base, e.slices, single};
 }
 // ('T','N') products with k % 4 != 0 and more than three stages stay with the
 // other paths, as the path query has always answered.
@@ -435,8 +463,8 @@ int sgemm_impl(const char transa, const char transb, const int m, const int n,
   const bool direct_ok = a_ks == 1 && b_ks == 1 &&
                          direct_possible(k, p.terms, flags, a_rs, b_rs);
   const int rn = flags & WMMAE_FLAG_RN_MAIN;
-  Path path = choose_path(m, n, k, batch, rn, p.terms, policy,
-                          rows || fused_considered(k), rows, direct_ok);
+  Path path = Path::Packed;
+  int slices = 1; // of the single kernel; a forced one does not cut K
   if ((flags & WMMAE_FLAG_PATH_DIRECT) != 0) {
     if (!direct_ok)
       return WMMAE_STATUS_NOT_SUPPORTED;
@@ -446,8 +474,11 @@ int sgemm_impl(const char transa, const char transb, const int m, const int n,
                    policy != WMMAE_POLICY_BF16X3_EC))
       return WMMAE_STATUS_NOT_SUPPORTED;
     path = Path::Fused;
-  } else if ((flags & WMMAE_FLAG_PATH_PACKED) != 0) {
-    path = Path::Packed;
+  } else if ((flags & WMMAE_FLAG_PATH_PACKED) == 0) {
+    const Choice c = choose_path(m, n, k, batch, rn, p.terms, policy,
+                                 rows || fused_considered(k), rows, direct_ok);
+    path = c.single ? Path::Fused : c.path;
+    slices = c.slices;
   }
   if (path == Path::Direct) {
     // the planes of the K slices are the only workspace this path uses
@@ -519,6 +550,8 @@ int sgemm_impl(const char transa, const char transb, const int m, const int n,
     q.batch = batch;
     q.a_source = fused_source(a_rs, a_ks, k);
     q.b_source = fused_source(b_rs, b_ks, k);
+    q.slice_stages =
+        slices > 1 ? static_cast<int>(ceil_div(packed_k_tiles(k), slices)) : 0;
     q.alpha = *alpha;
     q.beta = *beta;
     q.inv_scale = p.inv_scale;
@@ -660,20 +693,12 @@ int wmmae_tcec_sgemm_path(const int m, const int n, const int k,
   if (m < 0 || n < 0 || k < 0 || batch < 0 || !policy_info(policy, p) ||
       (flags & ~WMMAE_FLAG_RN_MAIN) != 0)
     return WMMAE_STATUS_INVALID_VALUE;
-  const bool any = m > 0 && n > 0 && k > 0 && batch > 0;
-  const bool slices = any && choose_splits(p.terms, m, n, k, batch) > 1;
-  switch (choose_path(m, n, k, batch, flags, p.terms, policy,
-                      fused_considered(k), false,
-                      direct_possible(k, p.terms, flags, 1, 1))) {
-  case Path::Fused:
-    *path = 0;
-    break;
-  case Path::Direct:
-    *path = any && choose_splits(p.terms, m, n, k, batch, true) > 1 ? 4 : 3;
-    break;
-  default:
-    *path = slices ? 2 : 1;
-  }
+  const Choice c = choose_path(m, n, k, batch, flags, p.terms, policy,
+                               fused_considered(k), false,
+                               direct_possible(k, p.terms, flags, 1, 1));
+  *path = c.path == Path::Fused    ? 0
+          : c.path == Path::Direct ? (c.slices > 1 ? 4 : 3)
+                                   : (c.slices > 1 ? 2 : 1);
   return WMMAE_STATUS_SUCCESS;
 }
 
@@ -688,7 +713,11 @@ int wmmae_tcec_path_estimates(const int m, const int n, const int k,
   const PathEstimates e = estimate_paths(m, n, k, batch, p.terms,
                                          fused_considered(k), false,
                                          direct_possible(k, p.terms, 0, 1, 1));
-  seconds[0] = e.fused;
+  // (cut products: see the header)
+  seconds[0] = e.slices == 1 || std::isinf(e.fused)
+                   ? e.fused
+                   : std::max(fused_time(p.terms, m, n, k, batch, true, false),
+                              1.01 * e.base_time);
   seconds[1] = e.packed;
   seconds[2] = e.direct;
   return WMMAE_STATUS_SUCCESS;
@@ -725,19 +754,17 @@ int wmmae_tcec_sgemm_k_slices(const int m, const int n, const int k,
   if (m == 0 || n == 0 || k == 0 || batch == 0)
     return WMMAE_STATUS_SUCCESS;
   const bool direct_ok = direct_possible(k, p.terms, flags, 1, 1);
-  Path path = choose_path(m, n, k, batch, flags & WMMAE_FLAG_RN_MAIN, p.terms,
-                          policy, fused_considered(k), false, direct_ok);
   if ((flags & WMMAE_FLAG_PATH_DIRECT) != 0) {
     if (!direct_ok)
       return WMMAE_STATUS_NOT_SUPPORTED;
-    path = Path::Direct;
-  } else if ((flags & WMMAE_FLAG_PATH_FUSED) != 0) {
-    path = Path::Fused;
+    *slices = choose_splits(p.terms, m, n, k, batch, true);
   } else if ((flags & WMMAE_FLAG_PATH_PACKED) != 0) {
-    path = Path::Packed;
+    *slices = choose_splits(p.terms, m, n, k, batch);
+  } else if ((flags & WMMAE_FLAG_PATH_FUSED) == 0) {
+    *slices = choose_path(m, n, k, batch, flags & WMMAE_FLAG_RN_MAIN, p.terms,
+                          policy, fused_considered(k), false, direct_ok)
+                  .slices;
   }
-  if (path != Path::Fused)
-    *slices = choose_splits(p.terms, m, n, k, batch, path == Path::Direct);
   return WMMAE_STATUS_SUCCESS;
 }
 

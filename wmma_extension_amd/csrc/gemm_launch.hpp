@@ -271,11 +271,11 @@ template <class MT, int TERMS> int per_cu_by_shape(const int shape) {
   }
 }
 template <class T, int TERMS, int BM, int BN, int CW, int PW, int DEPTH, bool RN,
-          bool STREAM>
+          bool STREAM, bool SLICED>
 int launch_fused_grid(const FusedArgs &f, const long long grid) {
   using Cfg = wmmae_gemm::FusedConfig<TERMS, BM, BN, CW, PW>;
   auto kernel = wmmae_gemm::tcec_gemm_fused_kernel<T, TERMS, BM, BN, CW, PW,
-                                                   DEPTH, RN, STREAM>;
+                                                   DEPTH, RN, STREAM, SLICED>;
   static std::atomic<unsigned long long> lds_allowed{0};
   WMMAE_HIP_TRY(allow_dynamic_lds(reinterpret_cast<const void *>(kernel),
                                   Cfg::LDS_BYTES, lds_allowed));
@@ -284,7 +284,8 @@ int launch_fused_grid(const FusedArgs &f, const long long grid) {
   return launch_status();
 }
 
-template <class T, int TERMS, int BM, int BN, int CW, int PW, int DEPTH, bool RN>
+template <class T, int TERMS, int BM, int BN, int CW, int PW, int DEPTH, bool RN,
+          bool SLICED>
 int launch_fused(FusedArgs f) {
   wmmae_gemm::FusedParams &p = f.p;
   p.tiles_m = static_cast<int>(ceil_div(p.M, BM));
@@ -306,18 +307,20 @@ int launch_fused(FusedArgs f) {
   // one workgroup per tile when all of them are resident together, else
   // persistent workgroups
   if (spread <= resident)
-    return launch_fused_grid<T, TERMS, BM, BN, CW, PW, DEPTH, RN, false>(f,
-                                                                         spread);
-  return launch_fused_grid<T, TERMS, BM, BN, CW, PW, DEPTH, RN, true>(
+    return launch_fused_grid<T, TERMS, BM, BN, CW, PW, DEPTH, RN, false, SLICED>(
+        f, spread);
+  return launch_fused_grid<T, TERMS, BM, BN, CW, PW, DEPTH, RN, true, SLICED>(
       f, p.grouped ? 8 * per_xcd : resident);
 }
 
 template <class T, int TERMS, bool RN> int fused_by_size(const FusedArgs &f) {
+  if (f.p.slice_stages > 0) // (64x64 only: see fused_time)
+    return launch_fused<T, TERMS, 64, 64, 4, 4, 4, RN, true>(f);
   if (fused_small_tiles(TERMS, f.p.M, f.p.N, f.p.K, f.p.batch,
                         f.p.a_source != wmmae_gemm::kFusedKRows ||
                             f.p.b_source != wmmae_gemm::kFusedKRows))
-    return launch_fused<T, TERMS, 64, 64, 4, 4, 4, RN>(f);
-  return launch_fused<T, TERMS, 128, 128, 8, 4, 2, RN>(f);
+    return launch_fused<T, TERMS, 64, 64, 4, 4, 4, RN, false>(f);
+  return launch_fused<T, TERMS, 128, 128, 8, 4, 2, RN, false>(f);
 }
 
 // The table of one policy: split tag T, MFMA element type MT, stored terms; RN:

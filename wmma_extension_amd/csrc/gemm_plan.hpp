@@ -253,6 +253,15 @@ constexpr FusedRates kFused[3] = {
 // speak for, go by the times alone.
 constexpr double kFusedTnMargin[3] = {1.25, 1.4, 1.25}; // by terms
 constexpr int kFusedTnMarginBatch = 16;
+// Adding a K slice to the double-precision sums, for the workgroups of a compute
+// unit at a time: 110 products run with the cut and uncut, 0.17 us in the median
+// (one workgroup a unit), 0.10 (two), 3 % of a call.
+constexpr double kFusedSliceFold = 0.15e-6;
+// A product whose K is cut goes to the single kernel where this factor on its
+// time still leaves it ahead: of those 110, taken by the times alone, five ran
+// 1.06 to 1.27 times slower than the path it stood in for, their estimates 0.87
+// to 0.99 of that path's; all of them 0.71 of its time in the median.
+constexpr double kFusedSlicedMargin = 1.1;
 // Its workgroups that are resident on a compute unit: 12 waves of up to 168
 // registers (128x128), twice 8 waves of up to 128.
 constexpr int fused_resident(const int bm) { return bm > 64 ? 1 : 2; }
@@ -416,9 +425,12 @@ struct FusedArgs {
 };
 
 // Time of a call of the single kernel with its 64x64 or 128x128 tiles.  `rows`:
-// an operand does not have k contiguous.
+// an operand does not have k contiguous.  `slices`: K slices made in the kernel,
+// more than one with 64x64 tiles only (the double-precision sums of a 128x128
+// tile fit neither the registers nor LDS).
 inline double fused_time(const int terms, const int m, const int n, const int k,
-                         const int batch, const bool small, const bool rows) {
+                         const int batch, const bool small, const bool rows,
+                         const int slices = 1) {
   const fit::FusedRates &f = fit::kFused[terms - 1];
   const double kt = static_cast<double>(ceil_div(k, 32));
   const long long cus = device_cus();
@@ -433,7 +445,10 @@ inline double fused_time(const int terms, const int m, const int n, const int k,
     time = static_cast<double>(rounds / 2) *
                (kt * f.pair64 * factor * (1.0 + f.busy64 * full) +
                 f.pair_tile64) +
-           static_cast<double>(rounds % 2) * (kt * f.stage64 * factor + f.tile64);
+           static_cast<double>(rounds % 2) * (kt * f.stage64 * factor + f.tile64) +
+           (slices > 1 ? static_cast<double>(rounds) * slices *
+                             fit::kFusedSliceFold
+                       : 0.);
   } else {
     time = static_cast<double>(rounds) *
            (kt * f.stage128 * (rows ? f.rows128 : 1.0) *

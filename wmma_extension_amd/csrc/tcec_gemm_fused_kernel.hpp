@@ -82,6 +82,7 @@ struct FusedParams {
   // launcher for 8 or more entries that spread evenly enough)
   int grouped;
   int a_source, b_source; // FusedSource
+  int slice_stages; // SLICED: k stages of a slice
   float alpha, beta, inv_scale;
 };
 
@@ -103,11 +104,22 @@ template <int TERMS, int BM, int BN, int CW, int PW> struct FusedConfig {
 //             (the cursor's step to the next tile costs a stage 5 to 10 %, a
 //             pipeline refill per tile 2 to 3 us: 4096 tiles of 64x64 at k = 128
 //             46.6 -> 30.3 us)
+//   SLICED  : K is cut into slices of p.slice_stages stages.  A slice starts from
+//             cleared accumulators, its sums are rounded to fp32 as the plane of
+//             a slice in memory is, and the slices are added in double precision
+//             in ascending order: the bits of the other kernels' K slices
+//             (reduce_splits_kernel), without planes, fold launch or workspace.
+//             1024^3 in four slices, whole calls: two fp16 terms 17.0 us (16.1
+//             over an uncut K, 27.2 with packed operands, their GEMM and its
+//             fold), three bf16 terms 22.9 (21.8, 27.2)
 //   DEPTH   : stages of fp32 values in flight in registers (even: the LDS
 //             buffer and fragment set of a step are then compile-time choices)
 template <class T, int TERMS, int BM, int BN, int CW, int PW, int DEPTH,
-          bool RN_MAIN, bool STREAM>
-__global__ void __launch_bounds__(64 * (CW + PW))
+          bool RN_MAIN, bool STREAM, bool SLICED>
+// (SLICED: the double-precision sums must not cost the second workgroup of a
+// compute unit, four waves a SIMD; three bf16 terms with RN_MAIN took 130
+// registers of the 128 that leaves)
+__global__ void __launch_bounds__(64 * (CW + PW), SLICED ? 4 : 1)
     tcec_gemm_fused_kernel(const FusedParams p) {
   using traits = mtk::wmma::tcec::detail::split_traits<T>;
   using S = typename traits::storage;
@@ -123,7 +135,8 @@ __global__ void __launch_bounds__(64 * (CW + PW))
   // Two sets of fragments where they fit the registers that two workgroups (64x64
   // tile) or three waves a SIMD (128x128) leave a wave; else one set, a term's
   // fragments refilled for the next stage once its last product has been issued.
-  constexpr bool RECYCLE = TERMS == 3 || BM > 64;
+  // (SLICED: the double-precision sums take the registers of the second set)
+  constexpr bool RECYCLE = TERMS == 3 || BM > 64 || SLICED;
 
   extern __shared__ __attribute__((aligned(1024))) unsigned char lds_raw[];
 
@@ -162,6 +175,22 @@ __global__ void __launch_bounds__(64 * (CW + PW))
   };
 
   f32x4 acc_main[MT_][NT_], acc_err[MT_][NT_];
+  auto clear_acc = [&]() __attribute__((always_inline)) {
+#pragma unroll
+    for (int i = 0; i < MT_; i++)
+#pragma unroll
+      for (int j = 0; j < NT_; j++) {
+        acc_main[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+        acc_err[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+      }
+  };
+  // the accumulated value of tile (i, j), before alpha
+  auto folded = [&](const int i, const int j) {
+    f32x4 o = acc_main[i][j];
+    if constexpr (TERMS >= 2)
+      o = epilogue_fold(o, acc_err[i][j], p.inv_scale);
+    return o;
+  };
   struct Frags {
     ab_vec a[TERMS][MT_], b[TERMS][NT_];
   };
@@ -560,25 +589,45 @@ __global__ void __launch_bounds__(64 * (CW + PW))
       held = next;
     }
   };
+  typedef double f64x4 __attribute__((ext_vector_type(4)));
   for (int tile = 0; tile < n_my; tile++) {
+    f64x4 sum[SLICED ? MT_ : 1][SLICED ? NT_ : 1]; // of the slices
+    if constexpr (SLICED) {
 #pragma unroll
-    for (int i = 0; i < MT_; i++)
+      for (int i = 0; i < MT_; i++)
 #pragma unroll
-      for (int j = 0; j < NT_; j++) {
-        acc_main[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
-        acc_err[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+        for (int j = 0; j < NT_; j++)
+          sum[i][j] = f64x4{0., 0., 0., 0.};
+      int s = num_k; // stages left of the tile
+      while (s > 0) {
+        clear_acc();
+        const bool last = s <= p.slice_stages;
+        const int n = last ? s - 1 : p.slice_stages;
+        for (int x = 0; x < n; x++)
+          step(ic<0>{}, std::false_type{});
+        if (last)
+          step(ic<0>{}, std::true_type{});
+        s -= p.slice_stages;
+#pragma unroll
+        for (int i = 0; i < MT_; i++)
+#pragma unroll
+          for (int j = 0; j < NT_; j++)
+            sum[i][j] += __builtin_convertvector(folded(i, j), f64x4);
       }
-    int s = num_k;
-    for (; s > (RECYCLE ? 2 : 1); s -= 2) {
-      step(ic<0>{}, std::false_type{});
-      step(ic<1>{}, std::false_type{});
-    }
-    if (RECYCLE && s == 2)
-      step(ic<0>{}, std::false_type{});
-    if (RECYCLE || s == 1) { // the next tile's first fragments arrive in the other set
-      step(ic<0>{}, std::true_type{});
-      if constexpr (!RECYCLE)
-        f[0] = f[1];
+    } else {
+      clear_acc();
+      int s = num_k;
+      for (; s > (RECYCLE ? 2 : 1); s -= 2) {
+        step(ic<0>{}, std::false_type{});
+        step(ic<1>{}, std::false_type{});
+      }
+      if (RECYCLE && s == 2)
+        step(ic<0>{}, std::false_type{});
+      if (RECYCLE || s == 1) { // the next tile's first fragments arrive in the other set
+        step(ic<0>{}, std::true_type{});
+        if constexpr (!RECYCLE)
+          f[0] = f[1];
+      }
     }
     int entry, tm, tn;
     decode(tile, entry, tm, tn);
@@ -588,10 +637,10 @@ __global__ void __launch_bounds__(64 * (CW + PW))
                           : p.C + static_cast<long long>(entry) * p.c_bs;
     const float alpha = p.alpha;
     const auto out_value = [&](const int i, const int j) {
-      f32x4 o = acc_main[i][j];
-      if constexpr (TERMS >= 2)
-        o = epilogue_fold(o, acc_err[i][j], p.inv_scale);
-      return o * alpha;
+      if constexpr (SLICED)
+        return __builtin_convertvector(sum[i][j], f32x4) * alpha;
+      else
+        return folded(i, j) * alpha;
     };
     store_piece<MT_, NT_, MT_ % 2 == 0, MT_>(
         out_value, Cb, p.ldc, tm * BM + wm * WM, tn * BN + wn * WN, M, N,
