@@ -378,3 +378,16 @@ def test_single_kernel_over_an_uncut_k_only_where_no_path_would_cut_it(h):
         seen.add(path)
     assert seen == {0, 1, 2, 3, 4}
     assert slices((1024, 1024, 1024, 1, 0), 0) == 4 and slices((1024, 1024, 1024, 1, 2), 0) == 4
+
+
+def test_products_of_the_single_kernel_need_no_workspace(h):
+    """Products of short k, and batches, that have always run in one launch without a workspace: the
+    path query must go on answering 0 for them (packed operands would turn down a call whose workspace
+    does not hold them)."""
+    out = ctypes.c_int(-1)
+    for args in ((800, 2016, 160, 4, 2, 0), (2634, 1516, 256, 1, 0, 0), (3424, 1056, 128, 2, 2, 0),
+                 (1120, 2272, 288, 1, 3, 0), (3840, 3264, 32, 3, 0, 1), (832, 448, 288, 15, 0, 1),
+                 (4221, 4924, 92, 4, 0, 0), (2912, 1856, 32, 12, 4, 0), (4768, 608, 160, 4, 0, 0),
+                 (1760, 192, 608, 8, 0, 0), (3584, 4256, 64, 1, 0, 1), (1376, 4576, 128, 15, 2, 0)):
+        assert h.wmmae_tcec_sgemm_path(*args, ctypes.byref(out)) == 0
+        assert out.value == 0, args

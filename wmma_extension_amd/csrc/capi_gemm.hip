@@ -110,9 +110,9 @@ inline PathEstimates estimate_paths(const int m, const int n, const int k,
       e.fused = fit::kFusedSlicedMargin *
                 fused_time(terms, m, n, k, batch, true, rows, e.slices);
     else
-      e.fused = (rows || batch >= fit::kFusedTnMarginBatch
-                     ? 1.0
-                     : fit::kFusedTnMargin[terms - 1]) *
+      e.fused = (!rows && batch == 1 && k >= fit::kFusedTnMarginK
+                     ? fit::kFusedTnMargin[terms - 1]
+                     : 1.0) *
                 std::min(fused_time(terms, m, n, k, batch, true, rows),
                          fused_time(terms, m, n, k, batch, false, rows));
     return e;
