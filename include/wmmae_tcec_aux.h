@@ -72,22 +72,21 @@ int wmmae_tcec_sgemm_k_slices(int m, int n, int k, int batch, int policy,
  * take.  The smallest is the path wmmae_tcec_sgemm* takes for these layouts
  * (none below the time the host needs to issue its launches).  For checking the
  * estimates against measured times.  seconds[0] is more than a time in two
- * cases: one product (batch 1) of 512 of k or more takes the single kernel only
- * where it is well ahead, and its seconds[0] holds that factor (1.25, 1.4, 1.25
- * for one, two, three terms); and a product whose K the faster of the
- * other two paths cuts does not run over an uncut K in the single kernel at all:
- * its seconds[0] lies above that path's. */
+ * cases: products of at least 1024 x 1024 x 512, and fewer than 16 entries, take
+ * the single kernel only where it is well ahead, and their seconds[0] holds that
+ * factor (1.25, 1.4, 1.25 for one, two, three terms); and a product whose K the
+ * faster of the other two paths cuts does not run over an uncut K in the single
+ * kernel at all: its seconds[0] lies above that path's. */
 int wmmae_tcec_path_estimates(int m, int n, int k, int batch, int policy,
                               double *seconds);
 
 /* Measurement hook (no counterpart in the reference): the calling thread's
  * next wmmae_tcec_sgemm* / wmmae_tcec_gemm_packed calls record `begin_event`
- * on their stream right before the MFMA GEMM kernel of the packed or the direct
- * path and `end_event` right after it (after the fold of its K slices, where
- * there is one), so that a caller can time that kernel inside a whole call
+ * on their stream right before the MFMA GEMM kernel of the path they take and
+ * `end_event` right after it (after the fold of its K slices, where there is
+ * one), so that a caller can time that kernel inside a whole call
  * (hipEventElapsedTime after the events have completed).  Both hipEvent_t, or
- * both NULL to switch the hook off.  The single-kernel ("fused") path records
- * nothing.  The events stay the caller's. */
+ * both NULL to switch the hook off.  The events stay the caller's. */
 int wmmae_tcec_time_gemm_kernel(void *begin_event, void *end_event);
 
 /* Test hook (no counterpart in the reference): the calling thread's next

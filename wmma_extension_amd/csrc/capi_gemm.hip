@@ -110,7 +110,7 @@ inline PathEstimates estimate_paths(const int m, const int n, const int k,
       e.fused = fit::kFusedSlicedMargin *
                 fused_time(terms, m, n, k, batch, true, rows, e.slices);
     else
-      e.fused = (!rows && batch == 1 && k >= fit::kFusedTnMarginK
+      e.fused = (!rows && fit::fused_tn_margin(m, n, k, batch)
                      ? fit::kFusedTnMargin[terms - 1]
                      : 1.0) *
                 std::min(fused_time(terms, m, n, k, batch, true, rows),

@@ -245,16 +245,20 @@ constexpr FusedRates kFused[3] = {
      0.551e-6, 2.12e-6, 0.522, 1.157, 4.74e12},
     {5.2e-6, 0.500e-6, 0.41e-6, 0.601e-6, 1.70e-6, 0.465, 1.101,
      0.909e-6, 2.02e-6, 0.434, 1.084, 3.95e12}};
-// One ('T','N') product of 512 of k or more takes the single kernel only where it
-// is well ahead: its time counts this much there.  The path query answers for
-// exactly these, and its answers for them are kept (1160x1544x1056, two terms:
-// packed operands, though the single kernel takes 0.8 of the time).  All others
-// go by the times alone: on batches and on shorter k the factor turned away
-// products the single kernel takes 0.81 of the packed and 0.78 of the direct
-// path's time for (medians of 63; 143 in all, where it is 0.65 to 1.18 of the
-// path taken, above 1.03 for three), and made them need a workspace.
+// ('T','N') products of at least 1024 x 1024 x 512, and fewer than 16 entries, take
+// the single kernel only where it is well ahead: its time counts this much there.
+// The path query answers for exactly these, and its answers for them are kept
+// (1160x1544x1056, two terms: packed operands, though the single kernel takes 0.8
+// of the time).  All others go by the times alone: on smaller outputs and shorter
+// k the factor turned away products the single kernel takes 0.81 of the packed
+// and 0.78 of the direct path's time for (medians of 63; 143 in all, where it is
+// 0.65 to 1.18 of the path taken, above 1.03 for three), and made them need a
+// workspace.
 constexpr double kFusedTnMargin[3] = {1.25, 1.4, 1.25}; // by terms
-constexpr int kFusedTnMarginK = 512;
+constexpr bool fused_tn_margin(const int m, const int n, const int k,
+                               const int batch) {
+  return m >= 1024 && n >= 1024 && k >= 512 && batch < 16;
+}
 // Adding a K slice to the double-precision sums, for the workgroups of a compute
 // unit at a time: 110 products run with the cut and uncut, 0.17 us in the median
 // (one workgroup a unit), 0.10 (two), 3 % of a call.
