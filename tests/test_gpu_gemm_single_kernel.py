@@ -66,3 +66,25 @@ def test_strides_beyond_the_offsets_of_a_load(tc, dev):
     longer fits its 32 bits)."""
     for ta, tb, m, n, k in (("T", "N", 5, 40, 36), ("N", "T", 40, 5, 6), ("N", "N", 33, 3, 5)):
         _same_bits(tc, dev, ta, tb, m, n, k, 1, 0, 0, (1 << 24) + 1, 0, 0.0)
+
+
+def test_events_around_the_single_kernel(tc, dev):
+    """wmmae_tcec_time_gemm_kernel on products that the driver gives to the single kernel, which a caller
+    of another layout than 'T','N' cannot ask for: the events enclose it, nearly all of the call."""
+    for policy, k in ((2, 515), (0, 900)):
+        m, n, batch = 777, 1333, 7
+        A, lda = _operand(torch.Generator().manual_seed(1), dev, batch, m, k, False, 0, 0)
+        B, ldb = _operand(torch.Generator().manual_seed(2), dev, batch, n, k, True, 0, 0)
+        C = torch.empty((batch, n, m), device=dev)
+        e0, e1, w0, w1 = (torch.cuda.Event(enable_timing=True) for _ in range(4))
+        inner, whole = [], []
+        for _ in range(5):
+            w0.record()
+            with tc.timed_gemm_kernel(e0, e1):
+                tc.sgemm_strided_batched("N", "N", m, n, k, 1.0, A, lda, A.stride(0), B, ldb, B.stride(0), 0.0, C, m,
+                                         m * n, batch, policy)
+            w1.record()
+            torch.cuda.synchronize()
+            inner.append(e0.elapsed_time(e1))
+            whole.append(w0.elapsed_time(w1))
+        assert 0.3 * min(whole) < min(inner) <= min(whole), (inner, whole)

@@ -279,9 +279,14 @@ int launch_fused_grid(const FusedArgs &f, const long long grid) {
   static std::atomic<unsigned long long> lds_allowed{0};
   WMMAE_HIP_TRY(allow_dynamic_lds(reinterpret_cast<const void *>(kernel),
                                   Cfg::LDS_BYTES, lds_allowed));
+  if (t_gemm_begin != nullptr)
+    WMMAE_HIP_TRY(hipEventRecord(t_gemm_begin, f.stream));
   hipLaunchKernelGGL(kernel, dim3(static_cast<unsigned>(grid)),
                      dim3(Cfg::NTHREADS), Cfg::LDS_BYTES, f.stream, f.p);
-  return launch_status();
+  const int st = launch_status();
+  if (st == WMMAE_STATUS_SUCCESS && t_gemm_end != nullptr)
+    WMMAE_HIP_TRY(hipEventRecord(t_gemm_end, f.stream));
+  return st;
 }
 
 template <class T, int TERMS, int BM, int BN, int CW, int PW, int DEPTH, bool RN,

@@ -149,7 +149,7 @@ def path_estimates(m, n, k, batch=1, policy=Policy.F16_EC):
 
 
 class timed_gemm_kernel:
-    """Within the block, this thread's packed- and direct-path calls record `begin` / `end`
+    """Within the block, this thread's GEMM calls record `begin` / `end`
     (torch.cuda.Event with timing) right before and after their MFMA GEMM kernel:
     begin.elapsed_time(end) after a synchronisation is that kernel's time inside the whole call."""
 
