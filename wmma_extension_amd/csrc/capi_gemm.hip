@@ -107,7 +107,9 @@ inline PathEstimates estimate_paths(const int m, const int n, const int k,
     if (!fused_ok)
       return e;
     if (e.slices > 1)
-      e.fused = fit::kFusedSlicedMargin *
+      e.fused = (e.base == Path::Direct
+                     ? fit::kFusedSlicedDirectMargin[terms - 1]
+                     : fit::kFusedSlicedMargin) *
                 fused_time(terms, m, n, k, batch, true, rows, e.slices);
     else
       e.fused = (!rows && fit::fused_tn_margin(m, n, k, batch)

@@ -264,10 +264,13 @@ constexpr bool fused_tn_margin(const int m, const int n, const int k,
 // (one workgroup a unit), 0.10 (two), 3 % of a call.
 constexpr double kFusedSliceFold = 0.15e-6;
 // A product whose K is cut goes to the single kernel where this factor on its
-// time still leaves it ahead: of those 110, taken by the times alone, five ran
-// 1.06 to 1.27 times slower than the path it stood in for, their estimates 0.87
-// to 0.99 of that path's; all of them 0.71 of its time in the median.
+// time still leaves it ahead.  In place of packed operands: of 120 products taken
+// with it, 0.72 of their time in the median, none above 1.02.  In place of the
+// direct kernel (by terms), whose one launch on 256x128 tiles loses least to long
+// k: with 1.1 there too, 15 of 70 products that the larger factor turns away ran
+// 1.03 to 1.74 times slower than the direct kernel, most of them with one term.
 constexpr double kFusedSlicedMargin = 1.1;
+constexpr double kFusedSlicedDirectMargin[2] = {1.25, 1.4};
 // Its workgroups that are resident on a compute unit: 12 waves of up to 168
 // registers (128x128), twice 8 waves of up to 128.
 constexpr int fused_resident(const int bm) { return bm > 64 ? 1 : 2; }
