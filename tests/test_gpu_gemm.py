@@ -643,8 +643,8 @@ def test_api_level_gemm_fp32_policy(tc, orc, dev):
 
 def test_pointer_array_entries_with_any_alignment(tc, orc, dev):
     """Pointer-array entries that are only 4-byte aligned (matrices carved out of a
-    larger buffer at odd offsets): the fused kernel finds out by itself and falls back
-    to 4-byte requests; results equal the aligned call bit for bit."""
+    larger buffer at odd offsets): the kernels read 16 bytes at any alignment a float can
+    have; results equal the aligned call bit for bit."""
     batch, m, n, k = 9, 72, 40, 96
     rng = np.random.default_rng(123)
     A = rng.standard_normal((batch, m, k)).astype(np.float32)

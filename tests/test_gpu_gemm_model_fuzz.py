@@ -77,7 +77,7 @@ def test_random_products_have_the_bits_of_the_model(tc, orc, dev, seed):
             got = dC.cpu().numpy()
             assert (got[:, m:] == 7.0).all(), (case, path)
             if path == 0 and (pad % 4 != 0 or (ta, tb) != ("T", "N")):
-                continue            # (the count the query reports holds for 'T', 'N' and tight leading dimensions)
+                continue            # (the count the query reports without a path flag holds for 'T', 'N')
             if slices not in models:
                 models[slices] = orc.epilogue(_model(orc, A, B, kind, ec, slices, rn), alpha, beta, C)
             want = models[slices]

@@ -76,8 +76,7 @@ def test_random_products_on_every_path(tc, dev, seed):
             res[flag] = C
         chosen = {0: FUSED, 1: PACKED, 2: PACKED, 3: DIRECT, 4: DIRECT}[tc.sgemm_path(m, n, k, batch, policy, 0)]
         if (ta, tb) == ("T", "N") and pad % 4 == 0:
-            # (the path query assumes op(A) = 'T', op(B) = 'N', tight leading dimensions and
-            # aligned bases: what the kernels can read 16 bytes at a time depends on those)
+            # (the path query answers for op(A) = 'T', op(B) = 'N')
             assert torch.equal(res[0], res[chosen]), (c, chosen)
         # (a single large product may also cut K for the tiles of a partly empty last round, with
         # planes in the workspace: those tiles then sum in another order)

@@ -68,6 +68,45 @@ def test_strides_beyond_the_offsets_of_a_load(tc, dev):
         _same_bits(tc, dev, ta, tb, m, n, k, 1, 0, 0, (1 << 24) + 1, 0, 0.0)
 
 
+@pytest.mark.parametrize("ta,tb", [("T", "N"), ("N", "N"), ("N", "T"), ("T", "T")])
+def test_pointer_arrays_in_every_layout(tc, dev, ta, tb):
+    """Matrices by pointer, scattered at every alignment a float can have, with one and with several tiles
+    per workgroup: the bits of the strided call on the same matrices."""
+    for m, n, k, batch, policy in ((70, 50, 77, 9, 0), (40, 60, 515, 3, 2), (61, 50, 37, 600, 0), (200, 150, 3, 300, 3)):
+        g = torch.Generator(device="cpu").manual_seed(m + k)
+        A, lda = _operand(g, dev, batch, m, k, ta == "T", 1, 0)
+        B, ldb = _operand(g, dev, batch, n, k, tb == "N", 2, 0)
+        C0 = (torch.rand((batch, n, m), generator=g) * 2 - 1).to(dev)
+        want = C0.clone()
+        tc.sgemm_strided_batched(ta, tb, m, n, k, 1.5, A, lda, A.stride(0), B, ldb, B.stride(0), -0.5, want, m, m * n,
+                                 batch, policy, FUSED)
+        rooms, arrays = [], []
+        for i, X in enumerate((A, B, C0)):
+            size = X[0].numel() + 11 + 2 * i                     # no multiple of four floats: all alignments
+            room = torch.full((batch, size), float("nan") if i < 2 else 7.0, device=dev)
+            order = [(5 * e + i) % batch if batch % 5 else batch - 1 - e for e in range(batch)]
+            for e in range(batch):
+                room[order[e], i + 1:i + 1 + X[0].numel()] = X[e].reshape(-1)
+            base = room.data_ptr()
+            arrays.append(torch.tensor([base + 4 * (order[e] * size + i + 1) for e in range(batch)], dtype=torch.int64,
+                                       device=dev))
+            rooms.append((room, order))
+        tc.sgemm_batched(ta, tb, m, n, k, 1.5, arrays[0], lda, arrays[1], ldb, -0.5, arrays[2], m, batch, policy, FUSED)
+        room, order = rooms[2]
+        got = room[order, 3:3 + n * m].view(batch, n, m)
+        assert torch.equal(got.view(torch.int32), want.view(torch.int32)), (ta, tb, m, n, k, batch)
+        assert (room[:, :3] == 7.0).all() and (room[:, 3 + n * m:] == 7.0).all()
+
+
+@pytest.mark.parametrize("policy", [0, 1, 2])
+def test_element_by_element_with_several_tiles_per_workgroup(tc, dev, policy):
+    """k < 4 with k contiguous (64-bit addresses, one element a load), more tiles than resident workgroups:
+    64x64 and 128x128 tiles, shared list and entries owned by an XCD."""
+    for m, n, k, batch in ((60, 50, 3, 1100), (60, 50, 1, 700), (130, 100, 2, 700), (1500, 1300, 3, 3),
+                           (4000, 3000, 2, 1)):
+        _same_bits(tc, dev, "T", "N", m, n, k, batch, policy, 0, 1, 1, 0.5)
+
+
 def test_events_around_the_single_kernel(tc, dev):
     """wmmae_tcec_time_gemm_kernel on products that the driver gives to the single kernel, which a caller
     of another layout than 'T','N' cannot ask for: the events enclose it, nearly all of the call."""

@@ -17,6 +17,9 @@ An instruction takes, per cycle group, as many cycles as the most loaded bank ha
 addresses.  The literal cycle counts of the stride scans below are the counters' readings (per
 instruction, 1000 repetitions each), which the model has to reproduce; the kernels' own layouts
 are then evaluated with it and compared with what rocprofv3 reads for them."""
+import os
+import re
+
 import numpy as np
 
 QUADS_OF_CYCLE = ((0, 3, 5, 6), (1, 2, 4, 7), (8, 11, 13, 14), (9, 10, 12, 15))
@@ -71,38 +74,45 @@ def test_model_reproduces_the_measured_stride_scans():
 
 
 def test_fragment_major_chunks_are_conflict_free():
-    """Packed operands and the term buffers of the single-kernel path: lane l reads base + 16*l."""
+    """Packed operands: lane l reads base + 16*l."""
     assert cycles("read_b128", 16 * LANE) == free("read_b128")
-
-
-def test_fused_kernel_raw_layout():
-    """Raw fp32 row block of the single-kernel path: 16 rows x 128 bytes.  Lane l converts row
-    r = l % 16, floats 8 * (l / 16) .. +7.  Stored row-major, every read is a four-way conflict;
-    with the pieces of a row permuted as the kernel does (32-byte pair index XOR (r / 2) % 4,
-    halves swapped for r >= 8) both reads are conflict free (the counter reads 0 for it)."""
-    r, g = LANE % 16, LANE // 16
-    plain = r * 128 + g * 32
-    assert cycles("read_b128", plain) == 16 and cycles("read_b128", plain + 16) == 16
-    base = r * 128 + 32 * (g ^ ((r >> 1) & 3))
-    lo = base + 16 * (r >> 3)
-    hi = base + 16 * (1 - (r >> 3))
-    assert cycles("read_b128", lo) == 4 and cycles("read_b128", hi) == 4
-    # the permutation is the one the requests write: lane l of request h fetches row
-    # 8h + l/8, piece (l%8) ^ (2*((l/16)%4) + h) into slot h*1024 + 16*l
-    where = {}
-    for h in range(2):
-        for l in range(64):
-            row = 8 * h + l // 8
-            piece = (l % 8) ^ (2 * ((l // 16) % 4) + h)
-            where[(row, piece)] = h * 1024 + 16 * l
-    assert len(where) == 128                                    # every piece of every row once
-    for l in range(64):
-        assert where[(r[l], 2 * g[l])] == lo[l]                  # floats 8g .. 8g+3
-        assert where[(r[l], 2 * g[l] + 1)] == hi[l]              # floats 8g+4 .. 8g+7
 
 
 def _direct_swizzle(q):
     return (12 * (q & 1)) ^ (4 * (q >> 1))
+
+
+def _swizzle_of_the_kernels():
+    """direct_swizzle of tcec_gemm_kernels.hpp, evaluated from the source's own expression."""
+    path = os.path.join(os.path.dirname(__file__), "..", "wmma_extension_amd", "csrc", "tcec_gemm_kernels.hpp")
+    body = re.search(r"constexpr unsigned direct_swizzle\(const unsigned q\) \{\s*return ([^;]+);", open(path).read())
+    return [eval(re.sub(r"(\d)u", r"\1", body.group(1)), {"q": q}) for q in range(4)]
+
+
+def test_single_kernel_term_buffers():
+    """The single kernel's producers write terms into 1 KiB chunks (a row block's 16 rows x 32 k, position
+    (row r, k group g) at 16-byte slot 16g + (r ^ swizzle(g))) in one of two patterns.  Rows contiguous:
+    lane = row of 64, 16 bytes of one k group each, lanes l / 16 = 0 .. 3 in four chunks.  k contiguous: eight
+    lanes to a row, 8 bytes each, rows 8h .. 8h + 7.  The consumers read a chunk's 64 positions, 16 bytes a
+    lane.  Both sides cover a chunk exactly once."""
+    swz = np.array(_swizzle_of_the_kernels())
+    assert list(swz) == [_direct_swizzle(q) for q in range(4)]
+    for terms in (1, 2, 3):
+        for g in range(4):
+            addr = (LANE >> 4) * (terms * 1024) + 256 * g + 16 * ((LANE & 15) ^ swz[g])
+            assert cycles("write_b128", addr) == free("write_b128"), (terms, g)
+    rows = np.concatenate([256 * g + 16 * (np.arange(16) ^ swz[g]) for g in range(4)])
+    assert sorted(rows) == list(range(0, 1024, 16))
+    halves = []
+    for h in range(2):
+        r, g = 8 * h + (LANE >> 3), (LANE & 7) >> 1
+        addr = 256 * g + 16 * (r ^ swz[g]) + 8 * (LANE & 1)
+        assert cycles("write_b64", addr) == 8          # banks b and b + 32, as in the direct kernel below
+        halves += list(addr)
+    assert sorted(halves) == list(range(0, 1024, 8))
+    read = 16 * ((LANE & 48) + ((LANE & 15) ^ swz[LANE >> 4]))
+    assert cycles("read_b128", read) == free("read_b128")
+    assert sorted(read) == list(range(0, 1024, 16))
 
 
 def test_direct_kernel_image_writes_and_reads():
