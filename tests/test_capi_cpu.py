@@ -310,7 +310,7 @@ def test_path_query_is_the_smallest_estimate(h):
         assert all(x > 0 for x in est)
         terms = {0: 2, 1: 1, 2: 3, 3: 2, 4: 1}[policy]
         assert math.isinf(est[2]) == (terms == 3 or k < 4)           # the direct kernel: at most two terms, k >= 4
-        assert math.isinf(est[0]) == (k % 4 != 0 and k > 96)          # the single kernel wants 16-byte requests
+        assert math.isinf(est[0]) == (k % 4 != 0 and k > 96)          # the query's answers there are kept
         assert not math.isinf(est[1])
         assert h.wmmae_tcec_sgemm_path(m, n, k, batch, policy, 0, ctypes.byref(out)) == 0
         best = min(range(3), key=lambda i: (e[i], (1, 0, 2)[i]))      # ties go to packed, then fused

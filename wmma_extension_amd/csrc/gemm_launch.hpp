@@ -318,6 +318,10 @@ int launch_fused(FusedArgs f) {
       f, p.grouped ? 8 * per_xcd : resident);
 }
 
+// (RN has no rates of its own.  Three terms with RN are short of registers on the
+// 128x128 tile, 48 to 80 bytes of scratch in the K loop, and even so no slower:
+// 45 products for which it is chosen took 1.00 of its time with 64x64 tiles in
+// the median, 0.86 to 1.21, and 0.61 of what they took on packed operands.)
 template <class T, int TERMS, bool RN> int fused_by_size(const FusedArgs &f) {
   if (f.p.slice_stages > 0) // (64x64 only: see fused_time)
     return launch_fused<T, TERMS, 64, 64, 4, 4, 4, RN, true>(f);

@@ -100,7 +100,10 @@ __device__ __forceinline__ f32x4 epilogue_beta(const f32x4 scaled,
 //   * One decision per piece: all of it inside C, no guards at all, or the
 //     guarded loop (with the choice made per pair of tiles the compiler keeps
 //     the accumulators in sight of several store paths, and values of the
-//     direct kernel's K loop go to scratch: c5b 1.45 -> 1.60 ms).
+//     direct kernel's K loop go to scratch: c5b 1.45 -> 1.60 ms).  The 256x128
+//     kernels of two and three terms keep one address pair, 12 bytes of scratch
+//     a lane, that is stored and loaded once per tile, outside the K loop; with
+//     GROUP 4 no less, with GROUP 2 more in the direct ones.
 // --------------------------------------------------------------------------
 template <int MT_, int NT_, bool PAIRS, int GROUP, class Value>
 __device__ __forceinline__ void
