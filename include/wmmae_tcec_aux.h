@@ -71,10 +71,11 @@ int wmmae_tcec_sgemm_k_slices(int m, int n, int k, int batch, int policy,
  * that splits the fp32 operands itself; infinity for a path the product cannot
  * take.  The smallest is the path wmmae_tcec_sgemm* takes for these layouts
  * (none below the time the host needs to issue its launches).  For checking the
- * estimates against measured times.  seconds[0] is more than a time in two
+ * estimates against measured times.  seconds[0] is more than a time in three
  * cases: products of at least 1024 x 1024 x 512, and fewer than 16 entries, take
  * the single kernel only where it is well ahead, and their seconds[0] holds that
- * factor (1.25, 1.4, 1.25 for one, two, three terms); and a product whose K the
+ * factor (1.25, 1.4, 1.25 for one, two, three terms); so do large batches that
+ * suit the direct kernel (1.4); and a product whose K the
  * faster of the other two paths cuts does not run over an uncut K in the single
  * kernel at all: its seconds[0] lies above that path's. */
 int wmmae_tcec_path_estimates(int m, int n, int k, int batch, int policy,

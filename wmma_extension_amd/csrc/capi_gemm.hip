@@ -115,6 +115,9 @@ inline PathEstimates estimate_paths(const int m, const int n, const int k,
       e.fused = (!rows && fit::fused_tn_margin(m, n, k, batch)
                      ? fit::kFusedTnMargin[terms - 1]
                      : 1.0) *
+                (e.base == Path::Direct
+                     ? fit::fused_direct_margin(m, n, k, batch)
+                     : 1.0) *
                 std::min(fused_time(terms, m, n, k, batch, true, rows),
                          fused_time(terms, m, n, k, batch, false, rows));
     return e;

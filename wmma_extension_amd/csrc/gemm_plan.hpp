@@ -259,6 +259,26 @@ constexpr bool fused_tn_margin(const int m, const int n, const int k,
                                const int batch) {
   return m >= 1024 && n >= 1024 && k >= 512 && batch < 16;
 }
+// An uncut product that would run in the direct kernel and moves more than the
+// 256 MiB of the memory-side cache, with k above two stages and tiles of 256x128
+// that lie within C for two thirds or more: the single kernel overlaps its stages
+// with that traffic less well than its estimate says (1024^2 x 128, 256 entries:
+// 403 us for 355 estimated, the direct kernel 347; 1024x768x224 x 256, one term,
+// 393 against 287).  Of 119 products of the direct kernel that the times alone
+// moved to the single kernel 17 became more than 5 % slower, up to 1.36 times,
+// with this factor 4 stay so; none of 113 that had run in the single kernel before
+// loses more than 4 %.
+constexpr double kFusedStreamMargin = 1.4;
+inline double fused_direct_margin(const int m, const int n, const int k,
+                                  const int batch) {
+  const double c = static_cast<double>(m) * n,
+               bytes = 4.0 * batch * (c + (static_cast<double>(m) + n) * k),
+               tiles = 32768.0 * static_cast<double>(ceil_div(m, 256) *
+                                                     ceil_div(n, 128));
+  return bytes > 256.0 * (1 << 20) && k > 64 && tiles < 1.5 * c
+             ? kFusedStreamMargin
+             : 1.0;
+}
 // Adding a K slice to the double-precision sums, for the workgroups of a compute
 // unit at a time: 110 products run with the cut and uncut, 0.17 us in the median
 // (one workgroup a unit), 0.10 (two), 3 % of a call.
