@@ -16,7 +16,7 @@ PACKED, FUSED, DIRECT = 2, 4, 8
 @pytest.mark.parametrize("flag,policy", [(f, p) for f in (PACKED, FUSED, DIRECT) for p in (0, 1, 2)
                                          if (f, p) != (DIRECT, 2)])   # direct: one and two terms only
 @pytest.mark.parametrize("m,n,batch", [(1, 1, 1), (3, 17, 1), (61, 63, 2), (255, 129, 1), (258, 131, 1), (271, 127, 9),
-                                       (289, 257, 1), (384, 256, 1), (1030, 515, 3), (777, 200, 70)])
+                                       (289, 257, 1), (172, 384, 3), (384, 256, 1), (1030, 515, 3), (777, 200, 70)])
 def test_edges_of_a_piece_of_c(tc, orc, dev, flag, policy, m, n, batch):
     k = 100
     g = torch.Generator(device="cpu").manual_seed(m * 1000 + n)

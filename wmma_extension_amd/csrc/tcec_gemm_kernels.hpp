@@ -104,6 +104,11 @@ __device__ __forceinline__ f32x4 epilogue_beta(const f32x4 scaled,
 //     kernels of two and three terms keep one address pair, 12 bytes of scratch
 //     a lane, that is stored and loaded once per tile, outside the K loop; with
 //     GROUP 4 no less, with GROUP 2 more in the direct ones.
+//   * In the guarded loop a group of four tile rows past the end of C is left by
+//     the wave as a whole: with per-lane guards alone 172x384x128 x 1000 took
+//     160 us in the direct kernel and 252 on packed operands, now 133 and 227
+//     (tests per tile, or groups of two, cost the K loops registers: 1.01 to
+//     1.09 of that).
 // --------------------------------------------------------------------------
 template <int MT_, int NT_, bool PAIRS, int GROUP, class Value>
 __device__ __forceinline__ void
@@ -196,6 +201,8 @@ store_piece(const Value &value, float *const Cb, const long long ld,
     static_assert(MT_ % HALF == 0, "whole groups");
 #pragma unroll
     for (int i0 = 0; i0 < MT_; i0 += HALF) {
+      if (row0 + 16 * i0 >= M) // wave-uniform
+        break;
       f32x4 old[HALF];
       if (beta != 0.f) {
 #pragma unroll
