@@ -18,6 +18,17 @@ PACKED, FUSED, DIRECT = 2, 4, 8
 @pytest.mark.parametrize("m,n,batch", [(1, 1, 1), (3, 17, 1), (61, 63, 2), (255, 129, 1), (258, 131, 1), (271, 127, 9),
                                        (289, 257, 1), (172, 384, 3), (384, 256, 1), (1030, 515, 3), (777, 200, 70)])
 def test_edges_of_a_piece_of_c(tc, orc, dev, flag, policy, m, n, batch):
+    _edges(tc, orc, dev, flag, policy, m, n, batch)
+
+
+@pytest.mark.parametrize("flag,policy", [(f | 1, p) for f in (PACKED, FUSED) for p in (0, 2)])
+@pytest.mark.parametrize("m,n,batch", [(3, 17, 1), (61, 63, 2), (172, 384, 3), (258, 131, 1), (271, 127, 9),
+                                       (384, 256, 1), (777, 200, 70)])
+def test_edges_with_the_leading_product_outside(tc, orc, dev, flag, policy, m, n, batch):
+    _edges(tc, orc, dev, flag, policy, m, n, batch)
+
+
+def _edges(tc, orc, dev, flag, policy, m, n, batch):
     k = 100
     g = torch.Generator(device="cpu").manual_seed(m * 1000 + n)
     A = (torch.rand((batch, m, k), generator=g) * 2 - 1).to(dev)

@@ -109,14 +109,21 @@ __device__ __forceinline__ f32x4 epilogue_beta(const f32x4 scaled,
 //     160 us in the direct kernel and 252 on packed operands, now 133 and 227
 //     (tests per tile, or groups of two, cost the K loops registers: 1.01 to
 //     1.09 of that).
+//   * GROUP 0: one tile at a time, its old values loaded next to its store, one
+//     loop for all pieces.  For three terms with the leading product outside the
+//     matrix core: with any other form the compiler copies fragments back from
+//     accumulation registers right in front of the MFMAs that read them, which
+//     then need a wait of two states each (1 to 3.5 % of such a product).  No
+//     PAIRS with the leading product outside, for the same reason.
 // --------------------------------------------------------------------------
 template <int MT_, int NT_, bool PAIRS, int GROUP, class Value>
 __device__ __forceinline__ void
 store_piece(const Value &value, float *const Cb, const long long ld,
             const int row0, const int col0, const int M, const int N,
             const float beta, unsigned lane) {
-  static_assert(MT_ * NT_ % GROUP == 0 &&
-                    (!PAIRS || (MT_ % 2 == 0 && GROUP % 2 == 0)),
+  constexpr int AHEAD = GROUP ? GROUP : 1;
+  static_assert(MT_ * NT_ % AHEAD == 0 &&
+                    (!PAIRS || (MT_ % 2 == 0 && AHEAD % 2 == 0)),
                 "whole groups");
   // (device memory: global instructions, not generic ones, which count as LDS
   // operations too)
@@ -128,6 +135,34 @@ store_piece(const Value &value, float *const Cb, const long long ld,
   asm volatile("" : "+v"(lane));
   const int q4 = 4 * static_cast<int>(lane >> 4);
   const int c16 = static_cast<int>(lane & 15u);
+  if constexpr (GROUP == 0) {
+#pragma unroll
+    for (int j = 0; j < NT_; j++) {
+      const int col = col0 + 16 * j + c16;
+      if (col >= N)
+        continue;
+#pragma unroll
+      for (int i = 0; i < MT_; i++) {
+        const int left = M - (row0 + 16 * i + q4); // rows from the lane's first
+        if (left <= 0)
+          continue;
+        f32x4 v = value(i, j);
+        gfloat *const dst = (gfloat *)(Cb + row0 + 16 * i + q4 +
+                                       static_cast<long long>(col) * ld);
+        if (left > 3) {
+          if (beta != 0.f)
+            v = epilogue_beta(v, beta, *reinterpret_cast<gf32x4 *>(dst));
+          *reinterpret_cast<gf32x4 *>(dst) = v;
+        } else {
+#pragma unroll
+          for (int x = 0; x < 3; x++)
+            if (x < left)
+              dst[x] = beta != 0.f ? __builtin_fmaf(beta, dst[x], v[x]) : v[x];
+        }
+      }
+    }
+    return;
+  }
   if (row0 + 16 * MT_ <= M && col0 + 16 * NT_ <= N) { // wave-uniform
     const int odd = static_cast<int>(lane & 1u);
     // place of the lane's f32x4 number i of tile column j: rows of tile i, or
@@ -141,16 +176,16 @@ store_piece(const Value &value, float *const Cb, const long long ld,
           (gfloat *)(Cb + row + static_cast<long long>(col) * ld));
     };
 #pragma unroll
-    for (int t0 = 0; t0 < MT_ * NT_; t0 += GROUP) {
-      f32x4 old[GROUP];
+    for (int t0 = 0; t0 < MT_ * NT_; t0 += AHEAD) {
+      f32x4 old[AHEAD];
       if (beta != 0.f) {
 #pragma unroll
-        for (int g = 0; g < GROUP; g++)
+        for (int g = 0; g < AHEAD; g++)
           old[g] = *place((t0 + g) % MT_, (t0 + g) / MT_);
       }
       if constexpr (PAIRS) {
 #pragma unroll
-        for (int g = 0; g < GROUP; g += 2) {
+        for (int g = 0; g < AHEAD; g += 2) {
           const int i = (t0 + g) % MT_, j = (t0 + g) / MT_;
           const f32x4 v0 = value(i, j), v1 = value(i + 1, j);
           f32x4 d0, d1;
@@ -172,7 +207,7 @@ store_piece(const Value &value, float *const Cb, const long long ld,
         }
       } else {
 #pragma unroll
-        for (int g = 0; g < GROUP; g++) {
+        for (int g = 0; g < AHEAD; g++) {
           const int i = (t0 + g) % MT_, j = (t0 + g) / MT_;
           f32x4 v = value(i, j);
           if (beta != 0.f)
@@ -1085,23 +1120,15 @@ __global__ void __launch_bounds__(WGM *WGN * 64)
   // wait states (the compiler emits none for the builtin either).  Small wave
   // tiles use the builtin.
   constexpr bool USE_ASM = MT_ * NT_ >= 8;
-  // (The round-to-nearest variants keep fragments in accumulation registers and
-  // copy them back right in front of the MFMAs that read them: a wait of two
-  // states in front of each makes that safe.)
   auto mfma_acc = [](f32x4 &z, const ab_vec x, const ab_vec y) {
-#define WMMAE_MFMA_ACC(GUARD, TYPE)                                            \
-  asm volatile(GUARD "v_mfma_f32_16x16x32_" TYPE " %0, %1, %2, %0"             \
-               : "+a"(z)                                                       \
-               : "v"(x), "v"(y))
-    if constexpr (std::is_same<MT, _Float16>::value && RN_MAIN)
-      WMMAE_MFMA_ACC("s_nop 1\n\t", "f16");
-    else if constexpr (std::is_same<MT, _Float16>::value)
-      WMMAE_MFMA_ACC(WMMAE_MFMA_GUARD, "f16");
-    else if constexpr (RN_MAIN)
-      WMMAE_MFMA_ACC("s_nop 1\n\t", "bf16");
+    if constexpr (std::is_same<MT, _Float16>::value)
+      asm volatile(WMMAE_MFMA_GUARD "v_mfma_f32_16x16x32_f16 %0, %1, %2, %0"
+                   : "+a"(z)
+                   : "v"(x), "v"(y));
     else
-      WMMAE_MFMA_ACC(WMMAE_MFMA_GUARD, "bf16");
-#undef WMMAE_MFMA_ACC
+      asm volatile(WMMAE_MFMA_GUARD "v_mfma_f32_16x16x32_bf16 %0, %1, %2, %0"
+                   : "+a"(z)
+                   : "v"(x), "v"(y));
   };
   auto mfma = [](const ab_vec x, const ab_vec y, const f32x4 z) -> f32x4 {
     if constexpr (std::is_same<MT, _Float16>::value)
@@ -1347,7 +1374,10 @@ __global__ void __launch_bounds__(WGM *WGN * 64)
         v = epilogue_fold(v, acc_err[i][j], inv_scale);
       return v * a_out;
     };
-    store_piece<MT_, NT_, MT_ % 2 == 0, (MT_ * NT_ <= 16 ? MT_ * NT_ : MT_)>(
+    store_piece<MT_, NT_, !RN_MAIN && MT_ % 2 == 0,
+                (RN_MAIN && TERMS == 3 ? 0
+                 : MT_ * NT_ <= 16     ? MT_ * NT_
+                                       : MT_)>(
         out_value, Cb, ld_out, (to_tail ? 0 : it.tm * BM) + wm * Cfg::WM,
         (to_tail ? 0 : it.tn * BN) + wn * Cfg::WN, M, N, b_out, lane);
   };
