@@ -163,7 +163,8 @@ int wmmae_tcec_sgemm_strided_batched(char transa, char transb, int m, int n,
  * WMMAE_STATIC_SCRATCH_BYTES inside the library image (every GPU the library
  * runs on holds it until the process ends), so the call makes no hipMalloc /
  * hipFree of any kind.  On packed operands (wmmae_tcec_sgemm_path 1, and 2
- * where the single kernel does not make the slices) the array holds the split operands, and products whose split operands need more
+ * where the single kernel does not make the slices) the array holds the split
+ * operands, and products whose split operands need more
  * (wmmae_tcec_pack_bytes of A and of B; fp16 hi+lo: 4*(m+n)*k bytes rounded up
  * to 16 rows and 32 of k) return WMMAE_STATUS_WORKSPACE_TOO_SMALL; K slices
  * are made only when they fit behind the operands.  On the path that reads the

@@ -109,8 +109,10 @@ def test_element_by_element_with_several_tiles_per_workgroup(tc, dev, policy):
 
 def test_events_around_the_single_kernel(tc, dev):
     """wmmae_tcec_time_gemm_kernel on products that the driver gives to the single kernel, which a caller
-    of another layout than 'T','N' cannot ask for: the events enclose it, nearly all of the call."""
-    for policy, k in ((2, 515), (0, 900)):
+    of another layout than 'T','N' cannot ask for: the events enclose it.  No kernel takes less time than its
+    matrix products at the nominal 2.5 PFLOP/s (16 to 18 us here; two events with nothing between them are a few
+    microseconds apart)."""
+    for policy, k, products in ((2, 515, 6), (0, 900, 3)):
         m, n, batch = 777, 1333, 7
         A, lda = _operand(torch.Generator().manual_seed(1), dev, batch, m, k, False, 0, 0)
         B, ldb = _operand(torch.Generator().manual_seed(2), dev, batch, n, k, True, 0, 0)
@@ -126,4 +128,5 @@ def test_events_around_the_single_kernel(tc, dev):
             torch.cuda.synchronize()
             inner.append(e0.elapsed_time(e1))
             whole.append(w0.elapsed_time(w1))
-        assert 0.3 * min(whole) < min(inner) <= min(whole), (inner, whole)
+        floor_ms = products * 2.0 * batch * m * n * k / 2.5e15 * 1e3
+        assert floor_ms < min(inner) <= min(whole), (floor_ms, inner, whole)
