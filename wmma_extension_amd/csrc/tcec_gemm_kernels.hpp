@@ -484,16 +484,31 @@ __global__ void __launch_bounds__(256)
 #pragma unroll
   for (int x = 0; x < VEC; x++)
     s[x] = 0.;
-  for (int z = 0; z < splits; z++) {
-    const float *const src = partial + (z * batches + entry) * mn + e;
-    if constexpr (VEC == 4) {
-      const f32x4 v = *reinterpret_cast<const f32x4 *>(src);
+  // (eight slices are read before any is added, past the last one the last again,
+  // which is not added; one read after the other, whole calls on packed operands
+  // took 27.9 us for 256x256x8192 in 32 slices, now 23.6, 200x160x10735 36.2, now
+  // 31.8)
+  typedef typename std::conditional<VEC == 4, f32x4, float>::type piece;
+  constexpr int AHEAD = 8;
+  for (int z0 = 0; z0 < splits; z0 += AHEAD) {
+    piece v[AHEAD];
 #pragma unroll
-      for (int x = 0; x < 4; x++)
-        s[x] += static_cast<double>(v[x]);
-    } else {
-      s[0] += static_cast<double>(*src);
+    for (int a = 0; a < AHEAD; a++) {
+      const int z = z0 + a < splits ? z0 + a : splits - 1;
+      v[a] = *reinterpret_cast<const piece *>(partial +
+                                              (z * batches + entry) * mn + e);
     }
+#pragma unroll
+    for (int a = 0; a < AHEAD; a++)
+      if (z0 + a < splits) {
+        if constexpr (VEC == 4) {
+#pragma unroll
+          for (int x = 0; x < 4; x++)
+            s[x] += static_cast<double>(v[a][x]);
+        } else {
+          s[0] += static_cast<double>(v[a]);
+        }
+      }
   }
   float *const cb =
       c_ptrs != nullptr ? c_ptrs[entry] : C + entry * batch_stride_c;
