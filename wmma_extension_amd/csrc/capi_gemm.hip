@@ -4,6 +4,7 @@
 // live in include/wmmae_tcec.h.
 #include "gemm_plan.hpp"
 #include <cmath>
+#include <random>
 
 namespace {
 using namespace wmmae_driver;
@@ -193,6 +194,7 @@ struct Choice {
   Path path; // Path::Fused: the single kernel over an uncut K
   int slices;
   bool single;
+  double time = 0.; // estimated
 };
 inline Choice choose_path(const int m, const int n, const int k, const int batch,
                           const int flags, const int terms, const int policy,
@@ -212,7 +214,59 @@ inline Choice choose_path(const int m, const int n, const int k, const int batch
   const double fused = std::max(e.fused, fit::kCallFloor[0]);
   const bool single = e.base == Path::Direct ? fused <= e.base_time
                                              : fused < e.base_time;
-  return {single && e.slices == 1 ? Path::Fused : e.base, e.slices, single};
+  return {single && e.slices == 1 ? Path::Fused : e.base, e.slices, single,
+          single ? fused : e.base_time};
+}
+// Tile of the single kernel (64 or 128) that makes a cut product's slices with a
+// workgroup each, 0: the slices are made as chosen.  The products that run on
+// packed operands or in the direct kernel, or whose slices one workgroup of the
+// single kernel would make one after the other: too few output tiles to fill the
+// chip, and a split pass, a GEMM of at most a round and a fold launch for what is
+// one launch here.  The same cut of K, so the same bits.  Needs the caller's
+// workspace to have the room; without one it allocates only where the path it
+// stands in for would.
+inline int choose_spread(const Choice &c, const int m, const int n, const int k,
+                         const int batch, const int terms,
+                         const void *const workspace,
+                         const size_t workspace_bytes) {
+  if (c.slices <= 1 || c.time <= 0.)
+    return 0;
+  double best = c.time;
+  if (!c.single)
+    best = c.path == Path::Direct
+               ? c.time / fit::kSpreadDirectMargin
+               : std::max(c.time / fit::kSpreadPackedMargin,
+                          fit::kCutPacked + c.slices * fit::kCutPackedSlice);
+  int chosen = 0;
+  for (const int tile : {64, 128}) {
+    const double t =
+        fused_spread_time(terms, m, n, k, batch, tile == 64, c.slices);
+    if (t < best &&
+        (workspace == nullptr
+             ? !c.single
+             : reinterpret_cast<uintptr_t>(workspace) % 16 == 0 &&
+                   workspace_bytes >=
+                       fused_spread_bytes(m, n, batch, c.slices, tile))) {
+      chosen = tile;
+      best = t;
+    }
+  }
+  return chosen;
+}
+// Tells a launch's arrival counts in a workspace from whatever else it may hold:
+// 58 bits that no other launch of any process is likely to have used.
+unsigned long long launch_number() {
+  static const unsigned long long seed = [] {
+    std::random_device r;
+    return (static_cast<unsigned long long>(r()) << 32) ^ r();
+  }();
+  static std::atomic<unsigned long long> count{0};
+  unsigned long long z =
+      seed + 0x9E3779B97F4A7C15ull * count.fetch_add(1, std::memory_order_relaxed);
+  z = (z ^ (z >> 30)) * 0xBF58476D1CE4E5B9ull;
+  z = (z ^ (z >> 27)) * 0x94D049BB133111EBull;
+  z = (z ^ (z >> 31)) >> 6;
+  return z != 0 ? z : 1;
 }
 // ('T','N') products with k % 4 != 0 and more than three stages stay with the
 // other paths, as the path query has always answered.
@@ -470,6 +524,7 @@ int sgemm_impl(const char transa, const char transb, const int m, const int n,
   const int rn = flags & WMMAE_FLAG_RN_MAIN;
   Path path = Path::Packed;
   int slices = 1; // of the single kernel; a forced one does not cut K
+  int spread_tile = 0;
   if ((flags & WMMAE_FLAG_PATH_DIRECT) != 0) {
     if (!direct_ok)
       return WMMAE_STATUS_NOT_SUPPORTED;
@@ -484,6 +539,10 @@ int sgemm_impl(const char transa, const char transb, const int m, const int n,
                                  rows || fused_considered(k), rows, direct_ok);
     path = c.single ? Path::Fused : c.path;
     slices = c.slices;
+    spread_tile = choose_spread(c, m, n, k, batch, p.terms, workspace,
+                                workspace_bytes);
+    if (spread_tile > 0)
+      path = Path::Fused;
   }
   if (path == Path::Direct) {
     // the planes of the K slices are the only workspace this path uses
@@ -562,7 +621,27 @@ int sgemm_impl(const char transa, const char transb, const int m, const int n,
     q.inv_scale = p.inv_scale;
     f.stream = static_cast<hipStream_t>(stream);
     const PolicyKernels *const kernels = policy_kernels(policy);
-    return rn != 0 ? kernels->fused_rn(f) : kernels->fused(f);
+    if (spread_tile == 0)
+      return rn != 0 ? kernels->fused_rn(f) : kernels->fused(f);
+    // the slices' sums and the tiles' arrival words in the caller's workspace or
+    // in one allocated here
+    const bool own = workspace == nullptr;
+    if (own)
+      WMMAE_HIP_TRY(hipMallocAsync(
+          &workspace, fused_spread_bytes(m, n, batch, slices, spread_tile),
+          f.stream));
+    f.spread_tile = spread_tile;
+    q.slices = slices;
+    q.planes = static_cast<float *>(workspace);
+    q.arrivals = reinterpret_cast<unsigned long long *>(
+        static_cast<char *>(workspace) +
+        fused_spread_planes(m, n, batch, slices, spread_tile));
+    q.launch = launch_number();
+    int st = rn != 0 ? kernels->fused_rn(f) : kernels->fused(f);
+    if (own && hipFreeAsync(workspace, f.stream) != hipSuccess &&
+        st == WMMAE_STATUS_SUCCESS)
+      st = WMMAE_STATUS_RUNTIME_ERROR;
+    return st;
   }
 
   size_t bytes_a = 0, bytes_b = 0, bytes_c = 0;

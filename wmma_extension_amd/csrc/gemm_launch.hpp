@@ -271,11 +271,11 @@ template <class MT, int TERMS> int per_cu_by_shape(const int shape) {
   }
 }
 template <class T, int TERMS, int BM, int BN, int CW, int PW, int DEPTH, bool RN,
-          bool STREAM, bool SLICED>
+          bool STREAM, int CUT>
 int launch_fused_grid(const FusedArgs &f, const long long grid) {
   using Cfg = wmmae_gemm::FusedConfig<TERMS, BM, BN, CW, PW>;
   auto kernel = wmmae_gemm::tcec_gemm_fused_kernel<T, TERMS, BM, BN, CW, PW,
-                                                   DEPTH, RN, STREAM, SLICED>;
+                                                   DEPTH, RN, STREAM, CUT>;
   static std::atomic<unsigned long long> lds_allowed{0};
   WMMAE_HIP_TRY(allow_dynamic_lds(reinterpret_cast<const void *>(kernel),
                                   Cfg::LDS_BYTES, lds_allowed));
@@ -290,7 +290,7 @@ int launch_fused_grid(const FusedArgs &f, const long long grid) {
 }
 
 template <class T, int TERMS, int BM, int BN, int CW, int PW, int DEPTH, bool RN,
-          bool SLICED>
+          int CUT>
 int launch_fused(FusedArgs f) {
   wmmae_gemm::FusedParams &p = f.p;
   p.tiles_m = static_cast<int>(ceil_div(p.M, BM));
@@ -299,6 +299,14 @@ int launch_fused(FusedArgs f) {
   const long long items = p.batch * tpb;
   if (items >= (1ll << 30)) // the kernel counts tiles in 32 bits
     return WMMAE_STATUS_NOT_SUPPORTED;
+  if constexpr (CUT == wmmae_gemm::kFusedSpread) {
+    const long long all = items * p.slices;
+    if (all >= (1ll << 30))
+      return WMMAE_STATUS_NOT_SUPPORTED;
+    p.grouped = 0;
+    return launch_fused_grid<T, TERMS, BM, BN, CW, PW, DEPTH, RN, false, CUT>(
+        f, 8 * ceil_div(all, 8));
+  } else {
   // with 8 or more batch entries an XCD (block index mod 8) owns whole entries
   // (not when the XCD that owns one entry more than the others would need over
   // 15 % more rounds of tiles than an even spread)
@@ -312,10 +320,11 @@ int launch_fused(FusedArgs f) {
   // one workgroup per tile when all of them are resident together, else
   // persistent workgroups
   if (spread <= resident)
-    return launch_fused_grid<T, TERMS, BM, BN, CW, PW, DEPTH, RN, false, SLICED>(
+    return launch_fused_grid<T, TERMS, BM, BN, CW, PW, DEPTH, RN, false, CUT>(
         f, spread);
-  return launch_fused_grid<T, TERMS, BM, BN, CW, PW, DEPTH, RN, true, SLICED>(
+  return launch_fused_grid<T, TERMS, BM, BN, CW, PW, DEPTH, RN, true, CUT>(
       f, p.grouped ? 8 * per_xcd : resident);
+  }
 }
 
 // (RN has no rates of its own.  Three terms with RN are short of registers on the
@@ -323,13 +332,18 @@ int launch_fused(FusedArgs f) {
 // 45 products for which it is chosen took 1.00 of its time with 64x64 tiles in
 // the median, 0.86 to 1.21, and 0.61 of what they took on packed operands.)
 template <class T, int TERMS, bool RN> int fused_by_size(const FusedArgs &f) {
+  using namespace wmmae_gemm;
+  if (f.spread_tile == 64)
+    return launch_fused<T, TERMS, 64, 64, 4, 4, 4, RN, kFusedSpread>(f);
+  if (f.spread_tile == 128)
+    return launch_fused<T, TERMS, 128, 128, 8, 4, 2, RN, kFusedSpread>(f);
   if (f.p.slice_stages > 0) // (64x64 only: see fused_time)
-    return launch_fused<T, TERMS, 64, 64, 4, 4, 4, RN, true>(f);
+    return launch_fused<T, TERMS, 64, 64, 4, 4, 4, RN, kFusedSliced>(f);
   if (fused_small_tiles(TERMS, f.p.M, f.p.N, f.p.K, f.p.batch,
                         f.p.a_source != wmmae_gemm::kFusedKRows ||
                             f.p.b_source != wmmae_gemm::kFusedKRows))
-    return launch_fused<T, TERMS, 64, 64, 4, 4, 4, RN, false>(f);
-  return launch_fused<T, TERMS, 128, 128, 8, 4, 2, RN, false>(f);
+    return launch_fused<T, TERMS, 64, 64, 4, 4, 4, RN, kFusedWhole>(f);
+  return launch_fused<T, TERMS, 128, 128, 8, 4, 2, RN, kFusedWhole>(f);
 }
 
 // The table of one policy: split tag T, MFMA element type MT, stored terms; RN:

@@ -291,6 +291,30 @@ constexpr double kFusedSliceFold = 0.15e-6;
 // 1.03 to 1.74 times slower than the direct kernel, most of them with one term.
 constexpr double kFusedSlicedMargin = 1.1;
 constexpr double kFusedSlicedDirectMargin[2] = {1.25, 1.4};
+// The single kernel with a workgroup for every K slice, by tile (64x64, 128x128)
+// and terms: launch, a stage of a 64x64 tile with at most one workgroup on a
+// compute unit, a stage with all resident ones (twice that for 64x64) and how
+// much longer the fuller the chip is, pipeline fill and the slice's sums, the last
+// workgroup's reading of one slice.  Fit: 1000 random products that are cut (m, n
+// = 32 .. 8192, k up to 65536, 1 .. 1024 entries, all layouts), each with both
+// tiles: 5 to 9 % rms (three terms), 9 to 12 (two), 15 to 17 (one).
+struct SpreadRates {
+  double launch, alone, stage, busy, tile, fold;
+};
+constexpr SpreadRates kSpread[2][3] = {
+    {{4.9e-6, 0.184e-6, 0.300e-6, 1.03, 4.92e-6, 0.278e-6},
+     {6.6e-6, 0.280e-6, 0.466e-6, 0.325, 3.94e-6, 0.263e-6},
+     {6.1e-6, 0.496e-6, 0.782e-6, 0.093, 3.60e-6, 0.239e-6}},
+    {{2.5e-6, 0., 0.216e-6, 2.03, 7.46e-6, 0.874e-6},
+     {1.3e-6, 0., 0.469e-6, 0.772, 9.13e-6, 0.872e-6},
+     {4.8e-6, 0., 0.675e-6, 0.812, 6.64e-6, 0.880e-6}}};
+constexpr double kSpreadBytesPerS = 4.9e12;
+// ... in place of the direct kernel and of packed operands where it is this much
+// ahead of their estimates; cut products on packed operands take no less than 15 us
+// and 0.4 a slice (their estimate has 16 to 18 us for 64 x 46 x 4032 in 21 slices,
+// which takes 27).
+constexpr double kSpreadDirectMargin = 1.2, kSpreadPackedMargin = 1.1;
+constexpr double kCutPacked = 15e-6, kCutPackedSlice = 0.4e-6;
 // Its workgroups that are resident on a compute unit: 12 waves of up to 168
 // registers (128x128), twice 8 waves of up to 128.
 constexpr int fused_resident(const int bm) { return bm > 64 ? 1 : 2; }
@@ -449,9 +473,22 @@ constexpr int ring_depth(const int bm, const int bn, const int terms) {
 
 // ------------------------------------------------------ fused small GEMM
 struct FusedArgs {
-  wmmae_gemm::FusedParams p;
+  wmmae_gemm::FusedParams p = {};
+  // > 0: K slices made by a workgroup each, with tiles of this size
+  int spread_tile = 0;
   hipStream_t stream;
 };
+// What those take of a workspace: a tile's sums for every slice, and a word a tile
+inline size_t fused_spread_planes(const int m, const int n, const int batch,
+                                  const int slices, const int tile) {
+  return static_cast<size_t>(ceil_div(m, tile) * ceil_div(n, tile)) * batch *
+         slices * tile * tile * 4u;
+}
+inline size_t fused_spread_bytes(const int m, const int n, const int batch,
+                                 const int slices, const int tile) {
+  return fused_spread_planes(m, n, batch, slices, tile) +
+         static_cast<size_t>(ceil_div(m, tile) * ceil_div(n, tile)) * batch * 8u;
+}
 
 // Time of a call of the single kernel with its 64x64 or 128x128 tiles.  `rows`:
 // an operand does not have k contiguous.  `slices`: K slices made in the kernel,
@@ -488,6 +525,32 @@ inline double fused_time(const int terms, const int m, const int n, const int k,
       4.0 * batch *
       (static_cast<double>(m) * n + (static_cast<double>(m) + n) * k);
   return f.launch + std::max(time, bytes / f.bytes_per_s);
+}
+// Time of a call whose K slices are made by a workgroup each.
+inline double fused_spread_time(const int terms, const int m, const int n,
+                                const int k, const int batch, const bool small,
+                                const int slices) {
+  const fit::SpreadRates &f = fit::kSpread[small ? 0 : 1][terms - 1];
+  const double kt = static_cast<double>(ceil_div(ceil_div(k, 32), slices));
+  const int t = small ? 64 : 128;
+  const double items = static_cast<double>(ceil_div(m, t) * ceil_div(n, t)) *
+                       batch * slices;
+  const double x =
+      items / (static_cast<double>(device_cus()) * fit::fused_resident(t));
+  double time;
+  if (small && x <= 0.5) {
+    time = kt * f.alone + 0.5 * f.tile;
+  } else {
+    // (workgroups follow one another as they end, not in rounds)
+    const double whole = std::ceil(x);
+    const double rounds = x <= 1. ? 1. : 0.35 * whole + 0.65 * x;
+    time = rounds * (kt * f.stage * (1. + f.busy * x / whole) + f.tile);
+  }
+  const double bytes =
+      4.0 * batch *
+      (static_cast<double>(m) * n + (static_cast<double>(m) + n) * k);
+  return f.launch + std::max(time, bytes / fit::kSpreadBytesPerS) +
+         slices * f.fold;
 }
 inline bool fused_small_tiles(const int terms, const int m, const int n,
                               const int k, const int batch, const bool rows) {

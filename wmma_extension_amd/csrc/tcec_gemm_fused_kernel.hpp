@@ -65,6 +65,9 @@
 namespace wmmae_gemm {
 
 enum FusedSource { kFusedKRows = 0, kFusedRRows = 1, kFusedAny = 2 };
+// K: whole, cut into slices that a workgroup makes one after the other, or cut
+// into slices that a workgroup each makes
+enum FusedCut { kFusedWhole = 0, kFusedSliced = 1, kFusedSpread = 2 };
 
 struct FusedParams {
   const float *A;
@@ -82,7 +85,13 @@ struct FusedParams {
   // launcher for 8 or more entries that spread evenly enough)
   int grouped;
   int a_source, b_source; // FusedSource
-  int slice_stages; // SLICED: k stages of a slice
+  int slice_stages; // CUT: k stages of a slice
+  // kFusedSpread: K slices; room for the slices' sums, slice z of tile t (entry
+  // by entry) at planes + (t*slices + z)*BM*BN, and a word per tile
+  // (last_of_tile), with what tells this launch's counts from other contents
+  int slices;
+  float *planes;
+  unsigned long long *arrivals, launch;
   float alpha, beta, inv_scale;
 };
 
@@ -98,6 +107,35 @@ template <int TERMS, int BM, int BN, int CW, int PW> struct FusedConfig {
   static_assert(LDS_BYTES <= 160 * 1024, "LDS of one compute unit");
 };
 
+// The word that counts the workgroups that have finished their slice of a tile
+// holds the launch's number above six bits of count.  A workspace holds what its
+// last user left there, so every workgroup, before it counts itself, replaces any
+// other contents by a count of zero: whoever's exchange fails finds the word
+// counting already.  The last one clears it, so that a captured launch, whose
+// number stays, finds no count when it is replayed.  (Counting itself by an
+// exchange that is tried until it succeeds takes 32 workgroups that finish
+// together up to 32 round trips: 64x64x34272 34.5 us, now 24.2.)
+__device__ __forceinline__ void
+start_count(unsigned long long *const word, const unsigned long long launch) {
+  unsigned long long seen = __hip_atomic_load(word, __ATOMIC_RELAXED,
+                                              __HIP_MEMORY_SCOPE_AGENT);
+  if ((seen >> 6) != launch)
+    __hip_atomic_compare_exchange_strong(word, &seen, launch << 6,
+                                         __ATOMIC_RELAXED, __ATOMIC_RELAXED,
+                                         __HIP_MEMORY_SCOPE_AGENT);
+}
+// Whether the calling workgroup is the last of the `count` (2 .. 32) of a tile.
+// One lane, behind the barrier at which the workgroup's sums have reached memory.
+__device__ __forceinline__ unsigned
+last_of_tile(unsigned long long *const word, const unsigned count) {
+  const unsigned long long before = __hip_atomic_fetch_add(
+      word, 1ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  const bool last = (before & 63u) + 1u >= count;
+  if (last)
+    __hip_atomic_store(word, 0ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  return last ? 1u : 0u;
+}
+
 //   RN_MAIN : accumulate the leading product with fp32 adds outside the matrix
 //             core (tcec_gemm_kernel's RN_MAIN; the reference's mma_rn_sync)
 //   STREAM  : a workgroup walks several tiles; else one, the grid covers them all
@@ -112,14 +150,26 @@ template <int TERMS, int BM, int BN, int CW, int PW> struct FusedConfig {
 //             1024^3 in four slices, whole calls: two fp16 terms 17.0 us (16.1
 //             over an uncut K, 27.2 with packed operands, their GEMM and its
 //             fold), three bf16 terms 22.9 (21.8, 27.2)
+//   SPREAD  : a workgroup makes one slice of a tile; the slices' sums meet in
+//             memory, and the last workgroup of a tile adds them in double
+//             precision in ascending order: the same bits again.  For few output
+//             tiles and long k, where a workgroup that makes all slices leaves the
+//             chip idle and packed operands cost three launches.  Whole calls,
+//             two fp16 terms: 2005x64x23136 (rows contiguous) 147 -> 42 us,
+//             64x3232x11712 91 -> 36, 32x480x7332 32.6 -> 19.4, 34x36x1874 20.2
+//             -> 11.6; 1000 random products that are cut: 0.74 of the time.  What
+//             bounds it with many slices: the last workgroup's reading of them,
+//             0.26 us each (128x128: 0.87), one compute unit's share of memory
 //   DEPTH   : stages of fp32 values in flight in registers (even: the LDS
 //             buffer and fragment set of a step are then compile-time choices)
 template <class T, int TERMS, int BM, int BN, int CW, int PW, int DEPTH,
-          bool RN_MAIN, bool STREAM, bool SLICED>
-// (SLICED: the double-precision sums must not cost the second workgroup of a
-// compute unit, four waves a SIMD; three bf16 terms with RN_MAIN took 130
-// registers of the 128 that leaves)
-__global__ void __launch_bounds__(64 * (CW + PW), SLICED ? 4 : 1)
+          bool RN_MAIN, bool STREAM, int CUT>
+// (SLICED, and SPREAD's fold: the double-precision sums must not cost the second
+// workgroup of a compute unit, four waves a SIMD; three bf16 terms with RN_MAIN
+// took 130 registers of the 128 that leaves)
+__global__ void __launch_bounds__(64 * (CW + PW), CUT == kFusedWhole ? 1
+                                                  : BM > 64          ? 3
+                                                                     : 4)
     tcec_gemm_fused_kernel(const FusedParams p) {
   using traits = mtk::wmma::tcec::detail::split_traits<T>;
   using S = typename traits::storage;
@@ -132,6 +182,8 @@ __global__ void __launch_bounds__(64 * (CW + PW), SLICED ? 4 : 1)
   constexpr int WM = BM / 2, WN = BN / WGN;
   constexpr int MT_ = WM / 16, NT_ = WN / 16;
   static_assert(DEPTH % 2 == 0 && DEPTH >= 2, "even ring");
+  constexpr bool SLICED = CUT == kFusedSliced, SPREAD = CUT == kFusedSpread;
+  static_assert(!(STREAM && SPREAD), "a workgroup makes one slice");
   // Two sets of fragments where they fit the registers that two workgroups (64x64
   // tile) or three waves a SIMD (128x128) leave a wave; else one set, a term's
   // fragments refilled for the next stage once its last product has been issued.
@@ -144,8 +196,7 @@ __global__ void __launch_bounds__(64 * (CW + PW), SLICED ? 4 : 1)
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int wm = wave & 1, wn = wave >> 1;
   const int M = p.M, N = p.N, K = p.K;
-  const int num_k = (K + 31) / 32;
-  const int k_left = K - 32 * (num_k - 1); // k of the last stage, 1 .. 32
+  const int all_k = (K + 31) / 32;
 
   // a producer's work: A or B, units unit0 .. unit0 + U-1 of it
   const bool loads_a = wave - CW < PW / 2;
@@ -155,23 +206,42 @@ __global__ void __launch_bounds__(64 * (CW + PW), SLICED ? 4 : 1)
 
   // ---- this workgroup's tiles: v = first + i*stride while v < count
   const int tpb = p.tiles_m * p.tiles_n;
-  const bool grouped = p.grouped != 0;
+  // SPREAD: the (slice, tile) pairs, slice by slice, in eight runs, one per XCD:
+  // what an XCD's tiles share is one slice of the operands
+  const int spread_tiles = tpb * p.batch;
+  int slice = 0, spread_tile = 0; // tile: entry by entry
+  if constexpr (SPREAD) {
+    const unsigned items = static_cast<unsigned>(spread_tiles * p.slices);
+    const unsigned run = (items + 7) >> 3;
+    const unsigned item = (blockIdx.x & 7u) * run + (blockIdx.x >> 3);
+    if ((blockIdx.x >> 3) >= run || item >= items)
+      return; // (before any barrier)
+    slice = static_cast<int>(item / static_cast<unsigned>(spread_tiles));
+    spread_tile = static_cast<int>(item) - slice * spread_tiles;
+  }
+  // the k stages this workgroup takes of a tile, stage0 the first
+  const int stage0 = SPREAD ? slice * p.slice_stages : 0;
+  const int num_k = SPREAD && all_k - stage0 > p.slice_stages ? p.slice_stages
+                                                              : all_k - stage0;
+  // k of the last stage, 1 .. 32
+  const int k_left = stage0 + num_k == all_k ? K - 32 * (all_k - 1) : 32;
+  const bool grouped = !SPREAD && p.grouped != 0;
   const int xcd = grouped ? static_cast<int>(blockIdx.x & 7u) : 0;
   const int first = grouped ? static_cast<int>(blockIdx.x >> 3)
                             : static_cast<int>(blockIdx.x);
   const int stride = grouped ? static_cast<int>(gridDim.x >> 3)
                              : static_cast<int>(gridDim.x);
   const int count = grouped ? ((p.batch - xcd + 7) >> 3) * tpb : p.batch * tpb;
-  if (first >= count)
+  if (!SPREAD && first >= count)
     return; // nothing for this workgroup (before any barrier)
   const int n_my = STREAM ? (count - first + stride - 1) / stride : 1;
   auto decode = [&](const int i, int &entry, int &tm, int &tn) {
-    const int v = first + i * stride;
+    const int v = SPREAD ? spread_tile : first + i * stride;
     const int bi = v / tpb;
     entry = grouped ? bi * 8 + xcd : bi;
     tile_of<8>(static_cast<unsigned>(v - bi * tpb), static_cast<unsigned>(tpb),
                static_cast<unsigned>(p.tiles_m),
-               static_cast<unsigned>(p.tiles_n), !grouped, tm, tn);
+               static_cast<unsigned>(p.tiles_n), !grouped && !SPREAD, tm, tn);
   };
 
   f32x4 acc_main[MT_][NT_], acc_err[MT_][NT_];
@@ -289,7 +359,7 @@ __global__ void __launch_bounds__(64 * (CW + PW), SLICED ? 4 : 1)
     // that read up to three floats before the stage); RRows: k clamped to the
     // last one.
     auto load_tail_stage = [&]() __attribute__((always_inline)) {
-      const int k0 = 32 * ld_stage;
+      const int k0 = 32 * (stage0 + ld_stage);
       int left = k_left;
       asm volatile("" : "+s"(left));
 #pragma unroll
@@ -327,8 +397,8 @@ __global__ void __launch_bounds__(64 * (CW + PW), SLICED ? 4 : 1)
 #pragma unroll
       for (int u = 0; u < U; u++) {
         const int row0 = unit_row(u);
-        src[u] = reinterpret_cast<unsigned long long>(X + row0 * rs +
-                                                      unit_k(u) * ks);
+        src[u] = reinterpret_cast<unsigned long long>(
+            X + row0 * rs + (32ll * stage0 + unit_k(u)) * ks);
         asm volatile("" : "+s"(src[u]));
 #pragma unroll
         for (int o = 0; o < NOFF; o++) {
@@ -378,7 +448,7 @@ __global__ void __launch_bounds__(64 * (CW + PW), SLICED ? 4 : 1)
       typedef const __attribute__((address_space(1))) float *flt_ptr;
       const gbytes_t base = reinterpret_cast<gbytes_t>(src[u]);
       if constexpr (src_kind == kFusedAny) {
-        const int k0 = 32 * ld_stage + unit_k(u);
+        const int k0 = 32 * (stage0 + ld_stage) + unit_k(u);
 #pragma unroll
         for (int e = 0; e < 8; e++) {
           const int k = k0 + e < K ? k0 + e : K - 1;
@@ -528,6 +598,91 @@ __global__ void __launch_bounds__(64 * (CW + PW), SLICED ? 4 : 1)
       steps(steps, ic<0>{});
   };
 
+  // the matrix C of a batch entry
+  auto c_of = [&](const int entry) {
+    typedef float *const __attribute__((address_space(4))) *out_array_t;
+    return p.c_ptrs != nullptr ? ((out_array_t)p.c_ptrs)[entry]
+                               : p.C + static_cast<long long>(entry) * p.c_bs;
+  };
+  // SPREAD: the sums of slice z of this workgroup's tile: wave, tile of the wave,
+  // halves of a lane's four rows, lane.  Written and read with the device's
+  // scope, past the XCDs' own L2: with ordinary accesses between agent-scope
+  // fences every wave writes its whole L2 back (0.5 us each, one after the other
+  // on an XCD: 1024x1376x7016, 1760 slices of 64x64, took 536 us, now 93).
+  typedef float f32x2 __attribute__((ext_vector_type(2)));
+  auto plane = [&](const int z) {
+    return reinterpret_cast<unsigned long long *>(p.planes) +
+           (static_cast<long long>(spread_tile) * p.slices + z) * (BM * BN / 2);
+  };
+  typedef double f64x2 __attribute__((ext_vector_type(2)));
+  typedef double f64x4 __attribute__((ext_vector_type(4)));
+  // SPREAD, every wave, after the consumers have written the slice's sums: the
+  // workgroup that is the last of its tile's adds the slices in double precision
+  // in ascending order (the bits of reduce_splits_kernel) and stores the tile.
+  // No workgroup waits for another.
+  auto fold_if_last = [&]() __attribute__((always_inline)) {
+    // the wave's stores have reached memory
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
+    __builtin_amdgcn_s_barrier();
+    unsigned *const flag = reinterpret_cast<unsigned *>(lds_raw);
+    if (wave == 0 && lane == 0)
+      *flag = last_of_tile(p.arrivals + spread_tile,
+                           static_cast<unsigned>(p.slices));
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
+    __builtin_amdgcn_s_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
+    if (__builtin_amdgcn_readfirstlane(*flag) == 0)
+      return;
+    int entry, tm, tn;
+    decode(0, entry, tm, tn);
+    float *const Cb = c_of(entry);
+    // a unit: one column of a consumer wave's tiles
+    for (int unit = wave; unit < CW * NT_; unit += CW + PW) {
+      const int w = unit / NT_, j = unit - w * NT_;
+      f64x2 sum[MT_][2];
+#pragma unroll
+      for (int i = 0; i < MT_; i++)
+        sum[i][0] = sum[i][1] = f64x2{0., 0.};
+      const unsigned long long *from = plane(0) + unit * (MT_ * 128) + lane;
+      constexpr int AHEAD = 16 / MT_; // planes read at a time
+      for (int z = 0; z < p.slices; z += AHEAD) {
+        unsigned long long v[AHEAD][MT_][2];
+#pragma unroll
+        for (int a = 0; a < AHEAD; a++) {
+          // (past the last plane the last one again, not added)
+          const int zz = z + a < p.slices ? z + a : p.slices - 1;
+          const unsigned long long *const src =
+              from + static_cast<long long>(zz) * (BM * BN / 2);
+#pragma unroll
+          for (int i = 0; i < MT_; i++)
+#pragma unroll
+            for (int h = 0; h < 2; h++)
+              v[a][i][h] =
+                  __hip_atomic_load(src + (i * 2 + h) * 64, __ATOMIC_RELAXED,
+                                    __HIP_MEMORY_SCOPE_AGENT);
+        }
+#pragma unroll
+        for (int a = 0; a < AHEAD; a++)
+          if (z + a < p.slices)
+#pragma unroll
+            for (int i = 0; i < MT_; i++)
+#pragma unroll
+              for (int h = 0; h < 2; h++)
+                sum[i][h] += __builtin_convertvector(
+                    __builtin_bit_cast(f32x2, v[a][i][h]), f64x2);
+      }
+      const auto value = [&](const int i, int) {
+        const f32x2 lo = __builtin_convertvector(sum[i][0], f32x2),
+                    hi = __builtin_convertvector(sum[i][1], f32x2);
+        return f32x4{lo[0], lo[1], hi[0], hi[1]} * p.alpha;
+      };
+      store_piece<MT_, 1, MT_ % 2 == 0, MT_>(
+          value, Cb, p.ldc, tm * BM + (w & 1) * WM,
+          tn * BN + (w >> 1) * WN + 16 * j, M, N, p.beta, lane);
+    }
+  };
+
   // (the waves of a workgroup meet at the same number of barriers, two and one
   // a stage, whatever their part; the producers' vector instructions are the
   // longest part of a step: they go first where they share a SIMD with a
@@ -541,11 +696,18 @@ __global__ void __launch_bounds__(64 * (CW + PW), SLICED ? 4 : 1)
       produce(ic<kFusedRRows>{});
     else
       produce(ic<kFusedAny>{});
+    if constexpr (SPREAD) {
+      __builtin_amdgcn_s_setprio(0);
+      fold_if_last();
+    }
     return;
   }
 
   // ---- consumer: step s of the stream, the MFMAs of stage s while the fragments
   // of stage s+1 (after a tile's last stage the next tile's first) are read
+  if constexpr (SPREAD)
+    if (wave == 0 && lane == 0) // (while the producers wait for their first loads)
+      start_count(p.arrivals + spread_tile, p.launch);
   asm volatile("s_barrier" ::: "memory"); // stages 0 and 1 are there
   Frags f[RECYCLE ? 1 : 2];
   unsigned held = 0; // LDS offset of the buffer whose stage is in registers
@@ -589,7 +751,6 @@ __global__ void __launch_bounds__(64 * (CW + PW), SLICED ? 4 : 1)
       held = next;
     }
   };
-  typedef double f64x4 __attribute__((ext_vector_type(4)));
   for (int tile = 0; tile < n_my; tile++) {
     f64x4 sum[SLICED ? MT_ : 1][SLICED ? NT_ : 1]; // of the slices
     if constexpr (SLICED) {
@@ -629,12 +790,29 @@ __global__ void __launch_bounds__(64 * (CW + PW), SLICED ? 4 : 1)
           f[0] = f[1];
       }
     }
+    if constexpr (SPREAD) {
+      if constexpr (RECYCLE) // (the producers' last barrier)
+        asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+      unsigned long long *const to = plane(slice) + wave * (NTILE * 128) + lane;
+#pragma unroll
+      for (int j = 0; j < NT_; j++)
+#pragma unroll
+        for (int i = 0; i < MT_; i++) {
+          const f32x4 v = folded(i, j);
+#pragma unroll
+          for (int h = 0; h < 2; h++)
+            __hip_atomic_store(to + ((j * MT_ + i) * 2 + h) * 64,
+                               __builtin_bit_cast(
+                                   unsigned long long,
+                                   f32x2{v[2 * h], v[2 * h + 1]}),
+                               __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        }
+      fold_if_last();
+      return;
+    }
     int entry, tm, tn;
     decode(tile, entry, tm, tn);
-    typedef float *const __attribute__((address_space(4))) *out_array_t;
-    float *const Cb = p.c_ptrs != nullptr
-                          ? ((out_array_t)p.c_ptrs)[entry]
-                          : p.C + static_cast<long long>(entry) * p.c_bs;
+    float *const Cb = c_of(entry);
     const float alpha = p.alpha;
     const auto out_value = [&](const int i, const int j) {
       if constexpr (SLICED)
