@@ -32,8 +32,7 @@ def _check(tc, dev, ta, tb, m, n, k, batch, policy, rn=0, pad=0, alpha=1.0, beta
 
     want = call(PACKED, torch.empty(tc.workspace_bytes(m, n, k, batch, policy), dtype=torch.uint8, device=dev))
     assert torch.isfinite(want).all()
-    # (a workspace that the path on packed operands would turn down, where it is smaller than they are)
-    size = _room(m, n, batch, slices)
+    size = max(_room(m, n, batch, slices), tc.workspace_bytes(m, n, k, batch, policy))
     room = torch.randint(0, 256, (size + 4096,), dtype=torch.uint8, device=dev)
     guard = room[size:].clone()
     for _ in range(3):
@@ -83,7 +82,7 @@ def test_replayed_graph(tc, dev):
     C = torch.zeros((n, m), device=dev)
     for slices in (2, 20, 32):
         with tc.forced_k_slices(slices):
-            ws = torch.randint(0, 256, (_room(m, n, 1, slices),), dtype=torch.uint8, device=dev)
+            ws = torch.randint(0, 256, (tc.workspace_bytes(m, n, k),), dtype=torch.uint8, device=dev)
 
             def call():
                 tc.sgemm("T", "N", m, n, k, 1.0, A, k, B, k, 0.0, C, m, 0, 0, ws)

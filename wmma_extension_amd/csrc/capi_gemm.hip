@@ -217,6 +217,68 @@ inline Choice choose_path(const int m, const int n, const int k, const int batch
   return {single && e.slices == 1 ? Path::Fused : e.base, e.slices, single,
           single ? fused : e.base_time};
 }
+// A call that its path turns down for the workspace it is given stays with it.
+inline bool refused_on_packed(const Choice &c, const int m, const int n,
+                              const int k, const int batch, const int terms,
+                              const void *const workspace,
+                              const size_t workspace_bytes) {
+  return !c.single && c.path == Path::Packed && workspace != nullptr &&
+         (reinterpret_cast<uintptr_t>(workspace) % 16 != 0 ||
+          workspace_bytes <
+              static_cast<size_t>(packed_elems(m, k, terms) +
+                                  packed_elems(n, k, terms)) *
+                  16u * static_cast<size_t>(batch));
+}
+// Bytes for the K slices of the tiles of a partly empty last round: the largest
+// need over the tile shapes and residencies the launch may choose; 0: no such
+// tiles.
+size_t tail_room(const int policy, const int m, const int n, const int k,
+                 const int batch) {
+  size_t need = 0;
+  if (batch != 1 || m <= 0 || n <= 0)
+    return need;
+  const int shapes[3][2] = {{256, 128}, {128, 128}, {64, 64}};
+  for (int i = 0; i < 3; i++) {
+    const int *const sh = shapes[i];
+    const TailPlan t =
+        plan_tail(ceil_div(m, sh[0]) * ceil_div(n, sh[1]),
+                  static_cast<long long>(device_cus()) *
+                      policy_kernels(policy)->per_cu(i),
+                  packed_k_tiles(k));
+    if (t.slices >= 2)
+      need = std::max<size_t>(need, static_cast<size_t>(t.slices) *
+                                        static_cast<size_t>(t.tail) * sh[0] *
+                                        sh[1] * 4u);
+  }
+  return need;
+}
+// Whether an uncut product that the path query gives to another path runs in the
+// single kernel all the same: same bits, and by its time alone it is ahead
+// (estimate_paths holds it back for the query's sake, ('T','N') products of k % 4
+// != 0 or of large outputs).
+inline bool single_is_ahead(const Choice &c, const int m, const int n,
+                            const int k, const int batch, const int flags,
+                            const int policy, const int terms, const bool rows,
+                            const void *const workspace,
+                            const size_t workspace_bytes) {
+  if (c.single || c.slices != 1 || c.time <= 0. || batch > (1 << 26) ||
+      refused_on_packed(c, m, n, k, batch, terms, workspace, workspace_bytes))
+    return false;
+  const double bytes =
+      4.0 * batch * (static_cast<double>(m) * n + (static_cast<double>(m) + n) * k);
+  const double ahead =
+      c.path == Path::Packed
+          ? ((flags & WMMAE_FLAG_RN_MAIN) != 0 ? fit::kSinglePackedRn
+                                               : fit::kSinglePacked)
+      : bytes > 256.0 * (1 << 20) ? fit::kSingleDirectLarge
+                                  : fit::kSingleDirect;
+  const double time =
+      std::max(fit::kCallFloor[0],
+               std::min(fused_time(terms, m, n, k, batch, true, rows),
+                        fused_time(terms, m, n, k, batch, false, rows)));
+  // (the other kernels cut the tiles of a partly empty last round along K)
+  return time < ahead * c.time && tail_room(policy, m, n, k, batch) == 0;
+}
 // Tile of the single kernel (64 or 128) that makes a cut product's slices with a
 // workgroup each, 0: the slices are made as chosen.  The products that run on
 // packed operands or in the direct kernel, or whose slices one workgroup of the
@@ -229,10 +291,13 @@ inline int choose_spread(const Choice &c, const int m, const int n, const int k,
                          const int batch, const int terms,
                          const void *const workspace,
                          const size_t workspace_bytes) {
-  if (c.slices <= 1 || c.time <= 0.)
+  if (c.slices <= 1 || c.time <= 0. ||
+      refused_on_packed(c, m, n, k, batch, terms, workspace, workspace_bytes))
     return 0;
   double best = c.time;
-  if (!c.single)
+  if (c.single)
+    best = c.time / fit::kSpreadSlicedMargin;
+  else
     best = c.path == Path::Direct
                ? c.time / fit::kSpreadDirectMargin
                : std::max(c.time / fit::kSpreadPackedMargin,
@@ -539,6 +604,9 @@ int sgemm_impl(const char transa, const char transb, const int m, const int n,
                                  rows || fused_considered(k), rows, direct_ok);
     path = c.single ? Path::Fused : c.path;
     slices = c.slices;
+    if (single_is_ahead(c, m, n, k, batch, rn, policy, p.terms, rows, workspace,
+                        workspace_bytes))
+      path = Path::Fused;
     spread_tile = choose_spread(c, m, n, k, batch, p.terms, workspace,
                                 workspace_bytes);
     if (spread_tile > 0)
@@ -744,26 +812,8 @@ int wmmae_tcec_gemm_packed_workspace_bytes(const int policy, const int m,
                          : 1);
   if (splits > 1) {
     *bytes = static_cast<size_t>(splits) * batch * m * n * 4u;
-  } else if (batch == 1 && m > 0 && n > 0) {
-    // K slices of the tiles of a partly empty last round: the largest need
-    // over the tile shapes and residencies the launch may choose
-    const int KT = packed_k_tiles(k);
-    size_t need = 0;
-    const int shapes[3][2] = {{256, 128}, {128, 128}, {64, 64}};
-    for (int i = 0; i < 3; i++) {
-      const int *const sh = shapes[i];
-      const int per_cu = policy_kernels(policy)->per_cu(i);
-      const TailPlan t =
-          plan_tail(ceil_div(m, sh[0]) * ceil_div(n, sh[1]),
-                    static_cast<long long>(device_cus()) * per_cu, KT);
-      if (t.slices >= 2)
-        need = std::max<size_t>(need, static_cast<size_t>(t.slices) *
-                                          static_cast<size_t>(t.tail) * sh[0] *
-                                          sh[1] * 4u);
-    }
-    *bytes = need;
   } else {
-    *bytes = 0;
+    *bytes = tail_room(policy, m, n, k, batch);
   }
   return WMMAE_STATUS_SUCCESS;
 }

@@ -279,6 +279,17 @@ inline double fused_direct_margin(const int m, const int n, const int k,
              ? kFusedStreamMargin
              : 1.0;
 }
+// An uncut product that the path query gives to another path runs in the single
+// kernel where its own time is below this much of that path's estimate.  Of 500
+// random ('T','N') products of those paths (m, n = 32 .. 8192, k up to 65536, 1 ..
+// 1024 entries; each run both ways): packed operands, 186 below 0.95, 0.67 of
+// the time in the median, two above 1.03 (the leading product outside the matrix
+// core: 25 below 1.15, 0.55, none above 1.05); the direct kernel below 0.88, 39,
+// 0.83, three above 1.03 by up to 5 %, and below 0.6 where the batch exceeds the
+// 256 MiB of the memory-side cache, 0.82 (95x125x10978 x 172 at 0.64 is 1.3 times
+// slower: the single kernel's estimate overlaps stages and traffic too well there).
+constexpr double kSinglePacked = 0.95, kSinglePackedRn = 1.15,
+                 kSingleDirect = 0.88, kSingleDirectLarge = 0.6;
 // Adding a K slice to the double-precision sums, for the workgroups of a compute
 // unit at a time: 110 products run with the cut and uncut, 0.17 us in the median
 // (one workgroup a unit), 0.10 (two), 3 % of a call.
@@ -313,7 +324,8 @@ constexpr double kSpreadBytesPerS = 4.9e12;
 // ahead of their estimates; cut products on packed operands take no less than 15 us
 // and 0.4 a slice (their estimate has 16 to 18 us for 64 x 46 x 4032 in 21 slices,
 // which takes 27).
-constexpr double kSpreadDirectMargin = 1.2, kSpreadPackedMargin = 1.1;
+constexpr double kSpreadDirectMargin = 1.25, kSpreadPackedMargin = 1.1,
+                 kSpreadSlicedMargin = 1.25;
 constexpr double kCutPacked = 15e-6, kCutPackedSlice = 0.4e-6;
 // Its workgroups that are resident on a compute unit: 12 waves of up to 168
 // registers (128x128), twice 8 waves of up to 128.
