@@ -48,6 +48,47 @@ int api_gemm_impl(const int type, const int ec, const int m, const int n,
       using EC = typename decltype(te)::type;
       using P = typename harness_policy<T, EC, 16, 16, 32>::type;
       const auto launch = [&](auto rr) -> int {
+        if constexpr (!std::is_same<T, float>::value) {
+          const auto split = [&](auto shape) -> int {
+            using SS = decltype(shape);
+            auto kernel = wmmae_harness::tcec_api_gemm_split_kernel<
+                T, P, SS, decltype(rr)::value>;
+            static std::atomic<unsigned long long> lds_allowed{0};
+            WMMAE_HIP_TRY(
+                allow_dynamic_lds(reinterpret_cast<const void *>(kernel),
+                                  SS::LDS_BYTES, lds_allowed));
+            const long long grid =
+                static_cast<long long>(m / SS::BM) * (n / SS::BM) * batch;
+            hipLaunchKernelGGL(kernel, dim3(static_cast<unsigned>(grid)),
+                               dim3(SS::THREADS), SS::LDS_BYTES, s, m, n, k, al,
+                               A, a_ptrs, lda, stride_a, B, b_ptrs, ldb,
+                               stride_b, be, C, c_ptrs, ldc, stride_c);
+            return launch_status();
+          };
+          // Up to half a round of large tiles the smaller ones (two fp16 terms,
+          // against the large tile with eight waves: 18 tiles 7.8 us for 12.5, 88
+          // tiles 13.0 for 15.4, 144 tiles 51.6 for 46.5).  Up to one round of
+          // large tiles eight waves share a tile, which hide each other's
+          // conversions (198 tiles of k = 7008: 180 us, four waves 230); with more,
+          // two workgroups of four waves a compute unit do that and read a third
+          // less from LDS (1024 tiles of k = 4096: 446, eight waves 465), but three
+          // terms do not fit their registers (957 us for 712).
+          // The kernel that splits at the fragment load stays for more than a round
+          // of tiles of one term and a long k (its direct copies take no registers;
+          // 897 tiles, k = 4096: 245 us for 297, at k = 1024 91 for 81) and of three
+          // terms and a short one (two workgroups a compute unit; 828 tiles, k =
+          // 224: 48.7 for 53.1, at k = 512 102 for 103).
+          using wmmae_harness::ApiSplitShape;
+          constexpr int terms = ApiSplitShape<T, P, 128, 2>::TERMS;
+          const long long cus = device_cus();
+          if (2 * blocks <= cus)
+            return split(ApiSplitShape<T, P, 64, 2>{});
+          if (blocks <= cus || (terms == 3 && k >= 512))
+            return split(ApiSplitShape<T, P, 128, 4>{});
+          if constexpr (terms < 3)
+            if (terms == 2 || k < 3072)
+              return split(ApiSplitShape<T, P, 128, 2>{});
+        }
         auto kernel =
             wmmae_harness::tcec_api_gemm_kernel<T, P, 2, decltype(rr)::value>;
         static std::atomic<unsigned long long> lds_allowed{0};

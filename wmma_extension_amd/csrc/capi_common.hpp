@@ -54,6 +54,27 @@ inline hipError_t allow_dynamic_lds(const void *const kernel, const int bytes,
   return e;
 }
 
+// Compute units of the current device, looked up once per device.
+inline int device_cus() {
+  static std::atomic<int> cached[64];
+  int dev = 0;
+  if (hipGetDevice(&dev) != hipSuccess)
+    return 256; // MI355X; also the answer when no device is visible
+  const bool tracked = dev >= 0 && dev < 64;
+  if (tracked) {
+    const int c = cached[dev].load(std::memory_order_relaxed);
+    if (c > 0)
+      return c;
+  }
+  hipDeviceProp_t prop;
+  if (hipGetDeviceProperties(&prop, dev) != hipSuccess ||
+      prop.multiProcessorCount <= 0)
+    return 256;
+  if (tracked)
+    cached[dev].store(prop.multiProcessorCount, std::memory_order_relaxed);
+  return prop.multiProcessorCount;
+}
+
 // ---- type / policy dispatch of the device-API harness entry points
 template <class F> int with_type(const int type, F f) {
   switch (type) {

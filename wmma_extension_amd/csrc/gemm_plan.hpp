@@ -101,27 +101,6 @@ struct GemmArgs {
   wmmae_gemm::DirectSource direct = {};
 };
 
-// Compute units of the current device, looked up once per device.
-inline int device_cus() {
-  static std::atomic<int> cached[64];
-  int dev = 0;
-  if (hipGetDevice(&dev) != hipSuccess)
-    return 256; // MI355X; also the answer when no device is visible
-  const bool tracked = dev >= 0 && dev < 64;
-  if (tracked) {
-    const int c = cached[dev].load(std::memory_order_relaxed);
-    if (c > 0)
-      return c;
-  }
-  hipDeviceProp_t prop;
-  if (hipGetDeviceProperties(&prop, dev) != hipSuccess ||
-      prop.multiProcessorCount <= 0)
-    return 256;
-  if (tracked)
-    cached[dev].store(prop.multiProcessorCount, std::memory_order_relaxed);
-  return prop.multiProcessorCount;
-}
-
 // ------------------------------------------------ fitted cost parameters
 // Every number the path and tile choices below are made with, in one place.
 // All are fits to measurements on MI355X (256 compute units, one box of the
@@ -324,7 +303,7 @@ constexpr double kSpreadBytesPerS = 4.9e12;
 // ahead of their estimates; cut products on packed operands take no less than 15 us
 // and 0.4 a slice (their estimate has 16 to 18 us for 64 x 46 x 4032 in 21 slices,
 // which takes 27).
-constexpr double kSpreadDirectMargin = 1.25, kSpreadPackedMargin = 1.1,
+constexpr double kSpreadDirectMargin = 1.25, kSpreadPackedMargin = 1.2,
                  kSpreadSlicedMargin = 1.25;
 constexpr double kCutPacked = 15e-6, kCutPackedSlice = 0.4e-6;
 // Its workgroups that are resident on a compute unit: 12 waves of up to 168

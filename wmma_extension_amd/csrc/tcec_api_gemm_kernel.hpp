@@ -1,9 +1,11 @@
-// A tiled, batched SGEMM written only against the public device API of this
-// library (tcec::fragment, load_matrix_sync, mma_sync, store_matrix_sync,
+// A tiled, batched SGEMM written against the public device API of this library
+// (tcec::fragment, load_matrix_sync, mma_sync, store_matrix_sync,
 // utils::cp_async), the way a user of the reference writes one: the shape of
 // the reference's bgemm_kernel / mma_core / dmem2smem
 // (test/tcec/batch_gemm.cu:74-116, 196-257, 261-386).
 //
+// tcec_api_gemm_kernel (fp32 operands kept whole; most products of 16-bit terms
+// take tcec_api_gemm_split_kernel below):
 //   * fp32 tiles of A (row-major) and B (column-major) are staged in LDS by
 //     utils::cp_async, two stages: the copies of stage s+1 are in flight while
 //     stage s is multiplied;
@@ -188,6 +190,210 @@ __global__ void __launch_bounds__(ApiGemmShape::THREADS, WAVES_PER_SIMD)
   float *const cw = (c_ptrs != nullptr ? c_ptrs[entry] : C + entry * stride_c) +
                     (tm * S::BM + wm * S::WM) +
                     static_cast<long long>(tn * S::BN + wn * S::WN) * ldc;
+  if (beta == 0.f) {
+    tcec::store_matrix_sync_with_mul<w::col_major>(cw, fc, ldc, alpha);
+  } else {
+    FragC fin;
+    tcec::load_matrix_sync(fin, cw, ldc, w::mem_col_major);
+    fc.integrate();
+#pragma unroll
+    for (unsigned i = 0; i < fc.num_elements; i++) // (the roundings written out)
+      fc.x(i) = __builtin_fmaf(alpha, fc.x(i), beta * fin.x(i));
+    tcec::store_matrix_sync(cw, fc, ldc, w::mem_col_major);
+  }
+}
+
+// The same product for operands of 16-bit terms: every element is split once per
+// workgroup, not once per wave that needs it, and no fp32 tile passes through LDS.
+// A wave loads its share of a stage's row blocks (16 rows of op(A) or columns of
+// op(B), 32 of k) into registers a stage ahead, splits them (split4, what
+// load_matrix_sync splits with) and puts the terms into LDS where the lanes of a
+// 16x16x32 fragment find theirs 16 bytes at a time; the waves fill the registers
+// of their tcec:: fragments from there.  With a conversion per wave the kernel was
+// bound by its instruction issue (1.66e8 vector instructions beside 2.5e7 matrix
+// ones at 4096^3) and, on few tiles, by its own chain of copy, split and multiply.
+// Two fp16 terms, before -> now: 4096^3 498 -> 446 us, 1152x2816x7008 252 -> 180,
+// 1920x1920x1024 44.7 -> 32.5, 256x256x8192 285 -> 136, 768x384x352 17.5 -> 7.8;
+// three bf16 terms 4096^3 738 -> 712, 768x384x352 23.8 -> 10.0; one term
+// 2944x3456x608 41.3 -> 31.5.  What bounds it now: conversions, the adds of
+// mma_rn_sync and matrix instructions share a SIMD's one or two waves.  Loads of eight lanes to a row's 128 bytes: with a lane's
+// eight k in two loads of its own the rows' requests ran at 9.5 TB/s, half the rate.
+//   BM  : block tile (64 or 128), 2 x WGN waves
+template <class T, class Policy, int BM_, int WGN> struct ApiSplitShape {
+  static constexpr int BM = BM_, SK = 32, WM = BM / 2, WN = BM / WGN;
+  static constexpr int NW = 2 * WGN, THREADS = 64 * NW;
+  static constexpr int BLOCKS = 2 * BM / 16; // row blocks of a stage, A's first
+  static constexpr int PER_WAVE = BLOCKS / NW;
+  static constexpr int TERMS =
+      tcec::fragment<w::matrix_a, 16, 16, SK, T, w::row_major, Policy>::num_terms;
+  static constexpr int STAGE_BYTES = BLOCKS * TERMS * 1024;
+  // two stages where two workgroups of a compute unit have room for them, else
+  // one and a second barrier a stage
+  static constexpr int STAGES = 2 * STAGE_BYTES <= (NW > 4 ? 160 : 80) * 1024 ? 2 : 1;
+  static constexpr int LDS_BYTES = STAGES * STAGE_BYTES;
+};
+
+template <class T, class Policy, class S, int ROUNDING>
+__global__ void __launch_bounds__(S::THREADS, S::BM > 64 ? 2 : 3)
+    tcec_api_gemm_split_kernel(const int m, const int n, const int k,
+                               const float alpha, const float *const A,
+                               const float *const *const a_ptrs, const int lda,
+                               const long long stride_a, const float *const B,
+                               const float *const *const b_ptrs, const int ldb,
+                               const long long stride_b, const float beta,
+                               float *const C, float *const *const c_ptrs,
+                               const int ldc, const long long stride_c) {
+  constexpr int BM = S::BM, WGN = S::NW / 2;
+  extern __shared__ __attribute__((aligned(1024))) unsigned char terms_lds[];
+
+  const unsigned tiles_m = m / BM, tiles_n = n / BM;
+  const unsigned tiles = tiles_m * tiles_n;
+  const unsigned entry = blockIdx.x / tiles;
+  unsigned t = blockIdx.x - entry * tiles;
+  if (tiles % 8 == 0)
+    t = (t % 8) * (tiles / 8) + t / 8;
+  const unsigned band = t / (8 * tiles_n);
+  const unsigned band_rows = tiles_m - 8 * band < 8 ? tiles_m - 8 * band : 8;
+  const unsigned in_band = t - band * 8 * tiles_n;
+  const unsigned tn = in_band / band_rows;
+  const unsigned tm = 8 * band + in_band - tn * band_rows;
+
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / 64);
+  const int wm = wave % 2, wn = wave / 2;
+  const unsigned lane = threadIdx.x & 63u;
+
+  using FragA =
+      tcec::fragment<w::matrix_a, S::WM, S::WN, S::SK, T, w::row_major, Policy>;
+  using FragB =
+      tcec::fragment<w::matrix_b, S::WM, S::WN, S::SK, T, w::col_major, Policy>;
+  using FragC =
+      tcec::fragment<w::accumulator, S::WM, S::WN, S::SK, T, void, Policy>;
+  FragC fc;
+  tcec::fill_zero(fc);
+  const auto mma = [](FragC &d, const FragA &a, const FragB &b) {
+    if constexpr (ROUNDING == 1)
+      tcec::mma_rn_sync(d, a, b, d);
+    else if constexpr (ROUNDING == 2)
+      tcec::mma_rz_sync(d, a, b, d);
+    else
+      tcec::mma_sync(d, a, b, d);
+  };
+
+  // this wave's row blocks: the first half of the waves takes A's, the others B's
+  // (a lane's registers of a matrix_b fragment are those of a matrix_a fragment
+  // with rows and columns exchanged)
+  const bool is_a = wave < WGN;
+  const int ld = is_a ? lda : ldb;
+  const float *src =
+      (is_a ? (a_ptrs != nullptr ? a_ptrs[entry] : A + entry * stride_a) +
+                  static_cast<long long>(tm * BM) * lda
+            : (b_ptrs != nullptr ? b_ptrs[entry] : B + entry * stride_b) +
+                  static_cast<long long>(tn * BM) * ldb) +
+      static_cast<long long>(wave % WGN) * (S::PER_WAVE * 16) * ld;
+
+  // Load h of a row block takes its rows 8h .. 8h+7, eight lanes to a row's 128
+  // bytes: four k, half of what a lane of a 16x16x32 operand holds.
+  typedef float f32x4 __attribute__((ext_vector_type(4)));
+  f32x4 raw[S::PER_WAVE][2];
+  src += static_cast<long long>(lane >> 3) * ld + 4 * (lane & 7u);
+  const auto load_raw = [&]() {
+#pragma unroll
+    for (int p = 0; p < S::PER_WAVE; p++)
+#pragma unroll
+      for (int h = 0; h < 2; h++)
+        raw[p][h] = *static_cast<const f32x4 *>(__builtin_assume_aligned(
+            src + static_cast<long long>(16 * p + 8 * h) * ld, 16));
+  };
+  // 16-byte slot of (row r, k group q) in a chunk of 16 rows x 32 k of one term:
+  // 16 q + (r ^ spread(q)), so that the lanes of a write that hold the same row do
+  // not share their banks
+  const auto spread = [](const unsigned q) { return 12u * (q & 1u) ^ 4u * (q >> 1); };
+  const unsigned read_off =
+      16u * ((lane & 48u) + ((lane & 15u) ^ spread(lane >> 4)));
+  unsigned write_off[2];
+#pragma unroll
+  for (unsigned h = 0; h < 2; h++) {
+    const unsigned q = (lane & 7u) >> 1, r = 8u * h + (lane >> 3);
+    write_off[h] = 16u * (16u * q + (r ^ spread(q))) + 8u * (lane & 1u);
+  }
+  const auto chunk = [&](const int stage, const int block, const int term) {
+    return terms_lds + stage * S::STAGE_BYTES +
+           (block * S::TERMS + term) * 1024;
+  };
+  const auto get = [&](auto &sub, const unsigned char *const from) {
+    static_assert(sizeof(sub.x) == 16, "eight 16-bit values a lane");
+    __builtin_memcpy(sub.x, __builtin_assume_aligned(from + read_off, 16), 16);
+  };
+  const auto put_terms = [&](const int stage) {
+    using E = typename tcec::detail::split_traits<T>::storage;
+#pragma unroll
+    for (int p = 0; p < S::PER_WAVE; p++)
+#pragma unroll
+      for (int h = 0; h < 2; h++) {
+        E term[3][4];
+        tcec::detail::split4<T>(raw[p][h], term[0], term[1], term[2]);
+#pragma unroll
+        for (int x = 0; x < S::TERMS; x++)
+          __builtin_memcpy(__builtin_assume_aligned(
+                               chunk(stage, wave * S::PER_WAVE + p, x) +
+                                   write_off[h], 8),
+                           term[x], 8);
+      }
+  };
+  const auto get_frag = [&](auto &f, const int stage, const int block0) {
+#pragma unroll
+    for (int i = 0; i < std::remove_reference_t<decltype(f)>::num_sub_frags; i++) {
+      get(f.sub_frag[i], chunk(stage, block0 + i, 0));
+      if constexpr (S::TERMS >= 2)
+        get(f.sub_d_frag[i], chunk(stage, block0 + i, 1));
+      if constexpr (S::TERMS >= 3)
+        get(f.sub_d2_frag[i], chunk(stage, block0 + i, 2));
+    }
+  };
+
+  load_raw();
+  put_terms(0);
+  src += k > S::SK ? S::SK : 0;
+  load_raw();
+  __syncthreads();
+  int stage = 0;
+  for (int k0 = S::SK; k0 < k; k0 += S::SK) {
+    FragA fa;
+    FragB fb;
+    get_frag(fa, stage, wm * (S::WM / 16));
+    get_frag(fb, stage, S::BM / 16 + wn * (S::WN / 16));
+    if constexpr (S::STAGES == 1)
+      __syncthreads();
+    stage = S::STAGES - 1 - stage;
+    put_terms(stage);
+    // (the last one again where there is no other, never used)
+    src += k0 + S::SK < k ? S::SK : 0;
+    load_raw();
+    mma(fc, fa, fb);
+    // a stage's vector instructions go between its matrix instructions, two after
+    // each (three fp16 products, eight waves a tile: 1152x2816x7008 206 -> 180 us,
+    // 4096^3 496 -> 465; three or more after each 1 to 13 % slower, and one
+    // product is better left to the compiler)
+    if constexpr (S::TERMS >= 2) {
+#pragma unroll
+      for (int i = 0; i < 48; i++) {
+        __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+        __builtin_amdgcn_sched_group_barrier(0x002, 2, 0);
+      }
+    }
+    __syncthreads();
+  }
+  {
+    FragA fa;
+    FragB fb;
+    get_frag(fa, stage, wm * (S::WM / 16));
+    get_frag(fb, stage, S::BM / 16 + wn * (S::WN / 16));
+    mma(fc, fa, fb);
+  }
+
+  float *const cw = (c_ptrs != nullptr ? c_ptrs[entry] : C + entry * stride_c) +
+                    (tm * BM + wm * S::WM) +
+                    static_cast<long long>(tn * BM + wn * S::WN) * ldc;
   if (beta == 0.f) {
     tcec::store_matrix_sync_with_mul<w::col_major>(cw, fc, ldc, alpha);
   } else {
