@@ -1,0 +1,78 @@
+"""The native host path of the frequent calls takes plain arguments only: everything else comes back as
+"not taken" and meets the checks in Python, with the same errors as before."""
+import pytest
+import torch
+
+from wmma_extension_amd import tcec
+from wmma_extension_amd._lib import WmmaeError
+
+NOT_TAKEN = 1
+
+
+def test_what_is_not_plain_is_not_taken():
+    calls = tcec._native()
+    A = torch.zeros(8, 8)
+    for name in ("sgemm", "sgemm_strided_batched", "sgemm_batched", "matmul_tn", "pack", "gemm_packed", "api_gemm",
+                 "primitive_tiles"):
+        assert getattr(calls, name)() == NOT_TAKEN
+        assert getattr(calls, name)(*[None] * 17) == NOT_TAKEN
+    ok = ["T", "N", 8, 8, 8, 1.0, A, 8, A, 8, 0.0, A, 8, 0, 0, None, 0]
+    assert calls.sgemm(*ok) == NOT_TAKEN                      # tensors of the host
+    for i, v in ((0, "TT"), (0, ""), (0, b"T"), (0, "Τ"), (2, 8.0), (2, 1 << 70), (3, 1 << 40), (5, "1"), (6, 5),
+                 (15, [1]), (16, None), (16, 1.5)):
+        assert calls.sgemm(*(ok[:i] + [v] + ok[i + 1:])) == NOT_TAKEN, (i, v)
+    with pytest.raises(ValueError, match="device tensors"):
+        tcec.sgemm(*ok[:13])
+    with pytest.raises(ValueError, match="device tensors"):
+        tcec.matmul_tn(A, A)
+
+
+@pytest.mark.gpu
+def test_the_same_results_and_errors_on_either_path(tc, dev):
+    m, n, k = 96, 80, 160
+    A, B = torch.rand((m, k), device=dev), torch.rand((n, k), device=dev)
+    want = tc.matmul_tn(A, B, out=torch.empty((n, m), device=dev))      # (an output of the caller: checked in Python)
+    assert torch.equal(tc.matmul_tn(A, B), want)
+    C = torch.zeros((n, m), device=dev)
+    tc.sgemm("T", "N", m, n, k, 1, A, k, B, k, 0, C, m)
+    assert torch.equal(C, want)
+    # views that are not contiguous, numbers that are no plain floats, a parameter
+    wide = torch.rand((m, k + 12), device=dev)
+    view = wide[:, :k].copy_(A)
+    C.zero_()
+    tc.sgemm("T", "N", m, n, k, torch.tensor(1.0), view, k + 12, torch.nn.Parameter(B), k, 0.0, C, m)
+    assert torch.equal(C, want)
+    stream = torch.cuda.Stream()
+    with torch.cuda.stream(stream):
+        stream.wait_stream(torch.cuda.default_stream())
+        got = tc.matmul_tn(A, B)
+    stream.synchronize()
+    assert torch.equal(got, want)
+
+    class Seen(torch.utils._python_dispatch.TorchDispatchMode):
+        ops = ()
+
+        def __torch_dispatch__(self, func, types, args=(), kwargs=None):
+            self.ops += (str(func),)
+            return func(*args, **(kwargs or {}))
+    with Seen() as seen:
+        got = tc.matmul_tn(A, B)
+    assert torch.equal(got, want) and any("empty" in o for o in seen.ops)
+    with pytest.raises(ValueError, match="float32"):
+        tc.sgemm("T", "N", m, n, k, 1.0, A.double(), k, B, k, 0.0, C, m)
+    with pytest.raises(ValueError, match="bytes from its first element"):
+        tc.sgemm("T", "N", m, n, k + 1, 1.0, A, k + 1, B, k + 1, 0.0, C, m)
+    with pytest.raises(ValueError, match="device tensors"):
+        tc.sgemm("T", "N", m, n, k, 1.0, A.cpu(), k, B, k, 0.0, C, m)
+    with pytest.raises(AssertionError):
+        tc.matmul_tn(A, B[:, :-1])
+    for flags in (64, 2 | 8):
+        with pytest.raises(WmmaeError) as e:
+            tc.sgemm("T", "N", m, n, k, 1.0, A, k, B, k, 0.0, C, m, 0, flags)
+        assert e.value.status == -1
+    with pytest.raises(WmmaeError) as e:
+        tc.api_gemm(0, 1, 100, n, k, 1.0, A[:, :128].contiguous(), 128, B, k, 0.0, C, m)
+    assert e.value.status in (-3, -4)
+    # gradients and transforms: raw pointers of wrapped tensors are refused as before
+    with pytest.raises(RuntimeError):
+        torch.func.vmap(lambda a: tc.matmul_tn(a, B))(A.expand(2, m, k).contiguous())

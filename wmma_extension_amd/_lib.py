@@ -7,6 +7,7 @@ import ctypes
 import glob
 import os
 import subprocess
+import sysconfig
 
 _PKG = os.path.dirname(os.path.abspath(__file__))
 ROOT = os.path.dirname(_PKG)
@@ -78,6 +79,22 @@ ASM_MFMA_SOURCES = ["gemm_f16.hip", "gemm_bf16.hip", "gemm_bf16x3.hip"]
 SOURCES = ["capi_gemm.hip", "capi_harness.hip", "capi_api_gemm.hip"] + ASM_MFMA_SOURCES
 
 
+# the frequent calls of tcec.py from Python in native code (no device code: the host compiler)
+HOST_CALLS_SOURCE = "host_calls.cpp"
+HOST_CALLS_PATH = os.path.join(LIB_DIR, "_wmmae_host_calls.so")
+
+
+def _host_calls_command():
+    import torch
+    root = os.path.dirname(os.path.abspath(torch.__file__))
+    includes = [os.path.join(root, "include"), os.path.join(root, "include", "torch", "csrc", "api", "include"),
+                sysconfig.get_paths()["include"]]
+    return [os.environ.get("CXX", "g++"), "-std=c++17", "-O2", "-fPIC", "-shared", "-fvisibility=hidden",
+            f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}", *("-I" + i for i in includes),
+            os.path.join(CSRC_DIR, HOST_CALLS_SOURCE), "-o", HOST_CALLS_PATH, "-L" + os.path.join(root, "lib"),
+            "-lc10", "-ltorch_cpu", "-ltorch_python"]
+
+
 def device_asm_path(name):
     """Where build() leaves the gfx950 assembly of a translation unit with inline-asm MFMAs."""
     return os.path.join(LIB_DIR, name.replace(".hip", "") + "-hip-amdgcn-amd-amdhsa-gfx950.s")
@@ -88,7 +105,7 @@ def _run(cmd, verbose):
     if verbose or res.returncode != 0:
         print(res.stdout)
     if res.returncode != 0:
-        raise RuntimeError("hipcc failed building libwmmae_tcec.so:\n" + res.stdout[-4000:])
+        raise RuntimeError(f"{os.path.basename(cmd[0])} failed building libwmmae_tcec.so:\n" + res.stdout[-4000:])
 
 
 def build(verbose=False, only=None):
@@ -109,7 +126,9 @@ def build(verbose=False, only=None):
             keep = ["-save-temps=obj"] if name in ASM_MFMA_SOURCES else []
             jobs.append([hipcc, *flags, *keep, "-I" + INCLUDE_DIR, "-c",
                          os.path.join(CSRC_DIR, name), "-o", obj])
-    with ThreadPoolExecutor(max_workers=len(SOURCES)) as pool:
+    if only is None or HOST_CALLS_SOURCE in only or not os.path.exists(HOST_CALLS_PATH):
+        jobs.append(_host_calls_command())
+    with ThreadPoolExecutor(max_workers=len(SOURCES) + 1) as pool:
         list(pool.map(lambda c: _run(c, verbose), jobs))
     from . import isa_check
     for name in ASM_MFMA_SOURCES:
@@ -198,6 +217,24 @@ def lib():
             fn.argtypes = argtypes
         _LIB = handle
     return _LIB
+
+
+def host_calls():
+    """The extension module of HOST_CALLS_SOURCE, bound to the loaded library; raise if it has not been
+    built.  (torch's libraries, which it uses, must be loaded already.)"""
+    import importlib.util
+    handle = lib()
+    if not os.path.exists(HOST_CALLS_PATH):
+        raise RuntimeError(f"{HOST_CALLS_PATH} is missing: build it with __graft_entry__.build()")
+    spec = importlib.util.spec_from_file_location("_wmmae_host_calls", HOST_CALLS_PATH)
+    module = importlib.util.module_from_spec(spec)
+    spec.loader.exec_module(module)
+    for name in ("wmmae_tcec_sgemm", "wmmae_tcec_sgemm_strided_batched", "wmmae_tcec_sgemm_batched",
+                 "wmmae_tcec_pack_bytes", "wmmae_tcec_pack", "wmmae_tcec_gemm_packed", "wmmae_tcec_api_gemm",
+                 "wmmae_primitive_tiles"):
+        if hasattr(handle, name):
+            module.bind(name, ctypes.cast(getattr(handle, name), ctypes.c_void_p).value)
+    return module
 
 
 class WmmaeError(RuntimeError):

@@ -55,7 +55,7 @@ inline hipError_t allow_dynamic_lds(const void *const kernel, const int bytes,
 }
 
 // Compute units of the current device, looked up once per device.
-inline int device_cus() {
+inline int lookup_device_cus() {
   static std::atomic<int> cached[64];
   int dev = 0;
   if (hipGetDevice(&dev) != hipSuccess)
@@ -73,6 +73,21 @@ inline int device_cus() {
   if (tracked)
     cached[dev].store(prop.multiProcessorCount, std::memory_order_relaxed);
   return prop.multiProcessorCount;
+}
+// ... and once per call of an entry point where one of these stands in it: the
+// time estimates ask some thirty times, and asking the runtime which device is
+// current took 1.2 of the 5.3 us a 64^3 product took to issue.
+inline thread_local int t_call_cus = 0;
+struct OneDeviceCall {
+  const int before = t_call_cus;
+  OneDeviceCall() {
+    if (t_call_cus == 0)
+      t_call_cus = lookup_device_cus();
+  }
+  ~OneDeviceCall() { t_call_cus = before; }
+};
+inline int device_cus() {
+  return t_call_cus > 0 ? t_call_cus : lookup_device_cus();
 }
 
 // ---- type / policy dispatch of the device-API harness entry points

@@ -528,6 +528,7 @@ int gemm_packed_impl(const int policy, const int m, const int n, const int k,
                          static_cast<unsigned>(e0));
     return launch_status();
   }
+  const OneDeviceCall one_device;
   GemmArgs g;
   g.a = static_cast<const u32x4 *>(packed_a);
   g.b = static_cast<const u32x4 *>(packed_b);
@@ -575,6 +576,7 @@ int sgemm_impl(const char transa, const char transb, const int m, const int n,
       (k > 0 && ((A == nullptr && a_ptrs == nullptr) ||
                  (B == nullptr && b_ptrs == nullptr))))
     return WMMAE_STATUS_NULL_POINTER;
+  const OneDeviceCall one_device;
   const int a_rows = is_n(transa) ? m : k; // rows of A as stored (column major)
   const int b_rows = is_n(transb) ? k : n;
   if (lda < (a_rows > 1 ? a_rows : 1) || ldb < (b_rows > 1 ? b_rows : 1) ||

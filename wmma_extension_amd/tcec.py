@@ -45,6 +45,34 @@ def _stream():
     return _raw_stream(_raw_device())
 
 
+# The frequent calls go through native code (csrc/host_calls.cpp) when their arguments are plain: it
+# returns the entry point's status, or _NOT_TAKEN with nothing done, and the checks here follow.
+_NOT_TAKEN = 1
+_calls = None
+
+
+def _native():
+    global _calls
+    if _calls is None:
+        _calls = _lib.host_calls()
+    return _calls
+
+
+def _native_stream():
+    """The current stream's handle, or None (which native code does not take) before torch has set up the GPU."""
+    if _raw_stream is None or _raw_device is None or not torch.cuda.is_initialized():
+        return None
+    return _raw_stream(_raw_device())
+
+
+def _done(st, where):
+    """Whether native code has made the call; raises for a status that is an error."""
+    if st == _NOT_TAKEN:
+        return False
+    _lib.check(st, where)
+    return True
+
+
 def _ptr(t):
     return t.data_ptr() if t is not None else None
 
@@ -196,6 +224,9 @@ def pack_bytes(rows, k, batch=1, policy=Policy.F16_EC):
 def sgemm(transa, transb, m, n, k, alpha, A, lda, B, ldb, beta, C, ldc,
           policy=Policy.F16_EC, flags=0, workspace=None):
     """C = alpha*op(A)*op(B) + beta*C, column-major BLAS convention."""
+    if _done((_calls or _native()).sgemm(transa, transb, m, n, k, alpha, A, lda, B, ldb, beta, C, ldc, policy, flags,
+                                         workspace, _native_stream()), "wmmae_tcec_sgemm"):
+        return
     _need_cuda(A, B, C, workspace)
     _check_gemm_operands(transa, transb, m, n, k, A, lda, B, ldb, C, ldc)
     ws_bytes = _bytes(workspace)
@@ -222,6 +253,11 @@ def sgemm_static(transa, transb, m, n, k, alpha, A, lda, B, ldb, beta, C, ldc,
 def sgemm_strided_batched(transa, transb, m, n, k, alpha, A, lda, stride_a, B, ldb, stride_b,
                           beta, C, ldc, stride_c, batch, policy=Policy.F16_EC, flags=0,
                           workspace=None):
+    if _done((_calls or _native()).sgemm_strided_batched(transa, transb, m, n, k, alpha, A, lda, stride_a, B, ldb,
+                                                         stride_b, beta, C, ldc, stride_c, batch, policy, flags,
+                                                         workspace, _native_stream()),
+             "wmmae_tcec_sgemm_strided_batched"):
+        return
     _need_cuda(A, B, C, workspace)
     _check_gemm_operands(transa, transb, m, n, k, A, lda, B, ldb, C, ldc, batch,
                          stride_a, stride_b, stride_c)
@@ -237,6 +273,10 @@ def sgemm_batched(transa, transb, m, n, k, alpha, A_array, lda, B_array, ldb, be
                   batch, policy=Policy.F16_EC, flags=0, workspace=None):
     """A_array / B_array / C_array: int64 device tensors holding `batch` device pointers
     (the launch_bgemm / cublasSgemmBatched convention)."""
+    if _done((_calls or _native()).sgemm_batched(transa, transb, m, n, k, alpha, A_array, lda, B_array, ldb, beta,
+                                                 C_array, ldc, batch, policy, flags, workspace, _native_stream()),
+             "wmmae_tcec_sgemm_batched"):
+        return
     _need_cuda(A_array, B_array, C_array, workspace)
     for name, arr in (("A_array", A_array), ("B_array", B_array), ("C_array", C_array)):
         if arr is not None and (arr.dtype != torch.int64 or arr.numel() < batch):
@@ -249,6 +289,9 @@ def sgemm_batched(transa, transb, m, n, k, alpha, A_array, lda, B_array, ldb, be
 
 
 def pack(policy, rows, k, X, row_stride, k_stride, packed, batch=1, batch_stride=0):
+    if _done((_calls or _native()).pack(policy, rows, k, X, row_stride, k_stride, packed, batch, batch_stride,
+                                        _native_stream()), "wmmae_tcec_pack"):
+        return
     _need_cuda(X, packed)
     if X is not None and X.dtype != torch.float32:
         raise ValueError(f"X: float32 tensor required, got {X.dtype}")
@@ -271,6 +314,10 @@ def gemm_packed_workspace_bytes(policy, m, n, k, batch=1):
 
 def gemm_packed(policy, m, n, k, alpha, packed_a, packed_b, beta, C, ldc, batch=1,
                 stride_c=0, flags=0, workspace=None):
+    if _done((_calls or _native()).gemm_packed(policy, m, n, k, alpha, packed_a, packed_b, beta, C, ldc, batch,
+                                               stride_c, flags, workspace, _native_stream()),
+             "wmmae_tcec_gemm_packed"):
+        return
     _need_cuda(packed_a, packed_b, C, workspace)
     _check_matrix("C", C, m, n, ldc, batch, stride_c)
     if k > 0 and m > 0 and n > 0 and batch > 0:
@@ -287,6 +334,12 @@ def matmul_tn(A, B, policy=Policy.F16_EC, flags=0, workspace=None, out=None):
     """The reference harness layout: A is (m,k) row-major, B is given as (n,k)
     row-major (= k x n column-major), result (n,m) row-major (= m x n column-major,
     ldc = m).  Returns the tensor holding C column-major, i.e. C^T as a torch view."""
+    if out is None:
+        out = (_calls or _native()).matmul_tn(A, B, policy, flags, workspace, _native_stream())
+        if isinstance(out, torch.Tensor):
+            return out
+        _done(out, "wmmae_tcec_sgemm")
+        out = None
     m, k = A.shape
     n, k2 = B.shape
     assert k == k2 and A.is_contiguous() and B.is_contiguous()
@@ -301,6 +354,10 @@ def matmul_tn(A, B, policy=Policy.F16_EC, flags=0, workspace=None, out=None):
 # --------------------------------------------------------------- harness
 def primitive_tiles(tiles):
     """tiles: (T,256) fp32.  Returns dict of the per-tile outputs."""
+    out = (_calls or _native()).primitive_tiles(tiles, _native_stream())
+    if isinstance(out, dict):
+        return out
+    _done(out, "wmmae_primitive_tiles")
     _need_cuda(tiles)
     T = tiles.shape[0]
     dev = tiles.device
@@ -382,6 +439,9 @@ def elementwise(type_, ec, inst, base, do_neg, do_integrate, device="cuda"):
 def api_gemm(type_, ec, m, n, k, alpha, A, lda, B, ldb, beta, C, ldc, rounding=0):
     """Tiled GEMM written against the public device API only (rounding: 0 tcec::mma_sync,
     1 mma_rn_sync, 2 mma_rz_sync)."""
+    if rounding == 0 and _done((_calls or _native()).api_gemm(type_, ec, m, n, k, alpha, A, lda, B, ldb, beta, C, ldc,
+                                                              _native_stream()), "wmmae_tcec_api_gemm"):
+        return
     _need_cuda(A, B, C)
     _check_gemm_operands("T", "N", m, n, k, A, lda, B, ldb, C, ldc)
     if rounding == 0:
