@@ -269,9 +269,11 @@ inline bool single_is_ahead(const Choice &c, const int m, const int n,
   const double ahead =
       c.path == Path::Packed
           ? ((flags & WMMAE_FLAG_RN_MAIN) != 0 ? fit::kSinglePackedRn
+             : terms == 1                      ? fit::kSinglePackedOneTerm
                                                : fit::kSinglePacked)
-      : bytes > 256.0 * (1 << 20) ? fit::kSingleDirectLarge
-                                  : fit::kSingleDirect;
+      : bytes > 256.0 * (1 << 20)        ? fit::kSingleDirectLarge
+      : c.time < fit::kSingleDirectShort ? fit::kSinglePacked
+                                         : fit::kSingleDirect;
   const double time =
       std::max(fit::kCallFloor[0],
                std::min(fused_time(terms, m, n, k, batch, true, rows),

@@ -261,14 +261,17 @@ inline double fused_direct_margin(const int m, const int n, const int k,
 // An uncut product that the path query gives to another path runs in the single
 // kernel where its own time is below this much of that path's estimate.  Of 500
 // random ('T','N') products of those paths (m, n = 32 .. 8192, k up to 65536, 1 ..
-// 1024 entries; each run both ways): packed operands, 186 below 0.95, 0.67 of
-// the time in the median, two above 1.03 (the leading product outside the matrix
-// core: 25 below 1.15, 0.55, none above 1.05); the direct kernel below 0.88, 39,
-// 0.83, three above 1.03 by up to 5 %, and below 0.6 where the batch exceeds the
-// 256 MiB of the memory-side cache, 0.82 (95x125x10978 x 172 at 0.64 is 1.3 times
-// slower: the single kernel's estimate overlaps stages and traffic too well there).
-constexpr double kSinglePacked = 0.95, kSinglePackedRn = 1.15,
-                 kSingleDirect = 0.88, kSingleDirectLarge = 0.6;
+// 1024 entries; each run both ways): packed operands with two or three terms, 214
+// below 0.95, 0.66 of the time in the median, none above 1.03 (one term below 0.75:
+// 425x1440x1450 x 3 at 0.8 is 1.2 times slower; the leading product outside the
+// matrix core: 25 below 1.15, 0.55, none above 1.05); the direct kernel below 0.75,
+// 0.83, two above 1.03 (all of 20 that take it less than 20 us are faster), and
+// below 0.6 where the batch exceeds the 256 MiB of the memory-side cache, 0.82
+// (95x125x10978 x 172 at 0.64 is 1.3 times slower: the single kernel's estimate
+// overlaps stages and traffic too well there).
+constexpr double kSinglePacked = 0.95, kSinglePackedOneTerm = 0.75,
+                 kSinglePackedRn = 1.15, kSingleDirect = 0.75,
+                 kSingleDirectShort = 20e-6, kSingleDirectLarge = 0.6;
 // Adding a K slice to the double-precision sums, for the workgroups of a compute
 // unit at a time: 110 products run with the cut and uncut, 0.17 us in the median
 // (one workgroup a unit), 0.10 (two), 3 % of a call.
