@@ -104,7 +104,11 @@ int wmmae_query(int what, long long *out);
  * (as the reference's bgemm_kernel splits at fragment load,
  * batch_gemm.cu:196-386): they use no workspace, allocate nothing and ignore
  * the workspace arguments.  Where one of the other paths would cut K, that
- * kernel makes the same slices itself, with the same bits.  Batches of medium-sized matrices and K-heavy
+ * kernel makes the same slices itself, with the same bits: one after the other
+ * without a workspace, or a workgroup each with their sums in the workspace.  It
+ * also stands in for the other paths where they leave K whole and it is ahead,
+ * with the same bits again (and what those paths turn down for its workspace is
+ * still turned down).  Batches of medium-sized matrices and K-heavy
  * products with k contiguous in both operands run the packed path's GEMM
  * kernel on the fp32 operands directly (it splits them on their way into LDS):
  * no packed copy; the workspace then only holds K slices.  All paths give the
@@ -114,8 +118,9 @@ int wmmae_query(int what, long long *out);
  * wmmae_tcec_sgemm_workspace_bytes is an upper bound over the paths: packed
  * A + packed B + K slices, whichever path the call then takes.  A product the
  * library runs on the fp32 operands directly (wmmae_tcec_sgemm_path 3 or 4)
- * touches only the K slices, wmmae_tcec_gemm_packed_workspace_bytes of it, and
- * path 0 nothing; a caller that knows its products take those paths may pass
+ * touches only the K slices, wmmae_tcec_gemm_packed_workspace_bytes of it (where
+ * the single kernel makes them: their sums in whole tiles and eight bytes a tile,
+ * if what it is given holds that), and path 0 nothing; a caller that knows its products take those paths may pass
  * that much.  A workspace that is not 16-byte aligned is WMMAE_STATUS_MISALIGNED
  * on the packed path, which cannot do without it; the other two paths then run
  * without K slices. */
@@ -127,12 +132,13 @@ int wmmae_tcec_sgemm_workspace_bytes(int m, int n, int k, int batch, int policy,
  * batch_gemm.cu:408-431, 659): *path = 0 the single kernel that splits the
  * operands on the fly (no workspace), 1 packed operands in the workspace,
  * 2 packed operands and K slices (when the workspace has room for them; or the
- * same slices, without a workspace, inside the single kernel, where that is
- * estimated to take less time),
+ * same slices in the single kernel, where that is estimated to take less time),
  * 3 the packed path's GEMM kernel loading and splitting the fp32 operands
- * itself (no packed operands), 4 the same with K slices (or inside the single
+ * itself (no packed operands), 4 the same with K slices (or in the single
  * kernel, as 2).  3 and 4 assume
- * k contiguous in both operands ('T','N') and need k >= 4.
+ * k contiguous in both operands ('T','N') and need k >= 4.  For 1 and 3 the single
+ * kernel may run in the path's place too: the answer is the path whose bits,
+ * workspace and refusals a call has.
  * The answer is for op(A) = 'T', op(B) = 'N', whatever the leading dimensions
  * and bases.  Other layouts take 0, 1 or 2, and the single kernel more often: it
  * runs them at the same speed, the split pass of 1 and 2 does not.  Whichever

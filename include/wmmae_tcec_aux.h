@@ -69,8 +69,9 @@ int wmmae_tcec_sgemm_k_slices(int m, int n, int k, int batch, int policy,
  * leading dimensions and aligned bases: seconds[0] the single kernel,
  * seconds[1] split passes + GEMM on packed operands, seconds[2] the GEMM kernel
  * that splits the fp32 operands itself; infinity for a path the product cannot
- * take.  The smallest is the path wmmae_tcec_sgemm* takes for these layouts
- * (none below the time the host needs to issue its launches).  For checking the
+ * take.  The smallest is the path wmmae_tcec_sgemm_path answers for these layouts
+ * (none below the time the host needs to issue its launches); the single kernel
+ * may stand in for it (see there), by its time alone.  For checking the
  * estimates against measured times.  seconds[0] is more than a time in three
  * cases: products of at least 1024 x 1024 x 512, and fewer than 16 entries, take
  * the single kernel only where it is well ahead, and their seconds[0] holds that

@@ -4,7 +4,8 @@
 // live in include/wmmae_tcec.h.
 #include "gemm_plan.hpp"
 #include <cmath>
-#include <random>
+#include <chrono>
+#include <unistd.h>
 
 namespace {
 using namespace wmmae_driver;
@@ -323,10 +324,12 @@ inline int choose_spread(const Choice &c, const int m, const int n, const int k,
 // Tells a launch's arrival counts in a workspace from whatever else it may hold:
 // 58 bits that no other launch of any process is likely to have used.
 unsigned long long launch_number() {
-  static const unsigned long long seed = [] {
-    std::random_device r;
-    return (static_cast<unsigned long long>(r()) << 32) ^ r();
-  }();
+  // (std::random_device may throw, which must not reach a C caller)
+  static const unsigned long long seed =
+      static_cast<unsigned long long>(
+          std::chrono::system_clock::now().time_since_epoch().count()) ^
+      (static_cast<unsigned long long>(getpid()) << 40) ^
+      reinterpret_cast<uintptr_t>(&seed);
   static std::atomic<unsigned long long> count{0};
   unsigned long long z =
       seed + 0x9E3779B97F4A7C15ull * count.fetch_add(1, std::memory_order_relaxed);

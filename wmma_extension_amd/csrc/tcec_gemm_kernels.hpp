@@ -484,23 +484,24 @@ __global__ void __launch_bounds__(256)
 #pragma unroll
   for (int x = 0; x < VEC; x++)
     s[x] = 0.;
-  // (eight slices are read before any is added, past the last one the last again,
-  // which is not added; one read after the other, whole calls on packed operands
-  // took 27.9 us for 256x256x8192 in 32 slices, now 23.6, 200x160x10735 36.2, now
-  // 31.8)
+  // (slices are read eight, four or up to three at a time before any is added; one
+  // read after the other, whole calls on packed operands took 27.9 us for
+  // 256x256x8192 in 32 slices, now 21.9, 200x160x10735 36.4, now 30.6)
   typedef typename std::conditional<VEC == 4, f32x4, float>::type piece;
-  constexpr int AHEAD = 8;
-  for (int z0 = 0; z0 < splits; z0 += AHEAD) {
-    piece v[AHEAD];
+  int z = 0;
+  const auto add = [&](auto COUNT, const int valid) {
+    constexpr int count = decltype(COUNT)::value;
+    piece v[count];
 #pragma unroll
-    for (int a = 0; a < AHEAD; a++) {
-      const int z = z0 + a < splits ? z0 + a : splits - 1;
+    for (int a = 0; a < count; a++) {
+      // (past the last slice the last one again, not added)
+      const int za = a < valid ? z + a : splits - 1;
       v[a] = *reinterpret_cast<const piece *>(partial +
-                                              (z * batches + entry) * mn + e);
+                                              (za * batches + entry) * mn + e);
     }
 #pragma unroll
-    for (int a = 0; a < AHEAD; a++)
-      if (z0 + a < splits) {
+    for (int a = 0; a < count; a++)
+      if (a < valid) {
         if constexpr (VEC == 4) {
 #pragma unroll
           for (int x = 0; x < 4; x++)
@@ -509,7 +510,14 @@ __global__ void __launch_bounds__(256)
           s[0] += static_cast<double>(v[a]);
         }
       }
-  }
+    z += valid;
+  };
+  while (z + 8 <= splits)
+    add(ic<8>{}, 8);
+  if (z + 4 <= splits)
+    add(ic<4>{}, 4);
+  if (z < splits)
+    add(ic<3>{}, splits - z);
   float *const cb =
       c_ptrs != nullptr ? c_ptrs[entry] : C + entry * batch_stride_c;
   float *const p = cb + (e % M) + (e / M) * ldc;
