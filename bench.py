@@ -515,7 +515,7 @@ def bench_api_gemm(torch, tcec, dev, n=4096, steps=100, warmup=10, also_rz=True)
         ms = e0.elapsed_time(e1) / steps
         return ms, 2.0 * n ** 3 / (ms * 1e-3) / 1e12
     ms, tf = timed(0)
-    out = {"kernel": "tcec_api_gemm_kernel (tcec::load_matrix_sync / mma_sync / utils::cp_async only)",
+    out = {"kernel": "tcec_api_gemm_split_kernel (tcec::fragment / mma_sync / store_matrix_sync, every element split once per workgroup)",
            "workload": f"M=N=K={n}, fp16 hi+lo with EC, uniform[-1,1]", "steps": steps,
            "ms_per_step": round(ms, 4), "value": round(tf, 2), "unit": "TFLOPS",
            "mfma_frac": round(3 * tf / PEAK_MFMA_TFLOPS, 4)}
@@ -747,7 +747,7 @@ def main():
             "config": {"workload": f"api: {w['desc']}"},
             "roofline": {"bound": "mfma", "achieved": round(3 * r["value"], 2), "peak": PEAK_MFMA_TFLOPS,
                          "unit": "TFLOP/s", "frac": r["mfma_frac"], "traffic": traffic,
-                         "traffic_source": traffic_source, "kernel": "tcec_api_gemm_kernel", "kernel_ms": r["ms_per_step"],
+                         "traffic_source": traffic_source, "kernel": "tcec_api_gemm_split_kernel", "kernel_ms": r["ms_per_step"],
                          "issued_flop_multiplier": 3},
             "cpu_baseline": None}))
         return
