@@ -1,0 +1,122 @@
+"""Which kernel a GEMM call runs and how it cuts K (wmmae_tcec_sgemm_route, host only): the kernel that
+stands in for another path makes that path's cut, whatever workspace the call is given."""
+import ctypes
+import os
+import random
+import re
+
+import pytest
+
+from wmma_extension_amd import _lib
+
+ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+ALIGNED = 1 << 20                     # an address that is never read
+SINGLE, PACKED, DIRECT = 0, 1, 3
+STATIC_BYTES = 64 << 20               # the fixed array of wmmae_tcec_sgemm_static
+
+
+@pytest.fixture(scope="module")
+def h():
+    if not os.path.exists(_lib.LIB_PATH):
+        _lib.build()
+    return _lib.lib()
+
+
+def _route(h, ta, tb, m, n, k, batch, policy, room, flags=0, address=ALIGNED, lda=None, ldb=None):
+    out = (ctypes.c_int * 3)()
+    st = h.wmmae_tcec_sgemm_route(ta, tb, m, n, k, lda or (k if ta == b"T" else m), ldb or (k if tb == b"N" else n),
+                                  batch, policy, flags, None if room is None else address, room or 0, out)
+    assert st == 0
+    return tuple(out)
+
+
+def _bytes(h, m, n, k, batch, policy):
+    """(packed operands, the slices' sums behind them)"""
+    a, b, c = (ctypes.c_size_t(0) for _ in range(3))
+    assert h.wmmae_tcec_pack_bytes(m, k, batch, policy, ctypes.byref(a)) == 0
+    assert h.wmmae_tcec_pack_bytes(n, k, batch, policy, ctypes.byref(b)) == 0
+    assert h.wmmae_tcec_gemm_packed_workspace_bytes(policy, m, n, k, batch, ctypes.byref(c)) == 0
+    return a.value + b.value, c.value
+
+
+def test_header_and_library_agree(h):
+    text = open(os.path.join(ROOT, "include", "wmmae_tcec_route.h")).read()
+    names = set(re.findall(r"\b(wmmae_[a-z0-9_]+)\s*\(", text))
+    assert names and names <= set(_lib._SIGNATURES) and all(getattr(h, x) is not None for x in names)
+
+
+def test_bad_arguments(h):
+    out = (ctypes.c_int * 3)()
+    ok = [b"T", b"N", 64, 64, 64, 64, 64, 1, 0, 0, None, 0, out]
+    assert h.wmmae_tcec_sgemm_route(*ok) == 0
+    for i, v in ((0, b"X"), (1, b"?"), (2, 0), (3, -1), (4, 0), (7, 0), (8, 9), (9, 2), (9, 64)):
+        assert h.wmmae_tcec_sgemm_route(*(ok[:i] + [v] + ok[i + 1:])) == -1, i
+    assert h.wmmae_tcec_sgemm_route(*ok[:-1], None) == -2
+
+
+# products whose path leaves K whole on a workspace that holds the packed operands alone (the last:
+# 58 MiB of operands and 26 MiB of sums in the 64 MiB of the fixed array)
+UNCUT = [(b"T", b"N", 63, 130, 6403, 2, 0), (b"N", b"N", 256, 256, 8192, 0, 0), (b"N", b"T", 200, 160, 10735, 2, 1),
+         (b"N", b"N", 700, 500, 12500, 0, 0)]
+
+
+@pytest.mark.parametrize("ta,tb,m,n,k,policy,flags", UNCUT)
+def test_no_room_for_the_sums_behind_packed_operands(h, ta, tb, m, n, k, policy, flags):
+    operands, sums = _bytes(h, m, n, k, 1, policy)
+    assert sums > 0 and _route(h, ta, tb, m, n, k, 1, policy, operands + sums, flags)[1] > 1
+    assert _route(h, ta, tb, m, n, k, 1, policy, operands, flags) == (PACKED, 1, 0)
+    assert _route(h, ta, tb, m, n, k, 1, policy, operands + sums - 1, flags) == (PACKED, 1, 0)
+    if operands <= STATIC_BYTES < operands + sums:
+        assert _route(h, ta, tb, m, n, k, 1, policy, STATIC_BYTES, flags) == (PACKED, 1, 0)
+
+
+def test_cut_of_random_products(h):
+    rng = random.Random(7)
+    cut = stood_in = 0
+    for _ in range(4000):
+        m, n, k = (int(2 ** rng.uniform(0, e)) for e in (12, 12, 16))
+        batch, policy = rng.choice([1, 1, 1, 2, 5, 40]), rng.randrange(5)
+        ta, tb = rng.choice([(b"T", b"N"), (b"N", b"N"), (b"N", b"T"), (b"T", b"T")])
+        flags = int(policy in (0, 2) and rng.random() < 0.2)
+        operands, sums = _bytes(h, m, n, k, batch, policy)
+        full = _route(h, ta, tb, m, n, k, batch, policy, operands + sums, flags)
+        if full[1] == 1:
+            assert full[2] == 0
+            continue
+        cut += 1
+        stood_in += full[2] > 0
+        # (what needs no packed operands is not turned down on sixteen bytes)
+        needs_operands = _route(h, ta, tb, m, n, k, batch, policy, 16, flags)[0] == PACKED
+        for room in (operands, operands + sums - 1):
+            got = _route(h, ta, tb, m, n, k, batch, policy, room, flags)
+            if needs_operands:
+                assert got == (PACKED, 1, 0), (ta, tb, m, n, k, batch, policy, flags, room)
+            elif got[0] == SINGLE:
+                assert got[1] == full[1]
+            else:                     # the direct kernel: its sums alone
+                assert got[0] == DIRECT and got[1] == (full[1] if room >= 4 * full[1] * batch * m * n else 1)
+        assert _route(h, ta, tb, m, n, k, batch, policy, operands + sums, flags, ALIGNED + 4)[2] == 0
+    assert cut > 300 and stood_in > 200
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("ta,tb,m,n,k,policy,flags", UNCUT)
+def test_bits_without_room_for_the_sums(tc, dev, ta, tb, m, n, k, policy, flags):
+    import torch
+    ta, tb = ta.decode(), tb.decode()
+    lda, ldb = (k if ta == "T" else m), (k if tb == "N" else n)
+    g = torch.Generator(device="cpu").manual_seed(m + n + k)
+    A, B = ((torch.rand((x, k), generator=g) * 2 - 1).to(dev).view(-1) for x in (m, n))
+    need = tc.pack_bytes(m, k, 1, policy) + tc.pack_bytes(n, k, 1, policy)
+    ws = torch.empty(need, dtype=torch.uint8, device=dev)
+
+    def call(flag):
+        C = torch.zeros((n, m), device=dev)
+        tc.sgemm(ta, tb, m, n, k, 1.0, A, lda, B, ldb, 0.0, C, m, policy, flag | flags, ws)
+        return C
+    want, got = call(tc.FLAG_PATH_PACKED), call(0)
+    assert torch.isfinite(want).all() and torch.equal(want, got)
+    if need <= STATIC_BYTES < tc.workspace_bytes(m, n, k, 1, policy):
+        C = torch.zeros((n, m), device=dev)
+        tc.sgemm_static(ta, tb, m, n, k, 1.0, A, lda, B, ldb, 0.0, C, m, policy, flags)
+        assert torch.equal(C, want)

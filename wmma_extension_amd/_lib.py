@@ -197,6 +197,8 @@ _SIGNATURES = {
     "wmmae_tcec_time_gemm_kernel": (_i, [_vp, _vp]),
     "wmmae_tcec_path_estimates": (_i, [_i, _i, _i, _i, _i, _c.POINTER(_c.c_double)]),
     "wmmae_mfma_source_hazard_probe": (_i, [_i, _i, _vp, _vp]),
+    # include/wmmae_tcec_route.h
+    "wmmae_tcec_sgemm_route": (_i, [_c.c_char, _c.c_char, _i, _i, _i, _i, _i, _i, _i, _i, _vp, _sz, _c.POINTER(_i)]),
 }
 
 

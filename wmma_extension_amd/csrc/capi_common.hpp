@@ -4,6 +4,7 @@
 #pragma once
 #include <wmmae_tcec.h>
 #include <wmmae_tcec_aux.h>
+#include <wmmae_tcec_route.h>
 
 #include <algorithm>
 #include <atomic>

@@ -218,6 +218,23 @@ inline Choice choose_path(const int m, const int n, const int k, const int batch
   return {single && e.slices == 1 ? Path::Fused : e.base, e.slices, single,
           single ? fused : e.base_time};
 }
+// what the direct kernel needs of a product (the operands' k strides are 1)
+inline bool direct_possible(const int k, const int terms, const int flags,
+                            const long long a_rs, const long long b_rs) {
+  return k >= 4 && terms <= 2 &&
+         (flags & WMMAE_FLAG_RN_MAIN) == 0 && a_rs < (1 << 24) &&
+         b_rs < (1 << 24);
+}
+
+// Whether a workspace holds packed operands and `more` bytes behind them.
+inline bool holds_packed(const int m, const int n, const int k, const int batch,
+                         const int terms, const size_t workspace_bytes,
+                         const size_t more) {
+  const size_t operands = static_cast<size_t>(packed_elems(m, k, terms) +
+                                              packed_elems(n, k, terms)) *
+                          16u * static_cast<size_t>(batch);
+  return workspace_bytes >= operands && workspace_bytes - operands >= more;
+}
 // A call that its path turns down for the workspace it is given stays with it.
 inline bool refused_on_packed(const Choice &c, const int m, const int n,
                               const int k, const int batch, const int terms,
@@ -225,10 +242,7 @@ inline bool refused_on_packed(const Choice &c, const int m, const int n,
                               const size_t workspace_bytes) {
   return !c.single && c.path == Path::Packed && workspace != nullptr &&
          (reinterpret_cast<uintptr_t>(workspace) % 16 != 0 ||
-          workspace_bytes <
-              static_cast<size_t>(packed_elems(m, k, terms) +
-                                  packed_elems(n, k, terms)) *
-                  16u * static_cast<size_t>(batch));
+          !holds_packed(m, n, k, batch, terms, workspace_bytes, 0));
 }
 // Bytes for the K slices of the tiles of a partly empty last round: the largest
 // need over the tile shapes and residencies the launch may choose; 0: no such
@@ -282,20 +296,38 @@ inline bool single_is_ahead(const Choice &c, const int m, const int n,
   // (the other kernels cut the tiles of a partly empty last round along K)
   return time < ahead * c.time && tail_room(policy, m, n, k, batch) == 0;
 }
+// Bytes for the K slices' sums of either GEMM kernel on packed operands or fp32
+// ones (the one that splits the fp32 operands itself plans its slices for its own
+// tile); 0: neither cuts K.
+size_t slices_room(const int terms, const int m, const int n, const int k,
+                   const int batch) {
+  if (m == 0 || n == 0 || k == 0 || batch == 0)
+    return 0;
+  const int splits = std::max(choose_splits(terms, m, n, k, batch),
+                              direct_possible(k, terms, 0, 1, 1)
+                                  ? choose_splits(terms, m, n, k, batch, true)
+                                  : 1);
+  return splits > 1 ? static_cast<size_t>(splits) * batch * m * n * 4u : 0;
+}
 // Tile of the single kernel (64 or 128) that makes a cut product's slices with a
 // workgroup each, 0: the slices are made as chosen.  The products that run on
 // packed operands or in the direct kernel, or whose slices one workgroup of the
 // single kernel would make one after the other: too few output tiles to fill the
 // chip, and a split pass, a GEMM of at most a round and a fold launch for what is
-// one launch here.  The same cut of K, so the same bits.  Needs the caller's
-// workspace to have the room; without one it allocates only where the path it
-// stands in for would.
+// one launch here.  The same cut of K, so the same bits: where packed operands
+// leave the workspace no room for the slices' sums, that path leaves K whole and
+// so does the call.  Needs the caller's workspace to have the room; without one it
+// allocates only where the path it stands in for would.
 inline int choose_spread(const Choice &c, const int m, const int n, const int k,
                          const int batch, const int terms,
                          const void *const workspace,
                          const size_t workspace_bytes) {
   if (c.slices <= 1 || c.time <= 0. ||
       refused_on_packed(c, m, n, k, batch, terms, workspace, workspace_bytes))
+    return 0;
+  if (!c.single && c.path == Path::Packed && workspace != nullptr &&
+      !holds_packed(m, n, k, batch, terms, workspace_bytes,
+                    slices_room(terms, m, n, k, batch)))
     return 0;
   double best = c.time;
   if (c.single)
@@ -341,12 +373,29 @@ unsigned long long launch_number() {
 // ('T','N') products with k % 4 != 0 and more than three stages stay with the
 // other paths, as the path query has always answered.
 inline bool fused_considered(const int k) { return k % 4 == 0 || k <= 96; }
-// what the direct kernel needs of a product (the operands' k strides are 1)
-inline bool direct_possible(const int k, const int terms, const int flags,
-                            const long long a_rs, const long long b_rs) {
-  return k >= 4 && terms <= 2 &&
-         (flags & WMMAE_FLAG_RN_MAIN) == 0 && a_rs < (1 << 24) &&
-         b_rs < (1 << 24);
+// Which kernel runs a call without a path flag, and how K is cut.
+struct Route {
+  Path path;
+  int slices;      // as chosen; what packed operands or the direct kernel make of
+                   // them depends on the workspace too (plan_k_slices)
+  int spread_tile; // > 0: made by a workgroup each, with tiles of this size
+};
+inline Route choose_route(const int m, const int n, const int k, const int batch,
+                          const int rn, const int policy, const int terms,
+                          const bool rows, const bool direct_ok,
+                          const void *const workspace,
+                          const size_t workspace_bytes) {
+  const Choice c = choose_path(m, n, k, batch, rn, terms, policy,
+                               rows || fused_considered(k), rows, direct_ok);
+  Route r{c.single ? Path::Fused : c.path, c.slices, 0};
+  if (single_is_ahead(c, m, n, k, batch, rn, policy, terms, rows, workspace,
+                      workspace_bytes))
+    r.path = Path::Fused;
+  r.spread_tile =
+      choose_spread(c, m, n, k, batch, terms, workspace, workspace_bytes);
+  if (r.spread_tile > 0)
+    r.path = Path::Fused;
+  return r;
 }
 
 // how the single kernel reads an operand (see its head comment)
@@ -607,17 +656,11 @@ int sgemm_impl(const char transa, const char transb, const int m, const int n,
       return WMMAE_STATUS_NOT_SUPPORTED;
     path = Path::Fused;
   } else if ((flags & WMMAE_FLAG_PATH_PACKED) == 0) {
-    const Choice c = choose_path(m, n, k, batch, rn, p.terms, policy,
-                                 rows || fused_considered(k), rows, direct_ok);
-    path = c.single ? Path::Fused : c.path;
-    slices = c.slices;
-    if (single_is_ahead(c, m, n, k, batch, rn, policy, p.terms, rows, workspace,
-                        workspace_bytes))
-      path = Path::Fused;
-    spread_tile = choose_spread(c, m, n, k, batch, p.terms, workspace,
-                                workspace_bytes);
-    if (spread_tile > 0)
-      path = Path::Fused;
+    const Route r = choose_route(m, n, k, batch, rn, policy, p.terms, rows,
+                                 direct_ok, workspace, workspace_bytes);
+    path = r.path;
+    slices = r.slices;
+    spread_tile = r.spread_tile;
   }
   if (path == Path::Direct) {
     // the planes of the K slices are the only workspace this path uses
@@ -808,20 +851,9 @@ int wmmae_tcec_gemm_packed_workspace_bytes(const int policy, const int m,
     return WMMAE_STATUS_NULL_POINTER;
   if (!policy_info(policy, p) || m < 0 || n < 0 || k < 0 || batch < 0)
     return WMMAE_STATUS_INVALID_VALUE;
-  // (room for the slices of either kernel: the one that splits the fp32
-  // operands itself plans them for its own tile)
-  const int splits =
-      (m == 0 || n == 0 || k == 0 || batch == 0)
-          ? 1
-          : std::max(choose_splits(p.terms, m, n, k, batch),
-                     direct_possible(k, p.terms, 0, 1, 1)
-                         ? choose_splits(p.terms, m, n, k, batch, true)
-                         : 1);
-  if (splits > 1) {
-    *bytes = static_cast<size_t>(splits) * batch * m * n * 4u;
-  } else {
+  *bytes = slices_room(p.terms, m, n, k, batch);
+  if (*bytes == 0)
     *bytes = tail_room(policy, m, n, k, batch);
-  }
   return WMMAE_STATUS_SUCCESS;
 }
 
@@ -840,6 +872,42 @@ int wmmae_tcec_sgemm_path(const int m, const int n, const int k,
   *path = c.path == Path::Fused    ? 0
           : c.path == Path::Direct ? (c.slices > 1 ? 4 : 3)
                                    : (c.slices > 1 ? 2 : 1);
+  return WMMAE_STATUS_SUCCESS;
+}
+
+int wmmae_tcec_sgemm_route(const char transa, const char transb, const int m,
+                           const int n, const int k, const int lda,
+                           const int ldb, const int batch, const int policy,
+                           const int flags, const void *const workspace,
+                           const size_t workspace_bytes, int *const route) {
+  PolicyInfo p;
+  if (route == nullptr)
+    return WMMAE_STATUS_NULL_POINTER;
+  if ((!is_n(transa) && !is_t(transa)) || (!is_n(transb) && !is_t(transb)) ||
+      m <= 0 || n <= 0 || k <= 0 || batch <= 0 || !policy_info(policy, p) ||
+      (flags & ~WMMAE_FLAG_RN_MAIN) != 0)
+    return WMMAE_STATUS_INVALID_VALUE;
+  const OneDeviceCall one_device;
+  const bool rows = is_n(transa) || !is_n(transb);
+  const Route r = choose_route(
+      m, n, k, batch, flags, policy, p.terms, rows,
+      !rows && direct_possible(k, p.terms, flags, lda, ldb), workspace,
+      workspace_bytes);
+  // (the slices those two make where the workspace holds their sums)
+  bool cut = true;
+  if (workspace != nullptr && r.path != Path::Fused) {
+    const size_t sums =
+        r.path == Path::Packed
+            ? slices_room(p.terms, m, n, k, batch)
+            : static_cast<size_t>(r.slices) * batch * m * n * 4u;
+    cut = reinterpret_cast<uintptr_t>(workspace) % 16 == 0 &&
+          (r.path == Path::Packed
+               ? holds_packed(m, n, k, batch, p.terms, workspace_bytes, sums)
+               : workspace_bytes >= sums);
+  }
+  route[0] = r.path == Path::Fused ? 0 : r.path == Path::Packed ? 1 : 3;
+  route[1] = cut ? r.slices : 1;
+  route[2] = r.spread_tile;
   return WMMAE_STATUS_SUCCESS;
 }
 
