@@ -711,7 +711,7 @@ int sgemm_impl(const char transa, const char transb, const int m, const int n,
     if (batch > (1 << 26)) // tile indices are 32-bit
       return WMMAE_STATUS_NOT_SUPPORTED;
     FusedArgs f;
-    wmmae_gemm::FusedParams &q = f.p;
+    wmmae_gemm::FusedSpreadParams &q = f.p;
     q.A = A;
     q.a_ptrs = a_ptrs;
     q.a_rs = a_rs;

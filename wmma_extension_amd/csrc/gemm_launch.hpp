@@ -270,6 +270,15 @@ template <class MT, int TERMS> int per_cu_by_shape(const int shape) {
     return workgroups_per_cu<MT, TERMS, 64, 64, 2, 2, false>();
   }
 }
+// the arguments that a kernel takes
+template <int CUT>
+wmmae_gemm::fused_params<CUT>
+launch_params(const wmmae_gemm::FusedSpreadParams &p) {
+  if constexpr (CUT == wmmae_gemm::kFusedSpread)
+    return p;
+  else
+    return {p, p.alpha, p.beta, p.inv_scale};
+}
 template <class T, int TERMS, int BM, int BN, int CW, int PW, int DEPTH, bool RN,
           bool STREAM, int CUT>
 int launch_fused_grid(const FusedArgs &f, const long long grid) {
@@ -282,7 +291,8 @@ int launch_fused_grid(const FusedArgs &f, const long long grid) {
   if (t_gemm_begin != nullptr)
     WMMAE_HIP_TRY(hipEventRecord(t_gemm_begin, f.stream));
   hipLaunchKernelGGL(kernel, dim3(static_cast<unsigned>(grid)),
-                     dim3(Cfg::NTHREADS), Cfg::LDS_BYTES, f.stream, f.p);
+                     dim3(Cfg::NTHREADS), Cfg::LDS_BYTES, f.stream,
+                     launch_params<CUT>(f.p));
   const int st = launch_status();
   if (st == WMMAE_STATUS_SUCCESS && t_gemm_end != nullptr)
     WMMAE_HIP_TRY(hipEventRecord(t_gemm_end, f.stream));
@@ -292,7 +302,7 @@ int launch_fused_grid(const FusedArgs &f, const long long grid) {
 template <class T, int TERMS, int BM, int BN, int CW, int PW, int DEPTH, bool RN,
           int CUT>
 int launch_fused(FusedArgs f) {
-  wmmae_gemm::FusedParams &p = f.p;
+  wmmae_gemm::FusedSpreadParams &p = f.p;
   p.tiles_m = static_cast<int>(ceil_div(p.M, BM));
   p.tiles_n = static_cast<int>(ceil_div(p.N, BN));
   const long long tpb = static_cast<long long>(p.tiles_m) * p.tiles_n;

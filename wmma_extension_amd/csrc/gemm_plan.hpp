@@ -467,7 +467,7 @@ constexpr int ring_depth(const int bm, const int bn, const int terms) {
 
 // ------------------------------------------------------ fused small GEMM
 struct FusedArgs {
-  wmmae_gemm::FusedParams p = {};
+  wmmae_gemm::FusedSpreadParams p = {};
   // > 0: K slices made by a workgroup each, with tiles of this size
   int spread_tile = 0;
   hipStream_t stream;

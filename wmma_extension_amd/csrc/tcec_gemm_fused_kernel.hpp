@@ -69,7 +69,7 @@ enum FusedSource { kFusedKRows = 0, kFusedRRows = 1, kFusedAny = 2 };
 // into slices that a workgroup each makes
 enum FusedCut { kFusedWhole = 0, kFusedSliced = 1, kFusedSpread = 2 };
 
-struct FusedParams {
+struct FusedOperands {
   const float *A;
   const float *const *a_ptrs;
   long long a_rs, a_ks, a_bs;
@@ -86,14 +86,30 @@ struct FusedParams {
   int grouped;
   int a_source, b_source; // FusedSource
   int slice_stages; // CUT: k stages of a slice
-  // kFusedSpread: K slices; room for the slices' sums, slice z of tile t (entry
-  // by entry) at planes + (t*slices + z)*BM*BN, and a word per tile
-  // (last_of_tile), with what tells this launch's counts from other contents
+};
+// What every workgroup reads of its launch, the number of workgroups behind it
+// included, lies in three lines of 64 bytes: with the fields of the slices among
+// them and a fourth line 1024^3 took 15.10 us for 14.92, calls of 9 us 0.1 more.
+struct FusedParams : FusedOperands {
+  float alpha, beta, inv_scale;
+  // (FusedSpreadParams' names, for code that is never reached with these)
+  static constexpr int slices = 1;
+  static constexpr float *planes = nullptr;
+  static constexpr unsigned long long *arrivals = nullptr, launch = 0;
+};
+static_assert(sizeof(FusedParams) + 4 <= 192, "three lines");
+// kFusedSpread: K slices; room for the slices' sums, slice z of tile t (entry by
+// entry) at planes + (t*slices + z)*BM*BN, and a word per tile (last_of_tile), with
+// what tells this launch's counts from other contents
+struct FusedSpreadParams : FusedOperands {
   int slices;
   float *planes;
   unsigned long long *arrivals, launch;
   float alpha, beta, inv_scale;
 };
+template <int CUT>
+using fused_params =
+    std::conditional_t<CUT == kFusedSpread, FusedSpreadParams, FusedParams>;
 
 // CW consumer waves (2 x CW/2 over the tile), PW producer waves
 template <int TERMS, int BM, int BN, int CW, int PW> struct FusedConfig {
@@ -170,7 +186,7 @@ template <class T, int TERMS, int BM, int BN, int CW, int PW, int DEPTH,
 __global__ void __launch_bounds__(64 * (CW + PW), CUT == kFusedWhole ? 1
                                                   : BM > 64          ? 3
                                                                      : 4)
-    tcec_gemm_fused_kernel(const FusedParams p) {
+    tcec_gemm_fused_kernel(const fused_params<CUT> p) {
   using traits = mtk::wmma::tcec::detail::split_traits<T>;
   using S = typename traits::storage;
   typedef S ab_vec __attribute__((ext_vector_type(8)));
