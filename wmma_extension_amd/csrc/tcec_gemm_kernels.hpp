@@ -464,7 +464,28 @@ __global__ void __launch_bounds__(256)
 // the launch geometry.  A thread owns VEC consecutive elements of a slice
 // (VEC == 4: M, ldc and the entries' bases are multiples of four floats, so
 // the four are rows of one column and every access is one 16-byte piece).
+// Slices are read in groups before any of a group is added.  One read after the
+// other, whole calls on packed operands took 27.9 us for 256x256x8192 in 32
+// slices, now 21.9, 200x160x10735 36.4, now 30.6.
 // --------------------------------------------------------------------------
+// Slices of the next group when `left` are to be added.  None is read twice (with a
+// group of three for the last one or two as well 4096x512x4096 took 71.3 us in two
+// slices for 70.5, 1024x1024x4096 in ten 50.4 for 49.8).
+__host__ __device__ constexpr int fold_group(const int left) {
+  return left >= 8 ? 8 : left >= 4 ? 4 : left;
+}
+constexpr bool fold_groups_cover(const int most) {
+  for (int splits = 1; splits <= most; splits++) {
+    int left = splits;
+    while (left > 0)
+      left -= fold_group(left) > 0 ? fold_group(left) : left + 1;
+    if (left != 0)
+      return false;
+  }
+  return true;
+}
+static_assert(fold_groups_cover(64), "every slice once");
+
 template <int VEC>
 __global__ void __launch_bounds__(256)
     reduce_splits_kernel(const float *__restrict__ partial, const int splits,
@@ -484,40 +505,47 @@ __global__ void __launch_bounds__(256)
 #pragma unroll
   for (int x = 0; x < VEC; x++)
     s[x] = 0.;
-  // (slices are read eight, four or up to three at a time before any is added; one
-  // read after the other, whole calls on packed operands took 27.9 us for
-  // 256x256x8192 in 32 slices, now 21.9, 200x160x10735 36.4, now 30.6)
   typedef typename std::conditional<VEC == 4, f32x4, float>::type piece;
-  int z = 0;
-  const auto add = [&](auto COUNT, const int valid) {
+  const float *from = partial + entry * mn + e;
+  const auto add = [&](auto COUNT) {
     constexpr int count = decltype(COUNT)::value;
     piece v[count];
 #pragma unroll
     for (int a = 0; a < count; a++) {
-      // (past the last slice the last one again, not added)
-      const int za = a < valid ? z + a : splits - 1;
-      v[a] = *reinterpret_cast<const piece *>(partial +
-                                              (za * batches + entry) * mn + e);
+      v[a] = *reinterpret_cast<const piece *>(from);
+      from += batches * mn;
     }
 #pragma unroll
-    for (int a = 0; a < count; a++)
-      if (a < valid) {
-        if constexpr (VEC == 4) {
+    for (int a = 0; a < count; a++) {
+      if constexpr (VEC == 4) {
 #pragma unroll
-          for (int x = 0; x < 4; x++)
-            s[x] += static_cast<double>(v[a][x]);
-        } else {
-          s[0] += static_cast<double>(v[a]);
-        }
+        for (int x = 0; x < 4; x++)
+          s[x] += static_cast<double>(v[a][x]);
+      } else {
+        s[0] += static_cast<double>(v[a]);
       }
-    z += valid;
+    }
   };
-  while (z + 8 <= splits)
-    add(ic<8>{}, 8);
-  if (z + 4 <= splits)
-    add(ic<4>{}, 4);
-  if (z < splits)
-    add(ic<3>{}, splits - z);
+  for (int left = splits; left > 0;) {
+    const int group = fold_group(left);
+    left -= group;
+    switch (group) {
+    case 8:
+      add(ic<8>{});
+      break;
+    case 4:
+      add(ic<4>{});
+      break;
+    case 3:
+      add(ic<3>{});
+      break;
+    case 2:
+      add(ic<2>{});
+      break;
+    default:
+      add(ic<1>{});
+    }
+  }
   float *const cb =
       c_ptrs != nullptr ? c_ptrs[entry] : C + entry * batch_stride_c;
   float *const p = cb + (e % M) + (e / M) * ldc;
