@@ -24,6 +24,12 @@ int wmmae_tcec_sgemm_route(char transa, char transb, int m, int n, int k,
                            const void *workspace, size_t workspace_bytes,
                            int *route);
 
+/* Test hook (no counterpart in the reference): where the calling thread's next
+ * wmmae_tcec_sgemm* calls cut K and the workspace has the room, the single kernel
+ * makes the slices a workgroup each, with tiles of this size (64 or 128); -1: it
+ * never does; 0: the estimates choose. */
+int wmmae_tcec_force_spread_tile(int tile);
+
 #ifdef __cplusplus
 }
 #endif

@@ -15,7 +15,8 @@ def _room(m, n, batch, slices):
     return max(-(-m // t) * -(-n // t) * batch * (slices * t * t * 4 + 8) for t in (64, 128))
 
 
-def _check(tc, dev, ta, tb, m, n, k, batch, policy, rn=0, pad=0, alpha=1.0, beta=0.0):
+def _check(tc, dev, ta, tb, m, n, k, batch, policy, rn=0, pad=0, alpha=1.0, beta=0.0, tile=0, pointers=False):
+    """tile: the one that has to run, 0 whichever is chosen, if any."""
     slices = tc.sgemm_k_slices(m, n, k, batch, policy, PACKED)
     assert slices > 1, (m, n, k)
     g = torch.Generator(device="cpu").manual_seed(m + 1000 * n + 7 * k + policy)
@@ -26,6 +27,13 @@ def _check(tc, dev, ta, tb, m, n, k, batch, policy, rn=0, pad=0, alpha=1.0, beta
 
     def call(flag, ws):
         C = C0.clone()
+        if flag == 0 and tile:
+            assert tc.sgemm_route(ta, tb, m, n, k, lda, ldb, batch, policy, rn, ws) == (0, slices, tile)
+        if pointers:
+            arrays = [torch.tensor([e.data_ptr() for e in X], dtype=torch.int64, device=dev) for X in (A, B, C)]
+            tc.sgemm_batched(ta, tb, m, n, k, alpha, arrays[0], lda, arrays[1], ldb, beta, arrays[2], ldc, batch,
+                             policy, flag | rn, ws)
+            return C
         tc.sgemm_strided_batched(ta, tb, m, n, k, alpha, A, lda, A.stride(0), B, ldb, B.stride(0), beta, C, ldc,
                                  n * ldc, batch, policy, flag | rn, ws)
         return C
@@ -40,6 +48,9 @@ def _check(tc, dev, ta, tb, m, n, k, batch, policy, rn=0, pad=0, alpha=1.0, beta
         assert torch.equal(want.view(torch.int32), got.view(torch.int32)), (ta, tb, m, n, k, batch, policy, rn)
         room[:size // 2].random_(0, 256)
     assert torch.equal(room[size:], guard)
+    if tile and tc.sgemm_route(ta, tb, m, n, k, lda, ldb, batch, policy, rn) == (0, slices, tile):
+        got = call(0, None)
+        assert torch.equal(want.view(torch.int32), got.view(torch.int32)), "workspace allocated by the call"
 
 
 @pytest.mark.parametrize("ta,tb", LAYOUTS)
@@ -60,10 +71,10 @@ def test_slices_of_a_workgroup_each(tc, dev, ta, tb, policy):
                                                  (3, 2150, 736, 1985, 2), (2, 1984, 800, 4100, 2)])
 def test_large_tiles(tc, dev, policy, m, n, k, slices):
     """Products that take 128x128 tiles."""
-    with tc.forced_k_slices(slices):
+    with tc.forced_k_slices(slices), tc.forced_spread_tile(128):
         for ta, tb in LAYOUTS[1:]:
-            _check(tc, dev, ta, tb, m, n, k, 1, policy, 0, 0, 1.0, 0.0)
-        _check(tc, dev, "N", "T", m, n, k, 1, policy, 0, 1, 0.5, 0.5)
+            _check(tc, dev, ta, tb, m, n, k, 1, policy, 0, 0, 1.0, 0.0, 128)
+        _check(tc, dev, "N", "T", m, n, k, 1, policy, 0, 1, 0.5, 0.5, 128)
 
 
 @pytest.mark.parametrize("policy", [0, 2])
@@ -72,6 +83,22 @@ def test_leading_product_outside_the_matrix_core(tc, dev, policy):
                                     ("N", "T", 1444, 448, 9000, 4)):
         with tc.forced_k_slices(slices):
             _check(tc, dev, ta, tb, m, n, k, 1, policy, tc.FLAG_RN_MAIN, 1, 1.25, -0.5)
+
+
+@pytest.mark.parametrize("tile", [64, 128])
+@pytest.mark.parametrize("ta,tb", LAYOUTS)
+@pytest.mark.parametrize("policy", [0, 1, 2, 3, 4])
+def test_each_tile(tc, dev, policy, ta, tb, tile):
+    """Every variant of the kernel, whatever the estimates would choose: tiles with a remainder of every
+    kind, several entries, k that ends inside a stage, matrices by pointer, and with fp32 adds outside
+    the matrix core where the policy has them."""
+    with tc.forced_spread_tile(tile):
+        for m, n, k, batch, slices in ((65, 60, 416, 3, 2), (1, 5, 700, 2, 3), (130, 259, 2048, 2, 10), (300, 129, 6403, 1, 32)):
+            with tc.forced_k_slices(slices):
+                _check(tc, dev, ta, tb, m, n, k, batch, policy, tile=tile)
+                _check(tc, dev, ta, tb, m, n, k, batch, policy, 0, 3, -0.75, 1.5, tile, pointers=True)
+                if policy in (0, 2):
+                    _check(tc, dev, ta, tb, m, n, k, batch, policy, tc.FLAG_RN_MAIN, 1, tile=tile)
 
 
 def test_replayed_graph(tc, dev):

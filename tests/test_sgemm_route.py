@@ -70,6 +70,23 @@ def test_no_room_for_the_sums_behind_packed_operands(h, ta, tb, m, n, k, policy,
         assert _route(h, ta, tb, m, n, k, 1, policy, STATIC_BYTES, flags) == (PACKED, 1, 0)
 
 
+def test_forced_tile(h):
+    """The hook chooses among what the rules allow: never more than the cut and the room there is."""
+    operands, sums = _bytes(h, 300, 129, 6403, 1, 0)
+    full = _route(h, b"N", b"N", 300, 129, 6403, 1, 0, operands + sums)
+    try:
+        for tile in (64, 128, -1):
+            assert h.wmmae_tcec_force_spread_tile(tile) == 0
+            got = _route(h, b"N", b"N", 300, 129, 6403, 1, 0, operands + sums)
+            assert got[1] == full[1] and got[2] == max(tile, 0) and (tile < 0 or got[0] == SINGLE)
+            assert _route(h, b"N", b"N", 300, 129, 6403, 1, 0, operands) == (PACKED, 1, 0)
+            assert _route(h, b"N", b"N", 64, 64, 64, 1, 0, operands) == (SINGLE, 1, 0)
+        assert h.wmmae_tcec_force_spread_tile(32) == -1
+    finally:
+        assert h.wmmae_tcec_force_spread_tile(0) == 0
+    assert _route(h, b"N", b"N", 300, 129, 6403, 1, 0, operands + sums) == full
+
+
 def test_cut_of_random_products(h):
     rng = random.Random(7)
     cut = stood_in = 0

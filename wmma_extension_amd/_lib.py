@@ -198,6 +198,7 @@ _SIGNATURES = {
     "wmmae_tcec_path_estimates": (_i, [_i, _i, _i, _i, _i, _c.POINTER(_c.c_double)]),
     "wmmae_mfma_source_hazard_probe": (_i, [_i, _i, _vp, _vp]),
     # include/wmmae_tcec_route.h
+    "wmmae_tcec_force_spread_tile": (_i, [_i]),
     "wmmae_tcec_sgemm_route": (_i, [_c.c_char, _c.c_char, _i, _i, _i, _i, _i, _i, _i, _i, _vp, _sz, _c.POINTER(_i)]),
 }
 

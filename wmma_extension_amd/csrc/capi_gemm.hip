@@ -309,6 +309,8 @@ size_t slices_room(const int terms, const int m, const int n, const int k,
                                   : 1);
   return splits > 1 ? static_cast<size_t>(splits) * batch * m * n * 4u : 0;
 }
+// Test hook (wmmae_tcec_force_spread_tile): 0 the estimates choose.
+thread_local int t_forced_spread_tile = 0;
 // Tile of the single kernel (64 or 128) that makes a cut product's slices with a
 // workgroup each, 0: the slices are made as chosen.  The products that run on
 // packed operands or in the direct kernel, or whose slices one workgroup of the
@@ -329,6 +331,17 @@ inline int choose_spread(const Choice &c, const int m, const int n, const int k,
       !holds_packed(m, n, k, batch, terms, workspace_bytes,
                     slices_room(terms, m, n, k, batch)))
     return 0;
+  const auto fits = [&](const int tile) {
+    return workspace == nullptr
+               ? !c.single
+               : reinterpret_cast<uintptr_t>(workspace) % 16 == 0 &&
+                     workspace_bytes >=
+                         fused_spread_bytes(m, n, batch, c.slices, tile);
+  };
+  if (t_forced_spread_tile != 0)
+    return t_forced_spread_tile > 0 && fits(t_forced_spread_tile)
+               ? t_forced_spread_tile
+               : 0;
   double best = c.time;
   if (c.single)
     best = c.time / fit::kSpreadSlicedMargin;
@@ -341,12 +354,7 @@ inline int choose_spread(const Choice &c, const int m, const int n, const int k,
   for (const int tile : {64, 128}) {
     const double t =
         fused_spread_time(terms, m, n, k, batch, tile == 64, c.slices);
-    if (t < best &&
-        (workspace == nullptr
-             ? !c.single
-             : reinterpret_cast<uintptr_t>(workspace) % 16 == 0 &&
-                   workspace_bytes >=
-                       fused_spread_bytes(m, n, batch, c.slices, tile))) {
+    if (t < best && fits(tile)) {
       chosen = tile;
       best = t;
     }
@@ -945,6 +953,13 @@ int wmmae_tcec_force_k_slices(const int slices) {
   if (slices < 0)
     return WMMAE_STATUS_INVALID_VALUE;
   t_forced_k_slices = slices;
+  return WMMAE_STATUS_SUCCESS;
+}
+
+int wmmae_tcec_force_spread_tile(const int tile) {
+  if (tile != -1 && tile != 0 && tile != 64 && tile != 128)
+    return WMMAE_STATUS_INVALID_VALUE;
+  t_forced_spread_tile = tile;
   return WMMAE_STATUS_SUCCESS;
 }
 

@@ -167,6 +167,16 @@ def sgemm_k_slices(m, n, k, batch=1, policy=Policy.F16_EC, flags=0):
     return out.value
 
 
+def sgemm_route(transa, transb, m, n, k, lda, ldb, batch=1, policy=Policy.F16_EC, flags=0, workspace=None):
+    """(kernel: 0 single, 1 packed operands, 3 direct; K slices; tile of slices made by a workgroup
+    each, else 0) of a GEMM call with this workspace (a tensor or None)."""
+    out = (ctypes.c_int * 3)()
+    _lib.check(_lib.lib().wmmae_tcec_sgemm_route(transa.encode(), transb.encode(), m, n, k, lda, ldb, batch,
+                                                 int(policy), flags, _ptr(workspace), _bytes(workspace), out),
+               "wmmae_tcec_sgemm_route")
+    return tuple(out)
+
+
 def path_estimates(m, n, k, batch=1, policy=Policy.F16_EC):
     """(fused, packed, direct) time estimates in seconds the driver chooses its path with
     (inf: the path cannot take the product)."""
@@ -211,6 +221,22 @@ class forced_k_slices:
 
     def __exit__(self, *exc):
         _lib.lib().wmmae_tcec_force_k_slices(0)
+        return False
+
+
+class forced_spread_tile:
+    """Test aid: within the block, this thread's GEMM calls make their K slices a workgroup each in the
+    single kernel with tiles of this size (64, 128), or never so (-1)."""
+
+    def __init__(self, tile):
+        self.tile = tile
+
+    def __enter__(self):
+        _lib.check(_lib.lib().wmmae_tcec_force_spread_tile(self.tile), "wmmae_tcec_force_spread_tile")
+        return self
+
+    def __exit__(self, *exc):
+        _lib.lib().wmmae_tcec_force_spread_tile(0)
         return False
 
 
