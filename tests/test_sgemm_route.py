@@ -87,6 +87,31 @@ def test_forced_tile(h):
     assert _route(h, b"N", b"N", 300, 129, 6403, 1, 0, operands + sums) == full
 
 
+@pytest.mark.parametrize("ta,tb,m,n,k,batch,policy,tile", [
+    # slower with a workgroup a slice than without (us, with and without), by the path they stand in for:
+    (b"T", b"N", 1248, 96, 1024, 4, 0, 0),        # the single kernel's slices one after the other: 20.6, 16.0
+    (b"T", b"N", 96, 5952, 1312, 1, 0, 0),        # 23.1, 18.2
+    (b"N", b"T", 68, 2738, 891, 1, 4, 0),         # 14.4, 11.5
+    (b"T", b"N", 256, 288, 6176, 1, 0, 0),        # packed operands: 30.2, 23.9
+    (b"T", b"T", 158, 92, 5248, 4, 1, 0),         # 25.7, 20.6
+    (b"T", b"N", 250, 381, 5798, 1, 0, 0),        # 29.3, 24.3
+    (b"T", b"N", 3616, 256, 1696, 3, 0, 0),       # the direct kernel: 56.7, 46.5
+    (b"T", b"N", 128, 5376, 7232, 1, 1, 0),       # one term: 41.0, 37.7
+    # faster so
+    (b"N", b"N", 2005, 64, 23136, 1, 0, 64),     # 42, 147
+    (b"T", b"N", 32, 480, 7332, 1, 0, 64),        # 18, 26
+    (b"T", b"N", 128, 96, 7463, 1, 0, 64),        # 17.3, 21.8
+    (b"T", b"N", 128, 658, 5052, 17, 4, 128),     # 91, 142
+    (b"T", b"N", 5632, 71, 36018, 1, 2, 128)])    # 322, 670
+def test_slices_of_a_workgroup_each_where_they_are_faster(h, ta, tb, m, n, k, batch, policy, tile):
+    """(256 compute units, which is also the answer without a device)"""
+    cu = ctypes.c_longlong(256)
+    h.wmmae_query(1, ctypes.byref(cu))
+    if cu.value != 256:
+        pytest.skip("measured on 256 compute units")
+    assert _route(h, ta, tb, m, n, k, batch, policy, sum(_bytes(h, m, n, k, batch, policy)))[2] == tile
+
+
 def test_cut_of_random_products(h):
     rng = random.Random(7)
     cut = stood_in = 0

@@ -321,7 +321,7 @@ thread_local int t_forced_spread_tile = 0;
 // so does the call.  Needs the caller's workspace to have the room; without one it
 // allocates only where the path it stands in for would.
 inline int choose_spread(const Choice &c, const int m, const int n, const int k,
-                         const int batch, const int terms,
+                         const int batch, const int terms, const bool rows,
                          const void *const workspace,
                          const size_t workspace_bytes) {
   if (c.slices <= 1 || c.time <= 0. ||
@@ -342,19 +342,24 @@ inline int choose_spread(const Choice &c, const int m, const int n, const int k,
     return t_forced_spread_tile > 0 && fits(t_forced_spread_tile)
                ? t_forced_spread_tile
                : 0;
-  double best = c.time;
-  if (c.single)
-    best = c.time / fit::kSpreadSlicedMargin;
-  else
-    best = c.path == Path::Direct
-               ? c.time / fit::kSpreadDirectMargin
-               : std::max(c.time / fit::kSpreadPackedMargin,
-                          fit::kCutPacked + c.slices * fit::kCutPackedSlice);
+  // (its own time: c.time holds margins against the other paths)
+  const double instead =
+      c.single ? fused_time(terms, m, n, k, batch, true, rows, c.slices) : c.time;
   int chosen = 0;
+  double best = std::numeric_limits<double>::infinity();
   for (const int tile : {64, 128}) {
     const double t =
         fused_spread_time(terms, m, n, k, batch, tile == 64, c.slices);
-    if (t < best && fits(tile)) {
+    const bool resident =
+        ceil_div(m, tile) * ceil_div(n, tile) * batch * c.slices <=
+        static_cast<long long>(device_cus()) * fit::fused_resident(tile);
+    const double margin =
+        c.single ? fit::kSpreadSlicedMargin[tile == 64 ? 0 : 1][terms - 1]
+        : c.path == Path::Packed
+            ? fit::kSpreadPackedMargin[tile == 64 && resident ? 0 : 1]
+        : tile == 128 && !resident ? fit::kSpreadDirectRounds
+                                   : fit::kSpreadDirectMargin[terms - 1];
+    if (t < best && t * margin < instead && fits(tile)) {
       chosen = tile;
       best = t;
     }
@@ -400,7 +405,7 @@ inline Route choose_route(const int m, const int n, const int k, const int batch
                       workspace_bytes))
     r.path = Path::Fused;
   r.spread_tile =
-      choose_spread(c, m, n, k, batch, terms, workspace, workspace_bytes);
+      choose_spread(c, m, n, k, batch, terms, rows, workspace, workspace_bytes);
   if (r.spread_tile > 0)
     r.path = Path::Fused;
   return r;

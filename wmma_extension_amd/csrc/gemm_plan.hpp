@@ -302,13 +302,28 @@ constexpr SpreadRates kSpread[2][3] = {
      {1.3e-6, 0., 0.469e-6, 0.772, 9.13e-6, 0.872e-6},
      {4.8e-6, 0., 0.675e-6, 0.812, 6.64e-6, 0.880e-6}}};
 constexpr double kSpreadBytesPerS = 4.9e12;
-// ... in place of the direct kernel and of packed operands where it is this much
-// ahead of their estimates; cut products on packed operands take no less than 15 us
-// and 0.4 a slice (their estimate has 16 to 18 us for 64 x 46 x 4032 in 21 slices,
-// which takes 27).
-constexpr double kSpreadDirectMargin = 1.25, kSpreadPackedMargin = 1.2,
-                 kSpreadSlicedMargin = 1.25;
-constexpr double kCutPacked = 15e-6, kCutPackedSlice = 0.4e-6;
+// ... in place of the other kernels where their estimates are this many times its
+// own.  1500 random products that are cut, each run without it and with both
+// tiles, and 110 more for the direct kernel beyond a round of 128x128 tiles:
+// * packed operands, 64x64 tiles that are all resident: 0.95 (both estimates are
+//   too long for tiny outputs); more of them, and 128x128 tiles: 1.2.  Of 973
+//   products 8 are more than 2 % slower than on packed operands, at most 10 %, all
+//   of 973 take 0.73 of their time.  (1.2 everywhere, and packed operands taken
+//   for no faster than 15 us and 0.4 a slice, which held before the fold read
+//   its slices in groups: 17 more than 2 % slower, 256x288x6176 in 28 slices 30.2
+//   us for 23.9.)
+// * the direct kernel: 1.35 and 1.25 for one and two terms (1.25 for one term:
+//   128x5376x7232 41.0 us for 37.7), 1.5 for 128x128 tiles of more than a round:
+//   of those 110 products one is faster so, 3616x256x1696 x 3 56.7 us for 46.5.
+// * the single kernel's slices one after the other, by tile and terms: of 244 such
+//   products three are more than 3 % slower, at most 6 %, all take 0.87 of their
+//   time.  (1.25 against an estimate that holds margins of its own: nine,
+//   1248x96x1024 x 4 20.6 us for 16.0, 68x2738x891 14.4 for 11.5.)
+constexpr double kSpreadPackedMargin[2] = {0.95, 1.2},
+                 kSpreadDirectMargin[2] = {1.35, 1.25},
+                 kSpreadDirectRounds = 1.5,
+                 kSpreadSlicedMargin[2][3] = {{1.2, 1.14, 1.12},
+                                              {1.1, 1.14, 1.12}};
 // Its workgroups that are resident on a compute unit: 12 waves of up to 168
 // registers (128x128), twice 8 waves of up to 128.
 constexpr int fused_resident(const int bm) { return bm > 64 ? 1 : 2; }
