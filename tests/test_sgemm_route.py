@@ -141,6 +141,16 @@ def test_cut_of_random_products(h):
     assert cut > 300 and stood_in > 200
 
 
+@pytest.mark.parametrize("m,n,k,batch,policy", [(1, 961, 101, 1 << 26, 0), (2, 1500, 103, 1 << 26, 0), (64, 961, 333, 1 << 26, 0),
+                                                (65, 4096, 333, 1 << 24, 2), (128, 961, 131, 1 << 25, 2)])
+def test_more_tiles_than_the_single_kernel_counts(h, m, n, k, batch, policy):
+    """It would turn them down; the path that the query reports has larger tiles and runs them."""
+    path = ctypes.c_int(-1)
+    assert h.wmmae_tcec_sgemm_path(m, n, k, batch, policy, 0, ctypes.byref(path)) == 0 and path.value in (PACKED, DIRECT)
+    assert -(-m // 64) * -(-n // 64) * batch >= 1 << 30
+    assert _route(h, b"T", b"N", m, n, k, batch, policy, 1 << 62) == (path.value, 1, 0)
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("ta,tb,m,n,k,policy,flags", UNCUT)
 def test_bits_without_room_for_the_sums(tc, dev, ta, tb, m, n, k, policy, flags):

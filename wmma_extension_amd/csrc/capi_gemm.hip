@@ -276,7 +276,9 @@ inline bool single_is_ahead(const Choice &c, const int m, const int n,
                             const int policy, const int terms, const bool rows,
                             const void *const workspace,
                             const size_t workspace_bytes) {
+  // (it counts its tiles in 32 bits, more of them than the other kernels make)
   if (c.single || c.slices != 1 || c.time <= 0. || batch > (1 << 26) ||
+      ceil_div(m, 64) * ceil_div(n, 64) * batch >= (1ll << 30) ||
       refused_on_packed(c, m, n, k, batch, terms, workspace, workspace_bytes))
     return false;
   const double bytes =
