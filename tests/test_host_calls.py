@@ -3,7 +3,7 @@
 import pytest
 import torch
 
-from wmma_extension_amd import tcec
+from wmma_extension_amd import _lib, tcec
 from wmma_extension_amd._lib import WmmaeError
 
 NOT_TAKEN = 1
@@ -25,6 +25,42 @@ def test_what_is_not_plain_is_not_taken():
         tcec.sgemm(*ok[:13])
     with pytest.raises(ValueError, match="device tensors"):
         tcec.matmul_tn(A, A)
+
+
+@pytest.fixture
+def no_module(monkeypatch):
+    """A package whose module was built for another torch, or not at all."""
+    monkeypatch.setattr(torch, "__version__", torch.__version__ + ".other")
+    monkeypatch.setattr(tcec, "_calls", None)
+
+
+def test_a_package_without_the_module(no_module):
+    """(built by the hipcc line alone): every call goes through the checks in Python, warned of once."""
+    assert _lib.host_calls_path() != _lib.host_calls_path().replace(".other", "")
+    A = torch.zeros(8, 8)
+    with pytest.warns(RuntimeWarning, match="ctypes"):
+        calls = tcec._native()
+    assert tcec._native() is calls
+    for name in ("sgemm", "sgemm_strided_batched", "sgemm_batched", "matmul_tn", "pack", "gemm_packed", "api_gemm",
+                 "primitive_tiles"):
+        assert getattr(calls, name)(A, 1) == NOT_TAKEN
+    with pytest.raises(ValueError, match="device tensors"):
+        tcec.sgemm("T", "N", 8, 8, 8, 1.0, A, 8, A, 8, 0.0, A, 8)
+    with pytest.raises(ValueError, match="device tensors"):
+        tcec.matmul_tn(A, A)
+
+
+@pytest.mark.gpu
+@pytest.mark.filterwarnings("ignore:.*ctypes.*:RuntimeWarning")
+def test_results_without_the_module(tc, dev, monkeypatch):
+    m, n, k = 96, 80, 160
+    A, B, C = torch.rand((m, k), device=dev), torch.rand((n, k), device=dev), torch.zeros((n, m), device=dev)
+    want = tc.matmul_tn(A, B)
+    monkeypatch.setattr(torch, "__version__", torch.__version__ + ".other")
+    monkeypatch.setattr(tcec, "_calls", None)
+    assert torch.equal(tc.matmul_tn(A, B), want)
+    tc.sgemm("T", "N", m, n, k, 1.0, A, k, B, k, 0.0, C, m)
+    assert torch.equal(C, want)
 
 
 @pytest.mark.gpu

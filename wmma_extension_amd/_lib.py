@@ -5,9 +5,12 @@ There is no fallback: if the shared object is missing, `lib()` raises.
 """
 import ctypes
 import glob
+import importlib.util
 import os
+import re
 import subprocess
 import sysconfig
+import warnings
 
 _PKG = os.path.dirname(os.path.abspath(__file__))
 ROOT = os.path.dirname(_PKG)
@@ -81,7 +84,14 @@ SOURCES = ["capi_gemm.hip", "capi_harness.hip", "capi_api_gemm.hip"] + ASM_MFMA_
 
 # the frequent calls of tcec.py from Python in native code (no device code: the host compiler)
 HOST_CALLS_SOURCE = "host_calls.cpp"
-HOST_CALLS_PATH = os.path.join(LIB_DIR, "_wmmae_host_calls.so")
+
+
+def host_calls_path():
+    """Where build() puts it for this interpreter and this torch: it uses torch's C++ interface, so a
+    module that was compiled for another one is not found under the name."""
+    import torch
+    version = re.sub(r"[^0-9A-Za-z.]", "_", torch.__version__)
+    return os.path.join(LIB_DIR, f"_wmmae_host_calls.torch-{version}{sysconfig.get_config_var('EXT_SUFFIX')}")
 
 
 def _host_calls_command():
@@ -91,7 +101,7 @@ def _host_calls_command():
                 sysconfig.get_paths()["include"]]
     return [os.environ.get("CXX", "g++"), "-std=c++17", "-O2", "-fPIC", "-shared", "-fvisibility=hidden",
             f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}", *("-I" + i for i in includes),
-            os.path.join(CSRC_DIR, HOST_CALLS_SOURCE), "-o", HOST_CALLS_PATH, "-L" + os.path.join(root, "lib"),
+            os.path.join(CSRC_DIR, HOST_CALLS_SOURCE), "-o", host_calls_path(), "-L" + os.path.join(root, "lib"),
             "-lc10", "-ltorch_cpu", "-ltorch_python"]
 
 
@@ -126,7 +136,7 @@ def build(verbose=False, only=None):
             keep = ["-save-temps=obj"] if name in ASM_MFMA_SOURCES else []
             jobs.append([hipcc, *flags, *keep, "-I" + INCLUDE_DIR, "-c",
                          os.path.join(CSRC_DIR, name), "-o", obj])
-    if only is None or HOST_CALLS_SOURCE in only or not os.path.exists(HOST_CALLS_PATH):
+    if only is None or HOST_CALLS_SOURCE in only or not os.path.exists(host_calls_path()):
         jobs.append(_host_calls_command())
     with ThreadPoolExecutor(max_workers=len(SOURCES) + 1) as pool:
         list(pool.map(lambda c: _run(c, verbose), jobs))
@@ -223,13 +233,16 @@ def lib():
 
 
 def host_calls():
-    """The extension module of HOST_CALLS_SOURCE, bound to the loaded library; raise if it has not been
-    built.  (torch's libraries, which it uses, must be loaded already.)"""
-    import importlib.util
+    """The extension module of HOST_CALLS_SOURCE, bound to the loaded library, or None, with a warning,
+    where there is none for this torch (a library built by the hipcc line alone): the calls then go
+    through ctypes, with the same results.  (torch's libraries, which it uses, must be loaded already.)"""
     handle = lib()
-    if not os.path.exists(HOST_CALLS_PATH):
-        raise RuntimeError(f"{HOST_CALLS_PATH} is missing: build it with __graft_entry__.build()")
-    spec = importlib.util.spec_from_file_location("_wmmae_host_calls", HOST_CALLS_PATH)
+    path = host_calls_path()
+    if not os.path.exists(path):
+        warnings.warn(f"{path} is missing (__graft_entry__.build() makes it): calls are issued through ctypes, which "
+                      "takes 2 to 4 us longer each", RuntimeWarning, stacklevel=3)
+        return None
+    spec = importlib.util.spec_from_file_location("_wmmae_host_calls", path)
     module = importlib.util.module_from_spec(spec)
     spec.loader.exec_module(module)
     for name in ("wmmae_tcec_sgemm", "wmmae_tcec_sgemm_strided_batched", "wmmae_tcec_sgemm_batched",

@@ -51,10 +51,17 @@ _NOT_TAKEN = 1
 _calls = None
 
 
+class _NoNativeCalls:
+    """In the native module's place where there is none: takes no call."""
+
+    def __getattr__(self, name):
+        return lambda *args: _NOT_TAKEN
+
+
 def _native():
     global _calls
     if _calls is None:
-        _calls = _lib.host_calls()
+        _calls = _lib.host_calls() or _NoNativeCalls()
     return _calls
 
 
