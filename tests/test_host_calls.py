@@ -112,3 +112,51 @@ def test_the_same_results_and_errors_on_either_path(tc, dev):
     # gradients and transforms: raw pointers of wrapped tensors are refused as before
     with pytest.raises(RuntimeError):
         torch.func.vmap(lambda a: tc.matmul_tn(a, B))(A.expand(2, m, k).contiguous())
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("policy", [0, 2])
+def test_plain_arguments_are_taken(tc, dev, policy, monkeypatch):
+    """Each function itself, so that one that turns every call away is seen, and its output against the
+    same call through the checks in Python."""
+    m, n, k, batch = 128, 256, 160, 3
+    calls, stream = tcec._native(), tcec._native_stream()
+    assert not isinstance(calls, tcec._NoNativeCalls) and stream is not None
+    A, B = (torch.rand((batch, x, k), device=dev) - 0.5 for x in (m, n))
+    C0 = torch.rand((batch, n, m), device=dev)
+    ws = torch.empty(tc.workspace_bytes(m, n, k, batch, policy), dtype=torch.uint8, device=dev)
+    pa, pb = (torch.empty(tc.pack_bytes(x, k, 1, policy), dtype=torch.uint8, device=dev) for x in (m, n))
+    tiles = torch.rand((5, 256), device=dev)
+    api = {0: (0, 1), 2: (2, 1)}[policy]
+    rows = [("sgemm", lambda C: ("T", "N", m, n, k, 0.5, A, k, B, k, 1, C, m, policy, 0, ws)),
+            ("sgemm_strided_batched", lambda C: ("T", "N", m, n, k, 0.5, A, k, m * k, B, k, n * k, 1.5, C, m, m * n, batch,
+                                                 tc.Policy(policy), 0, ws)),
+            ("sgemm_batched", lambda C: ("T", "N", m, n, k, 0.5, *sum(([p, ld] for p, ld in zip(
+                [torch.tensor([e.data_ptr() for e in X], device=dev) for X in (A, B)], (k, k))), []), 1.5,
+                torch.tensor([e.data_ptr() for e in C], device=dev), m, batch, policy, 0, None)),
+            ("gemm_packed", lambda C: (policy, m, n, k, 1.0, pa, pb, 1.0, C, m, 1, 0, 0, None)),
+            ("api_gemm", lambda C: (*api, m, n, k, 1.0, A, k, B, k, 1.0, C, m))]
+    for X, x, out in ((A, m, pa), (B, n, pb)):
+        args = (policy, x, k, X, k, 1, out, 1, 0)
+        assert calls.pack(*args, stream) == 0
+        got = out.clone()
+        with monkeypatch.context() as mp:
+            mp.setattr(tcec, "_calls", tcec._NoNativeCalls())
+            out.zero_()
+            tc.pack(*args)
+        assert torch.equal(got, out)
+    for name, args in rows:
+        C = C0.clone()
+        assert getattr(calls, name)(*args(C), stream) == 0, name
+        D = C0.clone()
+        with monkeypatch.context() as mp:
+            mp.setattr(tcec, "_calls", tcec._NoNativeCalls())
+            getattr(tc, name)(*args(D))
+        assert torch.equal(C, D) and not torch.equal(C, C0), name
+    got, dicts = calls.matmul_tn(A[0], B[0], policy, 0, ws, stream), calls.primitive_tiles(tiles, stream)
+    assert isinstance(got, torch.Tensor) and isinstance(dicts, dict)
+    with monkeypatch.context() as mp:
+        mp.setattr(tcec, "_calls", tcec._NoNativeCalls())
+        assert torch.equal(got, tc.matmul_tn(A[0], B[0], policy, 0, ws))
+        want = tc.primitive_tiles(tiles)
+    assert set(want) == set(dicts) and all(torch.equal(want[x], dicts[x]) for x in want)
