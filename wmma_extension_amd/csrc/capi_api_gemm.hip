@@ -79,7 +79,7 @@ int api_gemm_impl(const int type, const int ec, const int m, const int n,
           // terms and a short one (two workgroups a compute unit; 828 tiles, k =
           // 224: 48.7 for 53.1, at k = 512 102 for 103).
           using wmmae_harness::ApiSplitShape;
-          constexpr int terms = ApiSplitShape<T, P, 128, 2>::TERMS;
+          constexpr int terms = ApiSplitShape<T, P, 64, 2>::TERMS;
           const long long cus = device_cus();
           if (2 * blocks <= cus)
             return split(ApiSplitShape<T, P, 64, 2>{});

@@ -227,10 +227,9 @@ template <class T, class Policy, int BM_, int WGN> struct ApiSplitShape {
   static constexpr int TERMS =
       tcec::fragment<w::matrix_a, 16, 16, SK, T, w::row_major, Policy>::num_terms;
   static constexpr int STAGE_BYTES = BLOCKS * TERMS * 1024;
-  // two stages where two workgroups of a compute unit have room for them, else
-  // one and a second barrier a stage
-  static constexpr int STAGES = 2 * STAGE_BYTES <= (NW > 4 ? 160 : 80) * 1024 ? 2 : 1;
-  static constexpr int LDS_BYTES = STAGES * STAGE_BYTES;
+  static constexpr int LDS_BYTES = 2 * STAGE_BYTES;
+  static_assert(LDS_BYTES <= (NW > 4 ? 160 : 80) * 1024,
+                "two stages, of two workgroups a compute unit with four waves");
 };
 
 template <class T, class Policy, class S, int ROUNDING>
@@ -362,9 +361,7 @@ __global__ void __launch_bounds__(S::THREADS, S::BM > 64 ? 2 : 3)
     FragB fb;
     get_frag(fa, stage, wm * (S::WM / 16));
     get_frag(fb, stage, S::BM / 16 + wn * (S::WN / 16));
-    if constexpr (S::STAGES == 1)
-      __syncthreads();
-    stage = S::STAGES - 1 - stage;
+    stage = 1 - stage;
     put_terms(stage);
     // (the last one again where there is no other, never used)
     src += k0 + S::SK < k ? S::SK : 0;
