@@ -43,7 +43,7 @@ WORKLOADS = {
     "c5b": dict(m=1024, n=1024, k=262144, batch=1, policy="F16_EC", dist="normal", mult=3,
                 desc="K-heavy TCEC SGEMM, M=N=1024, K=262144"),
     "api": dict(kind="api", m=4096, n=4096, k=4096, dist="uniform",
-                desc="GEMM written against the public tcec:: device API only, fp16 hi+lo with EC, M=N=K=4096"),
+                desc="GEMM on the fragments of the tcec:: device API, fp16 hi+lo with EC, M=N=K=4096"),
 }
 # a timed region of a few milliseconds is measured while the power management still ramps
 DEFAULT_STEPS = {"c3": 200, "c5a": 400, "c5a_fused": 400, "c5a_packed": 200, "c5b": 50, "c2": 100, "api": 200}
@@ -492,10 +492,9 @@ def run_gemm_workload(args, torch, tcec, dev, name, steps, warmup):
 
 
 def bench_api_gemm(torch, tcec, dev, n=4096, steps=100, warmup=10, also_rz=True):
-    """The GEMM written only against the public tcec:: device API (what a user of the headers
-    gets), fp16 hi+lo with error correction, uniform[-1,1], M=N=K=n: with tcec::mma_sync, the
-    reference's default (the figure), and with mma_rz_sync, which on this hardware is as accurate
-    (`with_mma_rz_sync`)."""
+    """The GEMM on the fragments of the tcec:: device API (include/wmmae_tcec.h), fp16 hi+lo with
+    error correction, uniform[-1,1], M=N=K=n: with tcec::mma_sync, the reference's default (the
+    figure), and with mma_rz_sync, which on this hardware is as accurate (`with_mma_rz_sync`)."""
     g = torch.Generator(device=dev)
     g.manual_seed(0x5EED + 3)
     A = torch.rand((n, n), generator=g, device=dev, dtype=torch.float32) * 2 - 1

@@ -119,9 +119,12 @@ int wmmae_query(int what, long long *out);
  * A + packed B + K slices, whichever path the call then takes.  A product the
  * library runs on the fp32 operands directly (wmmae_tcec_sgemm_path 3 or 4)
  * touches only the K slices, wmmae_tcec_gemm_packed_workspace_bytes of it (where
- * the single kernel makes them: their sums in whole tiles and eight bytes a tile,
- * if what it is given holds that), and path 0 nothing; a caller that knows its products take those paths may pass
- * that much.  A workspace that is not 16-byte aligned is WMMAE_STATUS_MISALIGNED
+ * the single kernel makes them a workgroup each: their sums in whole tiles and
+ * eight bytes a tile, if what it is given holds that), and path 0 nothing; a
+ * caller that knows its products take those paths may pass that much.  K slices
+ * are made where the reported path makes them: on packed operands (2) where the
+ * slices' sums fit behind the operands, whichever kernel makes them, else K is
+ * not cut.  A workspace that is not 16-byte aligned is WMMAE_STATUS_MISALIGNED
  * on the packed path, which cannot do without it; the other two paths then run
  * without K slices. */
 int wmmae_tcec_sgemm_workspace_bytes(int m, int n, int k, int batch, int policy,
@@ -168,15 +171,18 @@ int wmmae_tcec_sgemm_strided_batched(char transa, char transb, int m, int n,
  * results as wmmae_tcec_sgemm; the workspace is a fixed device array of
  * WMMAE_STATIC_SCRATCH_BYTES inside the library image (every GPU the library
  * runs on holds it until the process ends), so the call makes no hipMalloc /
- * hipFree of any kind.  On packed operands (wmmae_tcec_sgemm_path 1, and 2
- * where the single kernel does not make the slices) the array holds the split
- * operands, and products whose split operands need more
- * (wmmae_tcec_pack_bytes of A and of B; fp16 hi+lo: 4*(m+n)*k bytes rounded up
- * to 16 rows and 32 of k) return WMMAE_STATUS_WORKSPACE_TOO_SMALL; K slices
- * are made only when they fit behind the operands.  On the path that reads the
- * fp32 operands directly (3, 4) the array holds K slices only, from its start,
- * and a product of any size succeeds (without K slices when they do not fit);
- * path 0 does not touch the array.  All calls on one GPU share the one array:
+ * hipFree of any kind.  Products of packed operands (wmmae_tcec_sgemm_path 1, and
+ * 2 where the single kernel does not make the slices one after the other) need
+ * the array to hold the split operands, whichever kernel runs them: those that
+ * need more (wmmae_tcec_pack_bytes of A and of B; fp16 hi+lo: 4*(m+n)*k bytes
+ * rounded up to 16 rows and 32 of k) return WMMAE_STATUS_WORKSPACE_TOO_SMALL; K
+ * slices are made only when they fit behind the operands.  On the path that
+ * reads the fp32 operands directly (3, 4) the array holds K slices only, from its
+ * start, and a product of any size succeeds (without K slices when they do not
+ * fit).  Where the single kernel makes the K slices of 2 or 4 with a workgroup
+ * each, the array holds their sums in whole tiles and a word a tile, from its
+ * start: only path 0 is sure to leave it untouched.  All calls on one GPU share
+ * the one array:
  * calls that overlap in time on the same GPU (two streams, two threads) race
  * and must be serialised by the caller.  Nothing in the array has to survive
  * between calls and nothing is assumed zero.
@@ -308,14 +314,22 @@ int wmmae_tcec_frag_dump(int use, int type, int ec, int frag_col,
 int wmmae_tcec_elementwise(int type, int ec, int inst, float *out, float base,
                            int do_neg, int do_integrate, void *stream);
 
-/* C = alpha*A*B + beta*C by a tiled kernel written only against the public
- * tcec:: device API: fp32 tiles staged in LDS by utils::cp_async (two stages),
- * split at fragment load in every wave (tcec::load_matrix_sync), tcec::mma_sync.
+/* C = alpha*A*B + beta*C by a tiled kernel on the tcec:: fragments of the device
+ * API.  Operands of 16-bit terms: every element is split once per workgroup and
+ * the waves take their fragments' registers from LDS; the products are
+ * tcec::mma_sync's, the stores tcec::store_matrix_sync's, but the split itself and
+ * the filling of the fragments reach below the public functions
+ * (tcec::detail::split4, fragment::sub_frag).  fp32 operands, one term from k =
+ * 3072 and three terms below k = 512, on more tiles than compute units, run a
+ * kernel written against the public functions alone: fp32 tiles staged in LDS
+ * by utils::cp_async (two stages), split at fragment load in every wave
+ * (tcec::load_matrix_sync); that one is what a user of the headers gets.  Same
+ * products in the same order, so the same bits.
  * A row-major m x k (lda), B column-major k x n (ldb), C column-major (ldc);
  * m, n multiples of 128, k of 32, lda/ldb multiples of 4, 16-byte aligned.
  * type/ec as in wmmae_tcec_mma_tile.
  * Replaces: bgemm_kernel + mma_core + dmem2smem, test/tcec/batch_gemm.cu:74-116,
- * 196-386: what a user of the headers gets, beside wmmae_tcec_sgemm. */
+ * 196-386. */
 int wmmae_tcec_api_gemm(int type, int ec, int m, int n, int k,
                         const float *alpha, const float *A, int lda,
                         const float *B, int ldb, const float *beta, float *C,

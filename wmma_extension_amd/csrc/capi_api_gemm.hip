@@ -1,6 +1,5 @@
-// extern "C" boundary of libwmmae_tcec.so: the tiled GEMM written against the
-// public tcec:: device API.  Declarations and documentation:
-// include/wmmae_tcec.h.
+// extern "C" boundary of libwmmae_tcec.so: the tiled GEMM on the fragments of the
+// tcec:: device API.  Declarations and documentation: include/wmmae_tcec.h.
 #include "capi_common.hpp"
 #include "tcec_api_gemm_kernel.hpp"
 
@@ -71,8 +70,8 @@ int api_gemm_impl(const int type, const int ec, const int m, const int n,
           // large tiles eight waves share a tile, which hide each other's
           // conversions (198 tiles of k = 7008: 180 us, four waves 230); with more,
           // two workgroups of four waves a compute unit do that and read a third
-          // less from LDS (1024 tiles of k = 4096: 446, eight waves 465), but three
-          // terms do not fit their registers (957 us for 712).
+          // less from LDS (1024 tiles of k = 4096: 4 % faster than eight waves),
+          // but three terms do not fit their registers (a third slower).
           // The kernel that splits at the fragment load stays for more than a round
           // of tiles of one term and a long k (its direct copies take no registers;
           // 897 tiles, k = 4096: 245 us for 297, at k = 1024 91 for 81) and of three

@@ -1,11 +1,13 @@
-// A tiled, batched SGEMM written against the public device API of this library
-// (tcec::fragment, load_matrix_sync, mma_sync, store_matrix_sync,
-// utils::cp_async), the way a user of the reference writes one: the shape of
-// the reference's bgemm_kernel / mma_core / dmem2smem
+// A tiled, batched SGEMM on the fragments of this library's device API, twice, in
+// the shape of the reference's bgemm_kernel / mma_core / dmem2smem
 // (test/tcec/batch_gemm.cu:74-116, 196-257, 261-386).
 //
-// tcec_api_gemm_kernel (fp32 operands kept whole; most products of 16-bit terms
-// take tcec_api_gemm_split_kernel below):
+// tcec_api_gemm_kernel is written against the public functions alone
+// (tcec::fragment, load_matrix_sync, mma_sync, store_matrix_sync,
+// utils::cp_async), the way a user of the reference writes one.  (It runs fp32
+// operands; most products of 16-bit terms take tcec_api_gemm_split_kernel below,
+// which splits with tcec::detail::split4 and fills the fragments' registers
+// itself.)
 //   * fp32 tiles of A (row-major) and B (column-major) are staged in LDS by
 //     utils::cp_async, two stages: the copies of stage s+1 are in flight while
 //     stage s is multiplied;
@@ -212,12 +214,15 @@ __global__ void __launch_bounds__(ApiGemmShape::THREADS, WAVES_PER_SIMD)
 // of their tcec:: fragments from there.  With a conversion per wave the kernel was
 // bound by its instruction issue (1.66e8 vector instructions beside 2.5e7 matrix
 // ones at 4096^3) and, on few tiles, by its own chain of copy, split and multiply.
-// Two fp16 terms, before -> now: 4096^3 498 -> 446 us, 1152x2816x7008 252 -> 180,
-// 1920x1920x1024 44.7 -> 32.5, 256x256x8192 285 -> 136, 768x384x352 17.5 -> 7.8;
-// three bf16 terms 4096^3 738 -> 712, 768x384x352 23.8 -> 10.0; one term
-// 2944x3456x608 41.3 -> 31.5.  What bounds it now: conversions, the adds of
-// mma_rn_sync and matrix instructions share a SIMD's one or two waves.  Loads of eight lanes to a row's 128 bytes: with a lane's
-// eight k in two loads of its own the rows' requests ran at 9.5 TB/s, half the rate.
+// Two fp16 terms, before -> now, calls of both in turn: 4096^3 504 -> 439 us (a
+// hundred of one in a row 505 -> 455 to 470), 1152x2816x7008 254 -> 180,
+// 1920x1920x1024 43.8 -> 32.4, 256x256x8192 288 -> 133, 768x384x352 17.5 -> 7.7;
+// three bf16 terms 4096^3 725 -> 691, 768x384x352 23.9 -> 10.0; one term
+// 2944x3456x608 41.0 -> 30.8.  What bounds it now: conversions, the adds of
+// mma_rn_sync and matrix instructions share a SIMD's one or two waves, and the
+// terms' 8-byte writes conflict (28 % of the LDS cycles at 4096^3).  Loads of
+// eight lanes to a row's 128 bytes: with a lane's eight k in two loads of its own
+// the rows' requests ran at 9.5 TB/s, half the rate.
 //   BM  : block tile (64 or 128), 2 x WGN waves
 template <class T, class Policy, int BM_, int WGN> struct ApiSplitShape {
   static constexpr int BM = BM_, SK = 32, WM = BM / 2, WN = BM / WGN;

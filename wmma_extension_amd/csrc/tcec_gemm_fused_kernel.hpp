@@ -171,9 +171,10 @@ last_of_tile(unsigned long long *const word, const unsigned count) {
 //             precision in ascending order: the same bits again.  For few output
 //             tiles and long k, where a workgroup that makes all slices leaves the
 //             chip idle and packed operands cost three launches.  Whole calls,
-//             two fp16 terms: 2005x64x23136 (rows contiguous) 147 -> 42 us,
-//             64x3232x11712 91 -> 36, 32x480x7332 32.6 -> 19.4, 34x36x1874 20.2
-//             -> 11.6; 1000 random products that are cut: 0.74 of the time.  What
+//             two fp16 terms, before -> now: 2005x64x23136 (rows contiguous) 148
+//             -> 44 us, 64x3232x11712 60 -> 34, 32x480x7332 27 -> 18, 34x36x1874
+//             18 -> 11; of 500 random products that are cut the 305 that it is
+//             chosen for take 0.73 of their time without it, the slowest 1.09.  What
 //             bounds it with many slices: the last workgroup's reading of them,
 //             0.26 us each (128x128: 0.87), one compute unit's share of memory
 //   DEPTH   : stages of fp32 values in flight in registers (even: the LDS

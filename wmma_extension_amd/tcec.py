@@ -470,7 +470,7 @@ def elementwise(type_, ec, inst, base, do_neg, do_integrate, device="cuda"):
 
 
 def api_gemm(type_, ec, m, n, k, alpha, A, lda, B, ldb, beta, C, ldc, rounding=0):
-    """Tiled GEMM written against the public device API only (rounding: 0 tcec::mma_sync,
+    """Tiled GEMM on the device API's fragments (include/wmmae_tcec.h; rounding: 0 tcec::mma_sync,
     1 mma_rn_sync, 2 mma_rz_sync)."""
     if rounding == 0 and _done((_calls or _native()).api_gemm(type_, ec, m, n, k, alpha, A, lda, B, ldb, beta, C, ldc,
                                                               _native_stream()), "wmmae_tcec_api_gemm"):
