@@ -121,10 +121,11 @@ int wmmae_query(int what, long long *out);
  * touches only the K slices, wmmae_tcec_gemm_packed_workspace_bytes of it (where
  * the single kernel makes them a workgroup each: their sums in whole tiles and
  * eight bytes a tile, if what it is given holds that), and path 0 nothing; a
- * caller that knows its products take those paths may pass that much.  K slices
- * are made where the reported path makes them: on packed operands (2) where the
- * slices' sums fit behind the operands, whichever kernel makes them, else K is
- * not cut.  A workspace that is not 16-byte aligned is WMMAE_STATUS_MISALIGNED
+ * caller that knows its products take those paths may pass that much.  Products
+ * of packed operands are cut into K slices where the slices' sums fit behind the
+ * operands, whichever kernel makes them, and else run over a whole K; those that
+ * the single kernel slices by itself are cut whatever the workspace.  A
+ * workspace that is not 16-byte aligned is WMMAE_STATUS_MISALIGNED
  * on the packed path, which cannot do without it; the other two paths then run
  * without K slices. */
 int wmmae_tcec_sgemm_workspace_bytes(int m, int n, int k, int batch, int policy,
