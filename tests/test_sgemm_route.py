@@ -112,6 +112,22 @@ def test_slices_of_a_workgroup_each_where_they_are_faster(h, ta, tb, m, n, k, ba
     assert _route(h, ta, tb, m, n, k, batch, policy, sum(_bytes(h, m, n, k, batch, policy)))[2] == tile
 
 
+@pytest.mark.parametrize("m,n,k,batch,kernel", [
+    # (us in the single kernel and on packed operands)
+    (1862, 1719, 3244, 24, PACKED),                # 3636, 3165
+    (1264, 6597, 1312, 1, PACKED),                 # 187.5, 174.0
+    (4842, 8160, 211, 1, PACKED),                  # 137.3, 126.2
+    (896, 3509, 1473, 1, SINGLE),                  # 67.6, 73.5
+    (64, 1122, 1088, 1, SINGLE),                   # 20.0, 25.7
+    (1061, 1472, 768, 7, SINGLE)])                 # 125.5, 130.5
+def test_three_terms_with_adds_outside_the_matrix_core(h, m, n, k, batch, kernel):
+    cu = ctypes.c_longlong(256)
+    h.wmmae_query(1, ctypes.byref(cu))
+    if cu.value != 256:
+        pytest.skip("measured on 256 compute units")
+    assert _route(h, b"T", b"N", m, n, k, batch, 2, sum(_bytes(h, m, n, k, batch, 2)), 1) == (kernel, 1, 0)
+
+
 def test_cut_of_random_products(h):
     rng = random.Random(7)
     cut = stood_in = 0

@@ -283,18 +283,19 @@ inline bool single_is_ahead(const Choice &c, const int m, const int n,
     return false;
   const double bytes =
       4.0 * batch * (static_cast<double>(m) * n + (static_cast<double>(m) + n) * k);
+  const double small = fused_time(terms, m, n, k, batch, true, rows),
+               large = fused_time(terms, m, n, k, batch, false, rows);
+  const double rn = terms == 3 && large < small ? fit::kSinglePackedRnThreeTerms
+                                                : fit::kSinglePackedRn;
   const double ahead =
       c.path == Path::Packed
-          ? ((flags & WMMAE_FLAG_RN_MAIN) != 0 ? fit::kSinglePackedRn
+          ? ((flags & WMMAE_FLAG_RN_MAIN) != 0 ? rn
              : terms == 1                      ? fit::kSinglePackedOneTerm
                                                : fit::kSinglePacked)
       : bytes > 256.0 * (1 << 20)        ? fit::kSingleDirectLarge
       : c.time < fit::kSingleDirectShort ? fit::kSinglePacked
                                          : fit::kSingleDirect;
-  const double time =
-      std::max(fit::kCallFloor[0],
-               std::min(fused_time(terms, m, n, k, batch, true, rows),
-                        fused_time(terms, m, n, k, batch, false, rows)));
+  const double time = std::max(fit::kCallFloor[0], std::min(small, large));
   // (the other kernels cut the tiles of a partly empty last round along K)
   return time < ahead * c.time && tail_room(policy, m, n, k, batch) == 0;
 }

@@ -264,13 +264,17 @@ inline double fused_direct_margin(const int m, const int n, const int k,
 // 1024 entries; each run both ways): packed operands with two or three terms, 214
 // below 0.95, 0.66 of the time in the median, none above 1.03 (one term below 0.75:
 // 425x1440x1450 x 3 at 0.8 is 1.2 times slower; the leading product outside the
-// matrix core: 25 below 1.15, 0.55, none above 1.05); the direct kernel below 0.75,
+// matrix core: 25 below 1.15, 0.55, none above 1.05; three terms of it in 128x128
+// tiles, which are short of registers, below 1.03: of 78 more seven are 6 to 15 %
+// slower between that and 1.15, 1862x1719x3244 x 24 3636 us for 3165, and one 3 %
+// faster); the direct kernel below 0.75,
 // 0.83, two above 1.03 (all of 20 that take it less than 20 us are faster), and
 // below 0.6 where the batch exceeds the 256 MiB of the memory-side cache, 0.82
 // (95x125x10978 x 172 at 0.64 is 1.3 times slower: the single kernel's estimate
 // overlaps stages and traffic too well there).
 constexpr double kSinglePacked = 0.95, kSinglePackedOneTerm = 0.75,
-                 kSinglePackedRn = 1.15, kSingleDirect = 0.75,
+                 kSinglePackedRn = 1.15, kSinglePackedRnThreeTerms = 1.03,
+                 kSingleDirect = 0.75,
                  kSingleDirectShort = 20e-6, kSingleDirectLarge = 0.6;
 // Adding a K slice to the double-precision sums, for the workgroups of a compute
 // unit at a time: 110 products run with the cut and uncut, 0.17 us in the median
